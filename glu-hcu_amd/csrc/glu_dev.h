@@ -176,6 +176,10 @@ struct SolveDev {
     DfDev tup_df, tlo_df;
     const uint32_t *tdf_src;
     uint32_t tdf_nval;
+    // the first sweep's right-hand side by position p (A x = b over lo_df,
+    // A' x = b over tup_df): float(v[rsrc[p]] * rscale[p]) [n]
+    const uint32_t *df_rsrc, *tdf_rsrc;
+    const double *df_rscale, *tdf_rscale;
     const uint32_t *row_perm, *row_perm_inv, *col_perm, *col_perm_inv;
     const double *row_scale, *col_scale_perm;
 };

@@ -1862,11 +1862,306 @@ __device__ __forceinline__ void df2_sweep(const DfDev &D, const float *__restric
     }
 }
 
+// ---------------------------------------------------------------------------
+// dataflow sweeps with the vector in LDS, values as their own ready marks
+// ---------------------------------------------------------------------------
+//
+// For orders whose whole sweep vector fits in LDS.  The vector starts as
+// kUnset everywhere; a row's result is published by storing it, and a reader
+// polls the value itself: one LDS read gives readiness and value, with no
+// ready bit, no fence and no second read between a row and its dependents.
+// What bounds these sweeps is that hop (n=20k: ~400 dependent rows a sweep).
+// Right-hand sides come from memory in position order (task order) with the
+// task's other prefetched loads, so nothing but the dependencies is read
+// while a row waits.  Measured against ready bits (flag, fence and value
+// read per hop): factor + exact solve n=640 238 -> 193 us, n=4,960 644 ->
+// 571 us, n=20,000 with GESP 2,127 -> 1,945 us; same bits.
+//
+// kUnset is a signalling NaN: no FP32 instruction produces one (results are
+// quieted), and sw_put replaces that pattern all the same, so a published
+// row never looks unset and every wait ends (the tables' order is checked on
+// the host, check_df).
+constexpr uint32_t kUnset = 0x7f8a5ca1u;
+
+__device__ __forceinline__ uint32_t sw_peek(const float *xs, uint32_t c)
+{
+    return __hip_atomic_load(reinterpret_cast<const uint32_t *>(xs) + c, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ void sw_put(float *xs, uint32_t r, float v)
+{
+    uint32_t b = __float_as_uint(v);
+    b = b == kUnset ? 0x7fc00000u : b;
+    __hip_atomic_store(reinterpret_cast<uint32_t *>(xs) + r, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// A task's prefetched data.  Slots that hold no entry have column n (a
+// zero that is always set) and value 0, so lanes need no length tests.
+struct SwTask {
+    uint32_t base, cnt, m, lg;
+    bool wave;
+    uint32_t row;
+    uint32_t idx[kDfK];
+    float val[kDfK];
+    float dval, rhs;
+};
+
+__device__ __forceinline__ void sw_issue(const DfDev &D, const float *__restrict__ sv, const float *__restrict__ rhs,
+                                         uint32_t n, uint4 d, uint32_t lane, SwTask &t)
+{
+    t.base = d.x;
+    t.wave = (d.z & kLongTask) != 0;
+    t.cnt = d.z & 0xffffffu;
+    t.lg = (d.z >> 24) & 0x7fu;
+    t.m = d.w;
+    const uint32_t p = d.y + (t.wave ? lane >> t.lg : lane);
+    t.row = D.rl[p].x;
+    t.rhs = rhs[min(p, n - 1)];
+    t.dval = 1.f;
+    if (D.div) t.dval = sv[D.nslots + p];   // the pivot
+    if (!t.wave) {
+#pragma unroll
+        for (uint32_t e = 0; e < kDfK; ++e) {   // entries past the task's longest row belong to later tasks
+            const uint32_t ix = D.idx[t.base + e * kWave + lane];
+            const float v = sv[t.base + e * kWave + lane];
+            t.idx[e] = e < t.m ? ix : n;
+            t.val[e] = e < t.m ? v : 0.f;
+        }
+    } else {
+        t.idx[0] = D.idx[t.base + lane];
+        t.val[0] = sv[t.base + lane];
+    }
+}
+
+// In each row of 16 lanes: a of lane k becomes a(k - 1) - p(k), k = 1..15 in
+// order (lane 0 keeps a), so lane 15 ends with a(0) - p(1) - ... - p(15),
+// each subtraction rounded.  row_shr:1 leaves lane 0 unwritten; after k steps
+// lane k holds its final value, and repeating the step does not change it.
+__device__ __forceinline__ float row_chain_sub(float a, float p)
+{
+#define GLU_CHAIN1 "s_nop 1\n\tv_sub_f32_dpp %0, %0, %1 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+#define GLU_CHAIN5 GLU_CHAIN1 GLU_CHAIN1 GLU_CHAIN1 GLU_CHAIN1 GLU_CHAIN1
+    asm volatile(GLU_CHAIN5 GLU_CHAIN5 GLU_CHAIN5 "s_nop 1" : "+v"(a) : "v"(p));
+#undef GLU_CHAIN5
+#undef GLU_CHAIN1
+    return a;
+}
+
+// One task.  kExact: each row's products subtracted one at a time in the
+// row's order (the arithmetic of Symbolic_Matrix::solve); otherwise a wave
+// row's products are summed by lane and then across the lanes.
+template <bool kExact>
+__device__ __forceinline__ void sw_run(const DfDev &D, const float *__restrict__ sv, float *xs, const SwTask &t,
+                                       uint32_t lane)
+{
+    if (!t.wave) {   // rows a lane each
+        bool pending = lane < t.cnt;
+        while (__ballot(pending)) {
+            uint32_t b[kDfK];
+            bool ok = pending;
+#pragma unroll
+            for (uint32_t e = 0; e < kDfK; ++e) b[e] = sw_peek(xs, t.idx[e]);
+#pragma unroll
+            for (uint32_t e = 0; e < kDfK; ++e) ok &= b[e] != kUnset;
+            if (ok) {
+                float acc = t.rhs;
+#pragma unroll
+                for (uint32_t e = 0; e < kDfK; ++e) acc = acc - t.val[e] * __uint_as_float(b[e]);
+                if (D.div) acc = acc / t.dval;
+                sw_put(xs, t.row, acc);
+                pending = false;
+            }
+        }
+        return;
+    }
+    const uint32_t gw = 1u << t.lg, j = lane & (gw - 1u);
+    const uint32_t *ix = D.idx + t.base + lane;   // passes past the first: a 64-lane row, t.m entries
+    const float *vx = sv + t.base + lane;
+    if (kExact) {
+        // 16 lanes at a time: wait for those entries only, subtract their
+        // products along the lanes, hand the running value on
+        float carry = t.rhs, a = 0.f;
+        uint32_t c = t.idx[0];
+        float v = t.val[0];
+        for (uint32_t c0 = 0;; c0 += kWave) {
+            const bool more = c0 + kWave < t.m;   // (uniform; only a 64-lane row)
+            uint32_t nc = 0;
+            float nv = 0.f;
+            if (more) {   // the next pass's entries load while this one is consumed
+                nc = ix[c0 + kWave];
+                nv = vx[c0 + kWave];
+            }
+            const uint32_t nseg = t.lg == 6 ? (more ? 4u : (t.m - c0 + 15u) / 16u) : gw / 16u;
+            uint64_t seg = t.lg == 4 ? ~0ull : t.lg == 5 ? 0x0000ffff0000ffffull : 0xffffull;
+            for (uint32_t r = 0; r < nseg; ++r, seg <<= 16) {
+                uint32_t b;
+                do {
+                    b = sw_peek(xs, c);
+                } while (__ballot(b == kUnset) & seg);
+                const float p = v * __uint_as_float(b);
+                a = row_chain_sub(carry - p, p);
+                // lane 15 of each row of 16 to the next row (row_bcast:15)
+                carry = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x142, 0xf, 0xf, false));
+            }
+            if (t.lg != 6) break;
+            carry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), (int)(16u * nseg - 1u)));
+            if (!more) break;
+            c = nc;
+            v = nv;
+        }
+        if (t.lg == 6) a = carry;
+        if (j == gw - 1u && (lane >> t.lg) < t.cnt) {
+            if (D.div) a = a / t.dval;
+            sw_put(xs, t.row, a);
+        }
+        return;
+    }
+    constexpr uint32_t kB = 4;   // passes of a long row loaded at a time, ahead of their use
+    uint32_t col[kB];
+    float w[kB];
+    if (t.m > kWave) {
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u) {
+            const uint32_t q = min((u + 1) * kWave, (t.m - 1) & ~(kWave - 1u));
+            col[u] = ix[q];
+            w[u] = vx[q];
+        }
+    }
+    uint32_t b;
+    do {
+        b = sw_peek(xs, t.idx[0]);
+    } while (__ballot(b == kUnset));
+    float sum = t.val[0] * __uint_as_float(b);
+    for (uint32_t c0 = kWave; c0 < t.m; c0 += kB * kWave) {   // gw == 64 here
+        uint32_t cc[kB];
+        float cw[kB];
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u) {
+            cc[u] = col[u];
+            cw[u] = w[u];
+        }
+        if (c0 + kB * kWave < t.m) {
+#pragma unroll
+            for (uint32_t u = 0; u < kB; ++u) {
+                const uint32_t q = min(c0 + (kB + u) * kWave, (t.m - 1) & ~(kWave - 1u));
+                col[u] = ix[q];
+                w[u] = vx[q];
+            }
+        }
+        uint32_t bb[kB];
+        bool un;
+        do {
+            un = false;
+#pragma unroll
+            for (uint32_t u = 0; u < kB; ++u) bb[u] = sw_peek(xs, cc[u]);
+#pragma unroll
+            for (uint32_t u = 0; u < kB; ++u) un |= bb[u] == kUnset;
+        } while (__ballot(un));
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u)
+            if (c0 + u * kWave + j < t.m) sum += cw[u] * __uint_as_float(bb[u]);
+    }
+    sum = group_sum(sum, gw);
+    if (j == 0 && (lane >> t.lg) < t.cnt) {
+        float acc = t.rhs - sum;
+        if (D.div) acc = acc / t.dval;
+        sw_put(xs, t.row, acc);
+    }
+}
+
+// All tasks of sweep D for the calling workgroup: right-hand sides rhs[p] by
+// position, results into xs (LDS; all kUnset but xs[n] = 0).  Waves, task
+// order and prefetch as df2_sweep.
+template <bool kExact>
+__device__ __forceinline__ void sw_sweep(const DfDev &D, const float *__restrict__ sv, const float *__restrict__ rhs,
+                                         uint32_t n, float *xs)
+{
+    const uint32_t lane = threadIdx.x & (kWave - 1), nw = blockDim.x / kWave;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // uniform: scalar loads below
+    const uint32_t mine = D.ntask > w ? (D.ntask - w + nw - 1) / nw : 0;
+    if (mine == 0) return;
+    const __attribute__((address_space(4))) uint32_t *tasks =
+        (const __attribute__((address_space(4))) uint32_t *)(uintptr_t)D.task;
+    auto desc = [&](uint32_t k) {
+        const uint32_t q = 4 * (w + (k < mine ? k : mine - 1) * nw);
+        const uint4 d = make_uint4(tasks[q], tasks[q + 1], tasks[q + 2], tasks[q + 3]);
+        return k < mine ? d : make_uint4(0u, 0u, 0u, 0u);
+    };
+    uint4 dn = desc(0), dn2 = desc(1);
+    SwTask cur, nxt;
+    sw_issue(D, sv, rhs, n, dn, lane, nxt);
+    for (uint32_t k = 0; k < mine; ++k) {
+        cur = nxt;
+        __builtin_amdgcn_s_waitcnt(0xF70);   // vmcnt(0): this task's loads (see df2_sweep)
+        dn = dn2;
+        dn2 = desc(k + 2);
+        sw_issue(D, sv, rhs, n, dn, lane, nxt);
+        sw_run<kExact>(D, sv, xs, cur, lane);
+    }
+}
+
+// Both sweeps of M = (LU)^-1 with the vector in LDS: rhs (n floats, memory)
+// holds the first sweep's right-hand sides by position and is used for the
+// second's; xs (n + 1 floats) ends with the results by row.  Starts with
+// everything before it visible only to this thread; ends with a barrier.
+template <bool kExact>
+__device__ __forceinline__ void sw_solve(const DfDev &first, const float *__restrict__ sv1, const DfDev &second,
+                                         const float *__restrict__ sv2, float *rhs, uint32_t n, float *xs)
+{
+    const uint32_t tid = threadIdx.x, nt = blockDim.x;
+    uint32_t *xb = reinterpret_cast<uint32_t *>(xs);
+    for (uint32_t i = tid; i <= n; i += nt) xb[i] = i < n ? kUnset : 0u;
+    __syncthreads();
+    sw_sweep<kExact>(first, sv1, rhs, n, xs);
+    __syncthreads();
+    constexpr uint32_t kU = 4;
+    for (uint32_t p0 = tid; p0 < n; p0 += kU * nt) {
+        uint32_t r[kU];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) r[u] = second.rl[min(p0 + u * nt, n - 1)].x;
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            if (p0 + u * nt < n) rhs[p0 + u * nt] = xs[r[u]];
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += nt) xb[i] = kUnset;
+    __syncthreads();
+    sw_sweep<kExact>(second, sv2, rhs, n, xs);
+    __syncthreads();
+}
+
+// rhs[p] = float(v[src[p]] * scale[p]): the right-hand side in the factors'
+// frame, by position of the first sweep (its loads four at a time).
+template <typename T>
+__device__ __forceinline__ void sw_scale(const T *__restrict__ v, const uint32_t *__restrict__ src,
+                                         const double *__restrict__ scale, float *rhs, uint32_t n)
+{
+    constexpr uint32_t kU = 4;
+    const uint32_t nt = blockDim.x;
+    for (uint32_t p0 = threadIdx.x; p0 < n; p0 += kU * nt) {
+        uint32_t s[kU];
+        double a[kU];
+        T x[kU];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) {
+            const uint32_t p = min(p0 + u * nt, n - 1);
+            s[u] = src[p];
+            a[u] = scale[p];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) x[u] = v[s[u]];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            if (p0 + u * nt < n) rhs[p0 + u * nt] = (float)((double)x[u] * a[u]);
+    }
+}
+
 // LDS placement of the batch pipeline's sweep state (dynamic LDS).
 enum : int {
     kSweepLevels = 0,   // level-synchronous sweeps, correction vector in global memory
     kSweepFlags = 1,    // dataflow sweeps, ready bits in LDS, vector in global memory
-    kSweepLds = 2,      // dataflow sweeps, ready bits and vector in LDS
+    kSweepLds = 2,      // dataflow sweeps, vector in LDS, values as their own ready marks
 };
 
 // One workgroup runs one matrix: value refresh, GESP value, factorization
@@ -2031,6 +2326,14 @@ __device__ __forceinline__ void wg_precond(const MatDesc *Md, const MatIO &io, c
 {
     const uint32_t n = Md->n;
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
+    if (kMode == kSweepLds) {
+        sw_scale(v, glb(kT ? Md->s.tdf_rsrc : Md->s.df_rsrc), glb(kT ? Md->s.tdf_rscale : Md->s.df_rscale), io.t32, n);
+        DfDev d1 = kT ? Md->s.tup_df : Md->s.lo_df, d2 = kT ? Md->s.tlo_df : Md->s.up_df;
+        globalize(d1);
+        globalize(d2);
+        sw_solve<false>(d1, io.lucsr + d1.voff, d2, io.lucsr + d2.voff, io.t32, n, xs);
+        return;
+    }
     const uint32_t nwords = (n + 31) / 32;
     if (!kT) {
         const uint32_t *cp = glb(Md->s.col_perm);
@@ -2285,13 +2588,14 @@ __device__ __forceinline__ void wg_refine(const MatDesc *Md, const MatIO &io, do
     }
 }
 
-// Dynamic LDS of the batch kernels: ready bits (ceil(n/32) words), then,
-// for kSweepLds, the n-float correction vector.
+// Dynamic LDS of the batch kernels: ready bits (ceil(n/32) words;
+// kSweepFlags), or the correction vector (kSweepLds: n + 1 floats, in the
+// n + ceil(n/32) that orders taken this way have room for).
 template <int kMode>
 __device__ __forceinline__ void batch_lds(uint32_t n, float *t32, uint32_t *&flags, float *&xs)
 {
-    flags = kMode == kSweepLevels ? nullptr : reinterpret_cast<uint32_t *>(g_lds_vec);
-    xs = kMode == kSweepLds ? g_lds_vec + (n + 31) / 32 : t32;
+    flags = kMode == kSweepFlags ? reinterpret_cast<uint32_t *>(g_lds_vec) : nullptr;
+    xs = kMode == kSweepLds ? g_lds_vec : t32;
 }
 
 // Same pattern: matrix b = blockIdx.x uses desc[0] and contiguous buffers.
@@ -2486,6 +2790,17 @@ __global__ void __launch_bounds__(1024) k_solve_one(const MatDesc *__restrict__ 
     uint32_t *flags;
     float *xs;
     batch_lds<kMode>(n, t32, flags, xs);
+    const uint32_t *rpi = glb(desc->s.row_perm_inv);
+    const double *rs = glb(desc->s.row_scale);
+    if (kMode == kSweepLds) {
+        sw_scale(b, glb(desc->s.df_rsrc), glb(desc->s.df_rscale), glb(t32), n);
+        DfDev d1 = desc->s.lo_df, d2 = desc->s.up_df;
+        globalize(d1);
+        globalize(d2);
+        sw_solve<true>(d1, glb(lucsr) + d1.voff, d2, glb(lucsr) + d2.voff, glb(t32), n, xs);
+        for (uint32_t j = tid; j < n; j += nt) x[j] = (float)((double)xs[rpi[j]] * rs[j]);
+        return;
+    }
     {
         const uint32_t *cp = glb(desc->s.col_perm);
         const double *csp = glb(desc->s.col_scale_perm);
@@ -2507,8 +2822,6 @@ __global__ void __launch_bounds__(1024) k_solve_one(const MatDesc *__restrict__ 
         }
         __syncthreads();
     }
-    const uint32_t *rpi = glb(desc->s.row_perm_inv);
-    const double *rs = glb(desc->s.row_scale);
     for (uint32_t j = tid; j < n; j += nt) x[j] = (float)((double)xs[rpi[j]] * rs[j]);
 }
 

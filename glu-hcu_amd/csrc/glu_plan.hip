@@ -1455,6 +1455,12 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     });
     for (int q = 0; q < 4; ++q)
         if (!ok[q]) return fail(GLU_ERR_INVALID, errs[q]);
+    // orders whose sweep vector fits in LDS: slots without an entry read the
+    // zero kept at column n (their value is 0)
+    if (!long_lanes)
+        for (DfHost *d : {&dlo, &dup, &dtu, &dtl})
+            for (size_t q = 0; q < d->idx.size(); ++q)
+                if (d->vpos[q] == UINT32_MAX) d->idx[q] = n;
     // the value copies are gathered in slot order (whole-line stores): the
     // CSC position of each slot, ~0 for padding slots (which get 0)
     std::vector<uint32_t> tdf_vpos(dtu.vpos);   // U' slots, U' pivots (+64 pad), L' slots
@@ -1491,7 +1497,8 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     // Refinement / refresh tables from the analysis.
     std::vector<uint32_t> a_rptr, a_cidx, a_src, lu_src, lu_col, a_rows, a_cols;
     std::vector<double> rs_col, a_rs, a_cs;
-    std::vector<uint32_t> a_dst, lu_fill;
+    std::vector<uint32_t> a_dst, lu_fill, df_rsrc, tdf_rsrc;
+    std::vector<double> df_rscale, tdf_rscale;
     const Analysis *an = a ? &a->an : nullptr;
     if (an) {
         const uint32_t nnz_a = an->nnz;
@@ -1549,6 +1556,18 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         long_first(an->in_ap.data(), a_cols, p->a_nlong_t);
         for (uint32_t i = 0; i < n; ++i)
             p->a_kmax = std::max({p->a_kmax, a_rptr[i + 1] - a_rptr[i], an->in_ap[i + 1] - an->in_ap[i]});
+        // the first sweeps' right-hand sides by position
+        df_rsrc.resize(n);
+        df_rscale.resize(n);
+        tdf_rsrc.resize(n);
+        tdf_rscale.resize(n);
+        for (uint32_t q = 0; q < n; ++q) {
+            const uint32_t r = dlo.rl[q].x, t = an->row_perm[dtu.rl[q].x];
+            df_rsrc[q] = an->col_perm[r];
+            df_rscale[q] = an->col_scale_perm[r];
+            tdf_rsrc[q] = t;
+            tdf_rscale[q] = an->row_scale[t];
+        }
         p->has_scaling = p->has_refine = true;
     }
 
@@ -1605,10 +1624,15 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         o_tlong[s] = U.put(p->tri[s].lvl_long);
         o_ttask[s] = U.put(p->tri[s].tasks);
     }
+    size_t o_rsrc = 0, o_rscale = 0, o_trsrc = 0, o_trscale = 0;
     size_t o_rp = 0, o_rpi = 0, o_cp = 0, o_cpi = 0, o_rs = 0, o_csp = 0;
     size_t o_arptr = 0, o_acidx = 0, o_asrc = 0, o_acptr = 0, o_aridx = 0, o_lusrc = 0, o_rscol = 0;
     size_t o_lucol = 0, o_arows = 0, o_acols = 0, o_adst = 0, o_ars = 0, o_acs = 0, o_lufill = 0;
     if (an) {
+        o_rsrc = U.put(df_rsrc);
+        o_rscale = U.put(df_rscale);
+        o_trsrc = U.put(tdf_rsrc);
+        o_trscale = U.put(tdf_rscale);
         o_rp = U.put(an->row_perm);
         o_rpi = U.put(an->row_perm_inv);
         o_cp = U.put(an->col_perm);
@@ -1743,6 +1767,10 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     S.df_cpy_range = p->copy_range;
     p->tri_dataflow = p->solve_df_opt >= 0 && p->lds_cap >= 4 * (size_t)((n + 31) / 32);
     if (an) {
+        S.df_rsrc = u32p(o_rsrc);
+        S.df_rscale = reinterpret_cast<const double *>(A + o_rscale);
+        S.tdf_rsrc = u32p(o_trsrc);
+        S.tdf_rscale = reinterpret_cast<const double *>(A + o_trscale);
         S.row_perm = u32p(o_rp);
         S.row_perm_inv = u32p(o_rpi);
         S.col_perm = u32p(o_cp);
