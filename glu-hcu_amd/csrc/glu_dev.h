@@ -53,20 +53,34 @@ constexpr uint32_t kFirstBit = 0x80000000u;
 //                barrier).
 
 // One LDS window: steps [l0, l1) with the nslot values they touch staged in
-// LDS.  Its items (cln / ctgt / cup / ment / msrc / dvd, indexed like the
-// factor's tables) address LDS slots instead of CSC positions; pos[slot] is
-// the slot's CSC position.
+// LDS (pos[slot] is the slot's CSC position), run from per-wave streams of
+// chunks: wave w takes chunks [wptr[w], wptr[w + 1]) in order, a chunk being
+// 16 bytes (eight 16-bit slots) per lane and a header
+// {kind << kWinKindShift | step - l0}:
+//   kWinCol    {l, d, u0, t0, u1, t1, u2, t2}: S[ti] += -(S[l] / S[d] * S[ui])
+//   kWinMerge  {t, flags, l0, u0, d0, l1, u1, d1}: two sources of the lane's
+//              merge entry t, the running value kept by the lane from the
+//              chunk with kWinFirst to the one with kWinLast
+//   kWinGroup  {l0, u0, d0, l1, u1, d1, t, flags}: 16 lanes share merge entry
+//              t, lane j holding sources j and 16 + j of the chunk's 32
+//              (kWinGroup1: only the first 16 are used)
+// Every wave passes one barrier per step.  Unused places address three kinds
+// of extra slots after the values: a 0 (slot nslot), a 1 (nslot + 1) and one
+// target a lane that nothing reads (nslot + 2 + lane), so that no chunk needs
+// tests: a missing update computes 0 / 1 * 0 and a missing source subtracts
+// +0, which changes no value.
+constexpr uint32_t kWinExtra = 66;        // extra slots
+constexpr uint32_t kWinKindShift = 30;
+constexpr uint32_t kWinCol = 0, kWinMerge = 1, kWinGroup1 = 2, kWinGroup = 3;
+constexpr uint32_t kWinFirst = 1, kWinLast = 2;
+
 struct WinDev {
     int32_t l0, l1;
-    uint32_t nslot, pad;
-    const uint32_t *pos;
-    const uint2 *cln;
-    const uint32_t *ctgt;
-    const uint32_t *cup;
-    const uint32_t *ment;
-    const MergeSrc *msrc;
-    const uint4 *mrec;
-    const uint2 *dvd;
+    uint32_t nslot, nwave;     // nwave: streams (waves past them only pass the barriers)
+    const uint32_t *pos;       // [nslot]
+    const uint4 *prog;         // [64 chunks]
+    const uint32_t *hdr;       // [chunks]
+    const uint32_t *wptr;      // [nwave + 1]
 };
 
 struct FactorDev {

@@ -882,13 +882,9 @@ constexpr int kMinWindow = 6;
 struct Window {
     int l0 = 0, l1 = 0;            // steps [l0, l1)
     std::vector<uint32_t> pos;     // slot -> CSC position
-    std::vector<uint2> cln;
-    std::vector<uint32_t> ctgt, cup;
-    std::vector<uint32_t> ment;
-    std::vector<MergeSrc> msrc;
-    std::vector<uint4> mrec;
-    std::vector<uint2> dvd;
-    uint32_t c0 = 0, g0 = 0, m0 = 0, s0 = 0, d0 = 0;   // first task / target / item of each kind
+    std::vector<uint16_t> prog;    // chunks, 64 lanes of eight slots each, stream by stream (WinDev)
+    std::vector<uint32_t> hdr;     // [chunks]
+    std::vector<uint32_t> wptr;    // [waves + 1]: each wave's chunks
 };
 
 // The records {target, L, U, pivot of source 0}, {L, U, pivot of source 1,
@@ -931,35 +927,167 @@ void step_positions(const Tables &T, int l, F f)
     }
 }
 
+// Chunks of one step under construction: chains of chunks that one wave runs
+// in order, with their rough relative costs.
+struct WinChain {
+    uint32_t first, count, cost;   // chunks [first, first + count) of the step's buffer
+};
+
+// The window's streams.  Per step: the single updates of each column as
+// column chunks (a lane: one L entry, up to three of its U entries; lanes
+// that share U entries side by side), merge entries of up to kWinLaneMerge
+// sources a lane each (two sources a chunk), larger ones 16 lanes each (a
+// chunk of 32 sources takes about two lane chunks' time).  A step's chains
+// go to its waves longest first, each to the wave with the least so far.
+constexpr uint32_t kWinLaneMerge = 4;
+
 void make_window(const Tables &T, int a, int b, const std::vector<uint32_t> &slot_of_pos,
-                 const std::vector<uint32_t> &pos, Window &w)
+                 const std::vector<uint32_t> &pos, uint32_t waves, Window &w)
 {
     w.l0 = a;
     w.l1 = b;
     w.pos = pos;
-    auto slot = [&](uint32_t q) { return slot_of_pos[q]; };
-    w.c0 = T.ctask_ptr[a];
-    const uint32_t c1 = T.ctask_ptr[b];
-    w.g0 = 256 * w.c0;
-    // padding entries (no update): ~0u targets, U position slot 0
-    for (size_t q = w.g0; q < 256 * (size_t)c1; ++q) {
-        w.ctgt.push_back(T.ctgt[q] == UINT32_MAX ? UINT32_MAX : slot(T.ctgt[q]));
-        w.cup.push_back(slot(T.cup[q]) != UINT32_MAX ? slot(T.cup[q]) : 0u);
+    const uint32_t zero = (uint32_t)pos.size(), one = zero + 1, sink = zero + 2;
+    auto slot = [&](uint32_t q) { return (uint16_t)slot_of_pos[q]; };
+    std::vector<std::vector<uint16_t>> data(waves);
+    std::vector<std::vector<uint32_t>> head(waves);
+    std::vector<uint16_t> buf;         // the step's chunks
+    std::vector<uint32_t> kind;
+    std::vector<WinChain> chains;
+    std::vector<std::vector<std::pair<uint16_t, uint16_t>>> lists;   // a column's single updates {u, t} by L entry
+    std::vector<uint32_t> lane_merges, group_merges;
+    std::vector<uint64_t> load(waves);
+    // a chunk of kind kd whose lanes do nothing
+    auto add_chunk = [&](uint32_t kd) {
+        const size_t at = buf.size();
+        buf.resize(at + 64 * 8);
+        kind.push_back(kd);
+        for (uint32_t lane = 0; lane < 64; ++lane) {
+            uint16_t *e = &buf[at + 8 * lane];
+            const uint16_t z = (uint16_t)zero, o = (uint16_t)one, t = (uint16_t)(sink + lane);
+            const uint16_t col[8] = {z, o, z, t, z, t, z, t};
+            const uint16_t mrg[8] = {t, 0, z, z, o, z, z, o};
+            const uint16_t grp[8] = {z, z, o, z, z, o, t, 0};
+            std::copy_n(kd == kWinCol ? col : kd == kWinMerge ? mrg : grp, 8, e);
+        }
+        return at;
+    };
+    for (int l = a; l < b; ++l) {
+        buf.clear();
+        kind.clear();
+        chains.clear();
+        // single updates
+        uint32_t used = 64;
+        const size_t q1 = 64 * (size_t)T.ctask_ptr[l + 1];
+        for (size_t q = 64 * (size_t)T.ctask_ptr[l]; q < q1;) {
+            if (T.cln[q].z == 0) {
+                ++q;
+                continue;
+            }
+            // the lanes of one column: its L entries for each four U entries
+            const size_t s = q;
+            size_t e = s;
+            while (e < q1 && T.cln[e].z && T.cln[e].y == T.cln[s].y) ++e;
+            size_t L = 1;
+            while (s + L < e && T.cln[s + L].x != T.cln[s].x) ++L;
+            if (lists.size() < L) lists.resize(L);
+            size_t longest = 0;
+            for (size_t ii = 0; ii < L; ++ii) {
+                lists[ii].clear();
+                for (size_t c = s + ii; c < e; c += L)
+                    for (uint32_t k = 0; k < T.cln[c].z; ++k) {
+                        const size_t at = 256 * (c / 64) + 64 * k + c % 64;
+                        if (T.ctgt[at] != UINT32_MAX) lists[ii].push_back({slot(T.cup[at]), slot(T.ctgt[at])});
+                    }
+                longest = std::max(longest, lists[ii].size());
+            }
+            for (size_t r = 0; r < longest; r += 3)
+                for (size_t ii = 0; ii < L; ++ii) {
+                    if (lists[ii].size() <= r) continue;
+                    if (used == 64) {
+                        chains.push_back(WinChain{(uint32_t)kind.size(), 1, 10});
+                        add_chunk(kWinCol);
+                        used = 0;
+                    }
+                    uint16_t *d = &buf[buf.size() - 512 + 8 * used++];
+                    d[0] = slot(T.cln[s + ii].x);
+                    d[1] = slot(T.cln[s].y);
+                    for (size_t k = r; k < std::min(r + 3, lists[ii].size()); ++k) {
+                        d[2 + 2 * (k - r)] = lists[ii][k].first;
+                        d[3 + 2 * (k - r)] = lists[ii][k].second;
+                    }
+                }
+            q = e;
+        }
+        // merge entries, those with the most sources first
+        lane_merges.clear();
+        group_merges.clear();
+        auto count = [&](uint32_t e) { return T.msrc_ptr[e + 1] - T.msrc_ptr[e]; };
+        for (uint32_t e = T.ment_ptr[l]; e < T.ment_ptr[l + 1]; ++e)
+            (count(e) <= kWinLaneMerge ? lane_merges : group_merges).push_back(e);
+        auto most = [&](uint32_t x, uint32_t y) { return count(x) > count(y); };
+        std::stable_sort(lane_merges.begin(), lane_merges.end(), most);
+        std::stable_sort(group_merges.begin(), group_merges.end(), most);
+        for (size_t i = 0; i < lane_merges.size(); i += 64) {
+            const uint32_t n = (count(lane_merges[i]) + 1) / 2;
+            chains.push_back(WinChain{(uint32_t)kind.size(), n, 12 * n});
+            for (uint32_t c = 0; c < n; ++c) {
+                const size_t at = add_chunk(kWinMerge);
+                for (size_t k = i; k < std::min(i + 64, lane_merges.size()); ++k) {
+                    const uint32_t e = lane_merges[k], cnt = count(e), own = (cnt + 1) / 2;
+                    if (c >= own) continue;   // this entry is done
+                    uint16_t *d = &buf[at + 8 * (k - i)];
+                    d[0] = slot(T.ment[e]);
+                    d[1] = (uint16_t)((c == 0 ? kWinFirst : 0) | (c + 1 == own ? kWinLast : 0));
+                    for (uint32_t x = 2 * c; x < std::min(2 * c + 2, cnt); ++x) {
+                        const MergeSrc &m = T.msrc[T.msrc_ptr[e] + x];
+                        uint16_t *f = d + 2 + 3 * (x - 2 * c);
+                        f[0] = slot(m.lpos), f[1] = slot(m.upos), f[2] = slot(m.dpos);
+                    }
+                }
+            }
+        }
+        for (size_t i = 0; i < group_merges.size(); i += 4) {
+            const uint32_t most_src = count(group_merges[i]), n = (most_src + 31) / 32;
+            const bool half_last = most_src - 32 * (n - 1) <= 16;   // the last chunk uses 16 sources only
+            chains.push_back(WinChain{(uint32_t)kind.size(), n, 35 * n - (half_last ? 10 : 0)});
+            for (uint32_t c = 0; c < n; ++c) {
+                const size_t at = add_chunk(half_last && c + 1 == n ? kWinGroup1 : kWinGroup);
+                for (size_t k = i; k < std::min(i + 4, group_merges.size()); ++k) {
+                    const uint32_t e = group_merges[k], cnt = count(e), own = (cnt + 31) / 32;
+                    if (c >= own) continue;
+                    for (uint32_t lane = 0; lane < 16; ++lane) {
+                        uint16_t *d = &buf[at + 8 * (16 * (k - i) + lane)];
+                        d[6] = slot(T.ment[e]);
+                        d[7] = (uint16_t)((c == 0 ? kWinFirst : 0) | (c + 1 == own ? kWinLast : 0));
+                        for (uint32_t x = 0; x < 2; ++x) {
+                            const uint32_t src = 32 * c + 16 * x + lane;
+                            if (src >= cnt) continue;
+                            const MergeSrc &m = T.msrc[T.msrc_ptr[e] + src];
+                            d[3 * x] = slot(m.lpos), d[3 * x + 1] = slot(m.upos), d[3 * x + 2] = slot(m.dpos);
+                        }
+                    }
+                }
+            }
+        }
+        std::stable_sort(chains.begin(), chains.end(),
+                         [](const WinChain &x, const WinChain &y) { return x.cost > y.cost; });
+        std::fill(load.begin(), load.end(), 0);
+        for (const WinChain &c : chains) {
+            const size_t to = std::min_element(load.begin(), load.end()) - load.begin();
+            load[to] += c.cost;
+            data[to].insert(data[to].end(), buf.begin() + 512 * (size_t)c.first,
+                            buf.begin() + 512 * (size_t)(c.first + c.count));
+            for (uint32_t k = c.first; k < c.first + c.count; ++k)
+                head[to].push_back(kind[k] << kWinKindShift | (uint32_t)(l - a));
+        }
     }
-    for (size_t q = (size_t)w.c0 * 64; q < (size_t)c1 * 64; ++q) {
-        const uint4 &ln = T.cln[q];
-        w.cln.push_back(ln.z ? make_uint2(slot(ln.x), slot(ln.y)) : make_uint2(0u, 0u));
+    w.wptr.assign(1, 0);
+    for (uint32_t v = 0; v < waves; ++v) {
+        w.prog.insert(w.prog.end(), data[v].begin(), data[v].end());
+        w.hdr.insert(w.hdr.end(), head[v].begin(), head[v].end());
+        w.wptr.push_back((uint32_t)w.hdr.size());
     }
-    w.m0 = T.ment_ptr[a];
-    const uint32_t m1 = T.ment_ptr[b];
-    w.s0 = T.msrc_ptr[w.m0];
-    for (uint32_t e = w.m0; e < m1; ++e) w.ment.push_back(slot(T.ment[e]));
-    merge_records(T.ment, T.msrc_ptr, T.msrc, w.m0, m1, slot, w.mrec);
-    for (uint32_t k = w.s0; k < T.msrc_ptr[m1]; ++k) {
-        const MergeSrc &m = T.msrc[k];
-        w.msrc.push_back(MergeSrc{slot(m.lpos), slot(m.upos), slot(m.dpos), 0});
-    }
-    w.d0 = 0;   // no division items inside a window (they run after the last step)
 }
 
 // Windows chosen backward from the last step, so that the final run (the
@@ -968,7 +1096,7 @@ void make_window(const Tables &T, int a, int b, const std::vector<uint32_t> &slo
 // runs in one workgroup, so a wide step inside it would give up the grid's
 // parallelism.
 void choose_windows(const Tables &T, int num_lev, uint32_t nnz, uint32_t budget, uint32_t narrow, int max_windows,
-                    std::vector<Window> &wins)
+                    uint32_t waves, std::vector<Window> &wins)
 {
     wins.clear();
     if (budget == 0 || max_windows <= 0) return;
@@ -1015,7 +1143,7 @@ void choose_windows(const Tables &T, int num_lev, uint32_t nnz, uint32_t budget,
         std::sort(pos.begin(), pos.end());
         for (uint32_t i = 0; i < pos.size(); ++i) slot_of_pos[pos[i]] = i;
         wins.emplace_back();
-        make_window(T, a, b, slot_of_pos, pos, wins.back());
+        make_window(T, a, b, slot_of_pos, pos, waves, wins.back());
         for (uint32_t q : pos) slot_of_pos[q] = UINT32_MAX;
         b = a;
     }
@@ -1355,9 +1483,12 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     HIP_TRY(hipGetDevice(&p->device));
     p->lds_cap = launch::enable_lds();
     std::vector<Window> wins;
-    uint32_t budget = (uint32_t)(p->lds_cap / sizeof(float));
+    // (slots are 16-bit numbers)
+    uint32_t budget = std::min<uint32_t>((uint32_t)(p->lds_cap / sizeof(float)), 0xffffu);
+    budget -= std::min(budget, kWinExtra);
     if (p->win_values) budget = std::min(budget, p->win_values);
-    choose_windows(T, P.num_lev, P.nnz, budget, (uint32_t)p->fuse_units, p->max_windows, wins);
+    choose_windows(T, P.num_lev, P.nnz, budget, (uint32_t)p->fuse_units, p->max_windows,
+                   (uint32_t)p->fused_threads / 64, wins);
     p->nwin = (int)wins.size();
     for (const Window &w : wins) {
         p->win_steps += w.l1 - w.l0;
@@ -1597,17 +1728,12 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     const size_t o_dvd = U.put(T.dvd);
     const size_t o_dptr = U.put(T.dvd_ptr);
     p->ndiv = (uint32_t)T.dvd.size();
-    std::vector<size_t> o_wpos(wins.size()), o_wcln(wins.size()), o_wctgt(wins.size()), o_wcup(wins.size()),
-        o_wment(wins.size()), o_wmsrc(wins.size()), o_wmrec(wins.size()), o_wdvd(wins.size());
+    std::vector<size_t> o_wpos(wins.size()), o_wprog(wins.size()), o_whdr(wins.size()), o_wptr(wins.size());
     for (size_t w = 0; w < wins.size(); ++w) {
         o_wpos[w] = U.put(wins[w].pos);
-        o_wcln[w] = U.put(wins[w].cln);
-        o_wctgt[w] = U.put(wins[w].ctgt);
-        o_wcup[w] = U.put(wins[w].cup);
-        o_wment[w] = U.put(wins[w].ment);
-        o_wmsrc[w] = U.put(wins[w].msrc);
-        o_wmrec[w] = U.put(wins[w].mrec);
-        o_wdvd[w] = U.put(wins[w].dvd);
+        o_wprog[w] = U.put(wins[w].prog);
+        o_whdr[w] = U.put(wins[w].hdr);
+        o_wptr[w] = U.put(wins[w].wptr);
     }
     const size_t o_wdev = U.reserve(sizeof(WinDev) * std::max<size_t>(wins.size(), 1));
     const size_t o_dlo_task = U.put(dlo.task), o_dlo_rl = U.put(dlo.rl), o_dlo_idx = U.put(dlo.idx);
@@ -1688,9 +1814,6 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     F.num_lev = P.num_lev;
     F.n = n;
     F.nnz = P.nnz;
-    // window items are indexed like the full tables: shift each base back
-    // by the index of its first item (only indices >= that are used)
-    auto shifted = [&](size_t off, size_t first, size_t item) { return (uintptr_t)(A + off) - first * item; };
     {
         std::vector<WinDev> wd(wins.size());
         for (size_t w = 0; w < wins.size(); ++w) {
@@ -1699,14 +1822,11 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
             d.l0 = x.l0;
             d.l1 = x.l1;
             d.nslot = (uint32_t)x.pos.size();
+            d.nwave = (uint32_t)x.wptr.size() - 1;
             d.pos = u32p(o_wpos[w]);
-            d.cln = reinterpret_cast<const uint2 *>(shifted(o_wcln[w], (size_t)x.c0 * 64, sizeof(uint2)));
-            d.ctgt = reinterpret_cast<const uint32_t *>(shifted(o_wctgt[w], x.g0, sizeof(uint32_t)));
-            d.cup = reinterpret_cast<const uint32_t *>(shifted(o_wcup[w], x.g0, sizeof(uint32_t)));
-            d.ment = reinterpret_cast<const uint32_t *>(shifted(o_wment[w], x.m0, sizeof(uint32_t)));
-            d.msrc = reinterpret_cast<const MergeSrc *>(shifted(o_wmsrc[w], x.s0, sizeof(MergeSrc)));
-            d.mrec = reinterpret_cast<const uint4 *>(shifted(o_wmrec[w], 2 * (size_t)x.m0, sizeof(uint4)));
-            d.dvd = reinterpret_cast<const uint2 *>(shifted(o_wdvd[w], x.d0, sizeof(uint2)));
+            d.prog = reinterpret_cast<const uint4 *>(A + o_wprog[w]);
+            d.hdr = u32p(o_whdr[w]);
+            d.wptr = u32p(o_wptr[w]);
         }
         if (!wd.empty())
             HIP_TRY(hipMemcpy(A + o_wdev, wd.data(), sizeof(WinDev) * wd.size(), hipMemcpyHostToDevice));
@@ -2358,7 +2478,7 @@ extern "C" glu_status glu_batch_solve(glu_plan *p, int batch, const double *d_ax
     batch_grid_steps(p, batch, d_ax, d_lu, p->d_bnorms, perturb, st);
     launch::batch_same(p->d_desc, batch, d_ax, d_b, d_x, d_lu, p->d_blucsr, p->d_bt32, p->d_br64, p->d_bnorms,
                        p->d_bkry, d_iters, d_eta, tol, maxit, perturb, p->fused_threads, mode,
-                       sizeof(float) * std::max(p->win_nslot, p->copy_range), launch::batch_lds_bytes(mode, p->n),
+                       sizeof(float) * std::max(p->win_nslot + kWinExtra, p->copy_range), launch::batch_lds_bytes(mode, p->n),
                        p->batch_grid_lev, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(GLU_ERR_DEVICE, std::string("batch launch: ") + hipGetErrorString(e));
@@ -2377,7 +2497,7 @@ extern "C" glu_status glu_batch_factor(glu_plan *p, int batch, const double *d_a
     if (s != GLU_OK) return s;
     batch_grid_steps(p, batch, d_ax, d_lu, p->d_fnorms, perturb, st);
     launch::batch_factor(p->d_desc, batch, d_ax, d_lu, p->d_fnorms, perturb, p->fused_threads,
-                         sizeof(float) * p->win_nslot, p->batch_grid_lev, st);
+                         sizeof(float) * (p->win_nslot + kWinExtra), p->batch_grid_lev, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(GLU_ERR_DEVICE, std::string("batch factor launch: ") + hipGetErrorString(e));
     return GLU_OK;
@@ -2580,7 +2700,7 @@ extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, c
     for (int i = nsplit; i < count; ++i) {
         const glu_plan *p = g->plans[g->order[i]];
         nmax = std::max<size_t>(nmax, p->n);
-        tmax = std::max<size_t>(tmax, sizeof(float) * std::max(p->win_nslot, p->copy_range));
+        tmax = std::max<size_t>(tmax, sizeof(float) * std::max(p->win_nslot + kWinExtra, p->copy_range));
     }
     const int mode = sweep_mode((uint32_t)nmax, cap);
     // ready bits only for the largest order: each matrix whose vector fits
