@@ -85,6 +85,8 @@ struct WinDev {
 
 struct FactorDev {
     const uint32_t *col_ptr;   // sym_c_ptr [n+1] (GESP column sums)
+    const uint32_t *gcols;     // columns, those with > kLongRow entries first [n]
+    uint32_t ngl;              // number of those
     // Column tasks, by level (tasks ctask_ptr[l] .. ctask_ptr[l+1]).  Lane
     // `lane` of task t owns one L entry of a pivot column k of the level and
     // up to four consecutive entries of U_k: cln[64 t + lane] = {L(i,k)

@@ -355,15 +355,68 @@ __device__ __forceinline__ void factor_levels_wg(const FactorDev &F, float *__re
     }
 }
 
-// GESP: pert = 3.45e-4 * max_c sum_p |val[p]| (FP32 sums in column order).
-__global__ void k_pert(const uint32_t *__restrict__ col_ptr, const float *__restrict__ val,
-                       uint32_t n, unsigned int *__restrict__ norm_bits)
+// sum_p |val[p]| over [p0, p1) in order, by one wave (in every lane): 64
+// entries at a time into the wave's LDS slice (64 floats), negated, and
+// subtracted in order (v - (-a) is v + a); the 256 entries after the current
+// 256 load meanwhile.  A rail's column has thousands of entries: one lane
+// walking it waits for memory at every step (n=20,000: GESP sums 498 us;
+// with the next 64 entries in flight 50 us, with the next 256 24 us).
+__device__ __forceinline__ float abs_col_sum_wave(const float *__restrict__ val, uint32_t p0, uint32_t p1,
+                                                  uint32_t lane, float *lds)
 {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n) return;
+    constexpr uint32_t U = 4;
+    float s = 0.f, v[U];
+    if (p0 >= p1) return s;
+    auto load = [&](uint32_t p) {   // 0 past the end
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t q = p + u * kWave + lane;
+            const float a = fabsf(val[min(q, p1 - 1)]);
+            v[u] = q < p1 ? a : 0.f;
+        }
+    };
+    load(p0);
+    for (uint32_t p = p0; p < p1; p += U * kWave) {
+        float c[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) c[u] = v[u];
+        load(p + U * kWave);
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            if (p + u * kWave >= p1) break;
+            lds[lane] = -c[u];   // lanes past the end hold -0: s + 0
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            s = serial_sub(s, lds, kWave, false);
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+    }
+    return s;
+}
+
+// GESP: pert = 3.45e-4 * max_c sum_p |val[p]| (FP32 sums in column order):
+// the first waves take a long column each, the lanes after them a short one.
+__global__ void __launch_bounds__(256) k_pert(FactorDev F, const float *__restrict__ val,
+                                              unsigned int *__restrict__ norm_bits)
+{
+    __shared__ __attribute__((aligned(16))) float lds[256 / kWave][kWave];
+    const uint32_t g = blockIdx.x * 256 + threadIdx.x, lane = g & (kWave - 1), w = g / kWave;
     float s = 0.f;
-    for (uint32_t p = col_ptr[c]; p < col_ptr[c + 1]; ++p) s += fabsf(val[p]);
-    if (s == s) atomicMax(norm_bits, __float_as_uint(s));
+    if (w < F.ngl) {
+        const uint32_t c = F.gcols[w];
+        s = abs_col_sum_wave(val, F.col_ptr[c], F.col_ptr[c + 1], lane, lds[threadIdx.x / kWave]);
+    } else {
+        const uint32_t t = F.ngl + (g - F.ngl * kWave);
+        if (t < F.n) {
+            const uint32_t c = F.gcols[t];
+            for (uint32_t p = F.col_ptr[c]; p < F.col_ptr[c + 1]; ++p) s += fabsf(val[p]);
+        }
+    }
+    // sums are >= 0, so their bits order as they do; a NaN sum does not count
+    uint32_t m = s == s ? __float_as_uint(s) : 0u;
+    for (int o = kWave / 2; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, kWave));
+    if (lane == 0 && m) atomicMax(norm_bits, m);
 }
 
 // Also re-arms the accumulator for the next call (no memset in the stream).
@@ -644,17 +697,43 @@ __global__ void __launch_bounds__(256) k_il_scatter(RefineDev R, const double *_
 }
 
 // GESP: bits[m] = max over columns of sum_p |val[p]| (FP32, column order)
-// for the matrices of group blockIdx.y, then k_il_pert_finish.
-__global__ void k_il_pert(const uint32_t *__restrict__ col_ptr, const float *__restrict__ S, uint32_t n,
-                          uint32_t nnz, uint32_t batch, unsigned int *__restrict__ bits)
+// for the matrices of group blockIdx.y, then k_il_pert_finish.  The first
+// blocks take a long column each: 64 positions at a time through LDS (whole
+// lines, all threads), summed by one lane a matrix; a block after them takes
+// a short column per kIl lanes.
+__global__ void __launch_bounds__(256) k_il_pert(FactorDev F, const float *__restrict__ S, uint32_t batch,
+                                                 unsigned int *__restrict__ bits)
 {
-    const uint32_t g = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t c = i / kIl, j = i % kIl, m = g * kIl + j;
-    if (c >= n || m >= batch) return;
-    const float *V = S + (size_t)g * nnz * kIl + j;
+    constexpr uint32_t kP = 64;   // positions a pass
+    __shared__ float tile[kP][kIl];
+    const uint32_t g = blockIdx.y, tid = threadIdx.x, j = tid % kIl, m = g * kIl + j;
+    const float *V = S + (size_t)g * F.nnz * kIl + j;
     float s = 0.f;
-    for (uint32_t p = col_ptr[c]; p < col_ptr[c + 1]; ++p) s += fabsf(V[(size_t)p * kIl]);
-    if (s == s) atomicMax(bits + m, __float_as_uint(s));
+    bool own = m < batch;
+    if (blockIdx.x < F.ngl) {
+        const uint32_t c = F.gcols[blockIdx.x], p1 = F.col_ptr[c + 1];
+        for (uint32_t p0 = F.col_ptr[c]; p0 < p1; p0 += kP) {
+            float v[kP * kIl / 256];
+#pragma unroll
+            for (uint32_t u = 0; u < kP * kIl / 256; ++u)
+                v[u] = V[(size_t)min(p0 + tid / kIl + u * (256 / kIl), p1 - 1) * kIl];
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < kP * kIl / 256; ++u) tile[tid / kIl + u * (256 / kIl)][j] = v[u];
+            __syncthreads();
+            if (tid < kIl)
+                for (uint32_t q = 0; q < min(kP, p1 - p0); ++q) s += fabsf(tile[q][j]);
+        }
+        own = own && tid < kIl;
+    } else {
+        const uint32_t t = F.ngl + ((blockIdx.x - F.ngl) * 256 + tid) / kIl;
+        own = own && t < F.n;
+        if (own) {
+            const uint32_t c = F.gcols[t];
+            for (uint32_t p = F.col_ptr[c]; p < F.col_ptr[c + 1]; ++p) s += fabsf(V[(size_t)p * kIl]);
+        }
+    }
+    if (own && s == s) atomicMax(bits + m, __float_as_uint(s));
 }
 
 // pertd[2 m] = the GESP value; re-arms bits for the next call.
@@ -1532,6 +1611,7 @@ __device__ __forceinline__ void wg_tri_refine(const TriDev &T, const float *__re
 __device__ __forceinline__ void globalize(FactorDev &F)
 {
     F.col_ptr = glb(F.col_ptr);
+    F.gcols = glb(F.gcols);
     F.ctask_ptr = glb(F.ctask_ptr);
     F.cln = glb(F.cln);
     F.ctgt = glb(F.ctgt);
@@ -2253,8 +2333,8 @@ enum : int {
 //
 // wg_values: steps 1-2 (the matrix's values, |b|_inf with x = 0 and
 // r64 = b, the GESP value).
-__device__ __forceinline__ void wg_values(const MatDesc *Md, const MatIO &io, int perturb, double *sh, double &bnorm,
-                                          float &pert)
+__device__ __forceinline__ void wg_values(const MatDesc *Md, const MatIO &io, int perturb, double *sh, float *wlds,
+                                          double &bnorm, float &pert)
 {
     const uint32_t n = Md->n, nnz = Md->nnz;
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
@@ -2299,9 +2379,16 @@ __device__ __forceinline__ void wg_values(const MatDesc *Md, const MatIO &io, in
     // 2. GESP value from the freshly placed values
     pert = 0.f;
     if (perturb) {
-        const uint32_t *col_ptr = glb(Md->f.col_ptr);
+        const uint32_t *col_ptr = glb(Md->f.col_ptr), *gcols = glb(Md->f.gcols);
+        const uint32_t ngl = Md->f.ngl;
         double cm = 0.0;
-        for (uint32_t c = tid; c < n; c += nt) {
+        for (uint32_t t = tid / kWave; t < ngl; t += nt / kWave) {   // long columns a wave each
+            const uint32_t c = gcols[t];
+            const float s = abs_col_sum_wave(io.lu, col_ptr[c], col_ptr[c + 1], tid & (kWave - 1), wlds);
+            if (s == s) cm = fmax(cm, (double)s);
+        }
+        for (uint32_t t = ngl + tid; t < n; t += nt) {
+            const uint32_t c = gcols[t];
             float s = 0.f;
             for (uint32_t p = col_ptr[c]; p < col_ptr[c + 1]; ++p) s += fabsf(io.lu[p]);
             if (s == s) cm = fmax(cm, (double)s);
@@ -2321,7 +2408,7 @@ __device__ __forceinline__ void wg_factor(const MatDesc *Md, const MatIO &io, in
     double bnorm = 0.0;
     float pert;
     if (l0 == 0) {
-        wg_values(Md, io, perturb, sh, bnorm, pert);
+        wg_values(Md, io, perturb, sh, wlds, bnorm, pert);
     } else {
         pert = perturb ? (float)io.norms[0] : 0.f;
         double bmax = 0.0;
@@ -3038,7 +3125,7 @@ static inline unsigned blocks_for(uint64_t work, unsigned per) { return (unsigne
 // norm_bits must be zero on entry; k_pert_finish leaves it zero again.
 void pert(const FactorDev &F, const float *val, unsigned int *norm_bits, float *d_pert, hipStream_t st)
 {
-    k_pert<<<blocks_for(F.n, 256), 256, 0, st>>>(F.col_ptr, val, F.n, norm_bits);
+    k_pert<<<blocks_for((uint64_t)F.ngl * kWave + (F.n - F.ngl), 256), 256, 0, st>>>(F, val, norm_bits);
     k_pert_finish<<<1, 1, 0, st>>>(norm_bits, d_pert);
 }
 
@@ -3235,8 +3322,8 @@ void il_values(const RefineDev &R, const FactorDev &F, const double *ax, float *
     }
     k_il_scatter<<<dim3(blocks_for(R.nnz_a, 64), groups), 256, 0, st>>>(R, ax, S, nnz, (uint32_t)batch);
     if (perturb) {
-        k_il_pert<<<dim3(blocks_for((uint64_t)n * kIl, 256), groups), 256, 0, st>>>(F.col_ptr, S, n, nnz,
-                                                                                      (uint32_t)batch, bits);
+        k_il_pert<<<dim3(F.ngl + blocks_for((uint64_t)(n - F.ngl) * kIl, 256), groups), 256, 0, st>>>(
+            F, S, (uint32_t)batch, bits);
         k_il_pert_finish<<<blocks_for(batch, 256), 256, 0, st>>>(bits, pertd, (uint32_t)batch);
     }
 }

@@ -1705,6 +1705,14 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     // ---------------- upload everything into one arena ------------------
     Uploader U;
     const size_t o_colptr = U.put(P.sym_c_ptr, n + 1);
+    std::vector<uint32_t> gcols;   // columns of the pattern, long ones first (GESP sums)
+    gcols.reserve(n);
+    for (int pass = 0; pass < 2; ++pass) {
+        for (uint32_t c = 0; c < n; ++c)
+            if ((P.sym_c_ptr[c + 1] - P.sym_c_ptr[c] > kLongRow) == (pass == 0)) gcols.push_back(c);
+        if (pass == 0) p->F.ngl = (uint32_t)gcols.size();
+    }
+    const size_t o_gcols = U.put(gcols);
     const size_t o_rowidx = U.put(P.sym_r_idx, P.nnz);
     const size_t o_diag = U.put(P.l_col_ptr, n);
     const size_t o_crptr = U.put(P.csr_r_ptr, n + 1);
@@ -1797,6 +1805,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     auto u32p = [&](size_t o) { return reinterpret_cast<const uint32_t *>(A + o); };
     FactorDev &F = p->F;
     F.col_ptr = u32p(o_colptr);
+    F.gcols = u32p(o_gcols);
     F.ctask_ptr = u32p(o_cptr);
     F.cln = reinterpret_cast<const uint2 *>(A + o_cln);
     F.ctgt = u32p(o_ctgt);
