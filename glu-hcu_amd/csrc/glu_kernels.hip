@@ -1378,12 +1378,32 @@ __device__ __forceinline__ void a_row_partial(const RefineDev &R, const double *
                                               const double *__restrict__ x, ARow row, uint32_t first,
                                               uint32_t step, int transpose, double &dot, double &asum)
 {
+    // four entries at a time: their index loads, then their value loads,
+    // issue together (past the end: the last entry again, not used); the
+    // sums stay in entry order
+    constexpr uint32_t U = 4;
     dot = 0.0;
     asum = 0.0;
-    for (uint32_t q = row.q0 + first; q < row.q1; q += step) {
-        const double a = transpose ? ax[q] : ax[R.a_src[q]];
-        if (x) dot = fma(a, x[transpose ? R.a_ridx[q] : R.a_cidx[q]], dot);
-        asum += fabs(a);
+    for (uint32_t q = row.q0 + first; q < row.q1; q += U * step) {
+        uint32_t src[U], col[U];
+        double a[U], xv[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t t = min(q + u * step, row.q1 - 1);
+            src[u] = transpose ? t : R.a_src[t];
+            col[u] = x ? (transpose ? R.a_ridx[t] : R.a_cidx[t]) : 0u;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            a[u] = ax[src[u]];
+            xv[u] = x ? x[col[u]] : 0.0;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (q + u * step < row.q1) {
+                if (x) dot = fma(a[u], xv[u], dot);
+                asum += fabs(a[u]);
+            }
     }
 }
 
@@ -1494,7 +1514,7 @@ __device__ __forceinline__ void wg_rows_of_a(const RefineDev &R, const double *_
 __device__ __forceinline__ void umax64(unsigned long long *p, double v)
 {
     unsigned long long bits = (v == v) ? (unsigned long long)__double_as_longlong(v) : 0x7ff8000000000000ull;
-    atomicMax(p, bits);
+    if (bits > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, bits);
 }
 
 // r = b - A x (or A' x); max norms.  Grid: one wave per long row plus one
@@ -1533,28 +1553,33 @@ __global__ void __launch_bounds__(256) k_residual(RefineDev R, const double *__r
             take(i, dot, asum);
         }
     }
-    rmax = wave_max(rmax);
-    xmax = wave_max(xmax);
-    amax = wave_max(amax);
-    bmax = wave_max(bmax);
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        umax64(norms + 0, rmax);
-        umax64(norms + 1, xmax);
-        if (with_anorm) {
-            umax64(norms + 2, amax);
-            umax64(norms + 3, bmax);
-        }
+    // the block's maxima, then one atomic each, and only where it would
+    // raise the norm (it only grows, so a stale read skips nothing): with an
+    // atomic per wave the four words were what the kernel waited for (n=100,000 67 -> 18 us)
+    __shared__ double sh[256 / kWave];
+    const double mx[4] = {wg_max(rmax, sh), wg_max(xmax, sh), with_anorm ? wg_max(amax, sh) : 0.0,
+                          with_anorm ? wg_max(bmax, sh) : 0.0};
+    if (threadIdx.x < (with_anorm ? 4u : 2u)) {
+        const double v = threadIdx.x == 0 ? mx[0] : threadIdx.x == 1 ? mx[1] : threadIdx.x == 2 ? mx[2] : mx[3];
+        umax64(norms + threadIdx.x, v);
     }
 }
 
-// grad[k] = -lam[row(k)] * x[col(k)] over the caller's CSC entries.
-__global__ void k_adjoint_values(RefineDev R, const double *__restrict__ lam, const double *__restrict__ x,
-                                 double *__restrict__ grad, uint32_t n)
+// grad[k] = -lam[row(k)] * x[col(k)] over the caller's CSC entries: the first
+// waves take a long column each, the lanes after them a short one (a rail's
+// column walked by one lane set the time: n=50,000 616 -> 10 us).
+__global__ void __launch_bounds__(256) k_adjoint_values(RefineDev R, const double *__restrict__ lam,
+                                                        const double *__restrict__ x, double *__restrict__ grad,
+                                                        uint32_t n)
 {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n) return;
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x, w = g / kWave;
+    const bool wide = w < R.a_nlong_t;
+    const uint32_t t = wide ? w : R.a_nlong_t + (g - R.a_nlong_t * kWave);
+    if (t >= n) return;
+    const uint32_t c = R.a_cols[t];
     const double xc = x[c];
-    for (uint32_t k = R.a_cptr[c]; k < R.a_cptr[c + 1]; ++k) grad[k] = -(lam[R.a_ridx[k]] * xc);
+    for (uint32_t k = R.a_cptr[c] + (wide ? g % kWave : 0u); k < R.a_cptr[c + 1]; k += wide ? kWave : 1u)
+        grad[k] = -(lam[R.a_ridx[k]] * xc);
 }
 
 // ---------------------------------------------------------------------------
@@ -3439,7 +3464,8 @@ size_t enable_lds()
 void adjoint_values(const RefineDev &R, const double *lam, const double *x, double *grad, uint32_t n,
                     hipStream_t st)
 {
-    k_adjoint_values<<<blocks_for(n, 256), 256, 0, st>>>(R, lam, x, grad, n);
+    k_adjoint_values<<<blocks_for((uint64_t)R.a_nlong_t * kWave + (n - R.a_nlong_t), 256), 256, 0, st>>>(R, lam, x, grad,
+                                                                                                    n);
 }
 
 void zero_u64(unsigned long long *p, int count, hipStream_t st)
