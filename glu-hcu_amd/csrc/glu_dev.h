@@ -175,7 +175,68 @@ struct DfDev {
     uint32_t voff;             // this sweep's first value in the per-matrix copy
 };
 
+// A triangular sweep as streams of chunks: the layout of the sweeps whose
+// vector is in LDS, values being their own ready marks.  A chunk is a wave's
+// unit: 64 lanes of four entries.  A row takes 1, 2, 4, 8 or 16 lanes
+// (aligned), lane j of the row its entries 4 j .. 4 j + 3 in the order the row
+// consumes them, rows of any size and level side by side in schedule order;
+// a row of more than 64 summed entries takes chunks of its own, lane j of
+// such a chunk holding entries j, 64 + j, 128 + j and 192 + j of its 256.
+//   meta[64 c + lane] = {slots of entries 0, 1 (16 bits each), of 2, 3,
+//     row slot | log2 lanes << 16 | kSwTree | kSwOn, 0}
+//   values: value c stride + 4 lane + e is entry e's, c stride + 256 + lane
+//     the row's pivot (div sweeps; at the lane that stores the row)
+//   a row's right-hand side: rhs[rpos[slot]], at its first lane
+// Slots number the rows of a part (one workgroup's rows); the two after them
+// hold 0 (places without an entry: value 0) and 1 (entries whose column is
+// not in the part: their value is the finished product).  kSwTree: the
+// refinement sums the row's products by lane and then across its lanes;
+// other rows, and every row in the exact solve, are subtracted in order.
+constexpr uint32_t kSwTree = 1u << 20, kSwOn = 1u << 21;
+constexpr uint32_t kSwLong = 1u << 31, kSwFirst = 1u << 30, kSwLast = 1u << 29;   // header bits
+constexpr uint32_t kSwHasTree = 1u << 28, kSwHasSeq = 1u << 27, kSwNarrow = 1u << 26;
+constexpr uint32_t kSwPassMask = 3u;   // header of a long chunk: passes of 64 used, less 1
+
+struct SwPart {
+    uint32_t wp;               // wptr[wp + w] .. wptr[wp + w + 1]: wave w's chunks
+    uint32_t s0, nslot;        // rows row[s0 + slot], right-hand sides rpos[s0 + slot]
+    uint32_t pad;
+};
+
+// An entry whose column belongs to an earlier launch: value[val] = lu[vpos] * x[col].
+struct SwProd {
+    uint32_t val, vpos, col;
+};
+
+struct SwDev {
+    const uint4 *meta;         // [64 chunks]
+    const uint32_t *hdr;       // [chunks]
+    const uint32_t *wptr;
+    const SwPart *part;
+    const uint32_t *row, *rpos;
+    const SwProd *prod;
+    uint32_t nprod, nwave;     // nwave: streams per part
+    uint32_t stride, voff;     // floats per chunk; this sweep's first value in the copy
+    int32_t div;
+    uint32_t pad;
+};
+
+// The split sweeps of one matrix (a vector beyond LDS): head parts and tail
+// of the first and the second sweep, over a value copy of their own.
+struct SplitDev {
+    SwDev head[2], tail[2];
+    const uint32_t *src;       // CSC position of each value of the copy (~0: 0) [nval]
+    uint32_t nval;
+    uint32_t parts;            // head parts
+    uint32_t head_slots;       // rows of the largest
+    uint32_t tail_slots;
+    const uint32_t *rsrc;      // SolveDev::df_rsrc / df_rscale, or the transposed ones
+    const double *rscale;
+};
+
 struct SolveDev {
+    // the vector in LDS, one part (slot = row): L, U and, for A' x = b, U', L'
+    SwDev sw[4];
     TriDev lo, up;             // A x = b:   L then U
     TriDev tup, tlo;           // A' x = b:  U' then L'
     DfDev lo_df, up_df;        // L, U over the per-matrix value copy
@@ -192,10 +253,11 @@ struct SolveDev {
     DfDev tup_df, tlo_df;
     const uint32_t *tdf_src;
     uint32_t tdf_nval;
-    // the first sweep's right-hand side by position p (A x = b over lo_df,
-    // A' x = b over tup_df): float(v[rsrc[p]] * rscale[p]) [n]
+    // the first sweep's right-hand side by row r of the factors (A x = b, and
+    // A' x = b): float(v[rsrc[r]] * rscale[r]) [n]
     const uint32_t *df_rsrc, *tdf_rsrc;
     const double *df_rscale, *tdf_rscale;
+    uint32_t t32_len;          // floats of a matrix's right-hand-side / correction vector scratch
     const uint32_t *row_perm, *row_perm_inv, *col_perm, *col_perm_inv;
     const double *row_scale, *col_scale_perm;
 };

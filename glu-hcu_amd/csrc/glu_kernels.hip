@@ -1591,7 +1591,7 @@ struct MatIO {
     const double *b;    // n
     double *x;          // n
     float *lu;          // nnz_lu
-    float *t32;         // n scratch
+    float *t32;         // t32_len scratch: the correction vector, or the sweeps' right-hand sides
     double *r64;        // n scratch
     float *lucsr;       // df_nval scratch: the sweeps' value copy
     double *norms;      // 2 scratch: [1] = |b|_inf (factor -> refine kernel), [0] unused
@@ -1663,6 +1663,17 @@ __device__ __forceinline__ void globalize(TriDev &T)
     T.lvl_ptr = glb(T.lvl_ptr);
     T.lvl_long = glb(T.lvl_long);
     T.dtask = glb(T.dtask);
+}
+
+__device__ __forceinline__ void globalize(SwDev &D)
+{
+    D.meta = glb(D.meta);
+    D.hdr = glb(D.hdr);
+    D.wptr = glb(D.wptr);
+    D.part = glb(D.part);
+    D.row = glb(D.row);
+    D.rpos = glb(D.rpos);
+    D.prod = glb(D.prod);
 }
 
 __device__ __forceinline__ void globalize(DfDev &D)
@@ -2065,28 +2076,20 @@ __device__ __forceinline__ void df2_sweep(const DfDev &D, const float *__restric
 // dataflow sweeps with the vector in LDS, values as their own ready marks
 // ---------------------------------------------------------------------------
 //
-// For orders whose whole sweep vector fits in LDS.  The vector starts as
+// A part is the rows one workgroup owns, their vector in LDS.  It starts as
 // kUnset everywhere; a row's result is published by storing it, and a reader
 // polls the value itself: one LDS read gives readiness and value, with no
 // ready bit, no fence and no second read between a row and its dependents.
 // What bounds these sweeps is that hop (n=20k: ~400 dependent rows a sweep).
-// Right-hand sides come from memory in position order (task order) with the
-// task's other prefetched loads, so nothing but the dependencies is read
-// while a row waits.  Measured against ready bits (flag, fence and value
-// read per hop): factor + exact solve n=640 238 -> 193 us, n=4,960 644 ->
-// 571 us, n=20,000 with GESP 2,127 -> 1,945 us; same bits.
+// Everything but the dependencies is loaded three chunks ahead.  Measured
+// (exact solve alone): n=4,960 235 -> 160 us, n=20,000 775 -> 430 us against
+// ready bits and one task of 16, 32 or 64 lanes a row.
 //
-// kUnset is a signalling NaN: no FP32 instruction produces one (results are
-// quieted), and sw_put replaces that pattern all the same, so a published
-// row never looks unset and every wait ends (the tables' order is checked on
-// the host, check_df).
-constexpr uint32_t kUnset = 0x7f8a5ca1u;
-
-__device__ __forceinline__ uint32_t sw_peek(const float *xs, uint32_t c)
-{
-    return __hip_atomic_load(reinterpret_cast<const uint32_t *>(xs) + c, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_WORKGROUP);
-}
+// kUnset is a NaN of the largest bit pattern, so the largest of several words
+// tells whether one is unset; sw_put never stores it (a row whose value is
+// that very NaN stores another), so a published row never looks unset and
+// every wait ends (the streams' order is checked on the host, check_sw).
+constexpr uint32_t kUnset = 0xffffffffu;
 
 __device__ __forceinline__ void sw_put(float *xs, uint32_t r, float v)
 {
@@ -2095,251 +2098,292 @@ __device__ __forceinline__ void sw_put(float *xs, uint32_t r, float v)
     __hip_atomic_store(reinterpret_cast<uint32_t *>(xs) + r, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// A task's prefetched data.  Slots that hold no entry have column n (a
-// zero that is always set) and value 0, so lanes need no length tests.
-struct SwTask {
-    uint32_t base, cnt, m, lg;
-    bool wave;
-    uint32_t row;
-    uint32_t idx[kDfK];
-    float val[kDfK];
-    float dval, rhs;
+// A chunk's prefetched data (SwDev).
+struct SwChunk {
+    uint4 m;
+    float4 v;
+    float r, d;
 };
 
-__device__ __forceinline__ void sw_issue(const DfDev &D, const float *__restrict__ sv, const float *__restrict__ rhs,
-                                         uint32_t n, uint4 d, uint32_t lane, SwTask &t)
+// a / d with the work on d done ahead (the divisor is known long before the
+// row's value is).  r: the reciprocal with one Newton step; the quotient then
+// takes the two corrections of the compiler's own division of operands that
+// need no scaling, so the result is its result, correctly rounded.  Operands
+// outside [2^-30, 2^30] (d) and [2^-64, 2^64] (a) take the full division.
+struct SwDiv {
+    float d, r;
+    bool plain;   // d in range
+};
+
+__device__ __forceinline__ bool sw_in_range(float v, uint32_t lo, uint32_t hi)
 {
-    t.base = d.x;
-    t.wave = (d.z & kLongTask) != 0;
-    t.cnt = d.z & 0xffffffu;
-    t.lg = (d.z >> 24) & 0x7fu;
-    t.m = d.w;
-    const uint32_t p = d.y + (t.wave ? lane >> t.lg : lane);
-    t.row = D.rl[p].x;
-    t.rhs = rhs[min(p, n - 1)];
-    t.dval = 1.f;
-    if (D.div) t.dval = sv[D.nslots + p];   // the pivot
-    if (!t.wave) {
-#pragma unroll
-        for (uint32_t e = 0; e < kDfK; ++e) {   // entries past the task's longest row belong to later tasks
-            const uint32_t ix = D.idx[t.base + e * kWave + lane];
-            const float v = sv[t.base + e * kWave + lane];
-            t.idx[e] = e < t.m ? ix : n;
-            t.val[e] = e < t.m ? v : 0.f;
-        }
-    } else {
-        t.idx[0] = D.idx[t.base + lane];
-        t.val[0] = sv[t.base + lane];
-    }
+    return (__float_as_uint(v) & 0x7fffffffu) - (lo << 23) < ((hi - lo) << 23);
 }
 
-// One task.  kExact: each row's products subtracted one at a time in the
-// row's order (the arithmetic of Symbolic_Matrix::solve); otherwise a wave
-// row's products are summed by lane and then across the lanes.
-template <bool kExact>
-__device__ __forceinline__ void sw_run(const DfDev &D, const float *__restrict__ sv, float *xs, const SwTask &t,
-                                       uint32_t lane)
+__device__ __forceinline__ SwDiv sw_div_prepare(float d)
 {
-    if (!t.wave) {   // rows a lane each
-        bool pending = lane < t.cnt;
-        while (__ballot(pending)) {
-            uint32_t b[kDfK];
-            bool ok = pending;
-#pragma unroll
-            for (uint32_t e = 0; e < kDfK; ++e) b[e] = sw_peek(xs, t.idx[e]);
-#pragma unroll
-            for (uint32_t e = 0; e < kDfK; ++e) ok &= b[e] != kUnset;
-            if (ok) {
-                float acc = t.rhs;
-#pragma unroll
-                for (uint32_t e = 0; e < kDfK; ++e) acc = acc - t.val[e] * __uint_as_float(b[e]);
-                if (D.div) acc = acc / t.dval;
-                sw_put(xs, t.row, acc);
-                pending = false;
-            }
-        }
-        return;
-    }
-    const uint32_t gw = 1u << t.lg, j = lane & (gw - 1u);
-    const uint32_t *ix = D.idx + t.base + lane;   // passes past the first: a 64-lane row, t.m entries
-    const float *vx = sv + t.base + lane;
-    if (kExact) {
-        // 16 lanes at a time: wait for those entries only, subtract their
-        // products along the lanes, hand the running value on
-        float carry = t.rhs, a = 0.f;
-        uint32_t c = t.idx[0];
-        float v = t.val[0];
-        for (uint32_t c0 = 0;; c0 += kWave) {
-            const bool more = c0 + kWave < t.m;   // (uniform; only a 64-lane row)
-            uint32_t nc = 0;
-            float nv = 0.f;
-            if (more) {   // the next pass's entries load while this one is consumed
-                nc = ix[c0 + kWave];
-                nv = vx[c0 + kWave];
-            }
-            const uint32_t nseg = t.lg == 6 ? (more ? 4u : (t.m - c0 + 15u) / 16u) : gw / 16u;
-            uint64_t seg = t.lg == 4 ? ~0ull : t.lg == 5 ? 0x0000ffff0000ffffull : 0xffffull;
-            for (uint32_t r = 0; r < nseg; ++r, seg <<= 16) {
-                uint32_t b;
-                do {
-                    b = sw_peek(xs, c);
-                } while (__ballot(b == kUnset) & seg);
-                const float p = v * __uint_as_float(b);
-                a = row_chain_sub(carry - p, p);
-                // lane 15 of each row of 16 to the next row (row_bcast:15)
-                carry = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x142, 0xf, 0xf, false));
-            }
-            if (t.lg != 6) break;
-            carry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), (int)(16u * nseg - 1u)));
-            if (!more) break;
-            c = nc;
-            v = nv;
-        }
-        if (t.lg == 6) a = carry;
-        if (j == gw - 1u && (lane >> t.lg) < t.cnt) {
-            if (D.div) a = a / t.dval;
-            sw_put(xs, t.row, a);
-        }
-        return;
-    }
-    constexpr uint32_t kB = 4;   // passes of a long row loaded at a time, ahead of their use
-    uint32_t col[kB];
-    float w[kB];
-    if (t.m > kWave) {
-#pragma unroll
-        for (uint32_t u = 0; u < kB; ++u) {
-            const uint32_t q = min((u + 1) * kWave, (t.m - 1) & ~(kWave - 1u));
-            col[u] = ix[q];
-            w[u] = vx[q];
-        }
-    }
-    uint32_t b;
-    do {
-        b = sw_peek(xs, t.idx[0]);
-    } while (__ballot(b == kUnset));
-    float sum = t.val[0] * __uint_as_float(b);
-    for (uint32_t c0 = kWave; c0 < t.m; c0 += kB * kWave) {   // gw == 64 here
-        uint32_t cc[kB];
-        float cw[kB];
-#pragma unroll
-        for (uint32_t u = 0; u < kB; ++u) {
-            cc[u] = col[u];
-            cw[u] = w[u];
-        }
-        if (c0 + kB * kWave < t.m) {
-#pragma unroll
-            for (uint32_t u = 0; u < kB; ++u) {
-                const uint32_t q = min(c0 + (kB + u) * kWave, (t.m - 1) & ~(kWave - 1u));
-                col[u] = ix[q];
-                w[u] = vx[q];
-            }
-        }
-        uint32_t bb[kB];
-        bool un;
-        do {
-            un = false;
-#pragma unroll
-            for (uint32_t u = 0; u < kB; ++u) bb[u] = sw_peek(xs, cc[u]);
-#pragma unroll
-            for (uint32_t u = 0; u < kB; ++u) un |= bb[u] == kUnset;
-        } while (__ballot(un));
-#pragma unroll
-        for (uint32_t u = 0; u < kB; ++u)
-            if (c0 + u * kWave + j < t.m) sum += cw[u] * __uint_as_float(bb[u]);
-    }
-    sum = group_sum(sum, gw);
-    if (j == 0 && (lane >> t.lg) < t.cnt) {
-        float acc = t.rhs - sum;
-        if (D.div) acc = acc / t.dval;
-        sw_put(xs, t.row, acc);
-    }
+    SwDiv q;
+    const float r = __builtin_amdgcn_rcpf(d);
+    q.d = d;
+    q.r = fmaf(fmaf(-d, r, 1.f), r, r);
+    q.plain = sw_in_range(d, 127 - 30, 127 + 30);
+    return q;
 }
 
-// All tasks of sweep D for the calling workgroup: right-hand sides rhs[p] by
-// position, results into xs (LDS; all kUnset but xs[n] = 0).  Waves, task
-// order and prefetch as df2_sweep.
-template <bool kExact>
-__device__ __forceinline__ void sw_sweep(const DfDev &D, const float *__restrict__ sv, const float *__restrict__ rhs,
-                                         uint32_t n, float *xs)
+// lanes: those whose quotient is used (uniform).
+__device__ __forceinline__ float sw_div(const SwDiv &q, float a, uint64_t lanes)
 {
-    const uint32_t lane = threadIdx.x & (kWave - 1), nw = blockDim.x / kWave;
-    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // uniform: scalar loads below
-    const uint32_t mine = D.ntask > w ? (D.ntask - w + nw - 1) / nw : 0;
-    if (mine == 0) return;
-    const __attribute__((address_space(4))) uint32_t *tasks =
-        (const __attribute__((address_space(4))) uint32_t *)(uintptr_t)D.task;
-    auto desc = [&](uint32_t k) {
-        const uint32_t q = 4 * (w + (k < mine ? k : mine - 1) * nw);
-        const uint4 d = make_uint4(tasks[q], tasks[q + 1], tasks[q + 2], tasks[q + 3]);
-        return k < mine ? d : make_uint4(0u, 0u, 0u, 0u);
+    const float q0 = a * q.r;
+    const float q1 = fmaf(fmaf(-q.d, q0, a), q.r, q0);
+    const float res = fmaf(fmaf(-q.d, q1, a), q.r, q1);
+    if (__ballot(!(q.plain && sw_in_range(a, 127 - 64, 127 + 64))) & lanes) {
+        asm volatile("");   // a branch: the full division is not to be computed beside
+        return a / q.d;
+    }
+    return res;
+}
+
+__device__ __forceinline__ float sw_f(uint32_t b) { return __uint_as_float(b); }
+
+// Chunks [k, k1) of sweep D, in order, by one wave: values sv, right-hand
+// sides rhs, results into xs (LDS; kUnset but for the two constant slots).
+// Chunks load three ahead (a chunk is four loads, so the waits count).
+// kExact: every row's products are subtracted one at a time in the row's
+// order (the arithmetic of Symbolic_Matrix::solve); slice: the wave's 64
+// floats of LDS for its long rows.  While a row waits, the subtractions that
+// can be done are: from the last entry's arrival only its own lane's remain.
+template <bool kExact>
+__device__ __forceinline__ void sw_wave(const SwDev &D, uint32_t k, uint32_t k1, const float *__restrict__ sv,
+                                        const float *__restrict__ rhs, float *xs, float *slice)
+{
+    if (k >= k1) return;
+    const uint32_t lane = threadIdx.x & (kWave - 1), doff = D.div ? 256u : 0u, stride = D.stride;
+    auto load = [&](uint32_t q) {
+        q = min(q, k1 - 1);
+        const float *c = sv + (size_t)q * stride;
+        SwChunk t;
+        t.m = D.meta[(size_t)q * kWave + lane];
+        t.v = reinterpret_cast<const float4 *>(c)[lane];
+        t.r = rhs[(size_t)q * kWave + lane];
+        t.d = c[doff + lane];
+        return t;
     };
-    uint4 dn = desc(0), dn2 = desc(1);
-    SwTask cur, nxt;
-    sw_issue(D, sv, rhs, n, dn, lane, nxt);
-    for (uint32_t k = 0; k < mine; ++k) {
-        cur = nxt;
-        __builtin_amdgcn_s_waitcnt(0xF70);   // vmcnt(0): this task's loads (see df2_sweep)
-        dn = dn2;
-        dn2 = desc(k + 2);
-        sw_issue(D, sv, rhs, n, dn, lane, nxt);
-        sw_run<kExact>(D, sv, xs, cur, lane);
+    auto header = [&](uint32_t q) { return D.hdr[min(q + lane, k1 - 1)]; };   // 64 chunks', one a lane
+    const uint32_t *X = reinterpret_cast<const uint32_t *>(xs);
+    auto peek = [&](uint32_t a) { return __hip_atomic_load(X + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    SwChunk c0 = load(k), c1 = load(k + 1), c2 = load(k + 2);
+    uint32_t hv = header(k), hn = header(k + kWave), j64 = 0;
+    float acc = 0.f, first = 0.f;   // a long row's running value (exact: the same in every lane), right-hand side
+    for (; k < k1; ++k, ++j64) {
+        const SwChunk t = c0;
+        c0 = c1;
+        c1 = c2;
+        c2 = load(k + 3);
+        if (j64 == (uint32_t)kWave) {
+            j64 = 0;
+            hv = hn;
+            hn = header(k + kWave);
+        }
+        const uint32_t h = __builtin_amdgcn_readlane(hv, j64);
+        const uint32_t a0 = t.m.x & 0xffffu, a1 = t.m.x >> 16, a2 = t.m.y & 0xffffu, a3 = t.m.y >> 16;
+        const uint32_t row = t.m.z & 0xffffu;
+        uint32_t b0, b1, b2, b3;
+        if (h & kSwLong) {
+            const uint32_t np = h & kSwPassMask;   // passes less 1 (uniform)
+            if (kExact) {
+                if (h & kSwFirst) acc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t.r)));
+                const uint32_t ad[4] = {a0, a1, a2, a3};
+                const float w[4] = {t.v.x, t.v.y, t.v.z, t.v.w};
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) {
+                    if (u > np) break;
+                    uint32_t b;
+                    for (;;) {
+                        b = peek(ad[u]);
+                        if (!__ballot(b == kUnset)) break;
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    slice[lane] = w[u] * sw_f(b);
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    acc = serial_sub(acc, slice, kWave, false);   // places without an entry hold +0
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                }
+                if ((h & kSwLast) && lane == 0) sw_put(xs, row, D.div ? acc / t.d : acc);
+            } else {
+                for (;;) {
+                    b0 = peek(a0), b1 = peek(a1), b2 = peek(a2), b3 = peek(a3);
+                    if (!__ballot(max(max(b0, b1), max(b2, b3)) == kUnset)) break;
+                    __builtin_amdgcn_s_sleep(1);
+                }
+                // (a place without an entry adds nothing, not even +0)
+                const bool e1 = t.m.w & 2u, e2 = t.m.w & 4u, e3 = t.m.w & 8u;
+                const float p0 = t.v.x * sw_f(b0), p1 = t.v.y * sw_f(b1), p2 = t.v.z * sw_f(b2), p3 = t.v.w * sw_f(b3);
+                if (h & kSwFirst) first = t.r;
+                float s = acc;
+                if (t.m.w & 1u) s = (h & kSwFirst) ? p0 : s + p0;
+                if (e1) s += p1;
+                if (e2) s += p2;
+                if (e3) s += p3;
+                acc = s;
+                if (h & kSwLast) {
+                    const float sum = group_sum(acc, 64);
+                    if (lane == 0) {
+                        const float v = first - sum;
+                        sw_put(xs, row, D.div ? v / t.d : v);
+                    }
+                }
+            }
+            continue;
+        }
+        const uint32_t lg = (t.m.z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
+        const bool on = t.m.z & kSwOn, tree = !kExact && (t.m.z & kSwTree);
+        const bool seq = kExact || (h & kSwHasSeq), sum = !kExact && (h & kSwHasTree);   // (uniform)
+        uint64_t left = __ballot(on && (tree ? j == 0 : j == g - 1u));   // lanes that store rows still to come
+        const uint64_t F = __ballot(j == 0), TR = __ballot(tree);
+        uint64_t V = 0;                            // lanes whose running value is final (rows in order)
+        const uint64_t rm = ((1ull << g) - 1ull) << (lane & ~(g - 1u));   // the row's lanes
+        const uint32_t rlo = (uint32_t)rm, rhi = (uint32_t)(rm >> 32);
+        SwDiv dv{1.f, 1.f, true};
+        if (D.div) dv = sw_div_prepare(t.d);
+        float a = 0.f;
+        // one of the few waves that carry the chain of narrow levels goes
+        // before the others, which give way while they wait
+        const bool narrow = h & kSwNarrow;
+        if (narrow) __builtin_amdgcn_s_setprio(2);
+        for (;;) {
+            b0 = peek(a0), b1 = peek(a1), b2 = peek(a2), b3 = peek(a3);
+            const uint64_t R = __ballot(max(max(b0, b1), max(b2, b3)) != kUnset);   // lanes whose entries are all set
+            const float p0 = t.v.x * sw_f(b0), p1 = t.v.y * sw_f(b1), p2 = t.v.z * sw_f(b2), p3 = t.v.w * sw_f(b3);
+            bool more;
+            do {
+                uint64_t fin = 0;
+                float res = 0.f;
+                more = false;
+                if (seq) {
+                    // lane j's value is lane j - 1's less its own four
+                    // products; a step settles the next ready lane of every
+                    // row, and does not change settled ones
+                    const float prev = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xf, 0xf, false));
+                    a = j == 0 ? t.r : prev;
+                    a = a - p0;
+                    a = a - p1;
+                    a = a - p2;
+                    a = a - p3;
+                    V = R & (F | (V << 1));
+                    fin = V & left & ~TR;
+                    res = a;
+                    more = (R & (F | (V << 1))) != V;
+                }
+                if (sum) {
+                    const bool rdy = ((uint32_t)R & rlo) == rlo && ((uint32_t)(R >> 32) & rhi) == rhi;
+                    float q = (p0 + p1) + (p2 + p3);
+                    q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0xB1, 0xf, 0xf, false));   // quad [1,0,3,2]
+                    q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x4E, 0xf, 0xf, false));   // quad [2,3,0,1]
+                    const float q8 = q + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x141, 0xf, 0xf, false));   // half mirror
+                    const float q16 = q8 + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q8), 0x140, 0xf, 0xf, false));  // mirror
+                    const float tv = t.r - (lg == 2u ? q : lg == 3u ? q8 : q16);
+                    fin |= __ballot(rdy) & left & TR;
+                    res = tree ? tv : res;
+                }
+                if (fin) {
+                    if (D.div) res = sw_div(dv, res, fin);
+                    if (__builtin_amdgcn_inverse_ballot_w64(fin)) sw_put(xs, row, res);
+                    left &= ~fin;
+                }
+            } while (more);
+            if (!left) break;
+            if (!narrow) __builtin_amdgcn_s_sleep(1);
+        }
+        if (narrow) __builtin_amdgcn_s_setprio(0);
     }
 }
 
-// Both sweeps of M = (LU)^-1 with the vector in LDS: rhs (n floats, memory)
-// holds the first sweep's right-hand sides by position and is used for the
-// second's; xs (n + 1 floats) ends with the results by row.  Starts with
-// everything before it visible only to this thread; ends with a barrier.
-template <bool kExact>
-__device__ __forceinline__ void sw_solve(const DfDev &first, const float *__restrict__ sv1, const DfDev &second,
-                                         const float *__restrict__ sv2, float *rhs, uint32_t n, float *xs)
+// The LDS vector of a part before its sweep: rows not set, then the constant
+// slots 0 and 1.
+__device__ __forceinline__ void sw_clear(float *xs, uint32_t nslot)
 {
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
     uint32_t *xb = reinterpret_cast<uint32_t *>(xs);
-    for (uint32_t i = tid; i <= n; i += nt) xb[i] = i < n ? kUnset : 0u;
-    __syncthreads();
-    sw_sweep<kExact>(first, sv1, rhs, n, xs);
-    __syncthreads();
-    constexpr uint32_t kU = 4;
-    for (uint32_t p0 = tid; p0 < n; p0 += kU * nt) {
-        uint32_t r[kU];
-#pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) r[u] = second.rl[min(p0 + u * nt, n - 1)].x;
-#pragma unroll
-        for (uint32_t u = 0; u < kU; ++u)
-            if (p0 + u * nt < n) rhs[p0 + u * nt] = xs[r[u]];
-    }
-    __syncthreads();
-    for (uint32_t i = tid; i < n; i += nt) xb[i] = kUnset;
-    __syncthreads();
-    sw_sweep<kExact>(second, sv2, rhs, n, xs);
-    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < nslot + 2; i += blockDim.x)
+        xb[i] = i < nslot ? kUnset : i == nslot ? 0u : 0x3f800000u;
 }
 
-// rhs[p] = float(v[src[p]] * scale[p]): the right-hand side in the factors'
-// frame, by position of the first sweep (its loads four at a time).
-template <typename T>
-__device__ __forceinline__ void sw_scale(const T *__restrict__ v, const uint32_t *__restrict__ src,
-                                         const double *__restrict__ scale, float *rhs, uint32_t n)
+// Part P of sweep D by the calling workgroup (vector cleared and right-hand
+// sides written, behind a barrier); wl: the workgroup's wave slices (kExact).
+template <bool kExact>
+__device__ __forceinline__ void sw_part(const SwDev &D, const SwPart &P, const float *sv, const float *rhs, float *xs,
+                                        float *wl)
 {
-    constexpr uint32_t kU = 4;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (w < D.nwave)
+        sw_wave<kExact>(D, D.wptr[P.wp + w], D.wptr[P.wp + w + 1], sv, rhs, xs, wl + w * kWave);
+}
+
+// rhs[rpos[i]] = float(v[src[r]] * scale[r]) for the rows r of part P (slot
+// i): the first sweep's right-hand side in the factors' frame.
+template <typename T>
+__device__ __forceinline__ void sw_scale(const SwDev &D, const SwPart &P, const T *__restrict__ v,
+                                         const uint32_t *__restrict__ src, const double *__restrict__ scale, float *rhs)
+{
+    constexpr uint32_t kU = 4;   // loads four at a time
     const uint32_t nt = blockDim.x;
-    for (uint32_t p0 = threadIdx.x; p0 < n; p0 += kU * nt) {
-        uint32_t s[kU];
+    for (uint32_t i0 = threadIdx.x; i0 < P.nslot; i0 += kU * nt) {
+        uint32_t r[kU], q[kU], s[kU];
         double a[kU];
         T x[kU];
 #pragma unroll
         for (uint32_t u = 0; u < kU; ++u) {
-            const uint32_t p = min(p0 + u * nt, n - 1);
-            s[u] = src[p];
-            a[u] = scale[p];
+            const uint32_t i = P.s0 + min(i0 + u * nt, P.nslot - 1);
+            r[u] = D.row[i];
+            q[u] = D.rpos[i];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) {
+            s[u] = src[r[u]];
+            a[u] = scale[r[u]];
         }
 #pragma unroll
         for (uint32_t u = 0; u < kU; ++u) x[u] = v[s[u]];
 #pragma unroll
         for (uint32_t u = 0; u < kU; ++u)
-            if (p0 + u * nt < n) rhs[p0 + u * nt] = (float)((double)x[u] * a[u]);
+            if (i0 + u * nt < P.nslot) rhs[q[u]] = (float)((double)x[u] * a[u]);
     }
+}
+
+// rhs[rpos[i]] = the first sweep's result of slot i (the second sweep's
+// right-hand side; both sweeps number the part's rows alike).
+__device__ __forceinline__ void sw_carry(const SwDev &D, const SwPart &P, const float *xs, float *rhs)
+{
+    constexpr uint32_t kU = 4;
+    const uint32_t nt = blockDim.x;
+    for (uint32_t i0 = threadIdx.x; i0 < P.nslot; i0 += kU * nt) {
+        uint32_t q[kU];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) q[u] = D.rpos[P.s0 + min(i0 + u * nt, P.nslot - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            if (i0 + u * nt < P.nslot) rhs[q[u]] = xs[i0 + u * nt];
+    }
+}
+
+// Both sweeps of M = (LU)^-1 over part 0 of each: right-hand sides already in
+// rhs (visible to this thread's later barrier), values sv, vector in LDS (xs:
+// nslot + 2 floats), results left there by slot.  Ends with a barrier.
+template <bool kExact>
+__device__ __forceinline__ void sw_both(const SwDev &A, const SwDev &B, const float *sv, float *rhs, float *xs, float *wl)
+{
+    const SwPart P = A.part[0], Q = B.part[0];
+    sw_clear(xs, P.nslot);
+    __syncthreads();
+    sw_part<kExact>(A, P, sv + A.voff, rhs, xs, wl);
+    __syncthreads();
+    sw_carry(B, Q, xs, rhs);
+    __syncthreads();
+    sw_clear(xs, Q.nslot);
+    __syncthreads();
+    sw_part<kExact>(B, Q, sv + B.voff, rhs, xs, wl);
+    __syncthreads();
 }
 
 // LDS placement of the batch pipeline's sweep state (dynamic LDS).
@@ -2519,11 +2563,12 @@ __device__ __forceinline__ void wg_precond(const MatDesc *Md, const MatIO &io, c
     const uint32_t n = Md->n;
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
     if (kMode == kSweepLds) {
-        sw_scale(v, glb(kT ? Md->s.tdf_rsrc : Md->s.df_rsrc), glb(kT ? Md->s.tdf_rscale : Md->s.df_rscale), io.t32, n);
-        DfDev d1 = kT ? Md->s.tup_df : Md->s.lo_df, d2 = kT ? Md->s.tlo_df : Md->s.up_df;
+        SwDev d1 = Md->s.sw[kT ? 2 : 0], d2 = Md->s.sw[kT ? 3 : 1];
         globalize(d1);
         globalize(d2);
-        sw_solve<false>(d1, io.lucsr + d1.voff, d2, io.lucsr + d2.voff, io.t32, n, xs);
+        sw_scale(d1, d1.part[0], v, glb(kT ? Md->s.tdf_rsrc : Md->s.df_rsrc), glb(kT ? Md->s.tdf_rscale : Md->s.df_rscale),
+                 io.t32);
+        sw_both<false>(d1, d2, io.lucsr, io.t32, xs, nullptr);
         return;
     }
     const uint32_t nwords = (n + 31) / 32;
@@ -2781,8 +2826,7 @@ __device__ __forceinline__ void wg_refine(const MatDesc *Md, const MatIO &io, do
 }
 
 // Dynamic LDS of the batch kernels: ready bits (ceil(n/32) words;
-// kSweepFlags), or the correction vector (kSweepLds: n + 1 floats, in the
-// n + ceil(n/32) that orders taken this way have room for).
+// kSweepFlags), or the correction vector (kSweepLds: n + 2 floats).
 template <int kMode>
 __device__ __forceinline__ void batch_lds(uint32_t n, float *t32, uint32_t *&flags, float *&xs)
 {
@@ -2802,7 +2846,7 @@ __device__ __forceinline__ MatIO batch_io(const MatDesc *desc, const double *ax,
     io.b = b + m * n;
     io.x = x + m * n;
     io.lu = lu + m * nnz;
-    io.t32 = t32 + m * n;
+    io.t32 = t32 + m * desc->s.t32_len;
     io.r64 = r64 + m * n;
     io.lucsr = lucsr ? lucsr + m * nval : nullptr;
     io.norms = norms + 2 * m;
@@ -2895,14 +2939,13 @@ __global__ void __launch_bounds__(1024) k_batch_same_fused(const MatDesc *__rest
 }
 
 // One matrix's factors gathered into the sweeps' layout (grid, a thread per
-// slot): lucsr[q] = lu[df_src[q]], 0 for padding slots.
-template <bool kT>
-__global__ void __launch_bounds__(256) k_copy_df(const MatDesc *__restrict__ desc, const float *__restrict__ lu,
-                                                 float *__restrict__ lucsr)
+// value): lucsr[q] = lu[src[q]], 0 where src is ~0.
+__global__ void __launch_bounds__(256) k_copy_df(const uint32_t *__restrict__ src, uint32_t nval,
+                                                 const float *__restrict__ lu, float *__restrict__ lucsr)
 {
     const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (kT ? desc->s.tdf_nval : desc->s.df_nval)) return;
-    const uint32_t p = glb(kT ? desc->s.tdf_src : desc->s.df_src)[q];
+    if (q >= nval) return;
+    const uint32_t p = src[q];
     lucsr[q] = p != ~0u ? lu[p] : 0.f;
 }
 
@@ -2972,7 +3015,7 @@ __global__ void __launch_bounds__(1024) k_sweeps_df(const MatDesc *__restrict__ 
 // copy of the factors, x = float(xs[row_perm_inv] * row_scale) — the
 // arithmetic of Symbolic_Matrix::solve (src/symbolic.cc:215-247).  Dynamic
 // LDS as k_batch_same_refine.
-template <int kMode, bool kSplit = false>
+template <int kMode, bool kSplit = false, bool kT = false>
 __global__ void __launch_bounds__(1024) k_solve_one(const MatDesc *__restrict__ desc,
                                                     const float *__restrict__ lucsr, const float *__restrict__ b,
                                                     float *__restrict__ x, float *__restrict__ t32, uint32_t r0)
@@ -2985,11 +3028,21 @@ __global__ void __launch_bounds__(1024) k_solve_one(const MatDesc *__restrict__ 
     const uint32_t *rpi = glb(desc->s.row_perm_inv);
     const double *rs = glb(desc->s.row_scale);
     if (kMode == kSweepLds) {
-        sw_scale(b, glb(desc->s.df_rsrc), glb(desc->s.df_rscale), glb(t32), n);
-        DfDev d1 = desc->s.lo_df, d2 = desc->s.up_df;
+        SwDev d1 = desc->s.sw[kT ? 2 : 0], d2 = desc->s.sw[kT ? 3 : 1];
         globalize(d1);
         globalize(d2);
-        sw_solve<true>(d1, glb(lucsr) + d1.voff, d2, glb(lucsr) + d2.voff, glb(t32), n, xs);
+        sw_scale(d1, d1.part[0], b, glb(kT ? desc->s.tdf_rsrc : desc->s.df_rsrc),
+                 glb(kT ? desc->s.tdf_rscale : desc->s.df_rscale), glb(t32));
+        sw_both<true>(d1, d2, glb(lucsr), glb(t32), xs, &wl[0][0]);
+        if (kT) {   // A' x = b: columns back by col_perm_inv, scaled by col_scale_perm
+            const uint32_t *cpi = glb(desc->s.col_perm_inv);
+            const double *csp = glb(desc->s.col_scale_perm);
+            for (uint32_t j = tid; j < n; j += nt) {
+                const uint32_t pj = cpi[j];
+                x[j] = (float)((double)xs[pj] * csp[pj]);
+            }
+            return;
+        }
         for (uint32_t j = tid; j < n; j += nt) x[j] = (float)((double)xs[rpi[j]] * rs[j]);
         return;
     }
@@ -3015,6 +3068,76 @@ __global__ void __launch_bounds__(1024) k_solve_one(const MatDesc *__restrict__ 
         __syncthreads();
     }
     for (uint32_t j = tid; j < n; j += nt) x[j] = (float)((double)xs[rpi[j]] * rs[j]);
+}
+
+// ---------------------------------------------------------------------------
+// split sweeps of one matrix: many workgroups, then one, then many
+// ---------------------------------------------------------------------------
+//
+// Orders whose vector does not fit in LDS.  The rows of little height in the
+// elimination order fall into independent components (head parts, a
+// workgroup each); the others, the tail, hold the dependency chain and fit in
+// one workgroup's LDS.  L: the head parts, then the tail with the products
+// by head values formed across the grid first.  U: the tail, then the head
+// parts likewise.  A product formed ahead meets a 1 in the sweep, so every
+// row's arithmetic and order are those of a sweep over the whole vector.
+// Against both sweeps in one workgroup with the vector in memory: n=50,000
+// exact solve 1,253 -> 404 us, n=200,003 9.0 -> 2.2 ms (of which the tail
+// takes 2.0 ms, its chain of ~2,150 rows and the rails' long rows).
+// Dynamic LDS: the part's slots.  xg: the vector by row.
+__device__ __forceinline__ void sw_out(const SwDev &D, const SwPart &P, const float *xs, float *__restrict__ xg)
+{
+    for (uint32_t i = threadIdx.x; i < P.nslot; i += blockDim.x) xg[D.row[P.s0 + i]] = xs[i];
+}
+
+template <bool kExact, typename T>
+__global__ void __launch_bounds__(1024) k_sw_first(SwDev D, const T *__restrict__ in, const uint32_t *__restrict__ src,
+                                                   const double *__restrict__ scale, const float *__restrict__ lucsr,
+                                                   float *rhs, float *__restrict__ xg)
+{
+    __shared__ __attribute__((aligned(16))) float wl[kExact ? 1024 / kWave : 1][kWave];
+    const SwPart P = D.part[blockIdx.x];
+    sw_scale(D, P, in, src, scale, rhs);
+    sw_clear(g_lds_vec, P.nslot);
+    __syncthreads();
+    sw_part<kExact>(D, P, lucsr + D.voff, rhs, g_lds_vec, &wl[0][0]);
+    __syncthreads();
+    sw_out(D, P, g_lds_vec, xg);
+}
+
+template <bool kExact, typename T>
+__global__ void __launch_bounds__(1024) k_sw_tail(SwDev A, SwDev B, const T *__restrict__ in,
+                                                  const uint32_t *__restrict__ src, const double *__restrict__ scale,
+                                                  const float *__restrict__ lucsr, float *rhs, float *__restrict__ xg)
+{
+    __shared__ __attribute__((aligned(16))) float wl[kExact ? 1024 / kWave : 1][kWave];
+    sw_scale(A, A.part[0], in, src, scale, rhs);
+    sw_both<kExact>(A, B, lucsr, rhs, g_lds_vec, &wl[0][0]);
+    sw_out(B, B.part[0], g_lds_vec, xg);
+}
+
+template <bool kExact>
+__global__ void __launch_bounds__(1024) k_sw_second(SwDev D, const float *__restrict__ lucsr, float *rhs,
+                                                    float *__restrict__ xg)
+{
+    __shared__ __attribute__((aligned(16))) float wl[kExact ? 1024 / kWave : 1][kWave];
+    const SwPart P = D.part[blockIdx.x];
+    for (uint32_t i = threadIdx.x; i < P.nslot; i += blockDim.x) rhs[D.rpos[P.s0 + i]] = xg[D.row[P.s0 + i]];
+    sw_clear(g_lds_vec, P.nslot);
+    __syncthreads();
+    sw_part<kExact>(D, P, lucsr + D.voff, rhs, g_lds_vec, &wl[0][0]);
+    __syncthreads();
+    sw_out(D, P, g_lds_vec, xg);
+}
+
+__global__ void __launch_bounds__(256) k_sw_prod(const SwProd *__restrict__ prod, uint32_t nprod,
+                                                 const float *__restrict__ lu, const float *__restrict__ xg,
+                                                 float *__restrict__ lucsr)
+{
+    const uint32_t q = blockIdx.x * 256 + threadIdx.x;
+    if (q >= nprod) return;
+    const SwProd p = prod[q];
+    lucsr[p.val] = lu[p.vpos] * xg[p.col];
 }
 
 // Distinct patterns: workgroup g runs matrix order[g] with its own tables.
@@ -3218,7 +3341,9 @@ void residual(const RefineDev &R, const double *ax, const double *b, const doubl
 size_t batch_lds_bytes(int mode, uint32_t n)
 {
     const size_t words = (n + 31) / 32;
-    return mode == kSweepLevels ? 0 : 4 * words + (mode == kSweepLds ? 4 * (size_t)n : 0);
+    // kSweepLds: the vector and its two constant slots, in no less than the
+    // ready bits and the vector take (so the same orders are taken this way)
+    return mode == kSweepLevels ? 0 : mode == kSweepLds ? 4 * (std::max<size_t>(words, 2) + n) : 4 * words;
 }
 
 // Sweep mode kSweepLds: one launch, factor then refine in each workgroup
@@ -3253,27 +3378,24 @@ void batch_same(const MatDesc *desc, int batch, const double *ax, const double *
 
 // glu_refine in one workgroup (orders whose sweep vector fits in LDS): the
 // factors into the sweeps' layout, then the refinement.
-void refine_one(const MatDesc *desc, uint32_t nval, const double *ax, const double *b, double *x,
+void refine_one(const MatDesc *desc, const uint32_t *src, uint32_t nval, const double *ax, const double *b, double *x,
                 const float *lu, float *lucsr, float *t32, double *r64, double *norms, double *kry, int32_t *iters,
                 double *eta, double tol, int maxit, int threads, size_t ref_lds, int transpose, hipStream_t st)
 {
-    const unsigned grid = blocks_for(nval, 256);
+    k_copy_df<<<blocks_for(nval, 256), 256, 0, st>>>(src, nval, lu, lucsr);
     if (transpose) {
-        k_copy_df<true><<<grid, 256, 0, st>>>(desc, lu, lucsr);
         k_refine_one<kSweepLds, true><<<1, threads, ref_lds, st>>>(desc, ax, b, x, lu, lucsr, t32, r64, norms, kry,
                                                                    iters, eta, tol, maxit);
     } else {
-        k_copy_df<false><<<grid, 256, 0, st>>>(desc, lu, lucsr);
         k_refine_one<kSweepLds, false><<<1, threads, ref_lds, st>>>(desc, ax, b, x, lu, lucsr, t32, r64, norms, kry,
                                                                     iters, eta, tol, maxit);
     }
 }
 
-// The factors into the sweeps' layout (A or A' tables), grid.
-void copy_df(const MatDesc *desc, uint32_t nval, const float *lu, float *lucsr, int transpose, hipStream_t st)
+// The factors into a sweep layout, grid.
+void copy_df(const uint32_t *src, uint32_t nval, const float *lu, float *lucsr, hipStream_t st)
 {
-    if (transpose) k_copy_df<true><<<blocks_for(nval, 256), 256, 0, st>>>(desc, lu, lucsr);
-    else k_copy_df<false><<<blocks_for(nval, 256), 256, 0, st>>>(desc, lu, lucsr);
+    k_copy_df<<<blocks_for(nval, 256), 256, 0, st>>>(src, nval, lu, lucsr);
 }
 
 // Both sweeps of the preconditioner in one workgroup over t32 (global).
@@ -3291,14 +3413,46 @@ void sweeps_df(const MatDesc *desc, const float *lucsr, float *t32, uint32_t r0,
 }
 
 // glu_solve in one workgroup: the factors into the sweep layout, then the
-// exact sweeps (mode: kSweepLds or kSweepFlags).
-void solve_one(const MatDesc *desc, uint32_t nval, const float *lu, float *lucsr, const float *b, float *x,
-               float *t32, uint32_t r0, int threads, int mode, size_t lds, hipStream_t st)
+// exact sweeps (mode: kSweepLds, or kSweepFlags for A x = b).
+void solve_one(const MatDesc *desc, const uint32_t *src, uint32_t nval, const float *lu, float *lucsr, const float *b,
+               float *x, float *t32, uint32_t r0, int threads, int mode, size_t lds, int transpose, hipStream_t st)
 {
-    k_copy_df<false><<<blocks_for(nval, 256), 256, 0, st>>>(desc, lu, lucsr);
-    if (mode == kSweepLds) k_solve_one<kSweepLds><<<1, threads, lds, st>>>(desc, lucsr, b, x, t32, r0);
+    copy_df(src, nval, lu, lucsr, st);
+    if (mode == kSweepLds && transpose)
+        k_solve_one<kSweepLds, false, true><<<1, threads, lds, st>>>(desc, lucsr, b, x, t32, r0);
+    else if (mode == kSweepLds) k_solve_one<kSweepLds><<<1, threads, lds, st>>>(desc, lucsr, b, x, t32, r0);
     else if (r0 != UINT32_MAX) k_solve_one<kSweepFlags, true><<<1, threads, lds, st>>>(desc, lucsr, b, x, t32, r0);
     else k_solve_one<kSweepFlags><<<1, threads, lds, st>>>(desc, lucsr, b, x, t32, r0);
+}
+
+// The split sweeps of one matrix (SplitDev) over the copy lucsr of its
+// factors lu: the right-hand side is float(in[rsrc[r]] * rscale[r]) by row r
+// of the factors, the result goes to xg by row.  T = float with kExact
+// (glu_solve), double without (glu_refine).
+template <bool kExact, typename T>
+static void split_sweeps_t(const SplitDev &S, const T *in, const float *lu, float *lucsr, float *rhs, float *xg,
+                           hipStream_t st)
+{
+    const unsigned hb = S.parts, ht = (unsigned)(S.head[0].nwave * kWave), tt = (unsigned)(S.tail[0].nwave * kWave);
+    const size_t hl = 4 * ((size_t)S.head_slots + 2), tl = 4 * ((size_t)S.tail_slots + 2);
+    if (hb) k_sw_first<kExact, T><<<hb, ht, hl, st>>>(S.head[0], in, S.rsrc, S.rscale, lucsr, rhs, xg);
+    if (S.tail[0].nprod)
+        k_sw_prod<<<blocks_for(S.tail[0].nprod, 256), 256, 0, st>>>(S.tail[0].prod, S.tail[0].nprod, lu, xg, lucsr);
+    k_sw_tail<kExact, T><<<1, tt, tl, st>>>(S.tail[0], S.tail[1], in, S.rsrc, S.rscale, lucsr, rhs, xg);
+    if (S.head[1].nprod)
+        k_sw_prod<<<blocks_for(S.head[1].nprod, 256), 256, 0, st>>>(S.head[1].prod, S.head[1].nprod, lu, xg, lucsr);
+    if (hb) k_sw_second<kExact><<<hb, ht, hl, st>>>(S.head[1], lucsr, rhs, xg);
+}
+
+void split_solve(const SplitDev &S, const float *b, const float *lu, float *lucsr, float *rhs, float *xg, hipStream_t st)
+{
+    split_sweeps_t<true, float>(S, b, lu, lucsr, rhs, xg, st);
+}
+
+void split_precond(const SplitDev &S, const double *r, const float *lu, float *lucsr, float *rhs, float *xg,
+                   hipStream_t st)
+{
+    split_sweeps_t<false, double>(S, r, lu, lucsr, rhs, xg, st);
 }
 
 void abft_cca(const FactorDev &F, const float *val, float *cca, int batch, hipStream_t st)
@@ -3423,6 +3577,13 @@ size_t enable_lds()
         reinterpret_cast<const void *>(&k_batch_same_factor<false>),
         reinterpret_cast<const void *>(&k_batch_factor),
         reinterpret_cast<const void *>(&k_solve_one<kSweepLds>),
+        reinterpret_cast<const void *>(&k_solve_one<kSweepLds, false, true>),
+        reinterpret_cast<const void *>(&k_sw_first<true, float>),
+        reinterpret_cast<const void *>(&k_sw_first<false, double>),
+        reinterpret_cast<const void *>(&k_sw_tail<true, float>),
+        reinterpret_cast<const void *>(&k_sw_tail<false, double>),
+        reinterpret_cast<const void *>(&k_sw_second<true>),
+        reinterpret_cast<const void *>(&k_sw_second<false>),
         reinterpret_cast<const void *>(&k_solve_one<kSweepFlags>),
         reinterpret_cast<const void *>(&k_refine_one<kSweepLds, false>),
         reinterpret_cast<const void *>(&k_refine_one<kSweepLds, true>),

@@ -73,12 +73,15 @@ size_t enable_lds();
 void factor_window(const FactorDev &F, int w, uint32_t nslot, float *val, const float *d_pert, int perturb,
                    int threads, hipStream_t st);
 void zero_u64(unsigned long long *p, int count, hipStream_t st);
-void solve_one(const MatDesc *desc, uint32_t nval, const float *lu, float *lucsr, const float *b, float *x,
-               float *t32, uint32_t r0, int threads, int mode, size_t lds, hipStream_t st);
-void refine_one(const MatDesc *desc, uint32_t nval, const double *ax, const double *b, double *x,
+void solve_one(const MatDesc *desc, const uint32_t *src, uint32_t nval, const float *lu, float *lucsr, const float *b,
+               float *x, float *t32, uint32_t r0, int threads, int mode, size_t lds, int transpose, hipStream_t st);
+void split_solve(const SplitDev &S, const float *b, const float *lu, float *lucsr, float *rhs, float *xg, hipStream_t st);
+void split_precond(const SplitDev &S, const double *r, const float *lu, float *lucsr, float *rhs, float *xg,
+                   hipStream_t st);
+void refine_one(const MatDesc *desc, const uint32_t *src, uint32_t nval, const double *ax, const double *b, double *x,
                 const float *lu, float *lucsr, float *t32, double *r64, double *norms, double *kry, int32_t *iters,
                 double *eta, double tol, int maxit, int threads, size_t ref_lds, int transpose, hipStream_t st);
-void copy_df(const MatDesc *desc, uint32_t nval, const float *lu, float *lucsr, int transpose, hipStream_t st);
+void copy_df(const uint32_t *src, uint32_t nval, const float *lu, float *lucsr, hipStream_t st);
 void sweeps_df(const MatDesc *desc, const float *lucsr, float *t32, uint32_t r0, int threads, size_t lds,
                int transpose, hipStream_t st);
 void adjoint_values(const RefineDev &R, const double *lam, const double *x, double *grad, uint32_t n,
@@ -323,6 +326,16 @@ struct glu_plan {
     uint32_t df_nval = 0;        // values of the per-matrix sweep copy
     uint32_t tdf_nval = 0;       // the same for A' x = b
     float *d_tlucsr = nullptr;   // glu_refine's A' x = b value copy
+    uint32_t t32_len = 0;        // floats of a matrix's sweep scratch (SolveDev::t32_len)
+    uint64_t scratch_nval[2] = {0, 0};   // value copies the scratch limit of glu_refine_noalloc counts (A, A')
+    // one matrix's sweeps outside the batch kernels (A, A'): value copy,
+    // right-hand sides, vector by row; allocated on first use, never moved
+    struct Single {
+        float *buf = nullptr, *lucsr = nullptr, *rhs = nullptr, *xg = nullptr;
+    } single[2];
+    bool has_split = false;      // vector beyond LDS: split sweeps (split[0]: A, [1]: A')
+    SplitDev split[2] = {};
+    uint32_t split_rhs = 0;      // floats of their right-hand sides
     // LDS windows allowed (from the last level); windows hold narrow steps
     // only, so small orders get one whatever the cap, and n=500k MNA gains
     // up to ~16 (refactor 14.3 -> 12.4 ms; no change beyond)
@@ -394,6 +407,8 @@ struct glu_plan {
         if (d_bkry) (void)hipFree(d_bkry);
         if (d_rout) (void)hipFree(d_rout);
         if (d_tlucsr) (void)hipFree(d_tlucsr);
+        for (Single &q : single)
+            if (q.buf) (void)hipFree(q.buf);
         if (d_abft) (void)hipFree(d_abft);
         if (d_bnorms) (void)hipFree(d_bnorms);
         if (d_fnorms) (void)hipFree(d_fnorms);
@@ -1414,6 +1429,410 @@ bool check_df(const DfHost &D, uint32_t n, uint32_t nnz, const char *name, std::
     return true;
 }
 
+// A sweep's streams (SwDev), from the dataflow table of the same sweep: its
+// rows in schedule order, each row's entries, and whether the refinement sums
+// the row's products (the rows that table gives a group of lanes).
+struct SwHost {
+    std::vector<uint4> meta;           // [64 chunks]
+    std::vector<uint32_t> hdr, wptr, row, rpos, vsrc;   // vsrc: CSC position of each value (~0: 0)
+    std::vector<SwPart> part;
+    std::vector<SwProd> prod;          // value index within this sweep
+    uint32_t nwave = 0, stride = 256, nslot_max = 0;
+};
+
+// Rows of parts: part_of[r] (UINT32_MAX: not in this sweep), slot_of[r] and
+// the part's row count.
+struct SwParts {
+    std::vector<uint32_t> part_of, slot_of, count;
+};
+
+constexpr uint32_t kSwEntries = 256;   // values of a chunk
+
+// Lanes a row of len entries takes, four entries a lane (a summed row: at
+// least the 16 entries whose sum is a fixed tree; 65 and more summed entries:
+// chunks of its own).
+inline uint32_t sw_lanes(uint32_t len, bool sum = false)
+{
+    uint32_t g = sum ? 4 : 1;
+    while (4 * g < len) g *= 2;
+    return g;
+}
+
+// A chunk that starts in a level of at most a chunk's lanes goes to one of a
+// few waves (one per SIMD): there the sweep is a chain, and more waves only
+// wait beside it (n=200,003: 6,434 us a factor and solve with all 16, 6,161
+// with 4, 6,605 with 1).
+constexpr uint32_t kSwNarrowLanes = 64, kSwNarrowWaves = 4;
+
+// Chunks go to the part's waves in turn, in schedule order; the rows of
+// several chunks, which take their time but can start early, to waves of
+// their own (each wave runs its chunks in order, and every dependency lies in
+// an earlier chunk of the schedule or an earlier lane of the same one, so the
+// first unfinished chunk can always finish: check_sw).
+void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwParts &Q, uint32_t waves, SwHost &S)
+{
+    const uint32_t nparts = (uint32_t)Q.count.size();
+    S.nwave = waves;
+    S.stride = kSwEntries + (div ? 64 : 0);
+    // by position: first entry's place in D, the step to the next, level, sum?
+    struct Pos {
+        uint32_t row, len, base, step, level, pivot;
+        bool sum;
+    };
+    std::vector<std::vector<Pos>> rows(nparts);
+    {
+        std::vector<uint32_t> base(n), step(n);
+        std::vector<uint8_t> sum(n);
+        for (const uint4 &d : D.task) {
+            const bool wave = (d.z & kLongTask) != 0;
+            const uint32_t lg = (d.z >> 24) & 0x7fu, cnt = d.z & 0xffffffu;
+            for (uint32_t k = 0; k < cnt; ++k) {
+                base[d.y + k] = d.x + (wave ? k << lg : k);
+                step[d.y + k] = wave ? 1 : 64;
+                sum[d.y + k] = wave;
+            }
+        }
+        uint32_t level = 0;
+        for (uint32_t p = 0; p < n; ++p) {
+            while (p >= H.lvl_ptr[level + 1]) ++level;
+            const uint32_t r = D.rl[p].x;
+            if (Q.part_of[r] != UINT32_MAX)
+                rows[Q.part_of[r]].push_back(
+                    Pos{r, D.rl[p].y, base[p], step[p], level, div ? D.pvpos[p] : 0u, sum[p] != 0});
+        }
+    }
+    for (uint32_t part = 0; part < nparts; ++part) {
+        std::vector<Pos> &R = rows[part];
+        const uint32_t nslot = Q.count[part], zero = nslot, one = nslot + 1;
+        S.nslot_max = std::max(S.nslot_max, nslot);
+        SwPart P{(uint32_t)S.wptr.size(), (uint32_t)S.row.size(), nslot, 0};
+        S.row.resize(P.s0 + nslot);
+        S.rpos.resize(P.s0 + nslot);
+        auto is_long = [](const Pos &x) { return x.sum && x.len > 64; };
+        // the part's chunks in schedule order
+        std::vector<uint4> meta;
+        std::vector<uint32_t> hdr, vsrc, wave, rpos(nslot);
+        struct Prod {
+            uint32_t chunk, at, vpos, col;
+        };
+        std::vector<Prod> prod;
+        auto add = [&](uint32_t h) {
+            hdr.push_back(h);
+            meta.resize(meta.size() + 64, make_uint4(zero | zero << 16, zero | zero << 16, 0u, 0u));
+            vsrc.resize(vsrc.size() + S.stride, UINT32_MAX);
+        };
+        auto put = [&](uint32_t lane, uint32_t e, const Pos &x, uint32_t k) {   // entry k of row x
+            const size_t c = hdr.size() - 1, q = x.base + (size_t)k * x.step;
+            const uint32_t col = D.idx[q], vp = D.vpos[q];
+            uint32_t slot;
+            if (Q.part_of[col] == part) {
+                slot = Q.slot_of[col];
+                vsrc[c * S.stride + 4 * lane + e] = vp;
+            } else {
+                slot = one;
+                prod.push_back(Prod{(uint32_t)c, 4 * lane + e, vp, col});
+            }
+            uint4 &m = meta[64 * c + lane];
+            uint32_t &w = e < 2 ? m.x : m.y;
+            w = (e & 1) ? (w & 0xffffu) | slot << 16 : (w & 0xffff0000u) | slot;
+        };
+        size_t multi = 0;
+        for (const Pos &x : R) multi += is_long(x) && x.len > kSwEntries;
+        const uint32_t own = waves >= 4 ? (uint32_t)std::min<size_t>(multi, std::max(1u, waves * 3 / 8)) : 0u;
+        std::vector<uint32_t> lanes_at(R.empty() ? 0 : R.back().level + 1, 0);   // lanes of each level
+        for (const Pos &x : R) lanes_at[x.level] += is_long(x) ? 0 : sw_lanes(x.len, x.sum);
+        uint32_t turn = 0, turn_long = 0, used = 64;
+        for (size_t i = 0; i < R.size();) {
+            size_t e = i;
+            while (e < R.size() && R[e].level == R[i].level) ++e;
+            // a level's rows are independent: long ones first, then by lanes,
+            // down on even levels and up on odd ones (alignment costs least)
+            const bool up = R[i].level & 1u;
+            std::stable_sort(R.begin() + i, R.begin() + e, [&](const Pos &x, const Pos &y) {
+                const bool lx = is_long(x), ly = is_long(y);
+                if (lx != ly) return lx;
+                if (lx) return false;
+                const uint32_t a = 2 * sw_lanes(x.len, x.sum) + x.sum, b = 2 * sw_lanes(y.len, y.sum) + y.sum;
+                return up ? a < b : a > b;
+            });
+            for (; i < e; ++i) {
+                const Pos &x = R[i];
+                const uint32_t slot = Q.slot_of[x.row];
+                S.row[P.s0 + slot] = x.row;
+                if (is_long(x)) {
+                    used = 64;   // (what is open may hold this row's dependencies: it stays before)
+                    const uint32_t nc = (x.len + kSwEntries - 1) / kSwEntries;
+                    const uint32_t to = nc > 1 && own ? turn_long++ % own : own + turn++ % (waves - own);
+                    for (uint32_t c = 0; c < nc; ++c) {
+                        const uint32_t left = std::min(x.len - c * kSwEntries, kSwEntries);
+                        add(kSwLong | (c == 0 ? kSwFirst : 0u) | (c + 1 == nc ? kSwLast : 0u) | ((left + 63) / 64 - 1));
+                        wave.push_back(to);
+                        for (uint32_t k = 0; k < left; ++k) {
+                            put(k % 64, k / 64, x, c * kSwEntries + k);
+                            meta[64 * (hdr.size() - 1) + k % 64].w |= 1u << (k / 64);
+                        }
+                        for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (hdr.size() - 1) + lane].z = slot;
+                        if (c == 0) rpos[slot] = 64 * (uint32_t)(hdr.size() - 1);
+                        if (c + 1 == nc && div) vsrc[(hdr.size() - 1) * S.stride + kSwEntries] = x.pivot;
+                    }
+                    continue;
+                }
+                const uint32_t g = sw_lanes(x.len, x.sum);
+                used = (used + g - 1) & ~(g - 1);
+                if (used + g > 64) {
+                    const bool few = lanes_at[x.level] <= kSwNarrowLanes;
+                    add(few ? kSwNarrow : 0u);
+                    wave.push_back(own + turn++ % (few ? std::min(kSwNarrowWaves, waves - own) : waves - own));
+                    used = 0;
+                }
+                const size_t c = hdr.size() - 1;
+                hdr[c] |= x.sum ? kSwHasTree : kSwHasSeq;
+                for (uint32_t lane = 0; lane < g; ++lane)
+                    meta[64 * c + used + lane].z = slot | (uint32_t)__builtin_ctz(g) << 16 | (x.sum ? kSwTree : 0u) | kSwOn;
+                for (uint32_t k = 0; k < x.len; ++k) put(used + k / 4, k % 4, x, k);
+                rpos[slot] = 64 * (uint32_t)c + used;
+                if (div)   // at the lane that stores the row: the last; a summed row's first too
+                    for (uint32_t lane : {used + g - 1, x.sum ? used : used + g - 1})
+                        vsrc[c * S.stride + kSwEntries + lane] = x.pivot;
+                used += g;
+            }
+        }
+        // stream by stream
+        std::vector<uint32_t> at(hdr.size());
+        for (uint32_t w = 0; w < waves; ++w) {
+            S.wptr.push_back((uint32_t)S.hdr.size());
+            for (size_t c = 0; c < hdr.size(); ++c) {
+                if (wave[c] != w) continue;
+                at[c] = (uint32_t)S.hdr.size();
+                S.hdr.push_back(hdr[c]);
+                S.meta.insert(S.meta.end(), meta.begin() + 64 * c, meta.begin() + 64 * (c + 1));
+                S.vsrc.insert(S.vsrc.end(), vsrc.begin() + c * S.stride, vsrc.begin() + (c + 1) * S.stride);
+            }
+        }
+        S.wptr.push_back((uint32_t)S.hdr.size());
+        for (uint32_t k = 0; k < nslot; ++k) S.rpos[P.s0 + k] = 64 * at[rpos[k] / 64] + rpos[k] % 64;
+        for (const Prod &q : prod) S.prod.push_back(SwProd{at[q.chunk] * S.stride + q.at, q.vpos, q.col});
+        S.part.push_back(P);
+    }
+}
+
+// Host check of a sweep's streams before any launch: every slot and value
+// position in range, every right-hand side at its row's first lane, every row
+// of a part stored once; and, running each part's streams side by side (a
+// wave moves on once its chunk's rows are done, a row is done once its
+// entries are set), every wave gets to its end: every wait of the sweep ends.
+bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
+{
+    auto bad = [&](const std::string &what) {
+        err = std::string(name) + " sweep streams: " + what;
+        return false;
+    };
+    const uint32_t nchunk = (uint32_t)S.hdr.size();
+    if (S.meta.size() != 64 * (size_t)nchunk || S.vsrc.size() != (size_t)S.stride * nchunk) return bad("sizes");
+    for (uint32_t v : S.vsrc)
+        if (v != UINT32_MAX && v >= nnz) return bad("value position out of range");
+    for (const SwProd &q : S.prod)
+        if (q.val >= S.vsrc.size() || q.vpos >= nnz) return bad("product out of range");
+    for (const SwPart &P : S.part) {
+        if ((size_t)P.wp + S.nwave >= S.wptr.size() || (size_t)P.s0 + P.nslot > S.row.size() || P.nslot > 0xfffdu)
+            return bad("part out of range");
+        std::vector<uint8_t> set(P.nslot + 2, 0);
+        set[P.nslot] = set[P.nslot + 1] = 1;
+        std::vector<uint32_t> at(S.nwave);
+        for (uint32_t w = 0; w < S.nwave; ++w) {
+            at[w] = S.wptr[P.wp + w];
+            if (at[w] > S.wptr[P.wp + w + 1] || S.wptr[P.wp + w + 1] > nchunk) return bad("stream out of range");
+        }
+        uint32_t done = 0;
+        for (bool moved = true; moved;) {
+            moved = false;
+            for (uint32_t w = 0; w < S.nwave; ++w)
+                for (; at[w] < S.wptr[P.wp + w + 1]; ++at[w]) {
+                    const uint32_t c = at[w], h = S.hdr[c];
+                    auto entry = [&](uint32_t lane, uint32_t e) {
+                        const uint4 &m = S.meta[64 * (size_t)c + lane];
+                        const uint32_t v = e < 2 ? m.x : m.y;
+                        return (e & 1) ? v >> 16 : v & 0xffffu;
+                    };
+                    bool whole = true;
+                    if (h & kSwLong) {
+                        for (uint32_t lane = 0; lane < 64; ++lane)
+                            for (uint32_t e = 0; e < 4; ++e) {
+                                if (entry(lane, e) > P.nslot + 1) return bad("slot out of range");
+                                whole = whole && set[entry(lane, e)];
+                            }
+                        const uint32_t slot = S.meta[64 * (size_t)c].z;
+                        if (slot >= P.nslot) return bad("row slot out of range");
+                        if (whole && (h & kSwFirst) && S.rpos[P.s0 + slot] != 64 * c) return bad("right-hand side misplaced");
+                        if (whole && (h & kSwLast)) {
+                            if (set[slot]) return bad("a row runs twice");
+                            set[slot] = 1, ++done;
+                        }
+                    } else {
+                        for (uint32_t lane = 0; lane < 64;) {
+                            const uint32_t z = S.meta[64 * (size_t)c + lane].z, slot = z & 0xffffu, g = 1u << ((z >> 16) & 7u);
+                            if (lane % g || lane + g > 64 || g > 16) return bad("row lanes out of place");
+                            bool rdy = true;
+                            for (uint32_t k = 0; k < g; ++k)
+                                for (uint32_t e = 0; e < 4; ++e) {
+                                    if (entry(lane + k, e) > P.nslot + 1) return bad("slot out of range");
+                                    rdy = rdy && set[entry(lane + k, e)];
+                                }
+                            if (z & kSwOn) {
+                                if (slot >= P.nslot) return bad("row slot out of range");
+                                if (S.rpos[P.s0 + slot] != 64 * c + lane) return bad("right-hand side misplaced");
+                                if (rdy && !set[slot]) set[slot] = 1, ++done, moved = true;
+                                whole = whole && set[slot];
+                            }
+                            lane += g;
+                        }
+                    }
+                    if (!whole) break;
+                    moved = true;
+                }
+        }
+        for (uint32_t w = 0; w < S.nwave; ++w)
+            if (at[w] != S.wptr[P.wp + w + 1]) return bad("a row waits for one that never runs");
+        if (done != P.nslot) return bad("a row never runs");
+    }
+    return true;
+}
+
+// The split of an order whose vector does not fit in LDS.  A row's height is
+// the longest chain of rows (entries of L or of U, either way) below it; the
+// rows of height h and more are closed under the dependencies of the U
+// sweeps, the others under those of the L sweeps, and fall into components
+// that share no entry.  Of the heights tried, the one with the least
+// estimated time: the tail's chunks on one workgroup and its chain, and the
+// largest head part's.  Components go to parts largest first, each to the
+// part with the least so far.
+struct SwSplit {
+    SwParts head, tail;
+};
+
+constexpr uint32_t kHeadWaves = 8;
+constexpr uint32_t kHeadParts = 512;    // two workgroups a CU
+constexpr uint32_t kHeadSlots = 16384;  // 64 KB of LDS
+
+bool choose_split(const glu_pattern &P, uint32_t cap_slots, uint32_t tail_waves, SwSplit &S)
+{
+    const uint32_t n = P.n;
+    std::vector<uint32_t> ht(n, 0), wgt(n);
+    uint32_t top = 0;
+    for (uint32_t r = 0; r < n; ++r) {
+        uint32_t h = 0;
+        for (uint32_t q = P.csr_r_ptr[r]; q < P.csr_diag_ptr[r]; ++q) h = std::max(h, ht[P.csr_c_idx[q]] + 1);
+        for (uint32_t q = P.sym_c_ptr[r]; q < P.l_col_ptr[r]; ++q) h = std::max(h, ht[P.sym_r_idx[q]] + 1);
+        ht[r] = h;
+        top = std::max(top, h);
+        // lanes of both sweeps
+        const uint32_t l = P.csr_diag_ptr[r] - P.csr_r_ptr[r], u = P.csr_r_ptr[r + 1] - P.csr_diag_ptr[r] - 1;
+        wgt[r] = (l > 64 ? l / 4 + 64 : sw_lanes(l)) + (u > 64 ? u / 4 + 64 : sw_lanes(u));
+    }
+    // components grow with h: one union-find over increasing heights
+    std::vector<uint32_t> parent(n), rows_at(top + 2, 0), by_h(n);
+    for (uint32_t r = 0; r < n; ++r) parent[r] = r, ++rows_at[ht[r] + 1];
+    for (uint32_t h = 0; h <= top; ++h) rows_at[h + 1] += rows_at[h];
+    {
+        std::vector<uint32_t> cur(rows_at.begin(), rows_at.end() - 1);
+        for (uint32_t r = 0; r < n; ++r) by_h[cur[ht[r]]++] = r;
+    }
+    std::vector<uint64_t> cw(wgt.begin(), wgt.end());
+    std::vector<uint32_t> cn(n, 1);
+    auto find = [&](uint32_t r) {
+        while (parent[r] != r) r = parent[r] = parent[parent[r]];
+        return r;
+    };
+    auto join = [&](uint32_t a, uint32_t b) {
+        a = find(a), b = find(b);
+        if (a == b) return a;
+        if (cn[a] < cn[b]) std::swap(a, b);
+        parent[b] = a;
+        cw[a] += cw[b];
+        cn[a] += cn[b];
+        return a;
+    };
+    uint64_t total = 0, head_w = 0, max_w = 0;
+    uint32_t max_n = 0, best_h = 0;
+    for (uint32_t r = 0; r < n; ++r) total += wgt[r];
+    double best = 0.0;
+    std::vector<uint32_t> best_parent;
+    constexpr double kChunk = 0.25, kHop = 0.2;   // us: a chunk of one wave, a hop of the chain
+    uint32_t next_try = 4;
+    for (uint32_t h = 1; h <= std::min(top, 512u); ++h) {   // rows of height < h in the head
+        for (uint32_t k = rows_at[h - 1]; k < rows_at[h]; ++k) {
+            const uint32_t r = by_h[k];
+            head_w += wgt[r];
+            uint32_t c = find(r);
+            for (uint32_t q = P.csr_r_ptr[r]; q < P.csr_diag_ptr[r]; ++q) c = join(c, P.csr_c_idx[q]);
+            for (uint32_t q = P.sym_c_ptr[r]; q < P.l_col_ptr[r]; ++q) c = join(c, P.sym_r_idx[q]);
+            max_w = std::max(max_w, cw[c]);
+            max_n = std::max(max_n, cn[c]);
+        }
+        if (h < next_try) continue;
+        next_try = h + std::max(1u, h / 4);
+        if (max_n > kHeadSlots) break;
+        const uint32_t tail = n - rows_at[h];
+        if (tail > cap_slots) continue;
+        const double head_chunks = std::max((double)max_w, (double)head_w / kHeadParts) / 64.0;
+        const double t = (double)(total - head_w) / 64.0 / tail_waves * kChunk + 2.0 * (top + 1 - h) * kHop +
+                         head_chunks / kHeadWaves * kChunk + 2.0 * h * kHop;
+        if (best_h == 0 || t < best) {
+            best = t;
+            best_h = h;
+            best_parent = parent;
+        }
+    }
+    if (best_h == 0) return false;
+    parent.swap(best_parent);
+    S.head.part_of.assign(n, UINT32_MAX);
+    S.head.slot_of.assign(n, 0);
+    S.tail.part_of.assign(n, UINT32_MAX);
+    S.tail.slot_of.assign(n, 0);
+    S.tail.count.assign(1, 0);
+    std::vector<uint32_t> comp(n, UINT32_MAX);
+    std::vector<uint64_t> weight;
+    std::vector<uint32_t> size;
+    for (uint32_t r = 0; r < n; ++r) {
+        if (ht[r] >= best_h) {
+            S.tail.part_of[r] = 0;
+            S.tail.slot_of[r] = S.tail.count[0]++;
+            continue;
+        }
+        const uint32_t c = find(r);
+        if (comp[c] == UINT32_MAX) {
+            comp[c] = (uint32_t)weight.size();
+            weight.push_back(0);
+            size.push_back(0);
+        }
+        weight[comp[c]] += wgt[r];
+        ++size[comp[c]];
+    }
+    std::vector<uint32_t> order(weight.size()), part(weight.size());
+    for (uint32_t c = 0; c < order.size(); ++c) order[c] = c;
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return weight[a] > weight[b]; });
+    const uint32_t nparts = (uint32_t)std::min<size_t>({weight.size(), kHeadParts, (size_t)(total / 1024 + 1)});
+    std::vector<uint64_t> load(nparts, 0);
+    std::vector<uint32_t> rows(nparts, 0);
+    for (uint32_t c : order) {
+        uint32_t to = UINT32_MAX;
+        for (uint32_t k = 0; k < nparts; ++k)
+            if (rows[k] + size[c] <= kHeadSlots && (to == UINT32_MAX || load[k] < load[to])) to = k;
+        if (to == UINT32_MAX) return false;
+        load[to] += weight[c];
+        rows[to] += size[c];
+        part[c] = to;
+    }
+    S.head.count.assign(nparts, 0);
+    for (uint32_t r = 0; r < n; ++r)
+        if (ht[r] < best_h) {
+            const uint32_t k = part[comp[find(r)]];
+            S.head.part_of[r] = k;
+            S.head.slot_of[r] = S.head.count[k]++;
+        }
+    return true;
+}
+
 struct Uploader {
     Arena arena;
     struct Item {
@@ -1487,8 +1906,102 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     uint32_t budget = std::min<uint32_t>((uint32_t)(p->lds_cap / sizeof(float)), 0xffffu);
     budget -= std::min(budget, kWinExtra);
     if (p->win_values) budget = std::min(budget, p->win_values);
-    choose_windows(T, P.num_lev, P.nnz, budget, (uint32_t)p->fuse_units, p->max_windows,
-                   (uint32_t)p->fused_threads / 64, wins);
+    // Built side by side on host threads: the windows, the four triangular
+    // sweeps (L, U; U', L' for A' x = b: rows of U' are columns of U with the
+    // pivot last, forward; rows of L' columns of L, backward: schedules,
+    // dataflow tables and, when the sweep vector fits in LDS, their streams),
+    // and, when it does not (then long lane rows in wide levels), the split.
+    const uint32_t n = P.n;
+    const bool long_lanes = launch::batch_lds_bytes(2, n) > p->lds_cap;
+    const uint32_t wg_waves = (uint32_t)p->fused_threads / 64;
+    DfHost dlo, dup, dtu, dtl;
+    DfHost *const dfs[4] = {&dlo, &dup, &dtu, &dtl};
+    const bool divs[4] = {false, true, true, false};
+    const char *const names[4] = {"L", "U", "U'", "L'"};
+    std::string errs[4];
+    bool good[4] = {false, false, false, false}, split = false;
+    SwSplit spl;
+    SwHost sw[4], hd[4];   // streams of the whole order, or of the tail; of the head parts
+    if (!long_lanes) {
+        spl.tail.part_of.assign(n, 0);
+        spl.tail.count.assign(1, n);
+        spl.tail.slot_of.resize(n);
+        for (uint32_t r = 0; r < n; ++r) spl.tail.slot_of[r] = r;
+    }
+    const auto sweep_tables = [&](int q) {
+        TriHost &H = p->tri[q];
+        const auto finish = [&](auto entries, auto pivot) {
+            tri_segments(*p, H);
+            tri_tasks(H);
+            build_df(H, entries, divs[q], pivot, long_lanes, *dfs[q]);
+            if (long_lanes) {
+                good[q] = check_df(*dfs[q], n, P.nnz, names[q], errs[q]);
+            } else {
+                build_sw(H, *dfs[q], n, divs[q], spl.tail, wg_waves, sw[q]);
+                good[q] = check_sw(sw[q], P.nnz, names[q], errs[q]);
+            }
+        };
+        const auto no_pivot = [](uint32_t) { return 0u; };
+        const auto diag = [&](uint32_t r) { return P.l_col_ptr[r]; };
+        switch (q) {
+        case 0:
+            tri_levels(n, +1, [&](uint32_t r, auto f) {
+                for (uint32_t k = P.csr_r_ptr[r]; k < P.csr_diag_ptr[r]; ++k) f(P.csr_c_idx[k]);
+            }, [&](uint32_t r) { return P.csr_diag_ptr[r] - P.csr_r_ptr[r]; }, H);
+            finish([&](uint32_t r, std::vector<uint2> &out) {
+                for (uint32_t k = P.csr_r_ptr[r]; k < P.csr_diag_ptr[r]; ++k)
+                    out.push_back(make_uint2(P.csr_c_idx[k], T.upos[k]));
+            }, no_pivot);
+            break;
+        case 1:
+            tri_levels(n, -1, [&](uint32_t r, auto f) {
+                for (uint32_t k = P.csr_diag_ptr[r] + 1; k < P.csr_r_ptr[r + 1]; ++k) f(P.csr_c_idx[k]);
+            }, [&](uint32_t r) { return P.csr_r_ptr[r + 1] - P.csr_diag_ptr[r] - 1; }, H);
+            finish([&](uint32_t r, std::vector<uint2> &out) {
+                for (uint32_t k = P.csr_r_ptr[r + 1]; k > P.csr_diag_ptr[r] + 1; --k)
+                    out.push_back(make_uint2(P.csr_c_idx[k - 1], T.upos[k - 1]));
+            }, diag);
+            break;
+        case 2:
+            tri_levels(n, +1, [&](uint32_t r, auto f) {
+                for (uint32_t k = P.sym_c_ptr[r]; k < P.l_col_ptr[r]; ++k) f(P.sym_r_idx[k]);
+            }, [&](uint32_t r) { return P.l_col_ptr[r] - P.sym_c_ptr[r]; }, H);
+            finish([&](uint32_t r, std::vector<uint2> &out) {
+                for (uint32_t k = P.sym_c_ptr[r]; k < P.l_col_ptr[r]; ++k) out.push_back(make_uint2(P.sym_r_idx[k], k));
+            }, diag);
+            break;
+        default:
+            tri_levels(n, -1, [&](uint32_t r, auto f) {
+                for (uint32_t k = P.l_col_ptr[r] + 1; k < P.sym_c_ptr[r + 1]; ++k) f(P.sym_r_idx[k]);
+            }, [&](uint32_t r) { return P.sym_c_ptr[r + 1] - P.l_col_ptr[r] - 1; }, H);
+            finish([&](uint32_t r, std::vector<uint2> &out) {
+                for (uint32_t k = P.sym_c_ptr[r + 1]; k > P.l_col_ptr[r] + 1; --k)
+                    out.push_back(make_uint2(P.sym_r_idx[k - 1], k - 1));
+            }, no_pivot);
+        }
+    };
+    parallel_items(long_lanes ? 6 : 5, table_threads(), [&](unsigned, size_t item) {
+        if (item == 0)
+            choose_windows(T, P.num_lev, P.nnz, budget, (uint32_t)p->fuse_units, p->max_windows, wg_waves, wins);
+        else if (item < 5)
+            sweep_tables((int)item - 1);
+        else
+            split = choose_split(P, (uint32_t)std::min<size_t>(p->lds_cap / sizeof(float), 0xffffu) - 2, wg_waves, spl);
+    });
+    for (int q = 0; q < 4; ++q)
+        if (!good[q]) return fail(GLU_ERR_INVALID, errs[q]);
+    if (split) {
+        std::string werr[8];
+        bool wgood[8] = {};
+        parallel_items(8, table_threads(), [&](unsigned, size_t item) {
+            const size_t q = item % 4;
+            SwHost &h = item < 4 ? hd[q] : sw[q];
+            build_sw(p->tri[q], *dfs[q], n, divs[q], item < 4 ? spl.head : spl.tail, item < 4 ? kHeadWaves : wg_waves, h);
+            wgood[item] = check_sw(h, P.nnz, names[q], werr[item]);
+        });
+        for (int i = 0; i < 8; ++i)
+            if (!wgood[i]) return fail(GLU_ERR_INVALID, werr[i]);
+    }
     p->nwin = (int)wins.size();
     for (const Window &w : wins) {
         p->win_steps += w.l1 - w.l0;
@@ -1527,85 +2040,43 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         std::sort(T.dvd.begin() + T.dvd_ptr[early], T.dvd.end(), by_pos);
     }
 
-    const uint32_t n = P.n;
-    // Solve schedules.
-    tri_levels(n, +1, [&](uint32_t r, auto f) {
-        for (uint32_t q = P.csr_r_ptr[r]; q < P.csr_diag_ptr[r]; ++q) f(P.csr_c_idx[q]);
-    }, [&](uint32_t r) { return P.csr_diag_ptr[r] - P.csr_r_ptr[r]; }, p->tri[0]);
-    tri_levels(n, -1, [&](uint32_t r, auto f) {
-        for (uint32_t q = P.csr_diag_ptr[r] + 1; q < P.csr_r_ptr[r + 1]; ++q) f(P.csr_c_idx[q]);
-    }, [&](uint32_t r) { return P.csr_r_ptr[r + 1] - P.csr_diag_ptr[r] - 1; }, p->tri[1]);
-    tri_levels(n, +1, [&](uint32_t r, auto f) {
-        for (uint32_t q = P.sym_c_ptr[r]; q < P.l_col_ptr[r]; ++q) f(P.sym_r_idx[q]);
-    }, [&](uint32_t r) { return P.l_col_ptr[r] - P.sym_c_ptr[r]; }, p->tri[2]);
-    tri_levels(n, -1, [&](uint32_t r, auto f) {
-        for (uint32_t q = P.l_col_ptr[r] + 1; q < P.sym_c_ptr[r + 1]; ++q) f(P.sym_r_idx[q]);
-    }, [&](uint32_t r) { return P.sym_c_ptr[r + 1] - P.l_col_ptr[r] - 1; }, p->tri[3]);
-    for (auto &h : p->tri) {
-        tri_segments(*p, h);
-        tri_tasks(h);
+    p->scratch_nval[0] = dlo.idx.size() + dup.idx.size() + n + 64;
+    p->scratch_nval[1] = dtu.idx.size() + dtl.idx.size() + n + 64;
+    uint32_t sw_rhs = 0;
+    for (const SwHost *h : {&sw[0], &sw[1], &sw[2], &sw[3], &hd[0], &hd[1], &hd[2], &hd[3]})
+        sw_rhs = std::max(sw_rhs, 64 * (uint32_t)h->hdr.size());
+    p->t32_len = long_lanes ? n : std::max(n, sw_rhs);
+    // the value copies (CSC position of each value, ~0 for places without
+    // one, which get 0) of A x = b and A' x = b; with the vector beyond LDS,
+    // those of the dataflow tables (slots, then the pivots), and the split
+    // sweeps' own beside them
+    std::vector<uint32_t> df_vpos, tdf_vpos, spl_vpos[2];
+    uint32_t sw_voff[4] = {0, 0, 0, 0}, hd_voff[4] = {0, 0, 0, 0}, tlo_voff = 0;
+    auto append = [](std::vector<uint32_t> &to, const SwHost &h) {
+        const uint32_t at = (uint32_t)to.size();
+        to.insert(to.end(), h.vsrc.begin(), h.vsrc.end());
+        return at;
+    };
+    if (!long_lanes) {
+        for (int q = 0; q < 4; ++q) sw_voff[q] = append(q < 2 ? df_vpos : tdf_vpos, sw[q]);
+    } else {
+        df_vpos = dlo.vpos;
+        df_vpos.insert(df_vpos.end(), dup.vpos.begin(), dup.vpos.end());
+        df_vpos.insert(df_vpos.end(), dup.pvpos.begin(), dup.pvpos.end());
+        df_vpos.resize(df_vpos.size() + 64, UINT32_MAX);   // pivot reads of the last positions' lanes
+        tdf_vpos = dtu.vpos;   // U' slots, U' pivots (+64 pad), L' slots
+        tdf_vpos.insert(tdf_vpos.end(), dtu.pvpos.begin(), dtu.pvpos.end());
+        tdf_vpos.resize(tdf_vpos.size() + 64, UINT32_MAX);
+        tlo_voff = (uint32_t)tdf_vpos.size();
+        tdf_vpos.insert(tdf_vpos.end(), dtl.vpos.begin(), dtl.vpos.end());
+        if (split)
+            for (int q = 0; q < 4; ++q) {
+                hd_voff[q] = append(spl_vpos[q / 2], hd[q]);
+                sw_voff[q] = append(spl_vpos[q / 2], sw[q]);
+            }
     }
-    // sweep vector beyond LDS (the richest sweep mode does not fit): long
-    // lane rows in wide levels
-    const bool long_lanes = launch::batch_lds_bytes(2, n) > p->lds_cap;
-    // the four sweeps' dataflow tables (L, U; U', L' for A' x = b: rows of
-    // U' are columns of U with the pivot last, forward; rows of L' columns
-    // of L, backward), built and checked on four host threads
-    DfHost dlo, dup, dtu, dtl;
-    std::string errs[4];
-    bool ok[4] = {false, false, false, false};
-    parallel_items(4, std::min(4u, table_threads()), [&](unsigned, size_t which) {
-        switch (which) {
-        case 0:
-            build_df(p->tri[0], [&](uint32_t r, std::vector<uint2> &out) {
-                for (uint32_t q = P.csr_r_ptr[r]; q < P.csr_diag_ptr[r]; ++q)
-                    out.push_back(make_uint2(P.csr_c_idx[q], T.upos[q]));
-            }, false, [&](uint32_t) { return 0u; }, long_lanes, dlo);
-            ok[0] = check_df(dlo, n, P.nnz, "L", errs[0]);
-            break;
-        case 1:
-            build_df(p->tri[1], [&](uint32_t r, std::vector<uint2> &out) {
-                for (uint32_t q = P.csr_r_ptr[r + 1]; q > P.csr_diag_ptr[r] + 1; --q)
-                    out.push_back(make_uint2(P.csr_c_idx[q - 1], T.upos[q - 1]));
-            }, true, [&](uint32_t r) { return P.l_col_ptr[r]; }, long_lanes, dup);
-            ok[1] = check_df(dup, n, P.nnz, "U", errs[1]);
-            break;
-        case 2:
-            build_df(p->tri[2], [&](uint32_t r, std::vector<uint2> &out) {
-                for (uint32_t q = P.sym_c_ptr[r]; q < P.l_col_ptr[r]; ++q) out.push_back(make_uint2(P.sym_r_idx[q], q));
-            }, true, [&](uint32_t r) { return P.l_col_ptr[r]; }, long_lanes, dtu);
-            ok[2] = check_df(dtu, n, P.nnz, "U'", errs[2]);
-            break;
-        default:
-            build_df(p->tri[3], [&](uint32_t r, std::vector<uint2> &out) {
-                for (uint32_t q = P.sym_c_ptr[r + 1]; q > P.l_col_ptr[r] + 1; --q)
-                    out.push_back(make_uint2(P.sym_r_idx[q - 1], q - 1));
-            }, false, [&](uint32_t) { return 0u; }, long_lanes, dtl);
-            ok[3] = check_df(dtl, n, P.nnz, "L'", errs[3]);
-        }
-    });
-    for (int q = 0; q < 4; ++q)
-        if (!ok[q]) return fail(GLU_ERR_INVALID, errs[q]);
-    // orders whose sweep vector fits in LDS: slots without an entry read the
-    // zero kept at column n (their value is 0)
-    if (!long_lanes)
-        for (DfHost *d : {&dlo, &dup, &dtu, &dtl})
-            for (size_t q = 0; q < d->idx.size(); ++q)
-                if (d->vpos[q] == UINT32_MAX) d->idx[q] = n;
-    // the value copies are gathered in slot order (whole-line stores): the
-    // CSC position of each slot, ~0 for padding slots (which get 0)
-    std::vector<uint32_t> tdf_vpos(dtu.vpos);   // U' slots, U' pivots (+64 pad), L' slots
-    tdf_vpos.insert(tdf_vpos.end(), dtu.pvpos.begin(), dtu.pvpos.end());
-    tdf_vpos.resize(tdf_vpos.size() + 64, UINT32_MAX);
-    const uint32_t tlo_voff = (uint32_t)tdf_vpos.size();
-    tdf_vpos.insert(tdf_vpos.end(), dtl.vpos.begin(), dtl.vpos.end());
-    p->tdf_nval = (uint32_t)tdf_vpos.size();
-    // per-matrix value copy: L slots, U slots, U pivots
-    std::vector<uint32_t> df_vpos(dlo.vpos);
-    df_vpos.insert(df_vpos.end(), dup.vpos.begin(), dup.vpos.end());
-    df_vpos.insert(df_vpos.end(), dup.pvpos.begin(), dup.pvpos.end());
-    df_vpos.resize(df_vpos.size() + 64, UINT32_MAX);   // pivot reads of the last positions' lanes
     p->df_nval = (uint32_t)df_vpos.size();
+    p->tdf_nval = (uint32_t)tdf_vpos.size();
     // The batch kernels build the copy in LDS, copy_range slots at a time:
     // per range, {CSC position, slot - range start} of its non-padding
     // slots in increasing position order (so that the reads sweep the
@@ -1687,15 +2158,15 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         long_first(an->in_ap.data(), a_cols, p->a_nlong_t);
         for (uint32_t i = 0; i < n; ++i)
             p->a_kmax = std::max({p->a_kmax, a_rptr[i + 1] - a_rptr[i], an->in_ap[i + 1] - an->in_ap[i]});
-        // the first sweeps' right-hand sides by position
+        // the first sweeps' right-hand sides by row
         df_rsrc.resize(n);
         df_rscale.resize(n);
         tdf_rsrc.resize(n);
         tdf_rscale.resize(n);
         for (uint32_t q = 0; q < n; ++q) {
-            const uint32_t r = dlo.rl[q].x, t = an->row_perm[dtu.rl[q].x];
-            df_rsrc[q] = an->col_perm[r];
-            df_rscale[q] = an->col_scale_perm[r];
+            const uint32_t t = an->row_perm[q];
+            df_rsrc[q] = an->col_perm[q];
+            df_rscale[q] = an->col_scale_perm[q];
             tdf_rsrc[q] = t;
             tdf_rscale[q] = an->row_scale[t];
         }
@@ -1744,6 +2215,20 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         o_wptr[w] = U.put(wins[w].wptr);
     }
     const size_t o_wdev = U.reserve(sizeof(WinDev) * std::max<size_t>(wins.size(), 1));
+    struct SwOff {
+        size_t meta, hdr, wptr, part, row, rpos, prod;
+    };
+    SwOff o_sw[4], o_hd[4];
+    for (int q = 0; q < 4; ++q)
+        for (int k = 0; k < 2; ++k) {
+            SwHost &h = k ? hd[q] : sw[q];
+            if (h.prod.size())   // product values count from the copy's start
+                for (SwProd &e : h.prod) e.val += k ? hd_voff[q] : sw_voff[q];
+            (k ? o_hd : o_sw)[q] = SwOff{U.put(h.meta), U.put(h.hdr), U.put(h.wptr), U.put(h.part),
+                                         U.put(h.row), U.put(h.rpos), U.put(h.prod)};
+        }
+    const size_t o_spl[2] = {U.put(spl_vpos[0]), U.put(spl_vpos[1])};
+    if (!long_lanes) dlo = dup = dtu = dtl = DfHost();   // (not uploaded: the streams replace them)
     const size_t o_dlo_task = U.put(dlo.task), o_dlo_rl = U.put(dlo.rl), o_dlo_idx = U.put(dlo.idx);
     const size_t o_dup_task = U.put(dup.task), o_dup_rl = U.put(dup.rl), o_dup_idx = U.put(dup.idx);
     const size_t o_dtu_task = U.put(dtu.task), o_dtu_rl = U.put(dtu.rl), o_dtu_idx = U.put(dtu.idx);
@@ -1883,6 +2368,40 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         d.voff = voff;
         return d;
     };
+    auto swd = [&](const SwHost &h, const SwOff &o, bool div, uint32_t voff) {
+        SwDev d{};
+        d.meta = reinterpret_cast<const uint4 *>(A + o.meta);
+        d.hdr = u32p(o.hdr);
+        d.wptr = u32p(o.wptr);
+        d.part = reinterpret_cast<const SwPart *>(A + o.part);
+        d.row = u32p(o.row);
+        d.rpos = u32p(o.rpos);
+        d.prod = reinterpret_cast<const SwProd *>(A + o.prod);
+        d.nprod = (uint32_t)h.prod.size();
+        d.nwave = h.nwave;
+        d.stride = h.stride;
+        d.voff = voff;
+        d.div = div;
+        return d;
+    };
+    if (!long_lanes)
+        for (int q = 0; q < 4; ++q) S.sw[q] = swd(sw[q], o_sw[q], divs[q], sw_voff[q]);
+    S.t32_len = p->t32_len;
+    p->has_split = split;
+    p->split_rhs = sw_rhs;
+    if (split)
+        for (int t = 0; t < 2; ++t) {
+            SplitDev &d = p->split[t];
+            for (int k = 0; k < 2; ++k) {
+                d.head[k] = swd(hd[2 * t + k], o_hd[2 * t + k], divs[2 * t + k], hd_voff[2 * t + k]);
+                d.tail[k] = swd(sw[2 * t + k], o_sw[2 * t + k], divs[2 * t + k], sw_voff[2 * t + k]);
+            }
+            d.src = u32p(o_spl[t]);
+            d.nval = (uint32_t)spl_vpos[t].size();
+            d.parts = (uint32_t)hd[2 * t].part.size();
+            d.head_slots = std::max(hd[2 * t].nslot_max, hd[2 * t + 1].nslot_max);
+            d.tail_slots = sw[2 * t].nslot_max;
+        }
     S.lo_df = df(dlo, o_dlo_task, o_dlo_rl, o_dlo_idx, 0, 0);
     S.up_df = df(dup, o_dup_task, o_dup_rl, o_dup_idx, 1, (uint32_t)dlo.idx.size());
     S.tup_df = df(dtu, o_dtu_task, o_dtu_rl, o_dtu_idx, 1, 0);
@@ -1900,6 +2419,10 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         S.df_rscale = reinterpret_cast<const double *>(A + o_rscale);
         S.tdf_rsrc = u32p(o_trsrc);
         S.tdf_rscale = reinterpret_cast<const double *>(A + o_trscale);
+        p->split[0].rsrc = S.df_rsrc;
+        p->split[0].rscale = S.df_rscale;
+        p->split[1].rsrc = S.tdf_rsrc;
+        p->split[1].rscale = S.tdf_rscale;
         S.row_perm = u32p(o_rp);
         S.row_perm_inv = u32p(o_rpi);
         S.col_perm = u32p(o_cp);
@@ -2038,13 +2561,28 @@ glu_status ensure_batch(glu_plan *p, int batch)
     p->d_blucsr = nullptr;
     p->d_bnorms = nullptr;
     p->batch_cap = 0;
-    HIP_TRY(hipMalloc(&p->d_bt32, sizeof(float) * (size_t)p->n * batch));
+    HIP_TRY(hipMalloc(&p->d_bt32, sizeof(float) * (size_t)p->t32_len * batch));
     HIP_TRY(hipMalloc(&p->d_br64, sizeof(double) * (size_t)p->n * batch));
     HIP_TRY(hipMalloc(&p->d_blucsr, sizeof(float) * (size_t)p->df_nval * batch));
     HIP_TRY(hipMalloc(&p->d_bnorms, 2 * sizeof(double) * (size_t)batch));
     if (p->krylov)
         HIP_TRY(hipMalloc(&p->d_bkry, sizeof(double) * (3 * (size_t)p->krylov + 1) * p->n * (size_t)batch));
     p->batch_cap = batch;
+    return GLU_OK;
+}
+
+// The buffers of one matrix's sweeps (p->single[transpose]).
+glu_status ensure_single(glu_plan *p, int transpose)
+{
+    glu_plan::Single &q = p->single[transpose];
+    if (q.buf) return GLU_OK;
+    const size_t nval = p->has_split ? p->split[transpose].nval : transpose ? p->tdf_nval : p->df_nval;
+    const size_t rhs = p->has_split ? p->split_rhs : p->t32_len;
+    const size_t a = (nval + 63) & ~(size_t)63, b = (rhs + 63) & ~(size_t)63;
+    HIP_TRY(hipMalloc(&q.buf, sizeof(float) * (a + b + p->n)));
+    q.lucsr = q.buf;
+    q.rhs = q.buf + a;
+    q.xg = q.rhs + b;
     return GLU_OK;
 }
 
@@ -2161,22 +2699,36 @@ extern "C" glu_status glu_solve(glu_plan *p, const float *d_lu, const float *d_b
     if (!p || !d_lu || !d_b || !d_x) return fail(GLU_ERR_ARGUMENT, "null argument");
     if (!p->has_scaling) return fail(GLU_ERR_ARGUMENT, "plan has no permutation/scaling (create it from an analysis)");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // A x = b in one workgroup (exact dataflow sweeps) when the ready bits
-    // fit in LDS and the dataflow solve is on
-    const int mode = !transpose && p->tri_dataflow ? sweep_mode(p->n, launch::enable_lds()) : 0;
+    transpose = transpose ? 1 : 0;
+    // mode 2: one workgroup, the vector in LDS (A x = b and A' x = b);
+    // 1: the split sweeps, or (A x = b) one workgroup with the ready bits in
+    // LDS; 0: level by level.  All give the reference's arithmetic.
+    int mode = p->tri_dataflow ? sweep_mode(p->n, launch::enable_lds()) : 0;
+    const bool split = mode == 1 && p->has_split;
+    if (mode == 1 && !split && transpose) mode = 0;
     if (mode != 0) {
-        glu_status s = ensure_batch(p, 1);   // the sweep-layout copy (before any graph capture)
+        glu_status s = ensure_single(p, transpose);   // (before any graph capture)
         if (s != GLU_OK) return s;
     }
     auto issue = [&](hipStream_t s) {
         const SolveDev &S = p->S;
-        if (mode != 0) {
+        const glu_plan::Single &q = p->single[transpose];
+        if (split) {
+            const SplitDev &d = p->split[transpose];
+            launch::copy_df(d.src, d.nval, d_lu, q.lucsr, s);
+            launch::split_solve(d, d_b, d_lu, q.lucsr, q.rhs, q.xg, s);
+            if (!transpose)
+                launch::perm_scale_f32(q.xg, d_x, S.row_perm_inv, S.row_scale, 0, p->n, s);
+            else
+                launch::perm_scale_f32(q.xg, d_x, S.col_perm_inv, S.col_scale_perm, 1, p->n, s);
+        } else if (mode != 0) {
             // mode 1: the LDS the ready bits leave free holds the last rows
             // (r0..n-1) when they are a quarter of the rows or more
             const size_t bits = launch::batch_lds_bytes(mode, p->n), cap = launch::enable_lds();
             const uint32_t keep = mode == 1 ? split_rows(p->n, bits, cap) : 0u;
-            launch::solve_one(p->d_desc, p->df_nval, d_lu, p->d_blucsr, d_b, d_x, p->d_bt32,
-                              keep ? p->n - keep : UINT32_MAX, p->fused_threads, mode, bits + sizeof(float) * keep, s);
+            launch::solve_one(p->d_desc, transpose ? S.tdf_src : S.df_src, transpose ? p->tdf_nval : p->df_nval, d_lu,
+                              q.lucsr, d_b, d_x, q.rhs, keep ? p->n - keep : UINT32_MAX, p->fused_threads, mode,
+                              bits + sizeof(float) * keep, transpose, s);
         } else if (!transpose) {
             launch::perm_scale_f32(d_b, p->d_t32, S.col_perm, S.col_scale_perm, 0, p->n, s);
             run_sweeps(p, d_lu, p->d_t32, 0, s);
@@ -2191,7 +2743,7 @@ extern "C" glu_status glu_solve(glu_plan *p, const float *d_lu, const float *d_b
         return GLU_OK;
     };
     if (!p->use_graph) return issue(st);
-    return replay(p, p->g_solve[transpose ? 1 : 0], d_lu, d_b, d_x, 0, st, issue);
+    return replay(p, p->g_solve[transpose], d_lu, d_b, d_x, 0, st, issue);
 }
 
 extern "C" glu_status glu_refresh(glu_plan *p, const double *d_ax, float *d_lu, int batch, void *stream)
@@ -2219,9 +2771,10 @@ namespace {
 // |r|, |x| (and |A|, |b| on the first pass), eta on the host.  The FP64 work
 // runs in grid kernels; the sweeps run in one workgroup over the
 // sweep-layout copy `lucsr` (dataflow, ready bits in LDS) or, when lucsr is
-// null, level by level over the factors.
+// null, level by level over the factors; with `rhs`, they are the split
+// sweeps (right-hand sides in rhs, lucsr their copy, t32 the vector by row).
 glu_status refine_host_loop(glu_plan *p, const double *d_ax, const float *d_lu, const double *d_b, double *d_x,
-                            double tol, int maxit, int transpose, const float *lucsr, float *t32, double *r64,
+                            double tol, int maxit, int transpose, float *lucsr, float *rhs, float *t32, double *r64,
                             unsigned long long *norms, int *h_iters, double *h_eta, hipStream_t st)
 {
     const SolveDev &S = p->S;
@@ -2236,11 +2789,15 @@ glu_status refine_host_loop(glu_plan *p, const double *d_ax, const float *d_lu, 
     double anorm = 0.0, bnorm = 0.0, eta = 0.0;
     int it = 0;
     for (;;) {
-        if (!transpose)
+        if (rhs)
+            launch::split_precond(p->split[transpose ? 1 : 0], r64, d_lu, lucsr, rhs, t32, st);
+        else if (!transpose)
             launch::perm_scale_f64(r64, t32, S.col_perm, S.col_scale_perm, 0, n, st);
         else
             launch::perm_scale_f64(r64, t32, S.row_perm, S.row_scale, 1, n, st);
-        if (lucsr)
+        if (rhs)
+            ;   // the split sweeps scaled the residual themselves
+        else if (lucsr)
             launch::sweeps_df(p->d_desc, lucsr, t32, r0, p->fused_threads, bits + sizeof(float) * keep, transpose, st);
         else
             run_sweeps(p, d_lu, t32, transpose, st);
@@ -2281,7 +2838,8 @@ glu_status refine_one_wg(glu_plan *p, const double *d_ax, const float *d_lu, con
     const uint32_t n = p->n;
     int32_t *d_it = reinterpret_cast<int32_t *>(out16);
     double *d_eta = reinterpret_cast<double *>(out16 + 8);
-    launch::refine_one(p->d_desc, transpose ? p->tdf_nval : p->df_nval, d_ax, d_b, d_x, d_lu, lucsr, t32, r64,
+    launch::refine_one(p->d_desc, transpose ? p->S.tdf_src : p->S.df_src, transpose ? p->tdf_nval : p->df_nval, d_ax, d_b,
+                       d_x, d_lu, lucsr, t32, r64,
                        bnorms, kry, d_it, d_eta, tol, maxit, p->fused_threads, launch::batch_lds_bytes(2, n),
                        transpose, st);
     HIP_TRY(hipGetLastError());
@@ -2311,6 +2869,15 @@ extern "C" glu_status glu_refine(glu_plan *p, const double *d_ax, const float *d
     // workgroup, FP64 work across the grid (plain refinement); 0: level by
     // level.
     const int mode = sweep_mode(n, launch::enable_lds());
+    if (mode == 1 && p->has_split) {
+        glu_status s = ensure_single(p, transpose ? 1 : 0);
+        if (s != GLU_OK) return s;
+        const glu_plan::Single &q = p->single[transpose ? 1 : 0];
+        const SplitDev &d = p->split[transpose ? 1 : 0];
+        launch::copy_df(d.src, d.nval, d_lu, q.lucsr, st);
+        return refine_host_loop(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, q.lucsr, q.rhs, q.xg, p->d_r64,
+                                p->d_norms, h_iters, h_eta, st);
+    }
     float *lucsr = nullptr;
     if (mode != 0) {
         glu_status s = ensure_batch(p, 1);
@@ -2326,9 +2893,10 @@ extern "C" glu_status glu_refine(glu_plan *p, const double *d_ax, const float *d
         return refine_one_wg(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, lucsr, p->d_bt32, p->d_br64,
                              p->d_bnorms, p->d_bkry, p->d_rout, h_iters, h_eta, st);
     }
-    if (mode == 1) launch::copy_df(p->d_desc, transpose ? p->tdf_nval : p->df_nval, d_lu, lucsr, transpose, st);
-    return refine_host_loop(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, lucsr, p->d_t32, p->d_r64, p->d_norms,
-                            h_iters, h_eta, st);
+    if (mode == 1)
+        launch::copy_df(transpose ? p->S.tdf_src : p->S.df_src, transpose ? p->tdf_nval : p->df_nval, d_lu, lucsr, st);
+    return refine_host_loop(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, lucsr, nullptr, p->d_t32, p->d_r64,
+                            p->d_norms, h_iters, h_eta, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -2338,7 +2906,7 @@ extern "C" glu_status glu_refine(glu_plan *p, const double *d_ax, const float *d
 
 namespace {
 
-constexpr size_t kScratchBytes = GLU_NOALLOC_SCRATCH_BYTES;
+constexpr size_t kScratchBytes = 2 * (size_t)GLU_NOALLOC_SCRATCH_BYTES;   // see glu_refine_noalloc's layout
 constexpr int kScratchDevices = 64;
 
 // One copy per device, held until the process ends.  Host code never uses
@@ -2384,10 +2952,19 @@ extern "C" glu_status glu_refine_noalloc(glu_plan *p, const double *d_ax, const 
         return fail(GLU_ERR_ARGUMENT, "order " + std::to_string(n) +
                                           " is beyond the dataflow sweeps (their ready bits exceed LDS): "
                                           "use glu_refine");
-    // scratch layout: sweep value copy, correction vector, residual, norms
-    // (one-workgroup path: FP64 |b| slots, FGMRES vectors, iteration count +
-    // eta; grid path: the four norm words)
-    const uint32_t nval = transpose ? p->tdf_nval : p->df_nval;
+    // The limit counts the copy with the dataflow tables' slots, the vector,
+    // the residual, the norms, the FGMRES vectors and the results; the
+    // layout below may take up to twice that (the array holds it).
+    const int t = transpose ? 1 : 0;
+    const size_t kry = mode == 2 && p->krylov ? sizeof(double) * (3 * (size_t)p->krylov + 1) * n : 0;
+    const size_t need = align256(sizeof(float) * (size_t)p->scratch_nval[t]) + align256(sizeof(float) * (size_t)n) +
+                        align256(sizeof(double) * (size_t)n) + align256(4 * sizeof(unsigned long long)) +
+                        align256(kry) + align256(16);
+    // scratch layout: sweep value copy, right-hand sides and vector,
+    // residual, norms (one-workgroup path: FP64 |b| slots, FGMRES vectors,
+    // iteration count + eta; grid path: the four norm words)
+    const bool split = mode == 1 && p->has_split;
+    const uint32_t nval = split ? p->split[t].nval : transpose ? p->tdf_nval : p->df_nval;
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t o = off;
@@ -2395,14 +2972,15 @@ extern "C" glu_status glu_refine_noalloc(glu_plan *p, const double *d_ax, const 
         return o;
     };
     const size_t o_val = take(sizeof(float) * (size_t)nval);
-    const size_t o_t32 = take(sizeof(float) * (size_t)n);
+    const size_t o_rhs = take(split ? sizeof(float) * (size_t)p->split_rhs : 0);
+    const size_t o_t32 = take(sizeof(float) * (size_t)std::max(p->t32_len, n));
     const size_t o_r64 = take(sizeof(double) * (size_t)n);
     const size_t o_norms = take(4 * sizeof(unsigned long long));
-    const size_t o_kry = take(mode == 2 && p->krylov ? sizeof(double) * (3 * (size_t)p->krylov + 1) * n : 0);
+    const size_t o_kry = take(kry);
     const size_t o_out = take(16);
-    if (off > kScratchBytes)
-        return fail(GLU_ERR_ARGUMENT, "refinement needs " + std::to_string(off) + " bytes of scratch; the static " +
-                                          "scratch holds " + std::to_string(kScratchBytes) + ": use glu_refine");
+    if (need > GLU_NOALLOC_SCRATCH_BYTES || off > kScratchBytes)
+        return fail(GLU_ERR_ARGUMENT, "refinement needs " + std::to_string(need) + " bytes of scratch; the static " +
+                                          "scratch holds " + std::to_string(GLU_NOALLOC_SCRATCH_BYTES) + ": use glu_refine");
     unsigned char *base = nullptr;
     glu_status s = scratch_base(&base);
     if (s != GLU_OK) return s;
@@ -2415,8 +2993,10 @@ extern "C" glu_status glu_refine_noalloc(glu_plan *p, const double *d_ax, const 
                              reinterpret_cast<double *>(base + o_norms),
                              p->krylov ? reinterpret_cast<double *>(base + o_kry) : nullptr,
                              reinterpret_cast<char *>(base + o_out), h_iters, h_eta, st);
-    launch::copy_df(p->d_desc, nval, d_lu, lucsr, transpose, st);   // as glu_refine: sweeps in one workgroup
-    return refine_host_loop(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, lucsr, t32, r64,
+    // as glu_refine: the split sweeps, or both sweeps in one workgroup
+    launch::copy_df(split ? p->split[t].src : transpose ? p->S.tdf_src : p->S.df_src, nval, d_lu, lucsr, st);
+    return refine_host_loop(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, lucsr,
+                            split ? reinterpret_cast<float *>(base + o_rhs) : nullptr, t32, r64,
                             reinterpret_cast<unsigned long long *>(base + o_norms), h_iters, h_eta, st);
 }
 
@@ -2570,7 +3150,8 @@ struct glu_group {
     float *d_lucsr = nullptr;
     double *d_norms = nullptr;
     double *d_kry = nullptr;
-    std::vector<size_t> voff;   // per-matrix offset into the scratch vectors
+    std::vector<size_t> voff;   // per-matrix offset into d_r64
+    std::vector<size_t> toff;   // per-matrix offset into d_t32
     std::vector<size_t> koff;   // per-matrix offset into d_kry (~0: plain refinement)
     std::vector<size_t> foff;   // per-matrix offset into d_lucsr
     std::vector<uint32_t> order;   // members, heaviest first (d_order)
@@ -2604,7 +3185,7 @@ extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_gr
     std::unique_ptr<glu_group> g(new glu_group());
     std::vector<MatDesc> descs(count);
     std::vector<std::pair<int64_t, uint32_t>> work(count);
-    size_t vtot = 0, ftot = 0, ktot = 0;
+    size_t vtot = 0, ttot = 0, ftot = 0, ktot = 0;
     for (int i = 0; i < count; ++i) {
         glu_plan *p = plans[i];
         if (!p || !p->has_refine) return fail(GLU_ERR_ARGUMENT, "every plan must come from an analysis");
@@ -2620,6 +3201,8 @@ extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_gr
         ktot += (3 * (size_t)p->krylov + 1) * p->n * (p->krylov != 0);
         g->voff.push_back(vtot);
         vtot += p->n;
+        g->toff.push_back(ttot);
+        ttot += p->t32_len;
         g->foff.push_back(ftot);
         ftot += p->df_nval;
         g->threads = std::max(g->threads, p->fused_threads);
@@ -2634,7 +3217,7 @@ extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_gr
     HIP_TRY(hipMalloc(&g->d_descs, sizeof(MatDesc) * count));
     HIP_TRY(hipMalloc(&g->d_ios, sizeof(MatIOHost) * count));
     HIP_TRY(hipMalloc(&g->d_order, sizeof(uint32_t) * count));
-    HIP_TRY(hipMalloc(&g->d_t32, sizeof(float) * vtot));
+    HIP_TRY(hipMalloc(&g->d_t32, sizeof(float) * ttot));
     HIP_TRY(hipMalloc(&g->d_r64, sizeof(double) * vtot));
     HIP_TRY(hipMalloc(&g->d_lucsr, sizeof(float) * ftot));
     HIP_TRY(hipMalloc(&g->d_norms, 2 * sizeof(double) * count));
@@ -2664,7 +3247,7 @@ extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, c
     std::vector<MatIOHost> ios(count);
     for (int i = 0; i < count; ++i) {
         if (!d_ax[i] || !d_b[i] || !d_x[i] || !d_lu[i]) return fail(GLU_ERR_ARGUMENT, "null matrix pointer");
-        ios[i] = MatIOHost{d_ax[i], d_b[i], d_x[i], d_lu[i], g->d_t32 + g->voff[i], g->d_r64 + g->voff[i],
+        ios[i] = MatIOHost{d_ax[i], d_b[i], d_x[i], d_lu[i], g->d_t32 + g->toff[i], g->d_r64 + g->voff[i],
                            g->d_lucsr + g->foff[i], g->d_norms + 2 * i,
                            g->koff[i] == ~(size_t)0 ? nullptr : g->d_kry + g->koff[i], d_iters + i, d_eta + i};
     }
@@ -2699,7 +3282,7 @@ extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, c
         launch::refresh(p->R, d_ax[m], d_lu[m], p->nnz, 1, as);
         s = run_factor(p, d_lu[m], perturb, as);
         if (s != GLU_OK) return s;
-        launch::refine_one(p->d_desc, p->df_nval, d_ax[m], d_b[m], d_x[m], d_lu[m], p->d_blucsr, p->d_bt32,
+        launch::refine_one(p->d_desc, p->S.df_src, p->df_nval, d_ax[m], d_b[m], d_x[m], d_lu[m], p->d_blucsr, p->d_bt32,
                            p->d_br64, p->d_bnorms, p->d_bkry, d_iters + m, d_eta + m, tol, maxit, g->threads,
                            launch::batch_lds_bytes(2, p->n), 0, as);
         HIP_TRY(hipGetLastError());

@@ -95,3 +95,53 @@ def test_sweeps_with_non_finite_values(bits):
         fin = np.isfinite(want)
         assert np.array_equal(fin, np.isfinite(x)) and np.array_equal(np.isnan(x), np.isnan(want))
         assert np.array_equal(x[fin].view(np.uint32), want[fin].view(np.uint32))
+
+
+def _solve_transposed(an, lu, b):
+    """A' x = b with the FP32 factors, row by row in order: U' forward with
+    the pivot division, then L' backward."""
+    one = np.float32
+    t = (b[an.row_perm].astype(np.float64) * an.row_scale[an.row_perm]).astype(one)
+    cp, ri, ld = an.sym_c_ptr.tolist(), an.sym_r_idx.tolist(), an.l_col_ptr.tolist()
+    for r in range(an.n):
+        acc = t[r]
+        for q in range(cp[r], ld[r]):
+            acc = acc - lu[q] * t[ri[q]]
+        t[r] = acc / lu[ld[r]]
+    for r in range(an.n - 1, -1, -1):
+        acc = t[r]
+        for q in range(cp[r + 1] - 1, ld[r], -1):
+            acc = acc - lu[q] * t[ri[q]]
+        t[r] = acc
+    back = an.col_perm_inv
+    return (t[back].astype(np.float64) * an.col_scale_perm[back]).astype(one)
+
+
+@pytest.mark.parametrize("name", ["mna600", "small", "batch", "grad"])
+def test_solves_are_sequential(name):
+    """A x = b and A' x = b (n=50k "grad": split over many workgroups) equal
+    the row-by-row solve bit for bit, with a second value set and right-hand
+    side over the same plan; the refinement of A' reaches its tolerance."""
+    import torch
+    from helpers import mna_case
+    from oracle import oracle as O
+    from pyglu import mna
+    from pyglu.analysis import Analysis
+    from pyglu.device import Plan
+    data, indices, indptr, n = mna_case(name)
+    an = Analysis(data, indices, indptr, n)
+    plan, pat = Plan(an), O.SymPattern(an)
+    for seed in (1, 2):
+        ax = torch.from_numpy(mna.perturb_values(data, seed)).cuda()
+        lu = plan.refresh(ax).reshape(-1)
+        plan.factor(lu)
+        b = mna.rhs(n, seed).astype(np.float32)
+        f = lu.cpu().numpy()
+        x = plan.solve(lu, torch.from_numpy(b).cuda()).cpu().numpy()
+        want = O.solve_f32(pat, f, an.col_perm, an.row_perm_inv, an.col_scale_perm, an.row_scale, b)
+        assert np.array_equal(x.view(np.uint32), want.view(np.uint32))
+        xt = plan.solve(lu, torch.from_numpy(b).cuda(), transpose=True).cpu().numpy()
+        assert np.array_equal(xt.view(np.uint32), _solve_transposed(an, f, b).view(np.uint32))
+    x, it, eta = plan.refine(ax, lu, torch.from_numpy(b.astype(np.float64)).cuda(), tol=1e-11, maxit=20, transpose=True)
+    print(f"[{name}] n={n} transposed refinement {it} solves eta {eta:.1e}", flush=True)
+    assert eta <= 1e-11
