@@ -64,14 +64,17 @@ constexpr uint32_t kFirstBit = 0x80000000u;
 //   kWinGroup  {l0, u0, d0, l1, u1, d1, t, flags}: 16 lanes share merge entry
 //              t, lane j holding sources j and 16 + j of the chunk's 32
 //              (kWinGroup1: only the first 16 are used)
+//   kWinOut    {l, d, u0, u1} and two 32-bit places o0, o1 (~0: none): the
+//              products S[l] / S[d] * S[ui] to out[oi] (phases, after the
+//              last step)
 // Every wave passes one barrier per step.  Unused places address three kinds
 // of extra slots after the values: a 0 (slot nslot), a 1 (nslot + 1) and one
 // target a lane that nothing reads (nslot + 2 + lane), so that no chunk needs
 // tests: a missing update computes 0 / 1 * 0 and a missing source subtracts
 // +0, which changes no value.
 constexpr uint32_t kWinExtra = 66;        // extra slots
-constexpr uint32_t kWinKindShift = 30;
-constexpr uint32_t kWinCol = 0, kWinMerge = 1, kWinGroup1 = 2, kWinGroup = 3;
+constexpr uint32_t kWinKindShift = 29;
+constexpr uint32_t kWinCol = 0, kWinMerge = 1, kWinGroup1 = 2, kWinGroup = 3, kWinOut = 4;
 constexpr uint32_t kWinFirst = 1, kWinLast = 2;
 
 struct WinDev {
@@ -81,6 +84,30 @@ struct WinDev {
     const uint4 *prog;         // [64 chunks]
     const uint32_t *hdr;       // [chunks]
     const uint32_t *wptr;      // [nwave + 1]
+};
+
+// One phase of the factorization: a run of leading steps whose columns fall
+// into components that share no entry (bins of components, a workgroup each,
+// their columns' and rows' entries in LDS as a window's).  Updates of entries
+// of later columns can come from several bins: their products go to out, the
+// products of one entry in the order of the steps and columns, and are
+// subtracted once the phase is done.  Entries of up to kAsmLane products come
+// first in groups of 64 (a lane each, product k of lane i at base + 64 k + i),
+// the rest a wave each (contiguous).
+constexpr uint32_t kAsmLane = 32;
+
+struct AsmWave {
+    uint32_t tgt, base, cnt, pad;
+};
+
+struct PhaseDev {
+    const WinDev *bin;         // [nbin]
+    const uint2 *grp;          // [ngrp]: {base, most products of a lane}
+    const uint32_t *tgt;       // [64 ngrp] entry (~0: none)
+    const uint8_t *cnt;        // [64 ngrp] its products
+    const AsmWave *wav;        // [nwav]
+    float *out;                // the products
+    uint32_t nbin, ngrp, nwav, nslot;   // nslot: the largest bin's
 };
 
 struct FactorDev {

@@ -831,7 +831,9 @@ __device__ __forceinline__ float row_chain_sub(float a, float p)
 // into addresses before the barrier.  Measured (n=20,000, 370 steps in one
 // window): 601 -> 206 us against the shared item code, whose table loads
 // depended on each other inside a step; n=640, 142 steps: 112 -> 48 us.
-__device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pert, int perturb)
+template <bool kOut = false>
+__device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pert, int perturb,
+                                             float *__restrict__ out = nullptr)
 {
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -868,7 +870,12 @@ __device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pe
             const uint32_t a6 = (q.w & 0xffffu) << 2, a7 = (q.w >> 14) & 0x3fffcu;
             const uint32_t step = h & ((1u << kWinKindShift) - 1u), kind = h >> kWinKindShift;
             for (; passed < step; ++passed) __syncthreads();
-            if (kind == kWinCol) {
+            if (kOut && kind == kWinOut) {
+                const float l = at(a0) / gesp(at(a1), pert, perturb);
+                const float u0 = at(a2), u1 = at(a3);
+                if (q.z != ~0u) out[q.z] = l * u0;
+                if (q.w != ~0u) out[q.w] = l * u1;
+            } else if (kind == kWinCol) {
                 const float lv = at(a0), dv = at(a1);
                 const float u0 = at(a2), t0 = at(a3), u1 = at(a4), t1 = at(a5), u2 = at(a6), t2 = at(a7);
                 const float l = lv / gesp(dv, pert, perturb);
@@ -906,8 +913,9 @@ __device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pe
 
 // Steps [W.l0, W.l1) inside one workgroup with the values they touch staged
 // in LDS (slots): load, the steps, store back.
+template <bool kOut = false>
 __device__ __forceinline__ void factor_window(const WinDev &W, float *__restrict__ val, float *slots, float pert,
-                                              int perturb)
+                                              int perturb, float *__restrict__ out = nullptr)
 {
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
     constexpr uint32_t U = 8;   // positions, then values, eight loads at a time
@@ -924,7 +932,7 @@ __device__ __forceinline__ void factor_window(const WinDev &W, float *__restrict
     }
     for (uint32_t i = tid; i < kWinExtra; i += nt) slots[W.nslot + i] = i == 1 ? 1.f : 0.f;
     __syncthreads();
-    window_steps(W, slots, pert, perturb);
+    window_steps<kOut>(W, slots, pert, perturb, out);
     for (uint32_t s0 = tid; s0 < W.nslot; s0 += U * nt) {
         uint32_t p[U];
 #pragma unroll
@@ -996,6 +1004,85 @@ __global__ void __launch_bounds__(1024) k_factor_window(FactorDev F, float *__re
     const float pert = perturb ? *d_pert : 0.f;
     const WinDev W = load_window(F, w);
     factor_window(W, val, g_lds_vec, pert, perturb);
+}
+
+// A phase: bin blockIdx.x in this workgroup (dynamic LDS: its entries and
+// kWinExtra slots).  The steps of a bin cost a barrier where a launch per step
+// cost ~7 us and read its values from memory; what remains is the largest
+// component's work.  n=20,000: 38 launches of 7.0 us -> 36 us + 18 us for the
+// assembly; n=200,003: 95 of 13.1 us -> two phases, 320 us + 96 us.
+__global__ void __launch_bounds__(1024) k_factor_phase(PhaseDev Ph, float *__restrict__ val,
+                                                       const float *__restrict__ d_pert, int perturb)
+{
+    const float pert = perturb ? *d_pert : 0.f;
+    WinDev W = Ph.bin[blockIdx.x];
+    W.pos = glb(W.pos);
+    W.prog = glb(W.prog);
+    W.hdr = glb(W.hdr);
+    W.wptr = glb(W.wptr);
+    factor_window<true>(W, val, g_lds_vec, pert, perturb, Ph.out);
+}
+
+// The products of a phase subtracted from their entries, each entry's in
+// order: waves [0, nwav) take an entry each (64 products at a time from the
+// wave's LDS slice, the next 256 loading), the groups after them 64 entries.
+__device__ __forceinline__ void phase_assemble(const PhaseDev &Ph, float *__restrict__ val, uint32_t w, uint32_t lane,
+                                               float *lds)
+{
+    constexpr uint32_t U = 4;
+    if (w < Ph.nwav) {
+        const AsmWave e = Ph.wav[w];
+        float v = val[e.tgt], p[U];
+        auto load = [&](uint32_t k) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                const uint32_t q = k + u * kWave + lane;
+                const float x = Ph.out[e.base + min(q, e.cnt - 1)];
+                p[u] = q < e.cnt ? x : 0.f;   // past the end: v - 0
+            }
+        };
+        load(0);
+        for (uint32_t k = 0; k < e.cnt; k += U * kWave) {
+            float c[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) c[u] = p[u];
+            load(k + U * kWave);
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                if (k + u * kWave >= e.cnt) break;
+                lds[lane] = c[u];
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                v = serial_sub(v, lds, kWave, false);
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            }
+        }
+        if (lane == 0) val[e.tgt] = v;
+        return;
+    }
+    const uint32_t g = w - Ph.nwav;
+    if (g >= Ph.ngrp) return;
+    const uint2 d = Ph.grp[g];
+    const uint32_t t = Ph.tgt[64 * g + lane], cnt = Ph.cnt[64 * g + lane];
+    if (t == ~0u) return;
+    float v = val[t];
+    constexpr uint32_t kB = 8;   // products loaded at a time
+    for (uint32_t k = 0; k < d.y; k += kB) {
+        float p[kB];
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u) p[u] = Ph.out[d.x + 64 * min(k + u, d.y - 1) + lane];
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u) v = k + u < cnt ? v - p[u] : v;
+    }
+    val[t] = v;
+}
+
+__global__ void __launch_bounds__(256) k_phase_assemble(PhaseDev Ph, float *__restrict__ val)
+{
+    __shared__ __attribute__((aligned(16))) float lds[256 / kWave][kWave];
+    const uint32_t w = __builtin_amdgcn_readfirstlane(blockIdx.x * (256 / kWave) + threadIdx.x / kWave);
+    phase_assemble(Ph, val, w, threadIdx.x & (kWave - 1), lds[threadIdx.x / kWave]);
 }
 
 // ---------------------------------------------------------------------------
@@ -3277,6 +3364,13 @@ void pert(const FactorDev &F, const float *val, unsigned int *norm_bits, float *
     k_pert_finish<<<1, 1, 0, st>>>(norm_bits, d_pert);
 }
 
+void factor_phase(const PhaseDev &Ph, float *val, const float *d_pert, int perturb, int threads, hipStream_t st)
+{
+    k_factor_phase<<<Ph.nbin, threads, 4 * (size_t)(Ph.nslot + kWinExtra), st>>>(Ph, val, d_pert, perturb);
+    if (Ph.nwav + Ph.ngrp)
+        k_phase_assemble<<<blocks_for(Ph.nwav + Ph.ngrp, 256 / kWave), 256, 0, st>>>(Ph, val);
+}
+
 // lanes: the lanes the level needs (column tasks and long merges 64 each)
 void factor_grid(const FactorDev &F, float *val, const float *d_pert, int lvl, uint32_t lanes,
                  int perturb, int threads, hipStream_t st)
@@ -3603,6 +3697,7 @@ size_t enable_lds()
         reinterpret_cast<const void *>(&k_batch_group_refine_mixed),
         reinterpret_cast<const void *>(&k_tri_df),
         reinterpret_cast<const void *>(&k_factor_window),
+        reinterpret_cast<const void *>(&k_factor_phase),
     };
     // the limit less the largest static LDS among them (their wave slices
     // and reduction arrays, ~4 KiB); 8 KiB if the attributes are unavailable

@@ -33,6 +33,7 @@ namespace launch {
 void pert(const FactorDev &F, const float *val, unsigned int *norm_bits, float *d_pert, hipStream_t st);
 void factor_grid(const FactorDev &F, float *val, const float *d_pert, int lvl, uint32_t items, int perturb,
                  int threads, hipStream_t st);
+void factor_phase(const PhaseDev &Ph, float *val, const float *d_pert, int perturb, int threads, hipStream_t st);
 void factor_fused(const FactorDev &F, float *val, const float *d_pert, int l0, int l1, int perturb,
                   int threads, hipStream_t st);
 void factor_divide(const FactorDev &F, float *val, const float *d_pert, uint32_t ndiv, int perturb, hipStream_t st);
@@ -281,6 +282,7 @@ struct Segment {
     uint32_t items;  // grid segments: items (factor) or rows (solve)
     uint32_t k0 = 0, k1 = 0;   // solve segments: dataflow tasks [k0, k1)
     int win = -1;              // factor segments: an LDS window
+    int phase = -1;            // factor segments: a phase
 };
 
 struct TriHost {
@@ -319,6 +321,7 @@ struct glu_plan {
     uint32_t a_kmax = 0;                   // most entries in a row or a column of A
 
     std::vector<Segment> fsegs;
+    std::vector<PhaseDev> phases;
     TriHost tri[4];          // lo, up, tup, tlo
     bool tri_dataflow = false;   // fused solve segments run barrier-free
     int solve_df_opt = 0;        // glu_plan_opts.solve_dataflow
@@ -529,6 +532,10 @@ bool validate_pattern(const glu_pattern &P, std::string &err)
 
 struct Tables {
     std::vector<uint32_t> upos;        // CSR position -> CSC position
+    // update map: target of (k, jj, ii) (its jj-th U and ii-th L entry) at
+    // moff[k] + jj L(k) + ii (until the phases are built)
+    std::vector<uint64_t> moff;
+    std::vector<uint32_t> umap;
     // column tasks, by level: task t has lanes 64 t .. 64 t + 63 in cln
     // ({L position, pivot position, update count <= 4, 0}); the lane's e-th
     // update reads U value cup[256 t + 64 e + lane] and targets ctgt[same]
@@ -617,7 +624,8 @@ bool build_factor_tables(const glu_pattern &P, Tables &T, int64_t &updates, std:
     }
     // Scatter targets per (k, jj, ii), built per target column j (columns
     // write disjoint ranges of umap).
-    std::vector<uint64_t> moff(n + 1);
+    std::vector<uint64_t> &moff = T.moff;
+    moff.resize(n + 1);
     uint64_t off = 0;
     for (uint32_t k = 0; k < n; ++k) {
         moff[k] = off;
@@ -627,7 +635,7 @@ bool build_factor_tables(const glu_pattern &P, Tables &T, int64_t &updates, std:
     }
     moff[n] = off;
     updates = (int64_t)off;
-    std::vector<uint32_t> umap;
+    std::vector<uint32_t> &umap = T.umap;
     try {
         umap.assign(off, 0);
     } catch (const std::bad_alloc &) {
@@ -778,7 +786,6 @@ bool build_factor_tables(const glu_pattern &P, Tables &T, int64_t &updates, std:
                 out.dvd.push_back(make_uint2(p, dpos | (p == dpos + 1 ? kFirstBit : 0u)));
         }
     });
-    umap = std::vector<uint32_t>();
     // concatenation in level order
     T.ctask_ptr.assign(nl + 2, 0);
     T.ment_ptr.assign(nl + 2, 0);
@@ -942,19 +949,185 @@ void step_positions(const Tables &T, int l, F f)
     }
 }
 
-// Chunks of one step under construction: chains of chunks that one wave runs
-// in order, with their rough relative costs.
-struct WinChain {
-    uint32_t first, count, cost;   // chunks [first, first + count) of the step's buffer
-};
-
-// The window's streams.  Per step: the single updates of each column as
-// column chunks (a lane: one L entry, up to three of its U entries; lanes
-// that share U entries side by side), merge entries of up to kWinLaneMerge
-// sources a lane each (two sources a chunk), larger ones 16 lanes each (a
-// chunk of 32 sources takes about two lane chunks' time).  A step's chains
-// go to its waves longest first, each to the wave with the least so far.
+// Merge entries of up to kWinLaneMerge sources take a lane each (two sources
+// a chunk), larger ones 16 lanes each (a chunk of 32 sources takes about two
+// lane chunks' time).
 constexpr uint32_t kWinLaneMerge = 4;
+
+// The streams of one window or of one bin of a phase, step by step.  A step's
+// single updates become column chunks (a lane: one L entry, up to three of
+// its U entries; lanes that share U entries side by side).  Its chains of
+// chunks go to the waves longest first, each to the wave with the least so
+// far.
+class WinBuilder {
+public:
+    struct Src {
+        uint16_t l, u, d;
+    };
+
+    void begin(uint32_t nslot, uint32_t waves)
+    {
+        zero = nslot, one = nslot + 1, sink = nslot + 2;
+        data.assign(waves, {});
+        head.assign(waves, {});
+        load.assign(waves, 0);
+        clear();
+    }
+    // The single updates of one column: pivot slot d, its L entries' slots,
+    // and {u, t} by L entry.
+    void column(uint16_t d, size_t L, const uint16_t *l, const std::vector<std::vector<std::pair<uint16_t, uint16_t>>> &ut)
+    {
+        size_t longest = 0;
+        for (size_t i = 0; i < L; ++i) longest = std::max(longest, ut[i].size());
+        for (size_t r = 0; r < longest; r += 3)
+            for (size_t i = 0; i < L; ++i) {
+                if (ut[i].size() <= r) continue;
+                uint16_t *e = lane(kWinCol, 10);
+                e[0] = l[i];
+                e[1] = d;
+                for (size_t k = r; k < std::min(r + 3, ut[i].size()); ++k) {
+                    e[2 + 2 * (k - r)] = ut[i][k].first;
+                    e[3 + 2 * (k - r)] = ut[i][k].second;
+                }
+            }
+    }
+    // A merge entry and its sources in order.
+    void merge(uint16_t t, const Src *src, uint32_t cnt)
+    {
+        merges.push_back(Merge{t, (uint32_t)srcs.size(), cnt});
+        srcs.insert(srcs.end(), src, src + cnt);
+    }
+    // Up to two products of L entry l (pivot d): u[i] times it to place o[i].
+    void product(uint16_t l, uint16_t d, uint32_t n, const uint16_t *u, const uint32_t *o)
+    {
+        uint16_t *e = lane(kWinOut, 10);
+        e[0] = l;
+        e[1] = d;
+        for (uint32_t i = 0; i < n; ++i) {
+            e[2 + i] = u[i];
+            std::memcpy(e + 4 + 2 * i, &o[i], 4);
+        }
+    }
+    void end_step(uint32_t step)
+    {
+        std::vector<Merge> one_lane, group;
+        for (const Merge &m : merges) (m.cnt <= kWinLaneMerge ? one_lane : group).push_back(m);
+        const auto most = [](const Merge &x, const Merge &y) { return x.cnt > y.cnt; };
+        std::stable_sort(one_lane.begin(), one_lane.end(), most);
+        std::stable_sort(group.begin(), group.end(), most);
+        for (size_t i = 0; i < one_lane.size(); i += 64) {
+            const uint32_t n = (one_lane[i].cnt + 1) / 2;
+            chains.push_back(Chain{(uint32_t)kind.size(), n, 12 * n});
+            for (uint32_t c = 0; c < n; ++c) {
+                const size_t at = chunk(kWinMerge);
+                for (size_t k = i; k < std::min(i + 64, one_lane.size()); ++k) {
+                    const Merge &m = one_lane[k];
+                    const uint32_t own = (m.cnt + 1) / 2;
+                    if (c >= own) continue;   // this entry is done
+                    uint16_t *e = &buf[at + 8 * (k - i)];
+                    e[0] = m.t;
+                    e[1] = (uint16_t)((c == 0 ? kWinFirst : 0) | (c + 1 == own ? kWinLast : 0));
+                    for (uint32_t x = 2 * c; x < std::min(2 * c + 2, m.cnt); ++x) put(e + 2 + 3 * (x - 2 * c), srcs[m.first + x]);
+                }
+            }
+        }
+        for (size_t i = 0; i < group.size(); i += 4) {
+            const uint32_t top = group[i].cnt, n = (top + 31) / 32;
+            const bool half_last = top - 32 * (n - 1) <= 16;   // the last chunk uses 16 sources only
+            chains.push_back(Chain{(uint32_t)kind.size(), n, 35 * n - (half_last ? 10 : 0)});
+            for (uint32_t c = 0; c < n; ++c) {
+                const size_t at = chunk(half_last && c + 1 == n ? kWinGroup1 : kWinGroup);
+                for (size_t k = i; k < std::min(i + 4, group.size()); ++k) {
+                    const Merge &m = group[k];
+                    const uint32_t own = (m.cnt + 31) / 32;
+                    if (c >= own) continue;
+                    for (uint32_t ln = 0; ln < 16; ++ln) {
+                        uint16_t *e = &buf[at + 8 * (16 * (k - i) + ln)];
+                        e[6] = m.t;
+                        e[7] = (uint16_t)((c == 0 ? kWinFirst : 0) | (c + 1 == own ? kWinLast : 0));
+                        for (uint32_t x = 0; x < 2; ++x)
+                            if (32 * c + 16 * x + ln < m.cnt) put(e + 3 * x, srcs[m.first + 32 * c + 16 * x + ln]);
+                    }
+                }
+            }
+        }
+        std::stable_sort(chains.begin(), chains.end(), [](const Chain &x, const Chain &y) { return x.cost > y.cost; });
+        std::fill(load.begin(), load.end(), 0);
+        for (const Chain &c : chains) {
+            const size_t to = std::min_element(load.begin(), load.end()) - load.begin();
+            load[to] += c.cost;
+            data[to].insert(data[to].end(), buf.begin() + 512 * (size_t)c.first, buf.begin() + 512 * (size_t)(c.first + c.count));
+            for (uint32_t k = c.first; k < c.first + c.count; ++k) head[to].push_back(kind[k] << kWinKindShift | step);
+        }
+        clear();
+    }
+    void finish(Window &w) const
+    {
+        w.wptr.assign(1, 0);
+        for (size_t v = 0; v < data.size(); ++v) {
+            w.prog.insert(w.prog.end(), data[v].begin(), data[v].end());
+            w.hdr.insert(w.hdr.end(), head[v].begin(), head[v].end());
+            w.wptr.push_back((uint32_t)w.hdr.size());
+        }
+    }
+
+private:
+    struct Chain {   // chunks [first, first + count) of the step, run in order by one wave
+        uint32_t first, count, cost;
+    };
+    struct Merge {
+        uint16_t t;
+        uint32_t first, cnt;
+    };
+    uint32_t zero = 0, one = 0, sink = 0;
+    std::vector<std::vector<uint16_t>> data;   // per wave
+    std::vector<std::vector<uint32_t>> head;
+    std::vector<uint64_t> load;
+    std::vector<uint16_t> buf;                 // the step's chunks
+    std::vector<uint32_t> kind;
+    std::vector<Chain> chains;
+    std::vector<Merge> merges;
+    std::vector<Src> srcs;
+    uint32_t used = 64, open = 0;              // lanes used in the open chunk, its kind
+
+    void clear()
+    {
+        buf.clear();
+        kind.clear();
+        chains.clear();
+        merges.clear();
+        srcs.clear();
+        used = 64;
+    }
+    static void put(uint16_t *e, const Src &s) { e[0] = s.l, e[1] = s.u, e[2] = s.d; }
+    // a chunk of kind kd whose lanes do nothing
+    size_t chunk(uint32_t kd)
+    {
+        const size_t at = buf.size();
+        buf.resize(at + 64 * 8);
+        kind.push_back(kd);
+        for (uint32_t ln = 0; ln < 64; ++ln) {
+            const uint16_t z = (uint16_t)zero, o = (uint16_t)one, t = (uint16_t)(sink + ln);
+            const uint16_t col[8] = {z, o, z, t, z, t, z, t};
+            const uint16_t mrg[8] = {t, 0, z, z, o, z, z, o};
+            const uint16_t grp[8] = {z, z, o, z, z, o, t, 0};
+            const uint16_t out[8] = {z, o, z, z, 0xffff, 0xffff, 0xffff, 0xffff};
+            std::copy_n(kd == kWinCol ? col : kd == kWinMerge ? mrg : kd == kWinOut ? out : grp, 8, &buf[at + 8 * ln]);
+        }
+        return at;
+    }
+    // the next lane of the open chunk of kind kd (one lane, one item)
+    uint16_t *lane(uint32_t kd, uint32_t cost)
+    {
+        if (used == 64 || open != kd) {
+            chains.push_back(Chain{(uint32_t)kind.size(), 1, cost});
+            chunk(kd);
+            used = 0;
+            open = kd;
+        }
+        return &buf[buf.size() - 512 + 8 * used++];
+    }
+};
 
 void make_window(const Tables &T, int a, int b, const std::vector<uint32_t> &slot_of_pos,
                  const std::vector<uint32_t> &pos, uint32_t waves, Window &w)
@@ -962,37 +1135,13 @@ void make_window(const Tables &T, int a, int b, const std::vector<uint32_t> &slo
     w.l0 = a;
     w.l1 = b;
     w.pos = pos;
-    const uint32_t zero = (uint32_t)pos.size(), one = zero + 1, sink = zero + 2;
     auto slot = [&](uint32_t q) { return (uint16_t)slot_of_pos[q]; };
-    std::vector<std::vector<uint16_t>> data(waves);
-    std::vector<std::vector<uint32_t>> head(waves);
-    std::vector<uint16_t> buf;         // the step's chunks
-    std::vector<uint32_t> kind;
-    std::vector<WinChain> chains;
+    WinBuilder B;
+    B.begin((uint32_t)pos.size(), waves);
     std::vector<std::vector<std::pair<uint16_t, uint16_t>>> lists;   // a column's single updates {u, t} by L entry
-    std::vector<uint32_t> lane_merges, group_merges;
-    std::vector<uint64_t> load(waves);
-    // a chunk of kind kd whose lanes do nothing
-    auto add_chunk = [&](uint32_t kd) {
-        const size_t at = buf.size();
-        buf.resize(at + 64 * 8);
-        kind.push_back(kd);
-        for (uint32_t lane = 0; lane < 64; ++lane) {
-            uint16_t *e = &buf[at + 8 * lane];
-            const uint16_t z = (uint16_t)zero, o = (uint16_t)one, t = (uint16_t)(sink + lane);
-            const uint16_t col[8] = {z, o, z, t, z, t, z, t};
-            const uint16_t mrg[8] = {t, 0, z, z, o, z, z, o};
-            const uint16_t grp[8] = {z, z, o, z, z, o, t, 0};
-            std::copy_n(kd == kWinCol ? col : kd == kWinMerge ? mrg : grp, 8, e);
-        }
-        return at;
-    };
+    std::vector<uint16_t> lslot;
+    std::vector<WinBuilder::Src> src;
     for (int l = a; l < b; ++l) {
-        buf.clear();
-        kind.clear();
-        chains.clear();
-        // single updates
-        uint32_t used = 64;
         const size_t q1 = 64 * (size_t)T.ctask_ptr[l + 1];
         for (size_t q = 64 * (size_t)T.ctask_ptr[l]; q < q1;) {
             if (T.cln[q].z == 0) {
@@ -1006,103 +1155,28 @@ void make_window(const Tables &T, int a, int b, const std::vector<uint32_t> &slo
             size_t L = 1;
             while (s + L < e && T.cln[s + L].x != T.cln[s].x) ++L;
             if (lists.size() < L) lists.resize(L);
-            size_t longest = 0;
+            lslot.resize(L);
             for (size_t ii = 0; ii < L; ++ii) {
                 lists[ii].clear();
+                lslot[ii] = slot(T.cln[s + ii].x);
                 for (size_t c = s + ii; c < e; c += L)
                     for (uint32_t k = 0; k < T.cln[c].z; ++k) {
                         const size_t at = 256 * (c / 64) + 64 * k + c % 64;
                         if (T.ctgt[at] != UINT32_MAX) lists[ii].push_back({slot(T.cup[at]), slot(T.ctgt[at])});
                     }
-                longest = std::max(longest, lists[ii].size());
             }
-            for (size_t r = 0; r < longest; r += 3)
-                for (size_t ii = 0; ii < L; ++ii) {
-                    if (lists[ii].size() <= r) continue;
-                    if (used == 64) {
-                        chains.push_back(WinChain{(uint32_t)kind.size(), 1, 10});
-                        add_chunk(kWinCol);
-                        used = 0;
-                    }
-                    uint16_t *d = &buf[buf.size() - 512 + 8 * used++];
-                    d[0] = slot(T.cln[s + ii].x);
-                    d[1] = slot(T.cln[s].y);
-                    for (size_t k = r; k < std::min(r + 3, lists[ii].size()); ++k) {
-                        d[2 + 2 * (k - r)] = lists[ii][k].first;
-                        d[3 + 2 * (k - r)] = lists[ii][k].second;
-                    }
-                }
+            B.column(slot(T.cln[s].y), L, lslot.data(), lists);
             q = e;
         }
-        // merge entries, those with the most sources first
-        lane_merges.clear();
-        group_merges.clear();
-        auto count = [&](uint32_t e) { return T.msrc_ptr[e + 1] - T.msrc_ptr[e]; };
-        for (uint32_t e = T.ment_ptr[l]; e < T.ment_ptr[l + 1]; ++e)
-            (count(e) <= kWinLaneMerge ? lane_merges : group_merges).push_back(e);
-        auto most = [&](uint32_t x, uint32_t y) { return count(x) > count(y); };
-        std::stable_sort(lane_merges.begin(), lane_merges.end(), most);
-        std::stable_sort(group_merges.begin(), group_merges.end(), most);
-        for (size_t i = 0; i < lane_merges.size(); i += 64) {
-            const uint32_t n = (count(lane_merges[i]) + 1) / 2;
-            chains.push_back(WinChain{(uint32_t)kind.size(), n, 12 * n});
-            for (uint32_t c = 0; c < n; ++c) {
-                const size_t at = add_chunk(kWinMerge);
-                for (size_t k = i; k < std::min(i + 64, lane_merges.size()); ++k) {
-                    const uint32_t e = lane_merges[k], cnt = count(e), own = (cnt + 1) / 2;
-                    if (c >= own) continue;   // this entry is done
-                    uint16_t *d = &buf[at + 8 * (k - i)];
-                    d[0] = slot(T.ment[e]);
-                    d[1] = (uint16_t)((c == 0 ? kWinFirst : 0) | (c + 1 == own ? kWinLast : 0));
-                    for (uint32_t x = 2 * c; x < std::min(2 * c + 2, cnt); ++x) {
-                        const MergeSrc &m = T.msrc[T.msrc_ptr[e] + x];
-                        uint16_t *f = d + 2 + 3 * (x - 2 * c);
-                        f[0] = slot(m.lpos), f[1] = slot(m.upos), f[2] = slot(m.dpos);
-                    }
-                }
-            }
+        for (uint32_t e = T.ment_ptr[l]; e < T.ment_ptr[l + 1]; ++e) {
+            src.clear();
+            for (uint32_t k = T.msrc_ptr[e]; k < T.msrc_ptr[e + 1]; ++k)
+                src.push_back({slot(T.msrc[k].lpos), slot(T.msrc[k].upos), slot(T.msrc[k].dpos)});
+            B.merge(slot(T.ment[e]), src.data(), (uint32_t)src.size());
         }
-        for (size_t i = 0; i < group_merges.size(); i += 4) {
-            const uint32_t most_src = count(group_merges[i]), n = (most_src + 31) / 32;
-            const bool half_last = most_src - 32 * (n - 1) <= 16;   // the last chunk uses 16 sources only
-            chains.push_back(WinChain{(uint32_t)kind.size(), n, 35 * n - (half_last ? 10 : 0)});
-            for (uint32_t c = 0; c < n; ++c) {
-                const size_t at = add_chunk(half_last && c + 1 == n ? kWinGroup1 : kWinGroup);
-                for (size_t k = i; k < std::min(i + 4, group_merges.size()); ++k) {
-                    const uint32_t e = group_merges[k], cnt = count(e), own = (cnt + 31) / 32;
-                    if (c >= own) continue;
-                    for (uint32_t lane = 0; lane < 16; ++lane) {
-                        uint16_t *d = &buf[at + 8 * (16 * (k - i) + lane)];
-                        d[6] = slot(T.ment[e]);
-                        d[7] = (uint16_t)((c == 0 ? kWinFirst : 0) | (c + 1 == own ? kWinLast : 0));
-                        for (uint32_t x = 0; x < 2; ++x) {
-                            const uint32_t src = 32 * c + 16 * x + lane;
-                            if (src >= cnt) continue;
-                            const MergeSrc &m = T.msrc[T.msrc_ptr[e] + src];
-                            d[3 * x] = slot(m.lpos), d[3 * x + 1] = slot(m.upos), d[3 * x + 2] = slot(m.dpos);
-                        }
-                    }
-                }
-            }
-        }
-        std::stable_sort(chains.begin(), chains.end(),
-                         [](const WinChain &x, const WinChain &y) { return x.cost > y.cost; });
-        std::fill(load.begin(), load.end(), 0);
-        for (const WinChain &c : chains) {
-            const size_t to = std::min_element(load.begin(), load.end()) - load.begin();
-            load[to] += c.cost;
-            data[to].insert(data[to].end(), buf.begin() + 512 * (size_t)c.first,
-                            buf.begin() + 512 * (size_t)(c.first + c.count));
-            for (uint32_t k = c.first; k < c.first + c.count; ++k)
-                head[to].push_back(kind[k] << kWinKindShift | (uint32_t)(l - a));
-        }
+        B.end_step((uint32_t)(l - a));
     }
-    w.wptr.assign(1, 0);
-    for (uint32_t v = 0; v < waves; ++v) {
-        w.prog.insert(w.prog.end(), data[v].begin(), data[v].end());
-        w.hdr.insert(w.hdr.end(), head[v].begin(), head[v].end());
-        w.wptr.push_back((uint32_t)w.hdr.size());
-    }
+    B.finish(w);
 }
 
 // Windows chosen backward from the last step, so that the final run (the
@@ -1165,13 +1239,347 @@ void choose_windows(const Tables &T, int num_lev, uint32_t nnz, uint32_t budget,
     std::reverse(wins.begin(), wins.end());
 }
 
+// A phase (PhaseDev): steps [l0, l1), the bins' streams (Window: entries and
+// programs) and the products' assembly.
+struct Phase {
+    int l0 = 0, l1 = 0;
+    std::vector<Window> bin;
+    std::vector<uint2> grp;
+    std::vector<uint32_t> tgt;
+    std::vector<uint8_t> cnt;
+    std::vector<AsmWave> wav;
+    uint32_t nout = 0, nslot = 0;
+};
+
+constexpr uint32_t kPhaseWaves = 8;
+constexpr uint32_t kPhaseBins = 512;       // two workgroups a CU
+constexpr uint32_t kPhaseSlots = 19000;    // entries of a bin (76 KB: two a CU)
+constexpr int kMinPhase = 4;               // steps
+
+// The steps from l0 on that make a phase, at most to `limit`: as many as keep
+// every component's entries within a bin.  Components of the columns of steps
+// [l0, e): joined by entries of L or U between them.  Returns e (l0: none)
+// and each column's component (UINT32_MAX: not in the phase).
+int phase_end(const glu_pattern &P, int l0, int limit, std::vector<uint32_t> &comp)
+{
+    const uint32_t n = P.n;
+    std::vector<uint32_t> parent(n), ent(n);
+    std::vector<uint8_t> seen(n);
+    auto find = [&](uint32_t r) {
+        while (parent[r] != r) r = parent[r] = parent[parent[r]];
+        return r;
+    };
+    // column k joins what it shares an entry with among the columns seen;
+    // returns its component's entries
+    auto add = [&](uint32_t k) {
+        seen[k] = 1;
+        auto join = [&](uint32_t r) {
+            if (!seen[r]) return;
+            const uint32_t a = find(r), c = find(k);
+            if (a == c) return;
+            parent[a] = c;
+            ent[c] += ent[a];
+        };
+        for (uint32_t q = P.csr_r_ptr[k]; q < P.csr_r_ptr[k + 1]; ++q) join(P.csr_c_idx[q]);
+        for (uint32_t q = P.sym_c_ptr[k]; q < P.sym_c_ptr[k + 1]; ++q) join(P.sym_r_idx[q]);
+        return ent[find(k)];
+    };
+    auto reset = [&]() {
+        for (uint32_t k = 0; k < n; ++k) {
+            parent[k] = k;
+            ent[k] = (P.sym_c_ptr[k + 1] - P.l_col_ptr[k]) + (P.csr_r_ptr[k + 1] - P.csr_diag_ptr[k] - 1);
+            seen[k] = 0;
+        }
+    };
+    reset();
+    int e = l0;
+    for (bool fits = true; e < limit && fits; e += fits)
+        for (int t = P.level_ptr[e]; t < P.level_ptr[e + 1]; ++t)
+            fits = add((uint32_t)P.level_idx[t]) <= kPhaseSlots && fits;
+    reset();   // (without the step that did not fit)
+    for (int l = l0; l < e; ++l)
+        for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) (void)add((uint32_t)P.level_idx[t]);
+    comp.assign(n, UINT32_MAX);
+    for (int l = l0; l < e; ++l)
+        for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) comp[P.level_idx[t]] = find((uint32_t)P.level_idx[t]);
+    return e;
+}
+
+// The streams and the assembly of the phase of steps [ph.l0, ph.l1) with the
+// columns' components comp.  False: an update would cross components (the
+// pattern's levels do not order it; the steps stay as they are).
+bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &level_of,
+                 const std::vector<uint32_t> &comp, Phase &ph)
+{
+    const uint32_t n = P.n;
+    const unsigned threads = table_threads();
+    // components -> bins, largest first, each to the bin with the least work
+    std::vector<uint32_t> id(n, UINT32_MAX), size;
+    std::vector<uint64_t> work;
+    uint64_t total = 0;
+    for (uint32_t k = 0; k < n; ++k) {
+        if (comp[k] == UINT32_MAX) continue;
+        uint32_t &c = id[comp[k]];
+        if (c == UINT32_MAX) {
+            c = (uint32_t)size.size();
+            size.push_back(0);
+            work.push_back(0);
+        }
+        const uint32_t e = (P.sym_c_ptr[k + 1] - P.l_col_ptr[k]) + (P.csr_r_ptr[k + 1] - P.csr_diag_ptr[k] - 1);
+        size[c] += e;
+        work[c] += T.moff[k + 1] - T.moff[k] + e;
+        total += T.moff[k + 1] - T.moff[k] + e;
+    }
+    std::vector<uint32_t> order(size.size()), bin_of(size.size());
+    for (uint32_t c = 0; c < order.size(); ++c) order[c] = c;
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return work[a] > work[b]; });
+    const uint32_t nbin = (uint32_t)std::min<uint64_t>({(uint64_t)size.size(), kPhaseBins, total / 2048 + 1});
+    std::vector<uint64_t> load(nbin, 0);
+    std::vector<uint32_t> fill(nbin, 0);
+    for (uint32_t c : order) {
+        uint32_t to = UINT32_MAX;
+        for (uint32_t b = 0; b < nbin; ++b)
+            if (fill[b] + size[c] <= kPhaseSlots && (to == UINT32_MAX || load[b] < load[to])) to = b;
+        if (to == UINT32_MAX) {   // no room: one more bin
+            to = (uint32_t)load.size();
+            load.push_back(0);
+            fill.push_back(0);
+        }
+        load[to] += work[c];
+        fill[to] += size[c];
+        bin_of[c] = to;
+    }
+    const uint32_t nb = (uint32_t)load.size();
+    // columns of each bin by step, and the bin and slot of each entry it owns
+    std::vector<std::vector<uint32_t>> cols(nb);
+    for (int l = ph.l0; l < ph.l1; ++l)
+        for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) {
+            const uint32_t k = (uint32_t)P.level_idx[t];
+            cols[bin_of[id[comp[k]]]].push_back(k);
+        }
+    std::vector<uint32_t> own(P.nnz, UINT32_MAX);   // bin of an entry
+    std::vector<uint16_t> slot(P.nnz, 0);
+    ph.bin.resize(nb);
+    parallel_items(nb, threads, [&](unsigned, size_t b) {
+        std::vector<uint32_t> &pos = ph.bin[b].pos;
+        for (uint32_t k : cols[b]) {
+            for (uint32_t p = P.l_col_ptr[k]; p < P.sym_c_ptr[k + 1]; ++p) pos.push_back(p);
+            for (uint32_t q = P.csr_diag_ptr[k] + 1; q < P.csr_r_ptr[k + 1]; ++q) pos.push_back(T.upos[q]);
+        }
+        std::sort(pos.begin(), pos.end());
+        for (uint32_t i = 0; i < pos.size(); ++i) {
+            own[pos[i]] = (uint32_t)b;
+            slot[pos[i]] = (uint16_t)i;
+        }
+    });
+    // products per later entry: column j's pivots of the phase in order of
+    // step and number; cnt by position, then each product's place
+    std::vector<uint32_t> cnt(P.nnz, 0), base(P.nnz, 0);
+    std::vector<uint32_t> csc2csr(P.nnz);
+    for (uint32_t q = 0; q < P.nnz; ++q) csc2csr[T.upos[q]] = q;
+    std::atomic<bool> crossed(false);
+    auto each_outside = [&](uint32_t j, std::vector<std::pair<int, uint32_t>> &ks, auto f) {
+        ks.clear();
+        for (uint32_t p = P.sym_c_ptr[j]; p < P.l_col_ptr[j]; ++p)
+            if (comp[P.sym_r_idx[p]] != UINT32_MAX) ks.push_back({level_of[P.sym_r_idx[p]], p});
+        std::sort(ks.begin(), ks.end());   // (positions of a column ascend with the pivots)
+        for (const auto &[lev, p] : ks) {
+            const uint32_t k = P.sym_r_idx[p], L = P.sym_c_ptr[k + 1] - P.l_col_ptr[k] - 1;
+            const uint64_t at = T.moff[k] + (uint64_t)(csc2csr[p] - P.csr_diag_ptr[k] - 1) * L;
+            for (uint32_t ii = 0; ii < L; ++ii) {
+                const uint32_t t = T.umap[at + ii];
+                if (own[t] == UINT32_MAX) f(at + ii, t);
+                else if (own[t] != bin_of[id[comp[k]]]) crossed.store(true);
+            }
+        }
+    };
+    std::vector<std::vector<std::pair<int, uint32_t>>> scratch(threads);
+    constexpr uint32_t kCols = 128;
+    const size_t items = (n + kCols - 1) / kCols;
+    parallel_items(items, threads, [&](unsigned w, size_t item) {
+        for (uint32_t j = (uint32_t)item * kCols; j < std::min<uint32_t>(n, (uint32_t)(item + 1) * kCols); ++j)
+            each_outside(j, scratch[w], [&](uint64_t, uint32_t t) { ++cnt[t]; });
+    });
+    if (crossed.load()) return false;
+    // entries by product count: groups of 64 of about the same, waves for the rest
+    std::vector<uint32_t> few, many;
+    for (uint32_t p = 0; p < P.nnz; ++p)
+        if (cnt[p]) (cnt[p] <= kAsmLane ? few : many).push_back(p);
+    const auto most = [&](uint32_t a, uint32_t b) { return cnt[a] > cnt[b]; };
+    std::stable_sort(few.begin(), few.end(), most);
+    std::stable_sort(many.begin(), many.end(), most);
+    uint64_t out = 0;
+    std::vector<uint8_t> lane64(P.nnz, 0);   // product stride 64 (grouped) or 1
+    for (size_t i = 0; i < few.size(); i += 64) {
+        const uint32_t m = cnt[few[i]];
+        ph.grp.push_back(make_uint2((uint32_t)out, m));
+        for (size_t k = i; k < i + 64; ++k) {
+            ph.tgt.push_back(k < few.size() ? few[k] : UINT32_MAX);
+            ph.cnt.push_back(k < few.size() ? (uint8_t)cnt[few[k]] : 0);
+            if (k < few.size()) {
+                base[few[k]] = (uint32_t)(out + (k - i));
+                lane64[few[k]] = 1;
+            }
+        }
+        out += 64 * (uint64_t)m;
+    }
+    for (uint32_t p : many) {
+        ph.wav.push_back(AsmWave{p, (uint32_t)out, cnt[p], 0});
+        base[p] = (uint32_t)out;
+        out += (cnt[p] + 63u) & ~63u;
+    }
+    if (out >= UINT32_MAX) return false;
+    ph.nout = (uint32_t)out;
+    std::vector<uint32_t> place(T.umap.size(), UINT32_MAX);   // by update, as umap
+    std::fill(cnt.begin(), cnt.end(), 0);
+    parallel_items(items, threads, [&](unsigned w, size_t item) {
+        for (uint32_t j = (uint32_t)item * kCols; j < std::min<uint32_t>(n, (uint32_t)(item + 1) * kCols); ++j)
+            each_outside(j, scratch[w], [&](uint64_t at, uint32_t t) {
+                place[at] = base[t] + cnt[t]++ * (lane64[t] ? 64u : 1u);
+            });
+    });
+    // each bin's program: its steps' inner updates, then all its products
+    struct Marks {
+        std::vector<uint32_t> stamp, count, first;
+        uint32_t gen = 0;
+    };
+    std::vector<Marks> marks(threads);
+    parallel_items(nb, threads, [&](unsigned wk, size_t b) {
+        Marks &M = marks[wk];
+        if (M.stamp.empty()) {   // by slot
+            M.stamp.assign(0x10000, 0);
+            M.count.assign(0x10000, 0);
+            M.first.assign(0x10000, 0);
+        }
+        Window &w = ph.bin[b];
+        w.l0 = 0;
+        w.l1 = ph.l1 - ph.l0;
+        WinBuilder B;
+        B.begin((uint32_t)w.pos.size(), kPhaseWaves);
+        std::vector<std::vector<std::pair<uint16_t, uint16_t>>> lists;
+        std::vector<uint16_t> lslot, order;
+        std::vector<WinBuilder::Src> src;
+        size_t i = 0;
+        for (int l = ph.l0; l < ph.l1; ++l) {
+            size_t e = i;
+            while (e < cols[b].size() && level_of[cols[b][e]] == l) ++e;
+            if (e == i) continue;
+            auto inner = [&](auto f) {   // f(column, jj, ii, L, target slot)
+                for (size_t c = i; c < e; ++c) {
+                    const uint32_t k = cols[b][c], L = P.sym_c_ptr[k + 1] - P.l_col_ptr[k] - 1;
+                    if (L == 0) continue;
+                    const uint32_t U = P.csr_r_ptr[k + 1] - P.csr_diag_ptr[k] - 1;
+                    for (uint32_t jj = 0; jj < U; ++jj)
+                        for (uint32_t ii = 0; ii < L; ++ii) {
+                            const uint64_t at = T.moff[k] + (uint64_t)jj * L + ii;
+                            if (place[at] == UINT32_MAX) f(k, jj, ii, slot[T.umap[at]]);
+                        }
+                }
+            };
+            ++M.gen;
+            order.clear();
+            inner([&](uint32_t, uint32_t, uint32_t, uint16_t t) {
+                if (M.stamp[t] != M.gen) {
+                    M.stamp[t] = M.gen;
+                    M.count[t] = 0;
+                    order.push_back(t);
+                }
+                ++M.count[t];
+            });
+            uint32_t nsrc = 0;
+            for (uint16_t t : order)
+                if (M.count[t] >= 2) {
+                    M.first[t] = nsrc;
+                    nsrc += M.count[t];
+                }
+            src.resize(nsrc);
+            std::vector<uint32_t> cur;   // next source of each merge entry
+            for (uint16_t t : order)
+                if (M.count[t] >= 2) cur.push_back(M.first[t]);
+            // the columns of a step ascend, so a merge entry's sources come in order
+            for (size_t c = i; c < e; ++c) {
+                const uint32_t k = cols[b][c], dpos = P.l_col_ptr[k], L = P.sym_c_ptr[k + 1] - dpos - 1;
+                if (L == 0) continue;
+                const uint32_t U = P.csr_r_ptr[k + 1] - P.csr_diag_ptr[k] - 1;
+                if (lists.size() < L) lists.resize(L);
+                lslot.resize(L);
+                for (uint32_t ii = 0; ii < L; ++ii) {
+                    lists[ii].clear();
+                    lslot[ii] = slot[dpos + 1 + ii];
+                }
+                for (uint32_t jj = 0; jj < U; ++jj) {
+                    const uint16_t u = slot[T.upos[P.csr_diag_ptr[k] + 1 + jj]];
+                    for (uint32_t ii = 0; ii < L; ++ii) {
+                        const uint64_t at = T.moff[k] + (uint64_t)jj * L + ii;
+                        if (place[at] != UINT32_MAX) continue;
+                        const uint16_t t = slot[T.umap[at]];
+                        if (M.count[t] >= 2) src[M.first[t]++] = {lslot[ii], u, slot[dpos]};
+                        else lists[ii].push_back({u, t});
+                    }
+                }
+                B.column(slot[dpos], L, lslot.data(), lists);
+            }
+            for (uint16_t t : order)
+                if (M.count[t] >= 2) B.merge(t, &src[M.first[t] - M.count[t]], M.count[t]);
+            B.end_step((uint32_t)(l - ph.l0));
+            i = e;
+        }
+        for (uint32_t k : cols[b]) {
+            const uint32_t dpos = P.l_col_ptr[k], L = P.sym_c_ptr[k + 1] - dpos - 1;
+            const uint32_t U = P.csr_r_ptr[k + 1] - P.csr_diag_ptr[k] - 1;
+            // two U entries a lane, the L entries side by side
+            for (uint32_t jj = 0; jj < U; jj += 2)
+                for (uint32_t ii = 0; ii < L; ++ii) {
+                    uint16_t u[2];
+                    uint32_t o[2], m = 0;
+                    for (uint32_t x = jj; x < std::min(jj + 2, U); ++x) {
+                        const uint32_t at = place[T.moff[k] + (uint64_t)x * L + ii];
+                        if (at == UINT32_MAX) continue;
+                        u[m] = slot[T.upos[P.csr_diag_ptr[k] + 1 + x]];
+                        o[m++] = at;
+                    }
+                    if (m) B.product(slot[dpos + 1 + ii], slot[dpos], m, u, o);
+                }
+        }
+        B.end_step((uint32_t)(ph.l1 - ph.l0));
+        B.finish(w);
+    });
+    for (const Window &w : ph.bin) ph.nslot = std::max<uint32_t>(ph.nslot, (uint32_t)w.pos.size());
+    return true;
+}
+
+// The phases ahead of step `limit` (the first LDS window's).
+void choose_phases(const glu_pattern &P, const Tables &T, int limit, std::vector<Phase> &phases)
+{
+    std::vector<int> level_of(P.n, 0);
+    for (int l = 0; l < P.num_lev; ++l)
+        for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) level_of[P.level_idx[t]] = l;
+    std::vector<uint32_t> comp;
+    for (int l = 0; l < limit;) {
+        const int e = phase_end(P, l, limit, comp);
+        if (e - l < kMinPhase) break;
+        Phase ph;
+        ph.l0 = l;
+        ph.l1 = e;
+        if (!build_phase(P, T, level_of, comp, ph)) break;
+        phases.push_back(std::move(ph));
+        l = e;
+    }
+}
+
 // Segments of the factorization schedule: windows (one workgroup each) and,
 // between them, runs of global-memory steps split into fused and grid
 // segments.
-void factor_segments(glu_plan &p, const Tables &T, const std::vector<Window> &wins)
+void factor_segments(glu_plan &p, const Tables &T, const std::vector<Phase> &phases, const std::vector<Window> &wins)
 {
     p.fsegs.clear();
     int l = 0;
+    for (size_t k = 0; k < phases.size(); ++k) {
+        Segment s{phases[k].l0, phases[k].l1, false, 0};
+        s.phase = (int)k;
+        p.fsegs.push_back(s);
+        l = phases[k].l1;
+    }
     auto global_run = [&](int a, int b) {
         if (a >= b) return;
         std::vector<uint32_t> work(b - a);
@@ -2008,7 +2416,10 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         p->win_nslot = std::max<uint32_t>(p->win_nslot, (uint32_t)w.pos.size());
         p->win_slots.push_back((uint32_t)w.pos.size());
     }
-    factor_segments(*p, T, wins);
+    std::vector<Phase> phases;
+    choose_phases(P, T, wins.empty() ? 0 : std::min(wins[0].l0, P.num_lev), phases);
+    T.umap = std::vector<uint32_t>();
+    factor_segments(*p, T, phases, wins);
     p->units = (int64_t)(T.cln.size() / 64);
     // The batched kernels' leading grid steps: those ahead of the first LDS
     // window with at least a workgroup's worth of lanes per matrix (a
@@ -2214,6 +2625,28 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         o_whdr[w] = U.put(wins[w].hdr);
         o_wptr[w] = U.put(wins[w].wptr);
     }
+    struct PhaseOff {
+        std::vector<size_t> pos, prog, hdr, wptr;
+        size_t bin, grp, tgt, cnt, wav;
+    };
+    std::vector<PhaseOff> o_ph(phases.size());
+    size_t most_out = 0;
+    for (size_t k = 0; k < phases.size(); ++k) {
+        PhaseOff &o = o_ph[k];
+        for (const Window &w : phases[k].bin) {
+            o.pos.push_back(U.put(w.pos));
+            o.prog.push_back(U.put(w.prog));
+            o.hdr.push_back(U.put(w.hdr));
+            o.wptr.push_back(U.put(w.wptr));
+        }
+        o.grp = U.put(phases[k].grp);
+        o.tgt = U.put(phases[k].tgt);
+        o.cnt = U.put(phases[k].cnt);
+        o.wav = U.put(phases[k].wav);
+        o.bin = U.reserve(sizeof(WinDev) * phases[k].bin.size());
+        most_out = std::max<size_t>(most_out, phases[k].nout);
+    }
+    const size_t o_out = U.reserve(sizeof(float) * most_out);
     const size_t o_wdev = U.reserve(sizeof(WinDev) * std::max<size_t>(wins.size(), 1));
     struct SwOff {
         size_t meta, hdr, wptr, part, row, rpos, prod;
@@ -2282,8 +2715,31 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
 
     HIP_TRY(hipMalloc(&p->d_arena, U.arena.total));
     p->arena_bytes = U.arena.total;
-    for (auto &it : U.items)
-        if (it.bytes) HIP_TRY(hipMemcpy(p->d_arena + it.off, it.src, it.bytes, hipMemcpyHostToDevice));
+    // large parts as they are, runs of small ones (a phase has a few per bin)
+    // gathered into one copy each
+    {
+        constexpr size_t kSmall = 1u << 20, kRun = 32u << 20;
+        std::vector<char> run;
+        size_t at = 0;
+        auto flush = [&]() -> hipError_t {
+            const hipError_t e = run.empty() ? hipSuccess
+                                             : hipMemcpy(p->d_arena + at, run.data(), run.size(), hipMemcpyHostToDevice);
+            run.clear();
+            return e;
+        };
+        for (auto &it : U.items) {
+            if (!it.bytes) continue;
+            if (it.bytes >= kSmall || (!run.empty() && it.off + it.bytes - at > kRun)) HIP_TRY(flush());
+            if (it.bytes >= kSmall) {
+                HIP_TRY(hipMemcpy(p->d_arena + it.off, it.src, it.bytes, hipMemcpyHostToDevice));
+                continue;
+            }
+            if (run.empty()) at = it.off;
+            run.resize(it.off + it.bytes - at);   // (reserved parts in between are filled later)
+            std::memcpy(run.data() + (it.off - at), it.src, it.bytes);
+        }
+        HIP_TRY(flush());
+    }
     HIP_TRY(hipMemset(p->d_arena + o_normbits, 0, sizeof(unsigned int)));
 
     char *A = p->d_arena;
@@ -2308,6 +2764,36 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     F.num_lev = P.num_lev;
     F.n = n;
     F.nnz = P.nnz;
+    for (size_t k = 0; k < phases.size(); ++k) {
+        const PhaseOff &o = o_ph[k];
+        std::vector<WinDev> wd;
+        for (size_t b = 0; b < phases[k].bin.size(); ++b) {
+            const Window &x = phases[k].bin[b];
+            WinDev d{};
+            d.l0 = x.l0;
+            d.l1 = x.l1;
+            d.nslot = (uint32_t)x.pos.size();
+            d.nwave = (uint32_t)x.wptr.size() - 1;
+            d.pos = u32p(o.pos[b]);
+            d.prog = reinterpret_cast<const uint4 *>(A + o.prog[b]);
+            d.hdr = u32p(o.hdr[b]);
+            d.wptr = u32p(o.wptr[b]);
+            wd.push_back(d);
+        }
+        HIP_TRY(hipMemcpy(A + o.bin, wd.data(), sizeof(WinDev) * wd.size(), hipMemcpyHostToDevice));
+        PhaseDev d{};
+        d.bin = reinterpret_cast<const WinDev *>(A + o.bin);
+        d.grp = reinterpret_cast<const uint2 *>(A + o.grp);
+        d.tgt = u32p(o.tgt);
+        d.cnt = reinterpret_cast<const uint8_t *>(A + o.cnt);
+        d.wav = reinterpret_cast<const AsmWave *>(A + o.wav);
+        d.out = reinterpret_cast<float *>(A + o_out);
+        d.nbin = (uint32_t)wd.size();
+        d.ngrp = (uint32_t)phases[k].grp.size();
+        d.nwav = (uint32_t)phases[k].wav.size();
+        d.nslot = phases[k].nslot;
+        p->phases.push_back(d);
+    }
     {
         std::vector<WinDev> wd(wins.size());
         for (size_t w = 0; w < wins.size(); ++w) {
@@ -2491,7 +2977,9 @@ glu_status run_factor(glu_plan *p, float *d_val, int perturb, hipStream_t st)
 {
     if (perturb) launch::pert(p->F, d_val, p->d_norm_bits, p->d_pert, st);
     for (const Segment &s : p->fsegs) {
-        if (s.win >= 0)
+        if (s.phase >= 0)
+            launch::factor_phase(p->phases[s.phase], d_val, p->d_pert, perturb, (int)kPhaseWaves * 64, st);
+        else if (s.win >= 0)
             launch::factor_window(p->F, s.win, p->win_slots[s.win], d_val, p->d_pert, perturb, p->fused_threads, st);
         else if (s.fused)
             launch::factor_fused(p->F, d_val, p->d_pert, s.l0, s.l1, perturb, p->fused_threads, st);
