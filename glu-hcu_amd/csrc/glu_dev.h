@@ -110,6 +110,17 @@ struct PhaseDev {
     uint32_t nbin, ngrp, nwav, nslot;   // nslot: the largest bin's
 };
 
+// The leading launches of a group of distinct patterns: items {member, block
+// of values | bin | first wave}, phase round by phase round.
+constexpr uint32_t kGroupRounds = 8;       // phases of a member taken this way, at most
+
+struct GroupLaunch {
+    const uint2 *values = nullptr, *bins[kGroupRounds] = {}, *asms[kGroupRounds] = {};
+    const PhaseDev *phase[kGroupRounds] = {};   // by member
+    uint32_t nvalues = 0, nbin[kGroupRounds] = {}, nasm[kGroupRounds] = {}, nslot[kGroupRounds] = {};
+    uint32_t rounds = 0, threads = 0;
+};
+
 struct FactorDev {
     const uint32_t *col_ptr;   // sym_c_ptr [n+1] (GESP column sums)
     const uint32_t *gcols;     // columns, those with > kLongRow entries first [n]

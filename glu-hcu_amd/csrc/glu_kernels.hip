@@ -946,14 +946,14 @@ __device__ __forceinline__ void factor_window(const WinDev &W, float *__restrict
 
 // Steps l0.. of one factorization by one workgroup: windows in LDS, the
 // steps between them in global memory; l0 is 0 or lies at or before the
-// first window's first step (the steps before it ran as
-// k_factor_grid_il launches).  The divisions L(i,k) /= U(k,k) of every
+// first window's first step (the steps before it ran as launches of
+// their own).  The divisions L(i,k) /= U(k,k) of every
 // column run after the last step, all at once: no step reads a divided L
 // value (updates divide on the fly) and no step writes L(:,k) or U(k,k)
 // after column k's step, so the values are those of the per-step order,
 // one barrier-bound pass per step less.
 __device__ __forceinline__ void factor_all_wg(const FactorDev &F, float *__restrict__ val, float *slots, float pert,
-                                              int perturb, float *wlds, int l0)
+                                              int perturb, float *wlds, int l0, uint32_t d0)
 {
     int l = l0;
     for (int w = 0; w < F.nwin; ++w) {
@@ -966,11 +966,12 @@ __device__ __forceinline__ void factor_all_wg(const FactorDev &F, float *__restr
     // the divisions, eight items a lane at a time (their loads issued
     // together); items are independent: an item writes its L entry and, for
     // a perturbed pivot, the pivot, which the column's other items divide
-    // by either way (see factor_divide).  Those of the columns of steps
-    // before l0 - 1 ran with the interleaved steps (k_factor_grid_il).
+    // by either way (see factor_divide).  Those before d0 ran with the
+    // interleaved steps (k_factor_grid_il: the columns of steps before
+    // l0 - 1).
     const uint32_t nd = F.dvd_ptr[F.num_lev], tid = threadIdx.x, nt = blockDim.x;
     constexpr int U = 8;
-    for (uint32_t t0 = (l0 > 0 ? F.dvd_ptr[l0 - 1] : 0u) + tid; t0 < nd; t0 += U * nt) {
+    for (uint32_t t0 = d0 + tid; t0 < nd; t0 += U * nt) {
         // loads without branches (past the end: the last item again), so
         // that the eight items' table loads, then value loads, issue together
         uint2 it[U];
@@ -2487,6 +2488,26 @@ enum : int {
 // each phase takes the (globalized) tables it needs from it, so the
 // descriptor is not held in registers as a whole.
 //
+// wg_pert: the GESP value of one matrix's values, by its workgroup.
+__device__ __forceinline__ float wg_pert(const MatDesc *Md, const float *__restrict__ lu, double *sh, float *wlds)
+{
+    const uint32_t *col_ptr = glb(Md->f.col_ptr), *gcols = glb(Md->f.gcols);
+    const uint32_t ngl = Md->f.ngl, n = Md->n, tid = threadIdx.x, nt = blockDim.x;
+    double cm = 0.0;
+    for (uint32_t t = tid / kWave; t < ngl; t += nt / kWave) {   // long columns a wave each
+        const uint32_t c = gcols[t];
+        const float s = abs_col_sum_wave(lu, col_ptr[c], col_ptr[c + 1], tid & (kWave - 1), wlds);
+        if (s == s) cm = fmax(cm, (double)s);
+    }
+    for (uint32_t t = ngl + tid; t < n; t += nt) {
+        const uint32_t c = gcols[t];
+        float s = 0.f;
+        for (uint32_t p = col_ptr[c]; p < col_ptr[c + 1]; ++p) s += fabsf(lu[p]);
+        if (s == s) cm = fmax(cm, (double)s);
+    }
+    return kPertFactor * (float)wg_max(cm, sh);
+}
+
 // wg_values: steps 1-2 (the matrix's values, |b|_inf with x = 0 and
 // r64 = b, the GESP value).
 __device__ __forceinline__ void wg_values(const MatDesc *Md, const MatIO &io, int perturb, double *sh, float *wlds,
@@ -2535,30 +2556,17 @@ __device__ __forceinline__ void wg_values(const MatDesc *Md, const MatIO &io, in
     // 2. GESP value from the freshly placed values
     pert = 0.f;
     if (perturb) {
-        const uint32_t *col_ptr = glb(Md->f.col_ptr), *gcols = glb(Md->f.gcols);
-        const uint32_t ngl = Md->f.ngl;
-        double cm = 0.0;
-        for (uint32_t t = tid / kWave; t < ngl; t += nt / kWave) {   // long columns a wave each
-            const uint32_t c = gcols[t];
-            const float s = abs_col_sum_wave(io.lu, col_ptr[c], col_ptr[c + 1], tid & (kWave - 1), wlds);
-            if (s == s) cm = fmax(cm, (double)s);
-        }
-        for (uint32_t t = ngl + tid; t < n; t += nt) {
-            const uint32_t c = gcols[t];
-            float s = 0.f;
-            for (uint32_t p = col_ptr[c]; p < col_ptr[c + 1]; ++p) s += fabsf(io.lu[p]);
-            if (s == s) cm = fmax(cm, (double)s);
-        }
-        pert = kPertFactor * (float)wg_max(cm, sh);
+        pert = wg_pert(Md, io.lu, sh, wlds);
     }
 }
 
-// Steps 1-4 (l0 = 0), or, after the interleaved launches of steps [0, l0)
-// (k_factor_grid_il; GESP value in io.norms[0]), |b|_inf into io.norms[1]
-// with x = 0 and r = b, steps l0.. of step 3 and step 4.
+// Steps 1-4 (l0 = 0), or, after the launches of steps [0, l0) (interleaved,
+// k_factor_grid_il, or phases; GESP value in io.norms[0]), |b|_inf into
+// io.norms[1] with x = 0 and r = b, steps l0.. of step 3 and step 4.
+// d0: the first division item still to do.
 template <bool kCopy>
 __device__ __forceinline__ void wg_factor(const MatDesc *Md, const MatIO &io, int perturb, double *sh, float *wlds,
-                                          int l0)
+                                          int l0, uint32_t d0)
 {
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
     double bnorm = 0.0;
@@ -2584,7 +2592,7 @@ __device__ __forceinline__ void wg_factor(const MatDesc *Md, const MatIO &io, in
     {
         FactorDev F = Md->f;
         globalize(F);
-        factor_all_wg(F, io.lu, g_lds_vec, pert, perturb, wlds, l0);
+        factor_all_wg(F, io.lu, g_lds_vec, pert, perturb, wlds, l0, d0);
     }
 
     // 4. the factors copied into the sweeps' task-contiguous layout, built
@@ -2958,7 +2966,7 @@ __global__ void __launch_bounds__(1024) k_batch_same_factor(const MatDesc *__res
     __shared__ double sh[1024 / kWave];
     __shared__ __attribute__((aligned(16))) float wl[1024 / kWave][kWave];
     const MatIO io = batch_io(desc, ax, b, x, lu, lucsr, t32, r64, norms, kry, iters, eta);
-    wg_factor<kCopy>(desc, io, perturb, sh, wl[threadIdx.x / kWave], l0);
+    wg_factor<kCopy>(desc, io, perturb, sh, wl[threadIdx.x / kWave], l0, l0 > 0 ? desc->f.dvd_ptr[l0 - 1] : 0u);
 }
 
 // Refresh + factor only (glu_batch_factor): matrix blockIdx.x of a
@@ -2975,7 +2983,7 @@ __global__ void __launch_bounds__(1024) k_batch_factor(const MatDesc *__restrict
     io.ax = glb(ax + (uint64_t)blockIdx.x * desc->r.nnz_a);
     io.lu = glb(lu + (uint64_t)blockIdx.x * desc->nnz);
     if (l0 > 0) io.norms = glb(norms + 2 * (uint64_t)blockIdx.x);
-    wg_factor<false>(desc, io, perturb, sh, wl[threadIdx.x / kWave], l0);
+    wg_factor<false>(desc, io, perturb, sh, wl[threadIdx.x / kWave], l0, l0 > 0 ? desc->f.dvd_ptr[l0 - 1] : 0u);
 }
 
 // Dynamic LDS: the sweeps' ready bits (and correction vector).
@@ -3014,7 +3022,7 @@ __global__ void __launch_bounds__(1024) k_batch_same_fused(const MatDesc *__rest
     __shared__ __attribute__((aligned(16))) float wl[1024 / kWave][kWave];
     static_assert(sizeof(double) * kKrylovLds <= sizeof(wl), "Arnoldi scalars exceed the wave slices");
     const MatIO io = batch_io(desc, ax, b, x, lu, lucsr, t32, r64, norms, kry, iters, eta);
-    wg_factor<true>(desc, io, perturb, sh, wl[threadIdx.x / kWave], l0);
+    wg_factor<true>(desc, io, perturb, sh, wl[threadIdx.x / kWave], l0, l0 > 0 ? desc->f.dvd_ptr[l0 - 1] : 0u);
     __syncthreads();
     // the refinement's Arnoldi scalars take the factorization's wave slices
     // (static LDS no larger than k_batch_same_factor's)
@@ -3227,18 +3235,82 @@ __global__ void __launch_bounds__(256) k_sw_prod(const SwProd *__restrict__ prod
     lucsr[p.val] = lu[p.vpos] * xg[p.col];
 }
 
-// Distinct patterns: workgroup g runs matrix order[g] with its own tables.
+// Distinct patterns.  Members with phases first: their values (blocks of
+// kGroupValues positions of a member), with GESP each one's value (a
+// workgroup a member) into norms[0], then phase by phase the bins and the
+// assembly of all of them side by side (items {member, block | bin | first
+// wave}).
+constexpr uint32_t kGroupValues = 1024;
+
+__global__ void __launch_bounds__(256) k_group_values(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
+                                                      const uint2 *__restrict__ items)
+{
+    const uint2 it = items[blockIdx.x];
+    RefineDev R = descs[it.x].r;
+    globalize(R);
+    const double *ax = glb(ios[it.x].ax);
+    float *lu = glb(ios[it.x].lu);
+    const uint32_t nnz = descs[it.x].nnz;
+#pragma unroll
+    for (uint32_t u = 0; u < kGroupValues / 256; ++u) {
+        const uint32_t p = it.y * kGroupValues + u * 256 + threadIdx.x;
+        if (p < nnz) refresh_entry(R, ax, lu, p);
+    }
+}
+
+__global__ void __launch_bounds__(1024) k_group_pert(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
+                                                     const uint32_t *__restrict__ order, const int32_t *__restrict__ l0)
+{
+    __shared__ double sh[1024 / kWave];
+    __shared__ __attribute__((aligned(16))) float wl[1024 / kWave][kWave];
+    const uint32_t m = order[blockIdx.x];
+    if (l0[m] == 0) return;   // its factor kernel forms the value itself
+    const float pert = wg_pert(descs + m, glb(ios[m].lu), sh, wl[threadIdx.x / kWave]);
+    if (threadIdx.x == 0) glb(ios[m].norms)[0] = (double)pert;
+}
+
+__global__ void __launch_bounds__(1024) k_group_phase(const PhaseDev *__restrict__ phases, const MatIO *__restrict__ ios,
+                                                      const uint2 *__restrict__ items, int perturb)
+{
+    const uint2 it = items[blockIdx.x];
+    const float pert = perturb ? (float)glb(ios[it.x].norms)[0] : 0.f;
+    WinDev W = glb(phases[it.x].bin)[it.y];
+    W.pos = glb(W.pos);
+    W.prog = glb(W.prog);
+    W.hdr = glb(W.hdr);
+    W.wptr = glb(W.wptr);
+    factor_window<true>(W, glb(ios[it.x].lu), g_lds_vec, pert, perturb, glb(phases[it.x].out));
+}
+
+__global__ void __launch_bounds__(256) k_group_assemble(const PhaseDev *__restrict__ phases,
+                                                        const MatIO *__restrict__ ios, const uint2 *__restrict__ items)
+{
+    __shared__ __attribute__((aligned(16))) float lds[256 / kWave][kWave];
+    const uint2 it = items[blockIdx.x];
+    PhaseDev Ph = phases[it.x];
+    Ph.grp = glb(Ph.grp);
+    Ph.tgt = glb(Ph.tgt);
+    Ph.cnt = glb(Ph.cnt);
+    Ph.wav = glb(Ph.wav);
+    Ph.out = glb(Ph.out);
+    phase_assemble(Ph, glb(ios[it.x].lu), __builtin_amdgcn_readfirstlane(it.y + threadIdx.x / kWave),
+                   threadIdx.x & (kWave - 1), lds[threadIdx.x / kWave]);
+}
+
+// Then workgroup g runs matrix order[g] with its own tables, from step
+// l0[order[g]].
 template <bool kCopy>
 __global__ void __launch_bounds__(1024) k_batch_group_factor(const MatDesc *__restrict__ descs,
                                                              const MatIO *__restrict__ ios,
-                                                             const uint32_t *__restrict__ order, int perturb)
+                                                             const uint32_t *__restrict__ order,
+                                                             const int32_t *__restrict__ l0, int perturb)
 {
     __shared__ double sh[1024 / kWave];
     __shared__ __attribute__((aligned(16))) float wl[1024 / kWave][kWave];
     const uint32_t m = order[blockIdx.x];
     MatIO io = ios[m];
     globalize(io);
-    wg_factor<kCopy>(descs + m, io, perturb, sh, wl[threadIdx.x / kWave], 0);
+    wg_factor<kCopy>(descs + m, io, perturb, sh, wl[threadIdx.x / kWave], l0[m], 0u);
 }
 
 template <int kMode>
@@ -3620,14 +3692,30 @@ void il_to_rows(const float *S, float *lu, uint32_t nnz, int batch, hipStream_t 
 uint32_t il_items_per_wave() { return kIlItems * kIlPer; }
 uint32_t il_group() { return kIl; }
 
-void batch_group(const MatDesc *descs, const void *ios, const uint32_t *order, int count, double tol,
+// The phases of a group's members (GroupLaunch: items on the device, their
+// counts by phase round).
+void group_phases(const MatDesc *descs, const void *ios, const uint32_t *order, int count, const int32_t *l0,
+                  const GroupLaunch &G, int perturb, int threads, hipStream_t st)
+{
+    const MatIO *io = static_cast<const MatIO *>(ios);
+    if (G.nvalues == 0) return;
+    k_group_values<<<G.nvalues, 256, 0, st>>>(descs, io, G.values);
+    if (perturb) k_group_pert<<<count, threads, 0, st>>>(descs, io, order, l0);
+    for (uint32_t r = 0; r < G.rounds; ++r) {
+        k_group_phase<<<G.nbin[r], G.threads, 4 * (size_t)(G.nslot[r] + kWinExtra), st>>>(G.phase[r], io, G.bins[r],
+                                                                                         perturb);
+        if (G.nasm[r]) k_group_assemble<<<G.nasm[r], 256, 0, st>>>(G.phase[r], io, G.asms[r]);
+    }
+}
+
+void batch_group(const MatDesc *descs, const void *ios, const uint32_t *order, int count, const int32_t *l0, double tol,
                  int maxit, int perturb, int threads, int mode, size_t fact_lds, size_t ref_lds, hipStream_t st)
 {
     const MatIO *io = static_cast<const MatIO *>(ios);
     if (mode == kSweepLevels)
-        k_batch_group_factor<false><<<count, threads, fact_lds, st>>>(descs, io, order, perturb);
+        k_batch_group_factor<false><<<count, threads, fact_lds, st>>>(descs, io, order, l0, perturb);
     else
-        k_batch_group_factor<true><<<count, threads, fact_lds, st>>>(descs, io, order, perturb);
+        k_batch_group_factor<true><<<count, threads, fact_lds, st>>>(descs, io, order, l0, perturb);
     if (mode == kSweepLds)
         k_batch_group_refine<kSweepLds><<<count, threads, ref_lds, st>>>(descs, io, order, tol, maxit);
     else if (mode == kSweepFlags)   // per matrix: vector in LDS where it fits ref_lds
@@ -3698,6 +3786,7 @@ size_t enable_lds()
         reinterpret_cast<const void *>(&k_tri_df),
         reinterpret_cast<const void *>(&k_factor_window),
         reinterpret_cast<const void *>(&k_factor_phase),
+        reinterpret_cast<const void *>(&k_group_phase),
     };
     // the limit less the largest static LDS among them (their wave slices
     // and reduction arrays, ~4 KiB); 8 KiB if the attributes are unavailable
@@ -3730,6 +3819,7 @@ void zero_u64(unsigned long long *p, int count, hipStream_t st)
 }
 
 size_t matio_size() { return sizeof(MatIO); }
+uint32_t group_values() { return kGroupValues; }
 
 }  // namespace launch
 }  // namespace glu

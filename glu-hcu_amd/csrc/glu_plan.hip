@@ -66,7 +66,9 @@ void abft_cca(const FactorDev &F, const float *val, float *cca, int batch, hipSt
 void abft_check(const FactorDev &F, const uint32_t *row_idx, const uint32_t *diag, const float *lu,
                 const float *cca, float *ccl, float tol, int32_t *first_bad, float *max_diff, int batch,
                 hipStream_t st);
-void batch_group(const MatDesc *descs, const void *ios, const uint32_t *order, int count, double tol,
+void group_phases(const MatDesc *descs, const void *ios, const uint32_t *order, int count, const int32_t *l0,
+                  const GroupLaunch &G, int perturb, int threads, hipStream_t st);
+void batch_group(const MatDesc *descs, const void *ios, const uint32_t *order, int count, const int32_t *l0, double tol,
                  int maxit, int perturb, int threads, int mode, size_t fact_lds, size_t ref_lds, hipStream_t st);
 void tri_df(const TriDev &T, const float *lu, float *x, int l0, int l1, uint32_t k0, uint32_t k1, uint32_t n,
             int threads, hipStream_t st);
@@ -88,6 +90,7 @@ void sweeps_df(const MatDesc *desc, const float *lucsr, float *t32, uint32_t r0,
 void adjoint_values(const RefineDev &R, const double *lam, const double *x, double *grad, uint32_t n,
                     hipStream_t st);
 size_t matio_size();
+uint32_t group_values();
 }  // namespace launch
 }  // namespace glu
 
@@ -322,6 +325,8 @@ struct glu_plan {
 
     std::vector<Segment> fsegs;
     std::vector<PhaseDev> phases;
+    std::vector<std::vector<uint32_t>> phase_work;   // chunks of each phase's bins
+    int phase_lev = 0;           // steps the phases cover
     TriHost tri[4];          // lo, up, tup, tlo
     bool tri_dataflow = false;   // fused solve segments run barrier-free
     int solve_df_opt = 0;        // glu_plan_opts.solve_dataflow
@@ -2793,6 +2798,9 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         d.nwav = (uint32_t)phases[k].wav.size();
         d.nslot = phases[k].nslot;
         p->phases.push_back(d);
+        p->phase_work.emplace_back();
+        for (const Window &w : phases[k].bin) p->phase_work.back().push_back((uint32_t)w.hdr.size());
+        p->phase_lev = phases[k].l1;
     }
     {
         std::vector<WinDev> wd(wins.size());
@@ -3633,6 +3641,9 @@ struct glu_group {
     MatDesc *d_descs = nullptr;
     MatIOHost *d_ios = nullptr;
     uint32_t *d_order = nullptr;
+    char *d_items = nullptr;       // the leading launches' items and phases, l0
+    int32_t *d_l0 = nullptr;       // by member: steps its phases cover
+    GroupLaunch lead[kMaxGroupSplit + 1];   // by the number of members split off
     float *d_t32 = nullptr;
     double *d_r64 = nullptr;
     float *d_lucsr = nullptr;
@@ -3660,6 +3671,7 @@ struct glu_group {
         if (d_descs) (void)hipFree(d_descs);
         if (d_ios) (void)hipFree(d_ios);
         if (d_order) (void)hipFree(d_order);
+        if (d_items) (void)hipFree(d_items);
         if (d_t32) (void)hipFree(d_t32);
         if (d_r64) (void)hipFree(d_r64);
     }
@@ -3710,6 +3722,69 @@ extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_gr
     HIP_TRY(hipMalloc(&g->d_lucsr, sizeof(float) * ftot));
     HIP_TRY(hipMalloc(&g->d_norms, 2 * sizeof(double) * count));
     if (ktot) HIP_TRY(hipMalloc(&g->d_kry, sizeof(double) * ktot));
+    // The leading launches (for every number of members that may be split
+    // off): blocks of values, then bins (those with the most work first) and
+    // assembly blocks of each phase round.
+    {
+        std::vector<int32_t> l0(count, 0);
+        for (int i = 0; i < count; ++i)
+            l0[i] = plans[i]->phases.size() <= kGroupRounds ? plans[i]->phase_lev : 0;
+        std::vector<PhaseDev> ph[kGroupRounds];
+        for (uint32_t r = 0; r < kGroupRounds; ++r) {
+            ph[r].resize(count);
+            for (int i = 0; i < count; ++i)
+                if (l0[i] && r < plans[i]->phases.size()) ph[r][i] = plans[i]->phases[r];
+        }
+        std::vector<uint2> items;
+        size_t first[kMaxGroupSplit + 1][1 + 2 * kGroupRounds];
+        for (int sp = 0; sp <= kMaxGroupSplit; ++sp) {
+            GroupLaunch &G = g->lead[sp];
+            G.threads = kPhaseWaves * 64;
+            std::vector<uint32_t> mem(order.begin() + std::min(sp, count), order.end());
+            first[sp][0] = items.size();
+            for (uint32_t m : mem)
+                for (uint32_t b = 0; l0[m] && b * (uint64_t)launch::group_values() < plans[m]->nnz; ++b)
+                    items.push_back(make_uint2(m, b));
+            G.nvalues = (uint32_t)(items.size() - first[sp][0]);
+            for (uint32_t r = 0; r < kGroupRounds; ++r) {
+                first[sp][1 + 2 * r] = items.size();
+                for (uint32_t m : mem)
+                    if (l0[m] && r < plans[m]->phases.size()) {
+                        G.rounds = std::max(G.rounds, r + 1);
+                        G.nslot[r] = std::max(G.nslot[r], ph[r][m].nslot);
+                        for (uint32_t b = 0; b < ph[r][m].nbin; ++b) items.push_back(make_uint2(m, b));
+                    }
+                std::stable_sort(items.begin() + first[sp][1 + 2 * r], items.end(), [&](const uint2 &a, const uint2 &b) {
+                    return plans[a.x]->phase_work[r][a.y] > plans[b.x]->phase_work[r][b.y];
+                });
+                G.nbin[r] = (uint32_t)(items.size() - first[sp][1 + 2 * r]);
+                first[sp][2 + 2 * r] = items.size();
+                for (uint32_t m : mem)
+                    if (l0[m] && r < plans[m]->phases.size())
+                        for (uint32_t w = 0; w < ph[r][m].nwav + ph[r][m].ngrp; w += 4) items.push_back(make_uint2(m, w));
+                G.nasm[r] = (uint32_t)(items.size() - first[sp][2 + 2 * r]);
+            }
+        }
+        const size_t o_items = sizeof(PhaseDev) * count * kGroupRounds, o_l0 = o_items + sizeof(uint2) * items.size();
+        HIP_TRY(hipMalloc(&g->d_items, o_l0 + sizeof(int32_t) * count));
+        for (uint32_t r = 0; r < kGroupRounds; ++r)
+            HIP_TRY(hipMemcpy(g->d_items + sizeof(PhaseDev) * count * r, ph[r].data(), sizeof(PhaseDev) * count,
+                              hipMemcpyHostToDevice));
+        if (!items.empty())
+            HIP_TRY(hipMemcpy(g->d_items + o_items, items.data(), sizeof(uint2) * items.size(), hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(g->d_items + o_l0, l0.data(), sizeof(int32_t) * count, hipMemcpyHostToDevice));
+        g->d_l0 = reinterpret_cast<int32_t *>(g->d_items + o_l0);
+        const uint2 *it = reinterpret_cast<const uint2 *>(g->d_items + o_items);
+        for (int sp = 0; sp <= kMaxGroupSplit; ++sp) {
+            GroupLaunch &G = g->lead[sp];
+            G.values = it + first[sp][0];
+            for (uint32_t r = 0; r < kGroupRounds; ++r) {
+                G.phase[r] = reinterpret_cast<const PhaseDev *>(g->d_items) + (size_t)count * r;
+                G.bins[r] = it + first[sp][1 + 2 * r];
+                G.asms[r] = it + first[sp][2 + 2 * r];
+            }
+        }
+    }
     HIP_TRY(hipMemcpy(g->d_descs, descs.data(), sizeof(MatDesc) * count, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(g->d_order, order.data(), sizeof(uint32_t) * count, hipMemcpyHostToDevice));
     *out = g.release();
@@ -3792,8 +3867,10 @@ extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, c
             const size_t full = launch::batch_lds_bytes(2, p->n);
             ref_lds = std::max(ref_lds, full <= cap ? full : launch::batch_lds_bytes(1, p->n));
         }
-    launch::batch_group(g->d_descs, g->d_ios, g->d_order + nsplit, count - nsplit, tol, maxit, perturb, g->threads,
-                        mode, tmax, ref_lds, st);
+    launch::group_phases(g->d_descs, g->d_ios, g->d_order + nsplit, count - nsplit, g->d_l0, g->lead[nsplit], perturb,
+                         g->threads, st);
+    launch::batch_group(g->d_descs, g->d_ios, g->d_order + nsplit, count - nsplit, g->d_l0, tol, maxit, perturb,
+                        g->threads, mode, tmax, ref_lds, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(GLU_ERR_DEVICE, std::string("group launch: ") + hipGetErrorString(e));
     for (int j = 0; j < nsplit; ++j) HIP_TRY(hipStreamWaitEvent(st, g->ev_aux[j], 0));

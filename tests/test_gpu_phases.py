@@ -84,3 +84,30 @@ def test_phases_match_oracle(name, values):
         want = factor(pat, lu.cpu().numpy(), perturb=perturb)[0]
         plan.factor(lu, perturb=perturb)
         assert np.array_equal(lu.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("perturb", [False, True])
+@pytest.mark.parametrize("split", [0, 1])
+def test_group_phases_match_single_path(split, perturb):
+    """Members with and without phases in one group: every member's factors
+    equal its own single-path factors, twice on other value sets, and every
+    backward error meets the tolerance."""
+    import torch
+    from pyglu import mna
+    from pyglu.analysis import Analysis
+    from pyglu.device import Group, Plan
+    mats = [CASES[k]() for k in ("unsym1500", "many", "mna2k", "lane", "one")] + [mna_case("small")]
+    plans = [Plan(Analysis(*m), lds_windows=1, lds_window_values=700) for m in mats]
+    plans.append(Plan(Analysis(*mats[2])))   # one window, no phase
+    mats.append(mats[2])
+    g = Group(plans, split=split)
+    for seed in (1, 2):
+        axs = [torch.from_numpy(mna.perturb_values(m[0], seed)).cuda() for m in mats]
+        bs = [torch.from_numpy(mna.rhs(m[3], seed)).cuda() for m in mats]
+        xs, lus, iters, eta = g.solve(axs, bs, tol=1e-10, maxit=20, perturb=perturb)
+        for i, (p, ax) in enumerate(zip(plans, axs)):
+            lu = p.refresh(ax).reshape(-1)
+            p.factor(lu, perturb=perturb)
+            assert torch.equal(lu.view(torch.int32), lus[i].view(torch.int32)), (seed, i)
+        assert float(eta.max()) <= 1e-10
+    g.close()
