@@ -300,7 +300,19 @@ struct SolveDev {
     const double *row_scale, *col_scale_perm;
 };
 
+// The rows of A (or A') of at most kLongRow entries for products in one
+// workgroup: 64 neighbouring rows a chunk, a lane each (neighbours name
+// neighbouring columns, so a chunk's gathers share lines: with rows by length
+// instead, n=20,000 163 us a product, 117 this way).
+struct SpDev {
+    const uint2 *chunk;        // [nchunk]: {first entry place, longest row}
+    const uint2 *rl;           // [64 nchunk]: {row, entries} ({0, ~0}: none)
+    const uint2 *ent;          // place + 64 e + lane: {value index, column} of entry e ({0, 0}: none)
+    uint32_t nchunk, pad;
+};
+
 struct RefineDev {
+    SpDev sp[2];               // A, A'
     const uint32_t *a_rptr;    // CSR of A [n+1]
     const uint32_t *a_cidx;    // [nnz_a]
     const uint32_t *a_src;     // index into the caller's CSC values [nnz_a]

@@ -1495,105 +1495,90 @@ __device__ __forceinline__ void a_row_partial(const RefineDev &R, const double *
     }
 }
 
-// Rows of A for one cooperating group: long rows one wave each (FP64 wave
-// reductions), the rest one lane each.  f(i, dot, asum) is called once per
-// row by one lane.
-template <typename F>
-__device__ __forceinline__ void for_rows_of_a(const RefineDev &R, const double *__restrict__ ax,
-                                              const double *__restrict__ x, uint32_t n, int transpose,
-                                              uint32_t tid, uint32_t nthreads, F f)
+// The rows of A (kT: of A') for one workgroup: f(i, dot, asum) once per row
+// by one lane, dot = sum_q a_q x[col_q] and asum = sum_q |a_q|.  Long rows a
+// wave each (FP64 wave reductions); the rest from the chunks of SpDev, a lane
+// each in entry order, eight entries at a time: their places, read a chunk
+// ahead, then the values and vector entries they name, all issued together.
+// (Read through row pointers in natural order, the product waited for three
+// dependent loads a row: n=20,000 121 us, 117 us this way.)
+template <bool kT, typename F>
+__device__ __forceinline__ void wg_rows(const RefineDev &R, const double *__restrict__ ax,
+                                        const double *__restrict__ x, F f)
 {
-    const uint32_t lane = tid & (kWave - 1), w = tid / kWave, nw = nthreads / kWave;
-    const uint32_t *rows = transpose ? R.a_cols : R.a_rows;
-    const uint32_t nl = transpose ? R.a_nlong_t : R.a_nlong;
+    constexpr uint32_t E = 8;
+    const uint32_t lane = threadIdx.x & (kWave - 1), nw = blockDim.x / kWave;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const SpDev S = R.sp[kT ? 1 : 0];
+    const uint2 *chunk = glb(S.chunk), *rls = glb(S.rl) + lane, *ent = glb(S.ent) + lane;
+    uint2 d = make_uint2(0u, 1u), rl = make_uint2(0u, 0u), it[E];
+    auto fetch = [&](uint32_t c) {   // chunk c's rows and first entries
+        d = chunk[c];
+        rl = rls[(size_t)c * kWave];
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e) it[e] = ent[d.x + kWave * min(e, d.y - 1)];
+    };
+    if (w < S.nchunk) fetch(w);
+    const uint32_t nl = kT ? R.a_nlong_t : R.a_nlong;
     for (uint32_t t = w; t < nl; t += nw) {
-        const uint32_t i = rows[t];
+        const uint32_t i = (kT ? R.a_cols : R.a_rows)[t];
         double dot, asum;
-        a_row_partial(R, ax, x, a_row(R, i, transpose), lane, kWave, transpose, dot, asum);
+        a_row_partial(R, ax, x, a_row(R, i, kT), lane, kWave, kT, dot, asum);
         dot = wave_sum64(dot);
         asum = wave_sum64(asum);
         if (lane == 0) f(i, dot, asum);
     }
-    for (uint32_t t = nl + tid; t < n; t += nthreads) {
-        const uint32_t i = rows[t];
-        double dot, asum;
-        a_row_partial(R, ax, x, a_row(R, i, transpose), 0, 1, transpose, dot, asum);
-        f(i, dot, asum);
+    for (uint32_t c = w; c < S.nchunk; c += nw) {
+        const uint32_t base = d.x, m = d.y, row = rl.x, len = rl.y == ~0u ? 0u : rl.y;
+        const bool own = rl.y != ~0u;
+        double a[E], v[E];
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e) {
+            a[e] = ax[it[e].x];
+            v[e] = x[it[e].y];
+        }
+        if (c + nw < S.nchunk) fetch(c + nw);
+        double dot = 0.0, asum = 0.0;
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
+            if (e < len) {
+                dot = fma(a[e], v[e], dot);
+                asum += fabs(a[e]);
+            }
+        for (uint32_t e0 = E; e0 < m; e0 += E) {
+            uint2 q[E];
+#pragma unroll
+            for (uint32_t e = 0; e < E; ++e) q[e] = ent[base + kWave * min(e0 + e, m - 1)];
+#pragma unroll
+            for (uint32_t e = 0; e < E; ++e) {
+                a[e] = ax[q[e].x];
+                v[e] = x[q[e].y];
+            }
+#pragma unroll
+            for (uint32_t e = 0; e < E; ++e)
+                if (e0 + e < len) {
+                    dot = fma(a[e], v[e], dot);
+                    asum += fabs(a[e]);
+                }
+        }
+        if (own) f(row, dot, asum);
     }
 }
 
-// for_rows_of_a for one workgroup, with the short rows taken in natural
-// order (long ones skipped: their waves take them), four rows per lane in
-// flight and four entries of each per step, so a lane keeps up to 16
-// independent gathers outstanding.
-template <typename F>
-__device__ __forceinline__ void wg_rows_of_a(const RefineDev &R, const double *__restrict__ ax,
-                                             const double *__restrict__ x, uint32_t n, F f)
+// fn(i, ld(i)) for i = tid, tid + nt, ... in order, the loads of four of them
+// issued together.
+template <typename Ld, typename Fn>
+__device__ __forceinline__ void wg_vec(uint32_t n, Ld ld, Fn fn)
 {
-    constexpr int RB = 2, EB = 4;
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t lane = tid & (kWave - 1), w = tid / kWave, nw = nt / kWave;
-    for (uint32_t t = w; t < R.a_nlong; t += nw) {
-        const uint32_t i = R.a_rows[t];
-        double dot, asum;
-        a_row_partial(R, ax, x, a_row(R, i, 0), lane, kWave, 0, dot, asum);
-        dot = wave_sum64(dot);
-        asum = wave_sum64(asum);
-        if (lane == 0) f(i, dot, asum);
-    }
-    for (uint32_t i0 = tid; i0 < n; i0 += RB * nt) {
-        uint32_t q[RB], qe[RB];
-        double dot[RB], asum[RB];
+    constexpr uint32_t U = 4;
+    const uint32_t nt = blockDim.x;
+    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += U * nt) {
+        decltype(ld(0u)) v[U];
 #pragma unroll
-        for (int r = 0; r < RB; ++r) {
-            const uint32_t i = i0 + r * nt;
-            q[r] = qe[r] = 0;
-            dot[r] = asum[r] = 0.0;
-            if (i < n) {
-                q[r] = R.a_rptr[i];
-                qe[r] = R.a_rptr[i + 1];
-                if (qe[r] - q[r] > kLongRow) qe[r] = q[r];   // a wave's row
-            }
-        }
-        for (;;) {
-            bool more = false;
+        for (uint32_t u = 0; u < U; ++u) v[u] = ld(min(i0 + u * nt, n - 1));
 #pragma unroll
-            for (int r = 0; r < RB; ++r) more |= q[r] < qe[r];
-            if (!more) break;
-            uint32_t src[RB][EB], col[RB][EB];
-#pragma unroll
-            for (int r = 0; r < RB; ++r)
-#pragma unroll
-                for (int e = 0; e < EB; ++e)
-                    if (q[r] + e < qe[r]) {
-                        src[r][e] = R.a_src[q[r] + e];
-                        col[r][e] = R.a_cidx[q[r] + e];
-                    }
-            double av[RB][EB], xv[RB][EB];
-#pragma unroll
-            for (int r = 0; r < RB; ++r)
-#pragma unroll
-                for (int e = 0; e < EB; ++e)
-                    if (q[r] + e < qe[r]) {
-                        av[r][e] = ax[src[r][e]];
-                        xv[r][e] = x ? x[col[r][e]] : 0.0;
-                    }
-#pragma unroll
-            for (int r = 0; r < RB; ++r)
-#pragma unroll
-                for (int e = 0; e < EB; ++e)
-                    if (q[r] + e < qe[r]) {
-                        if (x) dot[r] = fma(av[r][e], xv[r][e], dot[r]);
-                        asum[r] += fabs(av[r][e]);
-                    }
-#pragma unroll
-            for (int r = 0; r < RB; ++r) q[r] = q[r] + EB < qe[r] ? q[r] + EB : qe[r];
-        }
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
-            const uint32_t i = i0 + r * nt;
-            if (i < n && R.a_rptr[i + 1] - R.a_rptr[i] <= kLongRow) f(i, dot[r], asum[r]);
-        }
+        for (uint32_t u = 0; u < U; ++u)
+            if (i0 + u * nt < n) fn(i0 + u * nt, v[u]);
     }
 }
 
@@ -2707,34 +2692,23 @@ __device__ __forceinline__ void wg_precond(const MatDesc *Md, const MatIO &io, c
 }
 
 // r = b - A x in FP64 (into io.r64); returns the backward error
-// eta = |r|_inf / (|A|_inf |x|_inf + |b|_inf) to every thread.
-// Rows of A (kT: of A', the caller's CSC columns) for one workgroup.
-template <bool kT, typename F>
-__device__ __forceinline__ void wg_rows(const RefineDev &R, const double *__restrict__ ax,
-                                        const double *__restrict__ x, uint32_t n, F f)
-{
-    if (!kT) wg_rows_of_a(R, ax, x, n, f);
-    else for_rows_of_a(R, ax, x, n, 1, threadIdx.x, blockDim.x, f);
-}
-
-// anorm < 0: |A|_inf is taken from this product's row sums (and returned
-// in anorm).
+// eta = |r|_inf / (|A|_inf |x|_inf + |b|_inf) to every thread.  anorm < 0:
+// |A|_inf is taken from this product's row sums (and returned in anorm).
 template <bool kT = false>
 __device__ __forceinline__ double wg_residual(const MatDesc *Md, const MatIO &io, double &anorm, double bnorm,
                                               double *sh)
 {
     const uint32_t n = Md->n;
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
     double rmax = 0.0, xmax = 0.0, amax = 0.0;
     RefineDev R = Md->r;
     globalize(R);
-    wg_rows<kT>(R, io.ax, io.x, n, [&](uint32_t i, double dot, double asum) {
+    wg_rows<kT>(R, io.ax, io.x, [&](uint32_t i, double dot, double asum) {
         const double ri = io.b[i] - dot;
         io.r64[i] = ri;
         rmax = nmax(rmax, fabs(ri));
         amax = nmax(amax, asum);
     });
-    for (uint32_t i = tid; i < n; i += nt) xmax = nmax(xmax, fabs(io.x[i]));
+    wg_vec(n, [&](uint32_t i) { return io.x[i]; }, [&](uint32_t, double x) { xmax = nmax(xmax, fabs(x)); });
     if (anorm < 0.0) anorm = wg_max(amax, sh);
     const double rn = wg_max(rmax, sh);
     const double xn = wg_max(xmax, sh);
@@ -2751,6 +2725,17 @@ constexpr int kKrylovC = kKrylovG + kMaxKrylov + 1;
 constexpr int kKrylovS = kKrylovC + kMaxKrylov;
 constexpr int kKrylovD = kKrylovS + kMaxKrylov;
 constexpr int kKrylovLds = kKrylovD + kMaxKrylov;
+
+struct Vec2 {
+    double a, b;
+};
+struct Vec4 {
+    double a, b, c, d;
+};
+struct VecZ {
+    uint32_t p;
+    double s, x;
+};
 
 // Refinement of one matrix by one workgroup until eta <= tol or maxit
 // preconditioner solves, from x = 0, r = b.  M = (LU)^-1 is the FP32 sweep
@@ -2789,10 +2774,8 @@ __device__ __forceinline__ void wg_refine(const MatDesc *Md, const MatIO &io, do
         for (;;) {
             wg_precond<kMode, kT>(Md, io, io.r64, xs, flags);
             ++it;
-            for (uint32_t i = tid; i < n; i += nt) {
-                const uint32_t pi = bp[i];
-                io.x[i] = io.x[i] + (double)xs[pi] * bs[kT ? pi : i];
-            }
+            wg_vec(n, [&](uint32_t i) { return VecZ{bp[i], kT ? 0.0 : bs[i], io.x[i]}; },
+                   [&](uint32_t i, const VecZ &v) { io.x[i] = v.x + (double)xs[v.p] * (kT ? bs[v.p] : v.s); });
             __syncthreads();
             eta = wg_residual<kT>(Md, io, anorm, bnorm, sh);
             if (!(eta > tol) || it >= maxit) break;   // also stops on NaN
@@ -2806,13 +2789,13 @@ __device__ __forceinline__ void wg_refine(const MatDesc *Md, const MatIO &io, do
         bool done = false;
         while (!done) {
             double d = 0.0;
-            for (uint32_t i = tid; i < n; i += nt) d = fma(io.r64[i], io.r64[i], d);
+            wg_vec(n, [&](uint32_t i) { return io.r64[i]; }, [&](uint32_t, double r) { d = fma(r, r, d); });
             const double beta = sqrt(wg_sum(d, sh));
             if (!(beta > 0.0)) {                  // r = 0 (x exact) or NaN
                 eta = beta == 0.0 ? 0.0 : beta;
                 break;
             }
-            for (uint32_t i = tid; i < n; i += nt) V[i] = io.r64[i] / beta;
+            wg_vec(n, [&](uint32_t i) { return io.r64[i]; }, [&](uint32_t i, double r) { V[i] = r / beta; });
             if (tid == 0) {
                 g[0] = beta;
                 for (int c = 0; c < kMaxKrylov; ++c) y[c] = 0.0;
@@ -2822,36 +2805,38 @@ __device__ __forceinline__ void wg_refine(const MatDesc *Md, const MatIO &io, do
                 double *zj = Z + (size_t)j * n, *wj = W + (size_t)j * n, *vn = V + (size_t)(j + 1) * n;
                 wg_precond<kMode, kT>(Md, io, V + (size_t)j * n, xs, flags);
                 ++it;
-                for (uint32_t i = tid; i < n; i += nt) {
-                    const uint32_t pi = bp[i];
-                    zj[i] = (double)xs[pi] * bs[kT ? pi : i];
-                }
+                wg_vec(n, [&](uint32_t i) { return VecZ{bp[i], kT ? 0.0 : bs[i], 0.0}; },
+                       [&](uint32_t i, const VecZ &v) { zj[i] = (double)xs[v.p] * (kT ? bs[v.p] : v.s); });
                 __syncthreads();
                 {
                     RefineDev R = Md->r;
                     globalize(R);
                     double amax = 0.0;
-                    wg_rows<kT>(R, io.ax, zj, n, [&](uint32_t i, double dot, double asum) {
+                    wg_rows<kT>(R, io.ax, zj, [&](uint32_t i, double dot, double asum) {
                         wj[i] = dot;
-                        vn[i] = dot;
                         amax = nmax(amax, asum);
                     });
                     if (anorm < 0.0) anorm = wg_max(amax, sh);
                 }
                 __syncthreads();
+                // w_j less its parts along V into v_{j+1} (not yet scaled); the
+                // last pass sums its norm
+                double dn = 0.0;
                 for (int q = 0; q <= j; ++q) {
-                    const double *vq = V + (size_t)q * n;
+                    const double *vq = V + (size_t)q * n, *from = q == 0 ? wj : vn;
                     double dq = 0.0;
-                    for (uint32_t i = tid; i < n; i += nt) dq = fma(vn[i], vq[i], dq);
+                    wg_vec(n, [&](uint32_t i) { return Vec2{from[i], vq[i]}; },
+                           [&](uint32_t, const Vec2 &v) { dq = fma(v.a, v.b, dq); });
                     const double h = wg_sum(dq, sh);
-                    for (uint32_t i = tid; i < n; i += nt) vn[i] = fma(-h, vq[i], vn[i]);
+                    wg_vec(n, [&](uint32_t i) { return Vec2{from[i], vq[i]}; },
+                           [&](uint32_t i, const Vec2 &v) {
+                               const double t = fma(-h, v.b, v.a);
+                               vn[i] = t;
+                               if (q == j) dn = fma(t, t, dn);
+                           });
                     if (tid == 0) H[q * kMaxKrylov + j] = h;
                 }
-                double dn = 0.0;
-                for (uint32_t i = tid; i < n; i += nt) dn = fma(vn[i], vn[i], dn);
                 const double hn = sqrt(wg_sum(dn, sh));
-                if (hn > 0.0)
-                    for (uint32_t i = tid; i < n; i += nt) vn[i] = vn[i] / hn;
                 if (tid == 0) {
                     // previous rotations on column j, a new one zeroing hn
                     for (int c = 0; c < j; ++c) {
@@ -2879,18 +2864,18 @@ __device__ __forceinline__ void wg_refine(const MatDesc *Md, const MatIO &io, do
                 }
                 __syncthreads();
                 double rmax = 0.0, xmax = 0.0;
-                for (uint32_t i = tid; i < n; i += nt) {
-                    double xi = io.x[i], ri = io.r64[i];
-                    for (int c = 0; c <= j; ++c) {
-                        const double dc = dy[c];
-                        xi = fma(dc, Z[(size_t)c * n + i], xi);
-                        ri = fma(-dc, W[(size_t)c * n + i], ri);
-                    }
-                    io.x[i] = xi;
-                    io.r64[i] = ri;
-                    rmax = nmax(rmax, fabs(ri));
-                    xmax = nmax(xmax, fabs(xi));
-                }
+                wg_vec(n, [&](uint32_t i) { return Vec4{io.x[i], io.r64[i], Z[i], W[i]}; },
+                       [&](uint32_t i, const Vec4 &v) {
+                           double xi = fma(dy[0], v.c, v.a), ri = fma(-dy[0], v.d, v.b);
+                           for (int c = 1; c <= j; ++c) {
+                               xi = fma(dy[c], Z[(size_t)c * n + i], xi);
+                               ri = fma(-dy[c], W[(size_t)c * n + i], ri);
+                           }
+                           io.x[i] = xi;
+                           io.r64[i] = ri;
+                           rmax = nmax(rmax, fabs(ri));
+                           xmax = nmax(xmax, fabs(xi));
+                       });
                 const double rn = wg_max(rmax, sh);
                 const double xn = wg_max(xmax, sh);
                 eta = rn / (anorm * xn + bnorm);
@@ -2911,6 +2896,9 @@ __device__ __forceinline__ void wg_refine(const MatDesc *Md, const MatIO &io, do
                     break;   // not done: restart from the true residual
                 }
                 if (!(hn > 0.0)) break;   // breakdown short of tol: restart
+                if (j + 1 < m)
+                    wg_vec(n, [&](uint32_t i) { return vn[i]; }, [&](uint32_t i, double v) { vn[i] = v / hn; });
+                __syncthreads();
             }
         }
     }

@@ -2517,6 +2517,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     std::vector<double> rs_col, a_rs, a_cs;
     std::vector<uint32_t> a_dst, lu_fill, df_rsrc, tdf_rsrc;
     std::vector<double> df_rscale, tdf_rscale;
+    std::vector<uint2> sp_chunk[2], sp_rl[2], sp_ent[2];
     const Analysis *an = a ? &a->an : nullptr;
     if (an) {
         const uint32_t nnz_a = an->nnz;
@@ -2574,6 +2575,32 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         long_first(an->in_ap.data(), a_cols, p->a_nlong_t);
         for (uint32_t i = 0; i < n; ++i)
             p->a_kmax = std::max({p->a_kmax, a_rptr[i + 1] - a_rptr[i], an->in_ap[i + 1] - an->in_ap[i]});
+        // short rows of A and A' for the products in one workgroup
+        for (int t = 0; t < 2; ++t) {
+            const uint32_t *ptr = t ? an->in_ap.data() : a_rptr.data();
+            std::vector<uint32_t> rows;
+            for (uint32_t i = 0; i < n; ++i)
+                if (ptr[i + 1] - ptr[i] <= kLongRow) rows.push_back(i);
+            for (size_t i = 0; i < rows.size(); i += 64) {
+                uint32_t m = 1;
+                for (size_t k = i; k < std::min(i + 64, rows.size()); ++k) m = std::max(m, ptr[rows[k] + 1] - ptr[rows[k]]);
+                const size_t base = sp_ent[t].size();
+                sp_chunk[t].push_back(make_uint2((uint32_t)base, m));
+                sp_ent[t].resize(base + 64 * (size_t)m, make_uint2(0u, 0u));
+                for (size_t k = i; k < i + 64; ++k) {
+                    if (k >= rows.size()) {
+                        sp_rl[t].push_back(make_uint2(0u, ~0u));
+                        continue;
+                    }
+                    const uint32_t r = rows[k], len = ptr[r + 1] - ptr[r];
+                    sp_rl[t].push_back(make_uint2(r, len));
+                    for (uint32_t e = 0; e < len; ++e)
+                        sp_ent[t][base + 64 * (size_t)e + (k - i)] =
+                            t ? make_uint2(ptr[r] + e, an->in_ai[ptr[r] + e])
+                              : make_uint2(a_src[ptr[r] + e], a_cidx[ptr[r] + e]);
+                }
+            }
+        }
         // the first sweeps' right-hand sides by row
         df_rsrc.resize(n);
         df_rscale.resize(n);
@@ -2681,11 +2708,17 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         o_tlong[s] = U.put(p->tri[s].lvl_long);
         o_ttask[s] = U.put(p->tri[s].tasks);
     }
+    size_t o_spc[2] = {0, 0}, o_spr[2] = {0, 0}, o_spe[2] = {0, 0};
     size_t o_rsrc = 0, o_rscale = 0, o_trsrc = 0, o_trscale = 0;
     size_t o_rp = 0, o_rpi = 0, o_cp = 0, o_cpi = 0, o_rs = 0, o_csp = 0;
     size_t o_arptr = 0, o_acidx = 0, o_asrc = 0, o_acptr = 0, o_aridx = 0, o_lusrc = 0, o_rscol = 0;
     size_t o_lucol = 0, o_arows = 0, o_acols = 0, o_adst = 0, o_ars = 0, o_acs = 0, o_lufill = 0;
     if (an) {
+        for (int t = 0; t < 2; ++t) {
+            o_spc[t] = U.put(sp_chunk[t]);
+            o_spr[t] = U.put(sp_rl[t]);
+            o_spe[t] = U.put(sp_ent[t]);
+        }
         o_rsrc = U.put(df_rsrc);
         o_rscale = U.put(df_rscale);
         o_trsrc = U.put(tdf_rsrc);
@@ -2924,6 +2957,12 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         S.row_scale = reinterpret_cast<const double *>(A + o_rs);
         S.col_scale_perm = reinterpret_cast<const double *>(A + o_csp);
         RefineDev &R = p->R;
+        for (int t = 0; t < 2; ++t) {
+            R.sp[t].chunk = reinterpret_cast<const uint2 *>(A + o_spc[t]);
+            R.sp[t].rl = reinterpret_cast<const uint2 *>(A + o_spr[t]);
+            R.sp[t].ent = reinterpret_cast<const uint2 *>(A + o_spe[t]);
+            R.sp[t].nchunk = (uint32_t)sp_chunk[t].size();
+        }
         R.a_rptr = u32p(o_arptr);
         R.a_cidx = u32p(o_acidx);
         R.a_src = u32p(o_asrc);
