@@ -217,11 +217,12 @@ struct DfDev {
 // vector is in LDS, values being their own ready marks.  A chunk is a wave's
 // unit: 64 lanes of four entries.  A row takes 1, 2, 4, 8 or 16 lanes
 // (aligned), lane j of the row its entries 4 j .. 4 j + 3 in the order the row
-// consumes them, rows of any size and level side by side in schedule order;
+// consumes them, rows of any size side by side in schedule order;
 // a row of more than 64 summed entries takes chunks of its own, lane j of
 // such a chunk holding entries j, 64 + j, 128 + j and 192 + j of its 256.
 //   meta[64 c + lane] = {slots of entries 0, 1 (16 bits each), of 2, 3,
-//     row slot | log2 lanes << 16 | kSwTree | kSwOn, 0}
+//     row slot | log2 lanes << 16 | kSwTree | kSwOn, the chunk's header}; in a
+//     chunk of a long row kSwEntry << e: the lane has entry e
 //   values: value c stride + 4 lane + e is entry e's, c stride + 256 + lane
 //     the row's pivot (div sweeps; at the lane that stores the row)
 //   a row's right-hand side: rhs[rpos[slot]], at its first lane
@@ -230,15 +231,18 @@ struct DfDev {
 // not in the part: their value is the finished product).  kSwTree: the
 // refinement sums the row's products by lane and then across its lanes;
 // other rows, and every row in the exact solve, are subtracted in order.
-constexpr uint32_t kSwTree = 1u << 20, kSwOn = 1u << 21;
+constexpr uint32_t kSwTree = 1u << 20, kSwOn = 1u << 21, kSwEntry = 1u << 16;
 constexpr uint32_t kSwLong = 1u << 31, kSwFirst = 1u << 30, kSwLast = 1u << 29;   // header bits
 constexpr uint32_t kSwHasTree = 1u << 28, kSwHasSeq = 1u << 27, kSwNarrow = 1u << 26;
 constexpr uint32_t kSwPassMask = 3u;   // header of a long chunk: passes of 64 used, less 1
+// header: the chunk's step (its rows' level among the part's levels: a chunk
+// holds rows of one level, whose dependencies ran in earlier steps)
+constexpr uint32_t kSwStepShift = 2, kSwStepMask = 0xffffffu;
 
 struct SwPart {
     uint32_t wp;               // wptr[wp + w] .. wptr[wp + w + 1]: wave w's chunks
     uint32_t s0, nslot;        // rows row[s0 + slot], right-hand sides rpos[s0 + slot]
-    uint32_t pad;
+    uint32_t steps;
 };
 
 // An entry whose column belongs to an earlier launch: value[val] = lu[vpos] * x[col].
@@ -248,7 +252,6 @@ struct SwProd {
 
 struct SwDev {
     const uint4 *meta;         // [64 chunks]
-    const uint32_t *hdr;       // [chunks]
     const uint32_t *wptr;
     const SwPart *part;
     const uint32_t *row, *rpos;

@@ -1741,7 +1741,6 @@ __device__ __forceinline__ void globalize(TriDev &T)
 __device__ __forceinline__ void globalize(SwDev &D)
 {
     D.meta = glb(D.meta);
-    D.hdr = glb(D.hdr);
     D.wptr = glb(D.wptr);
     D.part = glb(D.part);
     D.row = glb(D.row);
@@ -2171,6 +2170,15 @@ __device__ __forceinline__ void sw_put(float *xs, uint32_t r, float v)
     __hip_atomic_store(reinterpret_cast<uint32_t *>(xs) + r, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// A pointer that is the same in every lane, in scalar registers.
+template <typename T>
+__device__ __forceinline__ T *uniform(T *p)
+{
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return glb(reinterpret_cast<T *>((uint64_t)hi << 32 | lo));
+}
+
 // A chunk's prefetched data (SwDev).
 struct SwChunk {
     uint4 m;
@@ -2221,103 +2229,65 @@ __device__ __forceinline__ float sw_f(uint32_t b) { return __uint_as_float(b); }
 // Chunks [k, k1) of sweep D, in order, by one wave: values sv, right-hand
 // sides rhs, results into xs (LDS; kUnset but for the two constant slots).
 // Chunks load three ahead (a chunk is four loads, so the waits count).
-// kExact: every row's products are subtracted one at a time in the row's
-// order (the arithmetic of Symbolic_Matrix::solve); slice: the wave's 64
-// floats of LDS for its long rows.  While a row waits, the subtractions that
-// can be done are: from the last entry's arrival only its own lane's remain.
-template <bool kExact>
+// Every row's products are subtracted one at a time in the row's order (the
+// arithmetic of Symbolic_Matrix::solve); slice: the wave's 64 floats of LDS
+// for its long rows.  While a row waits, the subtractions that can be done
+// are: from the last entry's arrival only its own lane's remain.
 __device__ __forceinline__ void sw_wave(const SwDev &D, uint32_t k, uint32_t k1, const float *__restrict__ sv,
                                         const float *__restrict__ rhs, float *xs, float *slice)
 {
     if (k >= k1) return;
     const uint32_t lane = threadIdx.x & (kWave - 1), doff = D.div ? 256u : 0u, stride = D.stride;
+    const uint4 *meta = uniform(D.meta);
+    const float *val = uniform(sv), *rh = uniform(rhs);
     auto load = [&](uint32_t q) {
         q = min(q, k1 - 1);
-        const float *c = sv + (size_t)q * stride;
+        const float *c = val + (size_t)q * stride, *rr = rh + (size_t)q * kWave;   // (scalar bases, the lane's offset)
+        const uint4 *m = meta + (size_t)q * kWave;
         SwChunk t;
-        t.m = D.meta[(size_t)q * kWave + lane];
+        t.m = m[lane];
         t.v = reinterpret_cast<const float4 *>(c)[lane];
-        t.r = rhs[(size_t)q * kWave + lane];
-        t.d = c[doff + lane];
+        t.r = rr[lane];
+        t.d = (c + doff)[lane];
         return t;
     };
-    auto header = [&](uint32_t q) { return D.hdr[min(q + lane, k1 - 1)]; };   // 64 chunks', one a lane
     const uint32_t *X = reinterpret_cast<const uint32_t *>(xs);
     auto peek = [&](uint32_t a) { return __hip_atomic_load(X + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
     SwChunk c0 = load(k), c1 = load(k + 1), c2 = load(k + 2);
-    uint32_t hv = header(k), hn = header(k + kWave), j64 = 0;
-    float acc = 0.f, first = 0.f;   // a long row's running value (exact: the same in every lane), right-hand side
-    for (; k < k1; ++k, ++j64) {
-        const SwChunk t = c0;
-        c0 = c1;
-        c1 = c2;
-        c2 = load(k + 3);
-        if (j64 == (uint32_t)kWave) {
-            j64 = 0;
-            hv = hn;
-            hn = header(k + kWave);
-        }
-        const uint32_t h = __builtin_amdgcn_readlane(hv, j64);
+    float acc = 0.f;   // a long row's running value, the same in every lane
+    auto run = [&](const SwChunk &t) __attribute__((always_inline)) {
+        const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w);
         const uint32_t a0 = t.m.x & 0xffffu, a1 = t.m.x >> 16, a2 = t.m.y & 0xffffu, a3 = t.m.y >> 16;
         const uint32_t row = t.m.z & 0xffffu;
         uint32_t b0, b1, b2, b3;
         if (h & kSwLong) {
             const uint32_t np = h & kSwPassMask;   // passes less 1 (uniform)
-            if (kExact) {
-                if (h & kSwFirst) acc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t.r)));
-                const uint32_t ad[4] = {a0, a1, a2, a3};
-                const float w[4] = {t.v.x, t.v.y, t.v.z, t.v.w};
+            if (h & kSwFirst) acc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t.r)));
+            const uint32_t ad[4] = {a0, a1, a2, a3};
+            const float w[4] = {t.v.x, t.v.y, t.v.z, t.v.w};
 #pragma unroll
-                for (uint32_t u = 0; u < 4; ++u) {
-                    if (u > np) break;
-                    uint32_t b;
-                    for (;;) {
-                        b = peek(ad[u]);
-                        if (!__ballot(b == kUnset)) break;
-                        __builtin_amdgcn_s_sleep(1);
-                    }
-                    slice[lane] = w[u] * sw_f(b);
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                    acc = serial_sub(acc, slice, kWave, false);   // places without an entry hold +0
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                }
-                if ((h & kSwLast) && lane == 0) sw_put(xs, row, D.div ? acc / t.d : acc);
-            } else {
+            for (uint32_t u = 0; u < 4; ++u) {
+                if (u > np) break;
+                uint32_t b;
                 for (;;) {
-                    b0 = peek(a0), b1 = peek(a1), b2 = peek(a2), b3 = peek(a3);
-                    if (!__ballot(max(max(b0, b1), max(b2, b3)) == kUnset)) break;
+                    b = peek(ad[u]);
+                    if (!__ballot(b == kUnset)) break;
                     __builtin_amdgcn_s_sleep(1);
                 }
-                // (a place without an entry adds nothing, not even +0)
-                const bool e1 = t.m.w & 2u, e2 = t.m.w & 4u, e3 = t.m.w & 8u;
-                const float p0 = t.v.x * sw_f(b0), p1 = t.v.y * sw_f(b1), p2 = t.v.z * sw_f(b2), p3 = t.v.w * sw_f(b3);
-                if (h & kSwFirst) first = t.r;
-                float s = acc;
-                if (t.m.w & 1u) s = (h & kSwFirst) ? p0 : s + p0;
-                if (e1) s += p1;
-                if (e2) s += p2;
-                if (e3) s += p3;
-                acc = s;
-                if (h & kSwLast) {
-                    const float sum = group_sum(acc, 64);
-                    if (lane == 0) {
-                        const float v = first - sum;
-                        sw_put(xs, row, D.div ? v / t.d : v);
-                    }
-                }
+                slice[lane] = w[u] * sw_f(b);
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                acc = serial_sub(acc, slice, kWave, false);   // places without an entry hold +0
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             }
-            continue;
+            if ((h & kSwLast) && lane == 0) sw_put(xs, row, D.div ? acc / t.d : acc);
+            return;
         }
         const uint32_t lg = (t.m.z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
-        const bool on = t.m.z & kSwOn, tree = !kExact && (t.m.z & kSwTree);
-        const bool seq = kExact || (h & kSwHasSeq), sum = !kExact && (h & kSwHasTree);   // (uniform)
-        uint64_t left = __ballot(on && (tree ? j == 0 : j == g - 1u));   // lanes that store rows still to come
-        const uint64_t F = __ballot(j == 0), TR = __ballot(tree);
+        uint64_t left = __ballot((t.m.z & kSwOn) && j == g - 1u);   // lanes that store rows still to come
+        const uint64_t F = __ballot(j == 0);
         uint64_t V = 0;                            // lanes whose running value is final (rows in order)
-        const uint64_t rm = ((1ull << g) - 1ull) << (lane & ~(g - 1u));   // the row's lanes
-        const uint32_t rlo = (uint32_t)rm, rhi = (uint32_t)(rm >> 32);
         SwDiv dv{1.f, 1.f, true};
         if (D.div) dv = sw_div_prepare(t.d);
         float a = 0.f;
@@ -2331,37 +2301,20 @@ __device__ __forceinline__ void sw_wave(const SwDev &D, uint32_t k, uint32_t k1,
             const float p0 = t.v.x * sw_f(b0), p1 = t.v.y * sw_f(b1), p2 = t.v.z * sw_f(b2), p3 = t.v.w * sw_f(b3);
             bool more;
             do {
-                uint64_t fin = 0;
-                float res = 0.f;
-                more = false;
-                if (seq) {
-                    // lane j's value is lane j - 1's less its own four
-                    // products; a step settles the next ready lane of every
-                    // row, and does not change settled ones
-                    const float prev = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xf, 0xf, false));
-                    a = j == 0 ? t.r : prev;
-                    a = a - p0;
-                    a = a - p1;
-                    a = a - p2;
-                    a = a - p3;
-                    V = R & (F | (V << 1));
-                    fin = V & left & ~TR;
-                    res = a;
-                    more = (R & (F | (V << 1))) != V;
-                }
-                if (sum) {
-                    const bool rdy = ((uint32_t)R & rlo) == rlo && ((uint32_t)(R >> 32) & rhi) == rhi;
-                    float q = (p0 + p1) + (p2 + p3);
-                    q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0xB1, 0xf, 0xf, false));   // quad [1,0,3,2]
-                    q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x4E, 0xf, 0xf, false));   // quad [2,3,0,1]
-                    const float q8 = q + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x141, 0xf, 0xf, false));   // half mirror
-                    const float q16 = q8 + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q8), 0x140, 0xf, 0xf, false));  // mirror
-                    const float tv = t.r - (lg == 2u ? q : lg == 3u ? q8 : q16);
-                    fin |= __ballot(rdy) & left & TR;
-                    res = tree ? tv : res;
-                }
+                // lane j's value is lane j - 1's less its own four products;
+                // a step settles the next ready lane of every row, and does
+                // not change settled ones
+                const float prev = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xf, 0xf, false));
+                a = j == 0 ? t.r : prev;
+                a = a - p0;
+                a = a - p1;
+                a = a - p2;
+                a = a - p3;
+                V = R & (F | (V << 1));
+                const uint64_t fin = V & left;
+                more = (R & (F | (V << 1))) != V;
                 if (fin) {
-                    if (D.div) res = sw_div(dv, res, fin);
+                    const float res = D.div ? sw_div(dv, a, fin) : a;
                     if (__builtin_amdgcn_inverse_ballot_w64(fin)) sw_put(xs, row, res);
                     left &= ~fin;
                 }
@@ -2370,7 +2323,137 @@ __device__ __forceinline__ void sw_wave(const SwDev &D, uint32_t k, uint32_t k1,
             if (!narrow) __builtin_amdgcn_s_sleep(1);
         }
         if (narrow) __builtin_amdgcn_s_setprio(0);
+    };
+    for (;;) {   // (three times the code: moved from one to the next, the chunks would be waited for)
+        run(c0);
+        c0 = load(k + 3);
+        if (++k >= k1) break;
+        run(c1);
+        c1 = load(k + 3);
+        if (++k >= k1) break;
+        run(c2);
+        c2 = load(k + 3);
+        if (++k >= k1) break;
     }
+}
+
+// Part P of sweep D, a level a step: every wave of the workgroup calls it and
+// meets the others once a step, so a chunk's entries are read once, without
+// asking whether they are set.  What does not depend on them (the wait for
+// the chunk's loads, three chunks ahead; addresses; the divisor's reciprocal)
+// is done in a step where the wave has no chunk.  Bound by the step: an LDS
+// round trip, 60 or so dependent instructions, the barrier of 16 waves.
+// (Waiting for each entry to be set, as the exact solve does, polled LDS from
+// 16 waves; a summed row has nothing to do early.  n=50,000, adjoint gradient
+// 2,814 -> 2,600 us; n=9,973 to 1e-12 730 -> 647 us; 16 patterns of about
+// 30,000 in one call 1,826 -> 1,512 us.)
+__device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const float *__restrict__ sv,
+                                         const float *__restrict__ rhs, float *xs)
+{
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    uint32_t k = __builtin_amdgcn_readfirstlane(w < D.nwave ? D.wptr[P.wp + w] : 0u);
+    const uint32_t k1 = __builtin_amdgcn_readfirstlane(w < D.nwave ? D.wptr[P.wp + w + 1] : 0u);
+    const uint32_t steps = __builtin_amdgcn_readfirstlane(P.steps);
+    if (k >= k1) {
+        for (uint32_t s = 0; s < steps; ++s) __syncthreads();
+        return;
+    }
+    const uint32_t lane = threadIdx.x & (kWave - 1), doff = D.div ? 256u : 0u, stride = D.stride;
+    const uint4 *meta = uniform(D.meta);
+    const float *val = uniform(sv), *rh = uniform(rhs);
+    auto load = [&](uint32_t q) {
+        q = min(q, k1 - 1);
+        const float *c = val + (size_t)q * stride, *rr = rh + (size_t)q * kWave;   // (scalar bases, the lane's offset)
+        const uint4 *m = meta + (size_t)q * kWave;
+        SwChunk t;
+        t.m = m[lane];
+        t.v = reinterpret_cast<const float4 *>(c)[lane];
+        t.r = rr[lane];
+        t.d = (c + doff)[lane];
+        return t;
+    };
+    SwChunk c0 = load(k);
+    asm volatile("" ::: "memory");   // (in this order, which the waits count on)
+    SwChunk c1 = load(k + 1), c2;
+    uint32_t done = 0;   // steps
+    float acc = 0.f, first = 0.f;   // a long row's running value, right-hand side
+    auto at = [&](uint32_t a) { return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(xs) + a); };
+    auto meet = [&]() {
+        __syncthreads();
+        ++done;
+    };
+    auto run = [&](const SwChunk &t, SwChunk &next) __attribute__((always_inline)) {
+        const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w), step = (h >> kSwStepShift) & kSwStepMask;
+        if (done < step) meet();
+        next = load(k + 2);
+        // (byte addresses)
+        uint32_t a0 = 4 * (t.m.x & 0xffffu), a1 = 4 * (t.m.x >> 16), a2 = 4 * (t.m.y & 0xffffu), a3 = 4 * (t.m.y >> 16);
+        uint32_t row = t.m.z & 0xffffu;
+        const uint32_t lg = (t.m.z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
+        const bool tree = t.m.z & kSwTree;
+        const bool stores = (h & kSwLong) ? lane == 0 : (t.m.z & kSwOn) && (tree ? j == 0 : j == g - 1u);
+        const uint64_t S = __ballot(stores);
+        uint32_t lanes = 1;   // of the chunk's widest row summed in order
+        if (!(h & kSwLong))
+            while (__ballot((t.m.z & kSwOn) && !tree && g > lanes)) lanes *= 2;
+        SwDiv dv{1.f, 1.f, true};
+        if (D.div) dv = sw_div_prepare(t.d);
+        asm volatile("" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(row));   // before the meeting, not after
+        asm volatile("" : "+v"(dv.r), "+v"(dv.d));
+        while (done < step) meet();
+        const float p0 = t.v.x * at(a0), p1 = t.v.y * at(a1), p2 = t.v.z * at(a2), p3 = t.v.w * at(a3);
+        float res;
+        if (h & kSwLong) {
+            // (a place without an entry adds nothing, not even +0)
+            if (h & kSwFirst) first = t.r;
+            float s = acc;
+            if (t.m.z & kSwEntry) s = (h & kSwFirst) ? p0 : s + p0;
+            if (t.m.z & (kSwEntry << 1)) s += p1;
+            if (t.m.z & (kSwEntry << 2)) s += p2;
+            if (t.m.z & (kSwEntry << 3)) s += p3;
+            acc = s;
+            if (!(h & kSwLast)) return;
+            res = first - group_sum(acc, 64);
+        } else {
+            res = t.r;
+            if (h & kSwHasSeq) {
+                float a = t.r - p0;
+                a = a - p1;
+                a = a - p2;
+                a = a - p3;
+                // lane j's value is lane j - 1's less its own four products
+                for (uint32_t s = 1; s < lanes; ++s) {
+                    float b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xf, 0xf, false));
+                    b = b - p0;
+                    b = b - p1;
+                    b = b - p2;
+                    b = b - p3;
+                    a = j == s ? b : a;
+                }
+                res = a;
+            }
+            if (h & kSwHasTree) {
+                float q = (p0 + p1) + (p2 + p3);
+                q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0xB1, 0xf, 0xf, false));   // quad [1,0,3,2]
+                q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x4E, 0xf, 0xf, false));   // quad [2,3,0,1]
+                const float q8 = q + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x141, 0xf, 0xf, false));   // half mirror
+                const float q16 = q8 + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q8), 0x140, 0xf, 0xf, false));  // mirror
+                const float tv = t.r - (lg == 2u ? q : lg == 3u ? q8 : q16);
+                res = tree ? tv : res;
+            }
+        }
+        if (D.div) res = sw_div(dv, res, S);
+        if (stores) sw_put(xs, row, res);
+    };
+    for (;;) {   // (three times the code: moved from one to the next, the chunks would be waited for)
+        run(c0, c2);
+        if (++k >= k1) break;
+        run(c1, c0);
+        if (++k >= k1) break;
+        run(c2, c1);
+        if (++k >= k1) break;
+    }
+    while (done < steps) meet();
 }
 
 // The LDS vector of a part before its sweep: rows not set, then the constant
@@ -2388,9 +2471,14 @@ template <bool kExact>
 __device__ __forceinline__ void sw_part(const SwDev &D, const SwPart &P, const float *sv, const float *rhs, float *xs,
                                         float *wl)
 {
+    if (!kExact) {
+        sw_steps(D, P, sv, rhs, xs);
+        return;
+    }
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (w < D.nwave)
-        sw_wave<kExact>(D, D.wptr[P.wp + w], D.wptr[P.wp + w + 1], sv, rhs, xs, wl + w * kWave);
+        sw_wave(D, __builtin_amdgcn_readfirstlane(D.wptr[P.wp + w]), __builtin_amdgcn_readfirstlane(D.wptr[P.wp + w + 1]),
+                sv, rhs, xs, wl + w * kWave);
 }
 
 // rhs[rpos[i]] = float(v[src[r]] * scale[r]) for the rows r of part P (slot

@@ -1955,7 +1955,10 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
         std::vector<uint32_t> lanes_at(R.empty() ? 0 : R.back().level + 1, 0);   // lanes of each level
         for (const Pos &x : R) lanes_at[x.level] += is_long(x) ? 0 : sw_lanes(x.len, x.sum);
         uint32_t turn = 0, turn_long = 0, used = 64;
-        for (size_t i = 0; i < R.size();) {
+        std::vector<uint32_t> step_of(nslot, 0), wave_step(waves, 0);   // a row's step; the step a wave's chunks got to
+        for (size_t i = 0; i < R.size(); ++P.steps) {
+            const uint32_t step = P.steps << kSwStepShift;
+            used = 64;
             size_t e = i;
             while (e < R.size() && R[e].level == R[i].level) ++e;
             // a level's rows are independent: long ones first, then by lanes,
@@ -1972,19 +1975,28 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
                 const Pos &x = R[i];
                 const uint32_t slot = Q.slot_of[x.row];
                 S.row[P.s0 + slot] = x.row;
+                step_of[slot] = P.steps;
                 if (is_long(x)) {
-                    used = 64;   // (what is open may hold this row's dependencies: it stays before)
                     const uint32_t nc = (x.len + kSwEntries - 1) / kSwEntries;
                     const uint32_t to = nc > 1 && own ? turn_long++ % own : own + turn++ % (waves - own);
                     for (uint32_t c = 0; c < nc; ++c) {
                         const uint32_t left = std::min(x.len - c * kSwEntries, kSwEntries);
-                        add(kSwLong | (c == 0 ? kSwFirst : 0u) | (c + 1 == nc ? kSwLast : 0u) | ((left + 63) / 64 - 1));
+                        // the row's step ends it; what is before runs as soon
+                        // as its entries are set and the wave is there
+                        uint32_t at = c + 1 == nc ? P.steps : wave_step[to];
+                        for (uint32_t k = 0; k < left && c + 1 < nc; ++k) {
+                            const uint32_t col = D.idx[x.base + (size_t)(c * kSwEntries + k) * x.step];
+                            if (Q.part_of[col] == part) at = std::max(at, step_of[Q.slot_of[col]] + 1);
+                        }
+                        wave_step[to] = at;
+                        add(at << kSwStepShift | kSwLong | (c == 0 ? kSwFirst : 0u) | (c + 1 == nc ? kSwLast : 0u) | ((left + 63) / 64 - 1));
                         wave.push_back(to);
+                        uint32_t bits[64] = {};
                         for (uint32_t k = 0; k < left; ++k) {
                             put(k % 64, k / 64, x, c * kSwEntries + k);
-                            meta[64 * (hdr.size() - 1) + k % 64].w |= 1u << (k / 64);
+                            bits[k % 64] |= kSwEntry << (k / 64);
                         }
-                        for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (hdr.size() - 1) + lane].z = slot;
+                        for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (hdr.size() - 1) + lane].z = slot | bits[lane];
                         if (c == 0) rpos[slot] = 64 * (uint32_t)(hdr.size() - 1);
                         if (c + 1 == nc && div) vsrc[(hdr.size() - 1) * S.stride + kSwEntries] = x.pivot;
                     }
@@ -1994,8 +2006,9 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
                 used = (used + g - 1) & ~(g - 1);
                 if (used + g > 64) {
                     const bool few = lanes_at[x.level] <= kSwNarrowLanes;
-                    add(few ? kSwNarrow : 0u);
+                    add(step | (few ? kSwNarrow : 0u));
                     wave.push_back(own + turn++ % (few ? std::min(kSwNarrowWaves, waves - own) : waves - own));
+                    wave_step[wave.back()] = P.steps;
                     used = 0;
                 }
                 const size_t c = hdr.size() - 1;
@@ -2018,6 +2031,7 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
                 if (wave[c] != w) continue;
                 at[c] = (uint32_t)S.hdr.size();
                 S.hdr.push_back(hdr[c]);
+                for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * c + lane].w = hdr[c];
                 S.meta.insert(S.meta.end(), meta.begin() + 64 * c, meta.begin() + 64 * (c + 1));
                 S.vsrc.insert(S.vsrc.end(), vsrc.begin() + c * S.stride, vsrc.begin() + (c + 1) * S.stride);
             }
@@ -2056,6 +2070,28 @@ bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
             at[w] = S.wptr[P.wp + w];
             if (at[w] > S.wptr[P.wp + w + 1] || S.wptr[P.wp + w + 1] > nchunk) return bad("stream out of range");
         }
+        // by steps: a stream's steps do not fall, an entry's row has an earlier one
+        std::vector<uint32_t> step_of(P.nslot + 2, 0);   // 1 + the row's step
+        for (uint32_t pass = 0; pass < 2; ++pass)
+            for (uint32_t w = 0; w < S.nwave; ++w)
+                for (uint32_t c = at[w], last = 0; c < S.wptr[P.wp + w + 1]; ++c) {
+                    const uint32_t h = S.hdr[c], step = (h >> kSwStepShift) & kSwStepMask;
+                    if (step < last || step >= P.steps) return bad("step out of range");
+                    if ((h & kSwLong) && !(h & kSwFirst) && (c == at[w] || !(S.hdr[c - 1] & kSwLong) || (S.hdr[c - 1] & kSwLast)))
+                        return bad("a row's chunks are apart");
+                    last = step;
+                    for (uint32_t lane = 0; lane < 64; ++lane) {
+                        const uint4 &m = S.meta[64 * (size_t)c + lane];
+                        if (pass == 0 && ((h & kSwLong) || (m.z & kSwOn))) {
+                            if ((m.z & 0xffffu) >= P.nslot) return bad("row slot out of range");
+                            if (!(h & kSwLong) || (h & kSwLast)) step_of[m.z & 0xffffu] = step + 1;
+                        }
+                        for (uint32_t v : {m.x & 0xffffu, m.x >> 16, m.y & 0xffffu, m.y >> 16}) {
+                            if (v > P.nslot + 1) return bad("slot out of range");
+                            if (pass == 1 && step_of[v] > step) return bad("an entry's row is not in an earlier step");
+                        }
+                    }
+                }
         uint32_t done = 0;
         for (bool moved = true; moved;) {
             moved = false;
@@ -2074,7 +2110,7 @@ bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
                                 if (entry(lane, e) > P.nslot + 1) return bad("slot out of range");
                                 whole = whole && set[entry(lane, e)];
                             }
-                        const uint32_t slot = S.meta[64 * (size_t)c].z;
+                        const uint32_t slot = S.meta[64 * (size_t)c].z & 0xffffu;
                         if (slot >= P.nslot) return bad("row slot out of range");
                         if (whole && (h & kSwFirst) && S.rpos[P.s0 + slot] != 64 * c) return bad("right-hand side misplaced");
                         if (whole && (h & kSwLast)) {
@@ -2681,7 +2717,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     const size_t o_out = U.reserve(sizeof(float) * most_out);
     const size_t o_wdev = U.reserve(sizeof(WinDev) * std::max<size_t>(wins.size(), 1));
     struct SwOff {
-        size_t meta, hdr, wptr, part, row, rpos, prod;
+        size_t meta, wptr, part, row, rpos, prod;
     };
     SwOff o_sw[4], o_hd[4];
     for (int q = 0; q < 4; ++q)
@@ -2689,7 +2725,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
             SwHost &h = k ? hd[q] : sw[q];
             if (h.prod.size())   // product values count from the copy's start
                 for (SwProd &e : h.prod) e.val += k ? hd_voff[q] : sw_voff[q];
-            (k ? o_hd : o_sw)[q] = SwOff{U.put(h.meta), U.put(h.hdr), U.put(h.wptr), U.put(h.part),
+            (k ? o_hd : o_sw)[q] = SwOff{U.put(h.meta), U.put(h.wptr), U.put(h.part),
                                          U.put(h.row), U.put(h.rpos), U.put(h.prod)};
         }
     const size_t o_spl[2] = {U.put(spl_vpos[0]), U.put(spl_vpos[1])};
@@ -2898,7 +2934,6 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     auto swd = [&](const SwHost &h, const SwOff &o, bool div, uint32_t voff) {
         SwDev d{};
         d.meta = reinterpret_cast<const uint4 *>(A + o.meta);
-        d.hdr = u32p(o.hdr);
         d.wptr = u32p(o.wptr);
         d.part = reinterpret_cast<const SwPart *>(A + o.part);
         d.row = u32p(o.row);
