@@ -808,6 +808,26 @@ __device__ __forceinline__ WinDev load_window(const FactorDev &F, int w)
     return W;
 }
 
+// A pointer that is the same in every lane, in scalar registers.
+template <typename T>
+__device__ __forceinline__ T *uniform(T *p)
+{
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return glb(reinterpret_cast<T *>((uint64_t)hi << 32 | lo));
+}
+
+// Byte addresses in LDS.
+typedef __attribute__((address_space(3))) float lds_float;
+__device__ __forceinline__ uint32_t lds_address(float *p)
+{
+    return (uint32_t)reinterpret_cast<uintptr_t>((lds_float *)p);
+}
+__device__ __forceinline__ lds_float *lds_at(uint32_t a)
+{
+    return reinterpret_cast<lds_float *>(static_cast<uintptr_t>(a));
+}
+
 // In each row of 16 lanes: a of lane k becomes a(k - 1) - p(k), k = 1..15 in
 // order (lane 0 keeps a), so lane 15 ends with a(0) - p(1) - ... - p(15),
 // each subtraction rounded.  row_shr:1 leaves lane 0 unwritten; after k steps
@@ -825,12 +845,16 @@ __device__ __forceinline__ float row_chain_sub(float a, float p)
 // The steps of one window over the staged values S (LDS), the caller having
 // staged them behind a barrier; ends with a barrier.  A step of a window is
 // short (one to a few columns), so its cost is the chain from one barrier to
-// the next: nothing but LDS reads, one division and LDS writes is on it.  The
-// chunks (all a lane needs, in one 16-byte load) are read three ahead, so no
-// memory load is ever waited for inside a step, and their slots are turned
-// into addresses before the barrier.  Measured (n=20,000, 370 steps in one
-// window): 601 -> 206 us against the shared item code, whose table loads
-// depended on each other inside a step; n=640, 142 steps: 112 -> 48 us.
+// the next: nothing but LDS reads, one division and LDS writes is on it, and
+// in a step of many chunks the waves' instructions.  The chunks (all a lane
+// needs, in one 16-byte load) are read three ahead into buffers that keep
+// their places, so no memory load is waited for inside a step, and their
+// slots are turned into addresses before the barrier.  Measured (n=20,000,
+// 370 steps in one window): 601 us with the shared item code, whose table
+// loads depended on each other inside a step, 206 us with chunks in buffers
+// moved from one to the next (each move waited for the newest load), 180 us
+// this way; n=640, 142 steps: 112, 48 and 37 us; n=200,003, 2,121 steps: 1,650
+// and 1,150 us with the two kinds of buffer.
 template <bool kOut = false>
 __device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pert, int perturb,
                                              float *__restrict__ out = nullptr)
@@ -841,35 +865,44 @@ __device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pe
     uint32_t passed = 0;
     uint32_t k = 0, k1 = 0;
     if (w < W.nwave) {
-        k = W.wptr[w];
-        k1 = W.wptr[w + 1];
+        k = __builtin_amdgcn_readfirstlane(W.wptr[w]);
+        k1 = __builtin_amdgcn_readfirstlane(W.wptr[w + 1]);
     }
     if (k < k1) {
-        const uint4 *g = W.prog + lane;
-        auto chunk = [&](uint32_t q) { return g[(size_t)min(q, k1 - 1) * kWave]; };
-        auto header = [&](uint32_t q) { return W.hdr[min(q + lane, k1 - 1)]; };   // 64 chunks', one a lane
-        uint4 q0 = chunk(k), q1 = chunk(k + 1), q2 = chunk(k + 2);
-        uint32_t hv = header(k), hn = header(k + kWave), j = 0;
+        const uint4 *prog = uniform(W.prog);
+        const uint32_t *hdr = uniform(W.hdr);
+        uint32_t zero = 0;   // (in a vector register: the header comes by a load that is waited for by count)
+        asm volatile("" : "+v"(zero));
+        struct Chunk {
+            uint4 q;
+            uint32_t h;
+        };
+        auto load = [&](uint32_t c) {
+            c = min(c, k1 - 1);
+            const uint4 *p = prog + (size_t)c * kWave;
+            const uint32_t *e = hdr + c;
+            return Chunk{p[lane], e[zero]};
+        };
         float acc = 0.f;   // kWinMerge: the lane's running value; groups: the running value, in lane 0 of 16
-        char *const B = reinterpret_cast<char *>(S);
-        auto at = [&](uint32_t a) -> float & { return *reinterpret_cast<float *>(B + a); };
-        for (; k < k1; ++k, ++j) {
-            const uint4 q = q0;
-            q0 = q1;
-            q1 = q2;
-            q2 = chunk(k + 3);
-            if (j == (uint32_t)kWave) {
-                j = 0;
-                hv = hn;
-                hn = header(k + kWave);
-            }
-            const uint32_t h = __builtin_amdgcn_readlane(hv, j);
-            const uint32_t a0 = (q.x & 0xffffu) << 2, a1 = (q.x >> 14) & 0x3fffcu;
-            const uint32_t a2 = (q.y & 0xffffu) << 2, a3 = (q.y >> 14) & 0x3fffcu;
-            const uint32_t a4 = (q.z & 0xffffu) << 2, a5 = (q.z >> 14) & 0x3fffcu;
-            const uint32_t a6 = (q.w & 0xffffu) << 2, a7 = (q.w >> 14) & 0x3fffcu;
+        const uint32_t base = lds_address(S);
+        auto at = [&](uint32_t a) -> lds_float & { return *lds_at(a); };
+        auto meet = [&]() {
+            __syncthreads();
+            ++passed;
+        };
+        auto run = [&](uint32_t c, const Chunk &t, Chunk &next) __attribute__((always_inline)) {
+            const uint32_t h = __builtin_amdgcn_readfirstlane(t.h);
             const uint32_t step = h & ((1u << kWinKindShift) - 1u), kind = h >> kWinKindShift;
-            for (; passed < step; ++passed) __syncthreads();
+            if (c < k1 && passed < step) meet();
+            next = load(c + 3);
+            if (c >= k1) return;
+            const uint4 q = t.q;
+            uint32_t a0 = base + ((q.x & 0xffffu) << 2), a1 = base + ((q.x >> 16) << 2);
+            uint32_t a2 = base + ((q.y & 0xffffu) << 2), a3 = base + ((q.y >> 16) << 2);
+            uint32_t a4 = base + ((q.z & 0xffffu) << 2), a5 = base + ((q.z >> 16) << 2);
+            uint32_t a6 = base + ((q.w & 0xffffu) << 2), a7 = base + ((q.w >> 16) << 2);
+            asm volatile("" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7));
+            while (passed < step) meet();
             if (kOut && kind == kWinOut) {
                 const float l = at(a0) / gesp(at(a1), pert, perturb);
                 const float u0 = at(a2), u1 = at(a3);
@@ -887,15 +920,15 @@ __device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pe
                 const float l0 = at(a2), u0 = at(a3), d0 = at(a4), l1 = at(a5), u1 = at(a6), d1 = at(a7);
                 const float p0 = (l0 / gesp(d0, pert, perturb)) * u0;
                 const float p1 = (l1 / gesp(d1, pert, perturb)) * u1;
-                if (a1 & (kWinFirst << 2)) acc = tv;
+                if (q.x & (kWinFirst << 16)) acc = tv;
                 acc = acc + (-p0);
                 acc = acc + (-p1);
-                if (a1 & (kWinLast << 2)) at(a0) = acc;
+                if (q.x & (kWinLast << 16)) at(a0) = acc;
             } else {
                 const float l0 = at(a0), u0 = at(a1), d0 = at(a2), tv = at(a6);
                 const float l1 = at(a3), u1 = at(a4), d1 = at(a5);
                 const float p0 = (l0 / gesp(d0, pert, perturb)) * u0;
-                if (a7 & (kWinFirst << 2)) acc = tv;
+                if (q.w & (kWinFirst << 16)) acc = tv;
                 float a = row_chain_sub(acc - p0, p0);
                 if (kind == kWinGroup) {
                     const float p1 = (l1 / gesp(d1, pert, perturb)) * u1;
@@ -903,9 +936,22 @@ __device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pe
                     const float c = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x121, 0xf, 0xf, false));
                     a = row_chain_sub(c - p1, p1);
                 }
-                if ((a7 & (kWinLast << 2)) && (lane & 15u) == 15u) at(a6) = a;
+                if ((q.w & (kWinLast << 16)) && (lane & 15u) == 15u) at(a6) = a;
                 acc = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x121, 0xf, 0xf, false));
             }
+        };
+        Chunk c0 = load(k);
+        asm volatile("" ::: "memory");   // (in this order, which the waits count on)
+        Chunk c1 = load(k + 1);
+        asm volatile("" ::: "memory");
+        Chunk c2 = load(k + 2), c3;
+        // (four times the code: moved from one to the next, the chunks would
+        // be waited for; loads and one exit on every path, for the counts)
+        for (; k < k1; k += 4) {
+            run(k, c0, c3);
+            run(k + 1, c1, c0);
+            run(k + 2, c2, c1);
+            run(k + 3, c3, c2);
         }
     }
     for (; passed < steps; ++passed) __syncthreads();
@@ -2170,15 +2216,6 @@ __device__ __forceinline__ void sw_put(float *xs, uint32_t r, float v)
     __hip_atomic_store(reinterpret_cast<uint32_t *>(xs) + r, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// A pointer that is the same in every lane, in scalar registers.
-template <typename T>
-__device__ __forceinline__ T *uniform(T *p)
-{
-    const uint64_t a = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-    return glb(reinterpret_cast<T *>((uint64_t)hi << 32 | lo));
-}
-
 // A chunk's prefetched data (SwDev).
 struct SwChunk {
     uint4 m;
@@ -2253,9 +2290,14 @@ __device__ __forceinline__ void sw_wave(const SwDev &D, uint32_t k, uint32_t k1,
     };
     const uint32_t *X = reinterpret_cast<const uint32_t *>(xs);
     auto peek = [&](uint32_t a) { return __hip_atomic_load(X + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
-    SwChunk c0 = load(k), c1 = load(k + 1), c2 = load(k + 2);
+    SwChunk c0 = load(k);
+    asm volatile("" ::: "memory");   // (in this order, which the waits count on)
+    SwChunk c1 = load(k + 1);
+    asm volatile("" ::: "memory");
+    SwChunk c2 = load(k + 2);
     float acc = 0.f;   // a long row's running value, the same in every lane
-    auto run = [&](const SwChunk &t) __attribute__((always_inline)) {
+    auto run = [&](uint32_t q, const SwChunk &t) __attribute__((always_inline)) {
+        if (q >= k1) return;
         const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w);
         const uint32_t a0 = t.m.x & 0xffffu, a1 = t.m.x >> 16, a2 = t.m.y & 0xffffu, a3 = t.m.y >> 16;
         const uint32_t row = t.m.z & 0xffffu;
@@ -2324,16 +2366,15 @@ __device__ __forceinline__ void sw_wave(const SwDev &D, uint32_t k, uint32_t k1,
         }
         if (narrow) __builtin_amdgcn_s_setprio(0);
     };
-    for (;;) {   // (three times the code: moved from one to the next, the chunks would be waited for)
-        run(c0);
+    // (three times the code: moved from one to the next, the chunks would be
+    // waited for; loads and one exit on every path, for the counts)
+    for (; k < k1; k += 3) {
+        run(k, c0);
         c0 = load(k + 3);
-        if (++k >= k1) break;
-        run(c1);
-        c1 = load(k + 3);
-        if (++k >= k1) break;
-        run(c2);
-        c2 = load(k + 3);
-        if (++k >= k1) break;
+        run(k + 1, c1);
+        c1 = load(k + 4);
+        run(k + 2, c2);
+        c2 = load(k + 5);
     }
 }
 
@@ -2377,17 +2418,20 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
     SwChunk c1 = load(k + 1), c2;
     uint32_t done = 0;   // steps
     float acc = 0.f, first = 0.f;   // a long row's running value, right-hand side
-    auto at = [&](uint32_t a) { return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(xs) + a); };
+    const uint32_t base = lds_address(xs);
+    auto at = [&](uint32_t a) -> float { return *lds_at(a); };
     auto meet = [&]() {
         __syncthreads();
         ++done;
     };
-    auto run = [&](const SwChunk &t, SwChunk &next) __attribute__((always_inline)) {
+    auto run = [&](uint32_t q, const SwChunk &t, SwChunk &next) __attribute__((always_inline)) {
         const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w), step = (h >> kSwStepShift) & kSwStepMask;
-        if (done < step) meet();
-        next = load(k + 2);
+        if (q < k1 && done < step) meet();
+        next = load(q + 2);
+        if (q >= k1) return;
         // (byte addresses)
-        uint32_t a0 = 4 * (t.m.x & 0xffffu), a1 = 4 * (t.m.x >> 16), a2 = 4 * (t.m.y & 0xffffu), a3 = 4 * (t.m.y >> 16);
+        uint32_t a0 = base + ((t.m.x & 0xffffu) << 2), a1 = base + ((t.m.x >> 16) << 2);
+        uint32_t a2 = base + ((t.m.y & 0xffffu) << 2), a3 = base + ((t.m.y >> 16) << 2);
         uint32_t row = t.m.z & 0xffffu;
         const uint32_t lg = (t.m.z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
         const bool tree = t.m.z & kSwTree;
@@ -2445,13 +2489,12 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
         if (D.div) res = sw_div(dv, res, S);
         if (stores) sw_put(xs, row, res);
     };
-    for (;;) {   // (three times the code: moved from one to the next, the chunks would be waited for)
-        run(c0, c2);
-        if (++k >= k1) break;
-        run(c1, c0);
-        if (++k >= k1) break;
-        run(c2, c1);
-        if (++k >= k1) break;
+    // (three times the code: moved from one to the next, the chunks would be
+    // waited for; loads and one exit on every path, for the counts)
+    for (; k < k1; k += 3) {
+        run(k, c0, c2);
+        run(k + 1, c1, c0);
+        run(k + 2, c2, c1);
     }
     while (done < steps) meet();
 }
