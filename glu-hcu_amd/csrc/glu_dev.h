@@ -222,7 +222,7 @@ struct DfDev {
 // such a chunk holding entries j, 64 + j, 128 + j and 192 + j of its 256.
 //   meta[64 c + lane] = {slots of entries 0, 1 (16 bits each), of 2, 3,
 //     row slot | log2 lanes << 16 | kSwTree | kSwOn, the chunk's header}; in a
-//     chunk of a long row kSwEntry << e: the lane has entry e
+//     chunk of a long row kSwEntry << e (the lane has entry e) and its entries
 //   values: value c stride + 4 lane + e is entry e's, c stride + 256 + lane
 //     the row's pivot (div sweeps; at the lane that stores the row)
 //   a row's right-hand side: rhs[rpos[slot]], at its first lane
@@ -233,11 +233,21 @@ struct DfDev {
 // other rows, and every row in the exact solve, are subtracted in order.
 constexpr uint32_t kSwTree = 1u << 20, kSwOn = 1u << 21, kSwEntry = 1u << 16;
 constexpr uint32_t kSwLong = 1u << 31, kSwFirst = 1u << 30, kSwLast = 1u << 29;   // header bits
-constexpr uint32_t kSwHasTree = 1u << 28, kSwHasSeq = 1u << 27, kSwNarrow = 1u << 26;
-constexpr uint32_t kSwPassMask = 3u;   // header of a long chunk: passes of 64 used, less 1
+constexpr uint32_t kSwHasTree = 1u << 28, kSwHasSeq = 1u << 27;
+constexpr uint32_t kSwTrack = 1u << 26;   // the second of the two long rows a wave can have open
 // header: the chunk's step (its rows' level among the part's levels: a chunk
-// holds rows of one level, whose dependencies ran in earlier steps)
-constexpr uint32_t kSwStepShift = 2, kSwStepMask = 0xffffffu;
+// holds rows of one level, whose dependencies ran in earlier steps; a chunk of
+// a long row that is not its last: a step by which its entries are set)
+constexpr uint32_t kSwStepMask = 0xffffu;
+// header, for the exact solve: what a wave can do ahead.  A long row's chunk:
+// its first entries set more than kSwLead steps before the chunk's (64 of them
+// a step, in the kSwLead steps before); other chunks: the lanes after the
+// first that the running values can pass in the step before, by entries set
+// two steps or more before the chunk's (pre), and those left for its own (rem).
+constexpr uint32_t kSwLead = 4;
+constexpr uint32_t kSwEarlyShift = 16, kSwEarlyMask = 0x1ffu;
+constexpr uint32_t kSwPreShift = 16, kSwPreMask = 15u, kSwRemShift = 20, kSwRemMask = 15u;
+constexpr uint32_t kSwCountShift = 20;   // meta.z of a long row's chunk: its entries
 
 struct SwPart {
     uint32_t wp;               // wptr[wp + w] .. wptr[wp + w + 1]: wave w's chunks

@@ -852,9 +852,9 @@ __device__ __forceinline__ float row_chain_sub(float a, float p)
 // slots are turned into addresses before the barrier.  Measured (n=20,000,
 // 370 steps in one window): 601 us with the shared item code, whose table
 // loads depended on each other inside a step, 206 us with chunks in buffers
-// moved from one to the next (each move waited for the newest load), 180 us
-// this way; n=640, 142 steps: 112, 48 and 37 us; n=200,003, 2,121 steps: 1,650
-// and 1,150 us with the two kinds of buffer.
+// moved from one to the next (each move waited for the newest load), 171 us
+// this way; n=640, 142 steps: 112, 48 and 39 us; n=200,003, 2,121 steps: 1,650
+// and 1,171 us with the two kinds of buffer.
 template <bool kOut = false>
 __device__ __forceinline__ void window_steps(const WinDev &W, float *S, float pert, int perturb,
                                              float *__restrict__ out = nullptr)
@@ -2191,30 +2191,11 @@ __device__ __forceinline__ void df2_sweep(const DfDev &D, const float *__restric
 }
 
 // ---------------------------------------------------------------------------
-// dataflow sweeps with the vector in LDS, values as their own ready marks
+// sweeps a level a step, the vector in LDS
 // ---------------------------------------------------------------------------
 //
-// A part is the rows one workgroup owns, their vector in LDS.  It starts as
-// kUnset everywhere; a row's result is published by storing it, and a reader
-// polls the value itself: one LDS read gives readiness and value, with no
-// ready bit, no fence and no second read between a row and its dependents.
-// What bounds these sweeps is that hop (n=20k: ~400 dependent rows a sweep).
-// Everything but the dependencies is loaded three chunks ahead.  Measured
-// (exact solve alone): n=4,960 235 -> 160 us, n=20,000 775 -> 430 us against
-// ready bits and one task of 16, 32 or 64 lanes a row.
-//
-// kUnset is a NaN of the largest bit pattern, so the largest of several words
-// tells whether one is unset; sw_put never stores it (a row whose value is
-// that very NaN stores another), so a published row never looks unset and
-// every wait ends (the streams' order is checked on the host, check_sw).
-constexpr uint32_t kUnset = 0xffffffffu;
-
-__device__ __forceinline__ void sw_put(float *xs, uint32_t r, float v)
-{
-    uint32_t b = __float_as_uint(v);
-    b = b == kUnset ? 0x7fc00000u : b;
-    __hip_atomic_store(reinterpret_cast<uint32_t *>(xs) + r, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
+// A part is the rows one workgroup owns, their vector in LDS; its chunks run
+// a level a step, every wave meeting the others between two (SwDev).
 
 // A chunk's prefetched data (SwDev).
 struct SwChunk {
@@ -2261,135 +2242,25 @@ __device__ __forceinline__ float sw_div(const SwDiv &q, float a, uint64_t lanes)
     return res;
 }
 
-__device__ __forceinline__ float sw_f(uint32_t b) { return __uint_as_float(b); }
-
-// Chunks [k, k1) of sweep D, in order, by one wave: values sv, right-hand
-// sides rhs, results into xs (LDS; kUnset but for the two constant slots).
-// Chunks load three ahead (a chunk is four loads, so the waits count).
-// Every row's products are subtracted one at a time in the row's order (the
-// arithmetic of Symbolic_Matrix::solve); slice: the wave's 64 floats of LDS
-// for its long rows.  While a row waits, the subtractions that can be done
-// are: from the last entry's arrival only its own lane's remain.
-__device__ __forceinline__ void sw_wave(const SwDev &D, uint32_t k, uint32_t k1, const float *__restrict__ sv,
-                                        const float *__restrict__ rhs, float *xs, float *slice)
-{
-    if (k >= k1) return;
-    const uint32_t lane = threadIdx.x & (kWave - 1), doff = D.div ? 256u : 0u, stride = D.stride;
-    const uint4 *meta = uniform(D.meta);
-    const float *val = uniform(sv), *rh = uniform(rhs);
-    auto load = [&](uint32_t q) {
-        q = min(q, k1 - 1);
-        const float *c = val + (size_t)q * stride, *rr = rh + (size_t)q * kWave;   // (scalar bases, the lane's offset)
-        const uint4 *m = meta + (size_t)q * kWave;
-        SwChunk t;
-        t.m = m[lane];
-        t.v = reinterpret_cast<const float4 *>(c)[lane];
-        t.r = rr[lane];
-        t.d = (c + doff)[lane];
-        return t;
-    };
-    const uint32_t *X = reinterpret_cast<const uint32_t *>(xs);
-    auto peek = [&](uint32_t a) { return __hip_atomic_load(X + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
-    SwChunk c0 = load(k);
-    asm volatile("" ::: "memory");   // (in this order, which the waits count on)
-    SwChunk c1 = load(k + 1);
-    asm volatile("" ::: "memory");
-    SwChunk c2 = load(k + 2);
-    float acc = 0.f;   // a long row's running value, the same in every lane
-    auto run = [&](uint32_t q, const SwChunk &t) __attribute__((always_inline)) {
-        if (q >= k1) return;
-        const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w);
-        const uint32_t a0 = t.m.x & 0xffffu, a1 = t.m.x >> 16, a2 = t.m.y & 0xffffu, a3 = t.m.y >> 16;
-        const uint32_t row = t.m.z & 0xffffu;
-        uint32_t b0, b1, b2, b3;
-        if (h & kSwLong) {
-            const uint32_t np = h & kSwPassMask;   // passes less 1 (uniform)
-            if (h & kSwFirst) acc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t.r)));
-            const uint32_t ad[4] = {a0, a1, a2, a3};
-            const float w[4] = {t.v.x, t.v.y, t.v.z, t.v.w};
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                if (u > np) break;
-                uint32_t b;
-                for (;;) {
-                    b = peek(ad[u]);
-                    if (!__ballot(b == kUnset)) break;
-                    __builtin_amdgcn_s_sleep(1);
-                }
-                slice[lane] = w[u] * sw_f(b);
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                acc = serial_sub(acc, slice, kWave, false);   // places without an entry hold +0
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            }
-            if ((h & kSwLast) && lane == 0) sw_put(xs, row, D.div ? acc / t.d : acc);
-            return;
-        }
-        const uint32_t lg = (t.m.z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
-        uint64_t left = __ballot((t.m.z & kSwOn) && j == g - 1u);   // lanes that store rows still to come
-        const uint64_t F = __ballot(j == 0);
-        uint64_t V = 0;                            // lanes whose running value is final (rows in order)
-        SwDiv dv{1.f, 1.f, true};
-        if (D.div) dv = sw_div_prepare(t.d);
-        float a = 0.f;
-        // one of the few waves that carry the chain of narrow levels goes
-        // before the others, which give way while they wait
-        const bool narrow = h & kSwNarrow;
-        if (narrow) __builtin_amdgcn_s_setprio(2);
-        for (;;) {
-            b0 = peek(a0), b1 = peek(a1), b2 = peek(a2), b3 = peek(a3);
-            const uint64_t R = __ballot(max(max(b0, b1), max(b2, b3)) != kUnset);   // lanes whose entries are all set
-            const float p0 = t.v.x * sw_f(b0), p1 = t.v.y * sw_f(b1), p2 = t.v.z * sw_f(b2), p3 = t.v.w * sw_f(b3);
-            bool more;
-            do {
-                // lane j's value is lane j - 1's less its own four products;
-                // a step settles the next ready lane of every row, and does
-                // not change settled ones
-                const float prev = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xf, 0xf, false));
-                a = j == 0 ? t.r : prev;
-                a = a - p0;
-                a = a - p1;
-                a = a - p2;
-                a = a - p3;
-                V = R & (F | (V << 1));
-                const uint64_t fin = V & left;
-                more = (R & (F | (V << 1))) != V;
-                if (fin) {
-                    const float res = D.div ? sw_div(dv, a, fin) : a;
-                    if (__builtin_amdgcn_inverse_ballot_w64(fin)) sw_put(xs, row, res);
-                    left &= ~fin;
-                }
-            } while (more);
-            if (!left) break;
-            if (!narrow) __builtin_amdgcn_s_sleep(1);
-        }
-        if (narrow) __builtin_amdgcn_s_setprio(0);
-    };
-    // (three times the code: moved from one to the next, the chunks would be
-    // waited for; loads and one exit on every path, for the counts)
-    for (; k < k1; k += 3) {
-        run(k, c0);
-        c0 = load(k + 3);
-        run(k + 1, c1);
-        c1 = load(k + 4);
-        run(k + 2, c2);
-        c2 = load(k + 5);
-    }
-}
-
-// Part P of sweep D, a level a step: every wave of the workgroup calls it and
-// meets the others once a step, so a chunk's entries are read once, without
-// asking whether they are set.  What does not depend on them (the wait for
-// the chunk's loads, three chunks ahead; addresses; the divisor's reciprocal)
-// is done in a step where the wave has no chunk.  Bound by the step: an LDS
-// round trip, 60 or so dependent instructions, the barrier of 16 waves.
-// (Waiting for each entry to be set, as the exact solve does, polled LDS from
-// 16 waves; a summed row has nothing to do early.  n=50,000, adjoint gradient
-// 2,814 -> 2,600 us; n=9,973 to 1e-12 730 -> 647 us; 16 patterns of about
-// 30,000 in one call 1,826 -> 1,512 us.)
+// Part P of sweep D by the calling workgroup (right-hand sides written, the
+// vector's constant slots set, behind a barrier): every wave meets the others
+// once a step, so a chunk's entries are read once, without asking whether
+// they are set.  What does not depend on the last of them is done in a step
+// where the wave has no chunk: the wait for the chunk's loads (three chunks
+// ahead), addresses, the divisor's reciprocal and, where a row's products are
+// subtracted one at a time in its order (kExact: every row, the arithmetic of
+// Symbolic_Matrix::solve; slice: the wave's 64 floats of LDS for long rows),
+// the subtractions of the entries set two steps ago, so that those of the
+// last step's remain.  Bound by the step: an LDS round trip, 60 or so
+// dependent instructions, the barrier of 16 waves.
+// (Waiting for each entry to be set polled LDS from 16 waves.  Refinement,
+// n=50,000, adjoint gradient 2,814 -> 2,600 us; n=9,973 to 1e-12 730 -> 647 us;
+// 16 patterns of about 30,000 in one call 1,826 -> 1,512 us.  Exact solves:
+// n=4,960 A' 166 -> 145 us, n=50,000 407 -> 374 us; factor and solve n=4,960
+// 314 -> 276 us, n=20,000 654 -> 605 us.)
+template <bool kExact>
 __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const float *__restrict__ sv,
-                                         const float *__restrict__ rhs, float *xs)
+                                         const float *__restrict__ rhs, float *xs, float *slice)
 {
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     uint32_t k = __builtin_amdgcn_readfirstlane(w < D.nwave ? D.wptr[P.wp + w] : 0u);
@@ -2417,7 +2288,8 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
     asm volatile("" ::: "memory");   // (in this order, which the waits count on)
     SwChunk c1 = load(k + 1), c2;
     uint32_t done = 0;   // steps
-    float acc = 0.f, first = 0.f;   // a long row's running value, right-hand side
+    // of the long rows open: running value (exact: the same in every lane), right-hand side
+    float acc_a = 0.f, acc_b = 0.f, first_a = 0.f, first_b = 0.f;
     const uint32_t base = lds_address(xs);
     auto at = [&](uint32_t a) -> float { return *lds_at(a); };
     auto meet = [&]() {
@@ -2425,7 +2297,7 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
         ++done;
     };
     auto run = [&](uint32_t q, const SwChunk &t, SwChunk &next) __attribute__((always_inline)) {
-        const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w), step = (h >> kSwStepShift) & kSwStepMask;
+        const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w), step = h & kSwStepMask;
         if (q < k1 && done < step) meet();
         next = load(q + 2);
         if (q >= k1) return;
@@ -2434,60 +2306,161 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
         uint32_t a2 = base + ((t.m.y & 0xffffu) << 2), a3 = base + ((t.m.y >> 16) << 2);
         uint32_t row = t.m.z & 0xffffu;
         const uint32_t lg = (t.m.z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
-        const bool tree = t.m.z & kSwTree;
+        const bool tree = !kExact && (t.m.z & kSwTree);
         const bool stores = (h & kSwLong) ? lane == 0 : (t.m.z & kSwOn) && (tree ? j == 0 : j == g - 1u);
         const uint64_t S = __ballot(stores);
-        uint32_t lanes = 1;   // of the chunk's widest row summed in order
-        if (!(h & kSwLong))
-            while (__ballot((t.m.z & kSwOn) && !tree && g > lanes)) lanes *= 2;
         SwDiv dv{1.f, 1.f, true};
         if (D.div) dv = sw_div_prepare(t.d);
         asm volatile("" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(row));   // before the meeting, not after
         asm volatile("" : "+v"(dv.r), "+v"(dv.d));
-        while (done < step) meet();
-        const float p0 = t.v.x * at(a0), p1 = t.v.y * at(a1), p2 = t.v.z * at(a2), p3 = t.v.w * at(a3);
         float res;
-        if (h & kSwLong) {
-            // (a place without an entry adds nothing, not even +0)
-            if (h & kSwFirst) first = t.r;
-            float s = acc;
-            if (t.m.z & kSwEntry) s = (h & kSwFirst) ? p0 : s + p0;
-            if (t.m.z & (kSwEntry << 1)) s += p1;
-            if (t.m.z & (kSwEntry << 2)) s += p2;
-            if (t.m.z & (kSwEntry << 3)) s += p3;
-            acc = s;
-            if (!(h & kSwLast)) return;
-            res = first - group_sum(acc, 64);
-        } else {
-            res = t.r;
-            if (h & kSwHasSeq) {
-                float a = t.r - p0;
-                a = a - p1;
-                a = a - p2;
-                a = a - p3;
-                // lane j's value is lane j - 1's less its own four products
-                for (uint32_t s = 1; s < lanes; ++s) {
+        if (kExact) {
+            const bool ahead = done < step;
+            if (h & kSwLong) {
+                const uint32_t early = (h >> kSwEarlyShift) & kSwEarlyMask, count = t.m.z >> kSwCountShift;   // (uniform)
+                const bool second = h & kSwTrack;
+                float acc = second ? acc_b : acc_a;
+                // the entries [lo, hi) of the chunk among its u-th 64
+                auto chain = [&](uint32_t u, uint32_t lo, uint32_t hi) __attribute__((always_inline)) {
+                    const uint32_t e = 64 * u + lane;
+                    const float p = (u == 0 ? t.v.x : u == 1 ? t.v.y : u == 2 ? t.v.z : t.v.w) *
+                                    at(u == 0 ? a0 : u == 1 ? a1 : u == 2 ? a2 : a3);
+                    slice[lane] = e >= lo && e < hi ? p : 0.f;   // (a - 0 is a)
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    const float4 *p4 = reinterpret_cast<const float4 *>(slice);
+                    if (lo <= 64 * u && 64 * u + 64 <= hi)
+                        acc = serial_sub(acc, slice, kWave, false);
+                    else {
+                        const uint32_t c1 = (min(hi - 64 * u, 64u) + 15) / 16;   // by 16 (uniform)
+                        for (uint32_t c = lo > 64 * u ? (lo - 64 * u) / 16 : 0u; c < c1; ++c) {
+                            const float4 q[4] = {p4[4 * c], p4[4 * c + 1], p4[4 * c + 2], p4[4 * c + 3]};
+#pragma unroll
+                            for (uint32_t i = 0; i < 4; ++i) {
+                                acc = acc - q[i].x;
+                                acc = acc - q[i].y;
+                                acc = acc - q[i].z;
+                                acc = acc - q[i].w;
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                };
+                if (h & kSwFirst) acc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(t.r)));
+                if (ahead) {
+                    while (done + kSwLead < step) meet();
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u) {
+                        if (64 * u >= early) break;
+                        chain(u, 0u, early);
+                        if (done + 1 < step) meet();
+                    }
+                }
+                while (done < step) meet();
+                const uint32_t lo = ahead ? early : 0u;
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u)
+                    if (64 * u < count && 64 * u + 64 > lo) chain(u, lo, count);
+                if (second) acc_b = acc;
+                else acc_a = acc;
+                if (!(h & kSwLast)) return;
+                res = acc;
+            } else {
+                const uint32_t pre = (h >> kSwPreShift) & kSwPreMask, rem = (h >> kSwRemShift) & kSwRemMask;   // (uniform)
+                float p0, p1, p2, p3, a = 0.f;
+                // lane j's value is lane j - 1's less its own four products;
+                // a step settles the next lane of every row, and does not
+                // change settled ones
+                auto link = [&]() __attribute__((always_inline)) {
                     float b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xf, 0xf, false));
                     b = b - p0;
                     b = b - p1;
                     b = b - p2;
                     b = b - p3;
-                    a = j == s ? b : a;
+                    a = j == 0 ? a : b;
+                };
+                auto links = [&](uint32_t k) __attribute__((always_inline)) {
+                    for (; k >= 4; k -= 4) {
+                        link();
+                        link();
+                        link();
+                        link();
+                    }
+                    if (k & 2) {
+                        link();
+                        link();
+                    }
+                    if (k & 1) link();
+                };
+                auto begin = [&]() __attribute__((always_inline)) {
+                    p0 = t.v.x * at(a0), p1 = t.v.y * at(a1), p2 = t.v.z * at(a2), p3 = t.v.w * at(a3);
+                    float b = t.r - p0;
+                    b = b - p1;
+                    b = b - p2;
+                    b = b - p3;
+                    a = j == 0 ? b : a;
+                };
+                while (done + 1 < step) meet();
+                if (ahead && pre) {   // (lanes with entries not set yet: anything, until the step itself)
+                    begin();
+                    links(pre);
                 }
+                while (done < step) meet();
+                begin();
+                links(ahead ? rem : pre + rem);
                 res = a;
             }
-            if (h & kSwHasTree) {
-                float q = (p0 + p1) + (p2 + p3);
-                q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0xB1, 0xf, 0xf, false));   // quad [1,0,3,2]
-                q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x4E, 0xf, 0xf, false));   // quad [2,3,0,1]
-                const float q8 = q + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x141, 0xf, 0xf, false));   // half mirror
-                const float q16 = q8 + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q8), 0x140, 0xf, 0xf, false));  // mirror
-                const float tv = t.r - (lg == 2u ? q : lg == 3u ? q8 : q16);
-                res = tree ? tv : res;
+        } else {
+            uint32_t lanes = 1;   // of the chunk's widest row summed in order
+            if (!(h & kSwLong))
+                while (__ballot((t.m.z & kSwOn) && !tree && g > lanes)) lanes *= 2;
+            while (done < step) meet();
+            const float p0 = t.v.x * at(a0), p1 = t.v.y * at(a1), p2 = t.v.z * at(a2), p3 = t.v.w * at(a3);
+            if (h & kSwLong) {
+                // (a place without an entry adds nothing, not even +0)
+                const bool second = h & kSwTrack;
+                const float first = (h & kSwFirst) ? t.r : second ? first_b : first_a;
+                float s = second ? acc_b : acc_a;
+                if (t.m.z & kSwEntry) s = (h & kSwFirst) ? p0 : s + p0;
+                if (t.m.z & (kSwEntry << 1)) s += p1;
+                if (t.m.z & (kSwEntry << 2)) s += p2;
+                if (t.m.z & (kSwEntry << 3)) s += p3;
+                if (second) acc_b = s, first_b = first;
+                else acc_a = s, first_a = first;
+                if (!(h & kSwLast)) return;
+                res = first - group_sum(s, 64);
+            } else {
+                res = t.r;
+                if (h & kSwHasSeq) {
+                    float a = t.r - p0;
+                    a = a - p1;
+                    a = a - p2;
+                    a = a - p3;
+                    // lane j's value is lane j - 1's less its own four products
+                    for (uint32_t s = 1; s < lanes; ++s) {
+                        float b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x111, 0xf, 0xf, false));
+                        b = b - p0;
+                        b = b - p1;
+                        b = b - p2;
+                        b = b - p3;
+                        a = j == s ? b : a;
+                    }
+                    res = a;
+                }
+                if (h & kSwHasTree) {
+                    float q = (p0 + p1) + (p2 + p3);
+                    q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0xB1, 0xf, 0xf, false));   // quad [1,0,3,2]
+                    q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x4E, 0xf, 0xf, false));   // quad [2,3,0,1]
+                    const float q8 = q + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x141, 0xf, 0xf, false));   // half mirror
+                    const float q16 = q8 + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q8), 0x140, 0xf, 0xf, false));  // mirror
+                    const float tv = t.r - (lg == 2u ? q : lg == 3u ? q8 : q16);
+                    res = tree ? tv : res;
+                }
             }
         }
         if (D.div) res = sw_div(dv, res, S);
-        if (stores) sw_put(xs, row, res);
+        if (stores) xs[row] = res;
     };
     // (three times the code: moved from one to the next, the chunks would be
     // waited for; loads and one exit on every path, for the counts)
@@ -2499,29 +2472,10 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
     while (done < steps) meet();
 }
 
-// The LDS vector of a part before its sweep: rows not set, then the constant
-// slots 0 and 1.
-__device__ __forceinline__ void sw_clear(float *xs, uint32_t nslot)
+// The constant slots of a part's vector in LDS.
+__device__ __forceinline__ void sw_constants(float *xs, uint32_t nslot)
 {
-    uint32_t *xb = reinterpret_cast<uint32_t *>(xs);
-    for (uint32_t i = threadIdx.x; i < nslot + 2; i += blockDim.x)
-        xb[i] = i < nslot ? kUnset : i == nslot ? 0u : 0x3f800000u;
-}
-
-// Part P of sweep D by the calling workgroup (vector cleared and right-hand
-// sides written, behind a barrier); wl: the workgroup's wave slices (kExact).
-template <bool kExact>
-__device__ __forceinline__ void sw_part(const SwDev &D, const SwPart &P, const float *sv, const float *rhs, float *xs,
-                                        float *wl)
-{
-    if (!kExact) {
-        sw_steps(D, P, sv, rhs, xs);
-        return;
-    }
-    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    if (w < D.nwave)
-        sw_wave(D, __builtin_amdgcn_readfirstlane(D.wptr[P.wp + w]), __builtin_amdgcn_readfirstlane(D.wptr[P.wp + w + 1]),
-                sv, rhs, xs, wl + w * kWave);
+    if (threadIdx.x < 2) xs[nslot + threadIdx.x] = threadIdx.x ? 1.f : 0.f;
 }
 
 // rhs[rpos[i]] = float(v[src[r]] * scale[r]) for the rows r of part P (slot
@@ -2578,15 +2532,15 @@ template <bool kExact>
 __device__ __forceinline__ void sw_both(const SwDev &A, const SwDev &B, const float *sv, float *rhs, float *xs, float *wl)
 {
     const SwPart P = A.part[0], Q = B.part[0];
-    sw_clear(xs, P.nslot);
+    sw_constants(xs, P.nslot);
     __syncthreads();
-    sw_part<kExact>(A, P, sv + A.voff, rhs, xs, wl);
+    sw_steps<kExact>(A, P, sv + A.voff, rhs, xs, wl);
     __syncthreads();
     sw_carry(B, Q, xs, rhs);
     __syncthreads();
-    sw_clear(xs, Q.nslot);
+    sw_constants(xs, Q.nslot);
     __syncthreads();
-    sw_part<kExact>(B, Q, sv + B.voff, rhs, xs, wl);
+    sw_steps<kExact>(B, Q, sv + B.voff, rhs, xs, wl);
     __syncthreads();
 }
 
@@ -3247,7 +3201,7 @@ __global__ void __launch_bounds__(1024) k_solve_one(const MatDesc *__restrict__ 
         globalize(d2);
         sw_scale(d1, d1.part[0], b, glb(kT ? desc->s.tdf_rsrc : desc->s.df_rsrc),
                  glb(kT ? desc->s.tdf_rscale : desc->s.df_rscale), glb(t32));
-        sw_both<true>(d1, d2, glb(lucsr), glb(t32), xs, &wl[0][0]);
+        sw_both<true>(d1, d2, glb(lucsr), glb(t32), xs, wl[threadIdx.x / kWave]);
         if (kT) {   // A' x = b: columns back by col_perm_inv, scaled by col_scale_perm
             const uint32_t *cpi = glb(desc->s.col_perm_inv);
             const double *csp = glb(desc->s.col_scale_perm);
@@ -3312,9 +3266,9 @@ __global__ void __launch_bounds__(1024) k_sw_first(SwDev D, const T *__restrict_
     __shared__ __attribute__((aligned(16))) float wl[kExact ? 1024 / kWave : 1][kWave];
     const SwPart P = D.part[blockIdx.x];
     sw_scale(D, P, in, src, scale, rhs);
-    sw_clear(g_lds_vec, P.nslot);
+    sw_constants(g_lds_vec, P.nslot);
     __syncthreads();
-    sw_part<kExact>(D, P, lucsr + D.voff, rhs, g_lds_vec, &wl[0][0]);
+    sw_steps<kExact>(D, P, lucsr + D.voff, rhs, g_lds_vec, kExact ? wl[threadIdx.x / kWave] : nullptr);
     __syncthreads();
     sw_out(D, P, g_lds_vec, xg);
 }
@@ -3326,7 +3280,7 @@ __global__ void __launch_bounds__(1024) k_sw_tail(SwDev A, SwDev B, const T *__r
 {
     __shared__ __attribute__((aligned(16))) float wl[kExact ? 1024 / kWave : 1][kWave];
     sw_scale(A, A.part[0], in, src, scale, rhs);
-    sw_both<kExact>(A, B, lucsr, rhs, g_lds_vec, &wl[0][0]);
+    sw_both<kExact>(A, B, lucsr, rhs, g_lds_vec, kExact ? wl[threadIdx.x / kWave] : nullptr);
     sw_out(B, B.part[0], g_lds_vec, xg);
 }
 
@@ -3337,9 +3291,9 @@ __global__ void __launch_bounds__(1024) k_sw_second(SwDev D, const float *__rest
     __shared__ __attribute__((aligned(16))) float wl[kExact ? 1024 / kWave : 1][kWave];
     const SwPart P = D.part[blockIdx.x];
     for (uint32_t i = threadIdx.x; i < P.nslot; i += blockDim.x) rhs[D.rpos[P.s0 + i]] = xg[D.row[P.s0 + i]];
-    sw_clear(g_lds_vec, P.nslot);
+    sw_constants(g_lds_vec, P.nslot);
     __syncthreads();
-    sw_part<kExact>(D, P, lucsr + D.voff, rhs, g_lds_vec, &wl[0][0]);
+    sw_steps<kExact>(D, P, lucsr + D.voff, rhs, g_lds_vec, kExact ? wl[threadIdx.x / kWave] : nullptr);
     __syncthreads();
     sw_out(D, P, g_lds_vec, xg);
 }

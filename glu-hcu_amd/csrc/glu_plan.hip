@@ -1871,17 +1871,9 @@ inline uint32_t sw_lanes(uint32_t len, bool sum = false)
     return g;
 }
 
-// A chunk that starts in a level of at most a chunk's lanes goes to one of a
-// few waves (one per SIMD): there the sweep is a chain, and more waves only
-// wait beside it (n=200,003: 6,434 us a factor and solve with all 16, 6,161
-// with 4, 6,605 with 1).
-constexpr uint32_t kSwNarrowLanes = 64, kSwNarrowWaves = 4;
-
-// Chunks go to the part's waves in turn, in schedule order; the rows of
+// Chunks go to the part's waves in turn, a level after the other; the rows of
 // several chunks, which take their time but can start early, to waves of
-// their own (each wave runs its chunks in order, and every dependency lies in
-// an earlier chunk of the schedule or an earlier lane of the same one, so the
-// first unfinished chunk can always finish: check_sw).
+// their own.
 void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwParts &Q, uint32_t waves, SwHost &S)
 {
     const uint32_t nparts = (uint32_t)Q.count.size();
@@ -1949,15 +1941,26 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
             uint32_t &w = e < 2 ? m.x : m.y;
             w = (e & 1) ? (w & 0xffffu) | slot << 16 : (w & 0xffff0000u) | slot;
         };
+        std::vector<uint32_t> step_of(nslot, 0);   // a row's step
+        auto ready = [&](const Pos &x, uint32_t k, uint32_t step, uint32_t before) {   // entry k of x: set that many steps before
+            const uint32_t col = D.idx[x.base + (size_t)k * x.step];
+            return Q.part_of[col] != part || step_of[Q.slot_of[col]] + before <= step;
+        };
+        // waves for the rows of several chunks, by their share of the work (a
+        // chunk of 256 subtractions in order takes about 0.75 us, another
+        // 0.2): at most three quarters
         size_t multi = 0;
-        for (const Pos &x : R) multi += is_long(x) && x.len > kSwEntries;
-        const uint32_t own = waves >= 4 ? (uint32_t)std::min<size_t>(multi, std::max(1u, waves * 3 / 8)) : 0u;
-        std::vector<uint32_t> lanes_at(R.empty() ? 0 : R.back().level + 1, 0);   // lanes of each level
-        for (const Pos &x : R) lanes_at[x.level] += is_long(x) ? 0 : sw_lanes(x.len, x.sum);
+        double rails = 0.0, rest = 1.0;
+        for (const Pos &x : R) {
+            const bool m = is_long(x) && x.len > kSwEntries;
+            multi += m;
+            (m ? rails : rest) += m ? 0.75 / kSwEntries * x.len : 0.2 / 64 * (is_long(x) ? 64 : sw_lanes(x.len, x.sum));
+        }
+        const uint32_t own = waves < 4 || !multi ? 0u
+            : (uint32_t)std::min<size_t>(multi, std::max(1u, (uint32_t)std::min(0.75 * waves, waves * rails / (rails + rest) + 0.5)));
         uint32_t turn = 0, turn_long = 0, used = 64;
-        std::vector<uint32_t> step_of(nslot, 0), wave_step(waves, 0);   // a row's step; the step a wave's chunks got to
+        std::vector<uint32_t> track_step(2 * own, 0);   // the step a wave's open rows got to
         for (size_t i = 0; i < R.size(); ++P.steps) {
-            const uint32_t step = P.steps << kSwStepShift;
             used = 64;
             size_t e = i;
             while (e < R.size() && R[e].level == R[i].level) ++e;
@@ -1978,25 +1981,34 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
                 step_of[slot] = P.steps;
                 if (is_long(x)) {
                     const uint32_t nc = (x.len + kSwEntries - 1) / kSwEntries;
-                    const uint32_t to = nc > 1 && own ? turn_long++ % own : own + turn++ % (waves - own);
+                    // a row of several chunks: its chunks spread over the
+                    // steps before its own, one of two rows a wave has open
+                    const bool rail = nc > 1 && own;
+                    const uint32_t track = rail ? turn_long++ % (2 * own) : 0u;
+                    const uint32_t to = rail ? track % own : own + turn++ % (waves - own);
                     for (uint32_t c = 0; c < nc; ++c) {
                         const uint32_t left = std::min(x.len - c * kSwEntries, kSwEntries);
-                        // the row's step ends it; what is before runs as soon
-                        // as its entries are set and the wave is there
-                        uint32_t at = c + 1 == nc ? P.steps : wave_step[to];
-                        for (uint32_t k = 0; k < left && c + 1 < nc; ++k) {
-                            const uint32_t col = D.idx[x.base + (size_t)(c * kSwEntries + k) * x.step];
-                            if (Q.part_of[col] == part) at = std::max(at, step_of[Q.slot_of[col]] + 1);
+                        uint32_t at = P.steps;   // the row's step ends it
+                        if (rail && c + 1 < nc) {
+                            const uint32_t from = track_step[track], gap = (P.steps - from) / (nc - c);
+                            at = std::min(from + std::min(std::max(gap, 1u), kSwLead), P.steps);
+                            for (uint32_t k = 0; k < left; ++k) {
+                                const uint32_t col = D.idx[x.base + (size_t)(c * kSwEntries + k) * x.step];
+                                if (Q.part_of[col] == part) at = std::max(at, step_of[Q.slot_of[col]] + 1);
+                            }
                         }
-                        wave_step[to] = at;
-                        add(at << kSwStepShift | kSwLong | (c == 0 ? kSwFirst : 0u) | (c + 1 == nc ? kSwLast : 0u) | ((left + 63) / 64 - 1));
+                        if (rail) track_step[track] = at;
+                        uint32_t early = 0;   // leading entries set well before
+                        while (early < left && ready(x, c * kSwEntries + early, at, kSwLead + 1)) ++early;
+                        add(at | kSwLong | (c == 0 ? kSwFirst : 0u) | (c + 1 == nc ? kSwLast : 0u) |
+                            (rail && track >= own ? kSwTrack : 0u) | early << kSwEarlyShift);
                         wave.push_back(to);
                         uint32_t bits[64] = {};
                         for (uint32_t k = 0; k < left; ++k) {
                             put(k % 64, k / 64, x, c * kSwEntries + k);
                             bits[k % 64] |= kSwEntry << (k / 64);
                         }
-                        for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (hdr.size() - 1) + lane].z = slot | bits[lane];
+                        for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (hdr.size() - 1) + lane].z = slot | bits[lane] | left << kSwCountShift;
                         if (c == 0) rpos[slot] = 64 * (uint32_t)(hdr.size() - 1);
                         if (c + 1 == nc && div) vsrc[(hdr.size() - 1) * S.stride + kSwEntries] = x.pivot;
                     }
@@ -2005,14 +2017,23 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
                 const uint32_t g = sw_lanes(x.len, x.sum);
                 used = (used + g - 1) & ~(g - 1);
                 if (used + g > 64) {
-                    const bool few = lanes_at[x.level] <= kSwNarrowLanes;
-                    add(step | (few ? kSwNarrow : 0u));
-                    wave.push_back(own + turn++ % (few ? std::min(kSwNarrowWaves, waves - own) : waves - own));
-                    wave_step[wave.back()] = P.steps;
+                    add(P.steps);
+                    wave.push_back(own + turn++ % (waves - own));
                     used = 0;
                 }
                 const size_t c = hdr.size() - 1;
                 hdr[c] |= x.sum ? kSwHasTree : kSwHasSeq;
+                uint32_t early = 0;   // leading lanes whose entries are set two steps before
+                while (early < g) {
+                    bool all = true;
+                    for (uint32_t k = 4 * early; k < std::min(4 * early + 4, x.len); ++k) all = all && ready(x, k, P.steps, 2);
+                    if (!all) break;
+                    ++early;
+                }
+                const uint32_t pre = early ? early - 1 : 0, rem = early ? g - early : g - 1;
+                hdr[c] = (hdr[c] & ~(kSwPreMask << kSwPreShift | kSwRemMask << kSwRemShift)) |
+                         std::max(pre, (hdr[c] >> kSwPreShift) & kSwPreMask) << kSwPreShift |
+                         std::max(rem, (hdr[c] >> kSwRemShift) & kSwRemMask) << kSwRemShift;
                 for (uint32_t lane = 0; lane < g; ++lane)
                     meta[64 * c + used + lane].z = slot | (uint32_t)__builtin_ctz(g) << 16 | (x.sum ? kSwTree : 0u) | kSwOn;
                 for (uint32_t k = 0; k < x.len; ++k) put(used + k / 4, k % 4, x, k);
@@ -2025,15 +2046,18 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
         }
         // stream by stream
         std::vector<uint32_t> at(hdr.size());
+        std::vector<std::vector<uint32_t>> stream(waves);
+        for (size_t c = 0; c < hdr.size(); ++c) stream[wave[c]].push_back((uint32_t)c);
         for (uint32_t w = 0; w < waves; ++w) {
             S.wptr.push_back((uint32_t)S.hdr.size());
-            for (size_t c = 0; c < hdr.size(); ++c) {
-                if (wave[c] != w) continue;
+            std::stable_sort(stream[w].begin(), stream[w].end(),
+                             [&](uint32_t a, uint32_t b) { return (hdr[a] & kSwStepMask) < (hdr[b] & kSwStepMask); });
+            for (uint32_t c : stream[w]) {
                 at[c] = (uint32_t)S.hdr.size();
                 S.hdr.push_back(hdr[c]);
-                for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * c + lane].w = hdr[c];
-                S.meta.insert(S.meta.end(), meta.begin() + 64 * c, meta.begin() + 64 * (c + 1));
-                S.vsrc.insert(S.vsrc.end(), vsrc.begin() + c * S.stride, vsrc.begin() + (c + 1) * S.stride);
+                for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (size_t)c + lane].w = hdr[c];
+                S.meta.insert(S.meta.end(), meta.begin() + 64 * (size_t)c, meta.begin() + 64 * ((size_t)c + 1));
+                S.vsrc.insert(S.vsrc.end(), vsrc.begin() + (size_t)c * S.stride, vsrc.begin() + ((size_t)c + 1) * S.stride);
             }
         }
         S.wptr.push_back((uint32_t)S.hdr.size());
@@ -2044,10 +2068,10 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
 }
 
 // Host check of a sweep's streams before any launch: every slot and value
-// position in range, every right-hand side at its row's first lane, every row
-// of a part stored once; and, running each part's streams side by side (a
-// wave moves on once its chunk's rows are done, a row is done once its
-// entries are set), every wave gets to its end: every wait of the sweep ends.
+// position in range, every row of a part stored once, with its right-hand
+// side at its first lane, a stream's steps in order, every entry's row in an
+// earlier step than the entry (and two before where the chunk's header takes
+// it ahead), the chunks of a long row together.
 bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
 {
     auto bad = [&](const std::string &what) {
@@ -2061,88 +2085,73 @@ bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
     for (const SwProd &q : S.prod)
         if (q.val >= S.vsrc.size() || q.vpos >= nnz) return bad("product out of range");
     for (const SwPart &P : S.part) {
-        if ((size_t)P.wp + S.nwave >= S.wptr.size() || (size_t)P.s0 + P.nslot > S.row.size() || P.nslot > 0xfffdu)
+        if ((size_t)P.wp + S.nwave >= S.wptr.size() || (size_t)P.s0 + P.nslot > S.row.size() || P.nslot > 0xfffdu ||
+            P.steps > kSwStepMask + 1)
             return bad("part out of range");
-        std::vector<uint8_t> set(P.nslot + 2, 0);
-        set[P.nslot] = set[P.nslot + 1] = 1;
-        std::vector<uint32_t> at(S.nwave);
-        for (uint32_t w = 0; w < S.nwave; ++w) {
-            at[w] = S.wptr[P.wp + w];
-            if (at[w] > S.wptr[P.wp + w + 1] || S.wptr[P.wp + w + 1] > nchunk) return bad("stream out of range");
-        }
-        // by steps: a stream's steps do not fall, an entry's row has an earlier one
-        std::vector<uint32_t> step_of(P.nslot + 2, 0);   // 1 + the row's step
+        std::vector<uint32_t> set(P.nslot + 2, 0);   // 1 + the row's step
         for (uint32_t pass = 0; pass < 2; ++pass)
-            for (uint32_t w = 0; w < S.nwave; ++w)
-                for (uint32_t c = at[w], last = 0; c < S.wptr[P.wp + w + 1]; ++c) {
-                    const uint32_t h = S.hdr[c], step = (h >> kSwStepShift) & kSwStepMask;
+            for (uint32_t w = 0; w < S.nwave; ++w) {
+                const uint32_t k0 = S.wptr[P.wp + w], k1 = S.wptr[P.wp + w + 1];
+                if (k0 > k1 || k1 > nchunk) return bad("stream out of range");
+                uint32_t last = 0;
+                bool open[2] = {false, false};   // in a long row
+                uint32_t row_open[2] = {0, 0};
+                for (uint32_t c = k0; c < k1; ++c) {
+                    const uint32_t h = S.hdr[c], step = h & kSwStepMask;
                     if (step < last || step >= P.steps) return bad("step out of range");
-                    if ((h & kSwLong) && !(h & kSwFirst) && (c == at[w] || !(S.hdr[c - 1] & kSwLong) || (S.hdr[c - 1] & kSwLast)))
-                        return bad("a row's chunks are apart");
                     last = step;
-                    for (uint32_t lane = 0; lane < 64; ++lane) {
-                        const uint4 &m = S.meta[64 * (size_t)c + lane];
-                        if (pass == 0 && ((h & kSwLong) || (m.z & kSwOn))) {
-                            if ((m.z & 0xffffu) >= P.nslot) return bad("row slot out of range");
-                            if (!(h & kSwLong) || (h & kSwLast)) step_of[m.z & 0xffffu] = step + 1;
-                        }
-                        for (uint32_t v : {m.x & 0xffffu, m.x >> 16, m.y & 0xffffu, m.y >> 16}) {
-                            if (v > P.nslot + 1) return bad("slot out of range");
-                            if (pass == 1 && step_of[v] > step) return bad("an entry's row is not in an earlier step");
-                        }
-                    }
-                }
-        uint32_t done = 0;
-        for (bool moved = true; moved;) {
-            moved = false;
-            for (uint32_t w = 0; w < S.nwave; ++w)
-                for (; at[w] < S.wptr[P.wp + w + 1]; ++at[w]) {
-                    const uint32_t c = at[w], h = S.hdr[c];
                     auto entry = [&](uint32_t lane, uint32_t e) {
                         const uint4 &m = S.meta[64 * (size_t)c + lane];
                         const uint32_t v = e < 2 ? m.x : m.y;
                         return (e & 1) ? v >> 16 : v & 0xffffu;
                     };
-                    bool whole = true;
+                    for (uint32_t lane = 0; lane < 64; ++lane)
+                        for (uint32_t e = 0; e < 4; ++e) {
+                            if (entry(lane, e) > P.nslot + 1) return bad("slot out of range");
+                            if (pass && set[entry(lane, e)] > step) return bad("an entry's row is not in an earlier step");
+                        }
+                    auto early = [&](uint32_t lane, uint32_t e) { return set[entry(lane, e)] < step || !set[entry(lane, e)]; };
+                    auto store = [&](uint32_t slot) {
+                        if (pass) return true;
+                        const bool once = !set[slot];
+                        set[slot] = step + 1;
+                        return once;
+                    };
                     if (h & kSwLong) {
-                        for (uint32_t lane = 0; lane < 64; ++lane)
-                            for (uint32_t e = 0; e < 4; ++e) {
-                                if (entry(lane, e) > P.nslot + 1) return bad("slot out of range");
-                                whole = whole && set[entry(lane, e)];
-                            }
-                        const uint32_t slot = S.meta[64 * (size_t)c].z & 0xffffu;
-                        if (slot >= P.nslot) return bad("row slot out of range");
-                        if (whole && (h & kSwFirst) && S.rpos[P.s0 + slot] != 64 * c) return bad("right-hand side misplaced");
-                        if (whole && (h & kSwLast)) {
-                            if (set[slot]) return bad("a row runs twice");
-                            set[slot] = 1, ++done;
-                        }
-                    } else {
-                        for (uint32_t lane = 0; lane < 64;) {
-                            const uint32_t z = S.meta[64 * (size_t)c + lane].z, slot = z & 0xffffu, g = 1u << ((z >> 16) & 7u);
-                            if (lane % g || lane + g > 64 || g > 16) return bad("row lanes out of place");
-                            bool rdy = true;
-                            for (uint32_t k = 0; k < g; ++k)
-                                for (uint32_t e = 0; e < 4; ++e) {
-                                    if (entry(lane + k, e) > P.nslot + 1) return bad("slot out of range");
-                                    rdy = rdy && set[entry(lane + k, e)];
-                                }
-                            if (z & kSwOn) {
-                                if (slot >= P.nslot) return bad("row slot out of range");
-                                if (S.rpos[P.s0 + slot] != 64 * c + lane) return bad("right-hand side misplaced");
-                                if (rdy && !set[slot]) set[slot] = 1, ++done, moved = true;
-                                whole = whole && set[slot];
-                            }
-                            lane += g;
-                        }
+                        const uint32_t z = S.meta[64 * (size_t)c].z, slot = z & 0xffffu;
+                        const uint32_t n_early = (h >> kSwEarlyShift) & kSwEarlyMask, count = z >> kSwCountShift;
+                        const uint32_t tr = (h & kSwTrack) ? 1 : 0;
+                        if (open[tr] ? (h & kSwFirst) || slot != row_open[tr] : !(h & kSwFirst)) return bad("a row's chunks are apart");
+                        open[tr] = !(h & kSwLast);
+                        row_open[tr] = slot;
+                        if (slot >= P.nslot || count > kSwEntries || n_early > count) return bad("long row out of range");
+                        for (uint32_t e = 0; e < n_early && pass; ++e)
+                            if (set[entry(e % 64, e / 64)] && set[entry(e % 64, e / 64)] + kSwLead > step) return bad("an entry is taken before it is set");
+                        if ((h & kSwFirst) && S.rpos[P.s0 + slot] != 64 * c) return bad("right-hand side misplaced");
+                        if ((h & kSwLast) && !store(slot)) return bad("a row runs twice");
+                        continue;
                     }
-                    if (!whole) break;
-                    moved = true;
+                    const uint32_t pre = (h >> kSwPreShift) & kSwPreMask, rem = (h >> kSwRemShift) & kSwRemMask;
+                    for (uint32_t lane = 0; lane < 64;) {
+                        const uint32_t z = S.meta[64 * (size_t)c + lane].z, slot = z & 0xffffu, g = 1u << ((z >> 16) & 7u);
+                        if (lane % g || lane + g > 64 || g > 16) return bad("row lanes out of place");
+                        if (z & kSwOn) {
+                            if (slot >= P.nslot) return bad("row slot out of range");
+                            if (S.rpos[P.s0 + slot] != 64 * c + lane) return bad("right-hand side misplaced");
+                            if (!store(slot)) return bad("a row runs twice");
+                            uint32_t n_early = 0;   // lanes done a step ahead
+                            while (n_early < std::min(g, pre + 1) && early(lane + n_early, 0) && early(lane + n_early, 1) &&
+                                   early(lane + n_early, 2) && early(lane + n_early, 3))
+                                ++n_early;
+                            if (pass && (g - std::max(n_early, 1u) > rem || g - 1 > pre + rem)) return bad("a row is cut short");
+                        }
+                        lane += g;
+                    }
                 }
-        }
-        for (uint32_t w = 0; w < S.nwave; ++w)
-            if (at[w] != S.wptr[P.wp + w + 1]) return bad("a row waits for one that never runs");
-        if (done != P.nslot) return bad("a row never runs");
+                if (open[0] || open[1]) return bad("a row does not end");
+            }
+        for (uint32_t k = 0; k < P.nslot; ++k)
+            if (!set[k]) return bad("a row never runs");
     }
     return true;
 }
