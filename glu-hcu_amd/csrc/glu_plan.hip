@@ -21,6 +21,7 @@
 #include <string>
 #include <atomic>
 #include <system_error>
+#include <future>
 #include <thread>
 #include <vector>
 
@@ -2438,11 +2439,21 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
             }, no_pivot);
         }
     };
-    parallel_items(long_lanes ? 6 : 5, table_threads(), [&](unsigned, size_t item) {
-        if (item == 0)
-            choose_windows(T, P.num_lev, P.nnz, budget, (uint32_t)p->fuse_units, p->max_windows, wg_waves, wins);
-        else if (item < 5)
-            sweep_tables((int)item - 1);
+    // (the phases, the longest, beside all that comes before they are needed)
+    std::vector<Phase> phases;
+    const auto windows_and_phases = [&]() {
+        choose_windows(T, P.num_lev, P.nnz, budget, (uint32_t)p->fuse_units, p->max_windows, wg_waves, wins);
+        choose_phases(P, T, wins.empty() ? 0 : std::min(wins[0].l0, P.num_lev), phases);
+    };
+    std::future<void> factor_steps;   // (waits in its destructor, before what it works on goes)
+    try {
+        factor_steps = std::async(std::launch::async, windows_and_phases);
+    } catch (const std::system_error &) {   // no thread to be had
+        windows_and_phases();
+    }
+    parallel_items(long_lanes ? 5 : 4, table_threads(), [&](unsigned, size_t item) {
+        if (item < 4)
+            sweep_tables((int)item);
         else
             split = choose_split(P, (uint32_t)std::min<size_t>(p->lds_cap / sizeof(float), 0xffffu) - 2, wg_waves, spl);
     });
@@ -2460,47 +2471,6 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         for (int i = 0; i < 8; ++i)
             if (!wgood[i]) return fail(GLU_ERR_INVALID, werr[i]);
     }
-    p->nwin = (int)wins.size();
-    for (const Window &w : wins) {
-        p->win_steps += w.l1 - w.l0;
-        p->win_nslot = std::max<uint32_t>(p->win_nslot, (uint32_t)w.pos.size());
-        p->win_slots.push_back((uint32_t)w.pos.size());
-    }
-    std::vector<Phase> phases;
-    choose_phases(P, T, wins.empty() ? 0 : std::min(wins[0].l0, P.num_lev), phases);
-    T.umap = std::vector<uint32_t>();
-    factor_segments(*p, T, phases, wins);
-    p->units = (int64_t)(T.cln.size() / 64);
-    // The batched kernels' leading grid steps: those ahead of the first LDS
-    // window with at least a workgroup's worth of lanes per matrix (a
-    // narrower step takes one pass of the per-matrix workgroup anyway).
-    {
-        const int lim = std::min({wins.empty() ? P.num_lev : std::min(wins[0].l0, P.num_lev),
-                                  p->batch_grid_opt < 0 ? 0 : p->batch_grid_opt > 0 ? p->batch_grid_opt : INT32_MAX});
-        const uint32_t per_wave = launch::il_items_per_wave();
-        for (int l = 0; l < lim && level_lanes(T, l) >= (uint32_t)p->fused_threads; ++l) {
-            const uint32_t ml = T.ment_long[l], nm = T.ment_ptr[l + 1] - T.ment_ptr[l];
-            const uint32_t items = (T.ctask_ptr[l + 1] - T.ctask_ptr[l]) * 64 + (nm - ml) +
-                                   (l > 0 ? T.dvd_ptr[l] - T.dvd_ptr[l - 1] : 0u);   // + previous step's divisions
-            p->grid_waves.push_back(ml + (items + per_wave - 1) / per_wave);
-        }
-        p->batch_grid_lev = (int)p->grid_waves.size();
-    }
-    // Division items: those of the columns of each of the batched kernels'
-    // grid steps but the last run with the next grid step (kept step by
-    // step); the rest run in one pass after the last step (the single path
-    // runs them all there).  Each step's items, and the rest, are in
-    // position order: a wave's items are then consecutive L entries of a
-    // column (each column's first entry first) and read and write whole
-    // lines.
-    {
-        const auto by_pos = [](const uint2 &a, const uint2 &b) { return a.x < b.x; };
-        const int early = std::max(p->batch_grid_lev - 1, 0);
-        for (int l = 0; l < early; ++l)
-            std::sort(T.dvd.begin() + T.dvd_ptr[l], T.dvd.begin() + T.dvd_ptr[l + 1], by_pos);
-        std::sort(T.dvd.begin() + T.dvd_ptr[early], T.dvd.end(), by_pos);
-    }
-
     p->scratch_nval[0] = dlo.idx.size() + dup.idx.size() + n + 64;
     p->scratch_nval[1] = dtu.idx.size() + dtl.idx.size() + n + 64;
     uint32_t sw_rhs = 0;
@@ -2546,15 +2516,20 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     if (p->copy_range == 0) return fail(GLU_ERR_DEVICE, "no LDS for the batch value copy");
     std::vector<uint2> df_cpy;
     std::vector<uint32_t> df_cpy_ptr(1, 0);
-    df_cpy.reserve(p->df_nval);
-    for (uint32_t b = 0; b < p->df_nval; b += p->copy_range) {
-        const uint32_t e = std::min<uint32_t>(p->df_nval, b + p->copy_range);
-        const size_t first = df_cpy.size();
-        for (uint32_t q = b; q < e; ++q)
-            if (df_vpos[q] != UINT32_MAX) df_cpy.push_back(make_uint2(df_vpos[q], q - b));
-        std::sort(df_cpy.begin() + first, df_cpy.end(),
-                  [](const uint2 &x, const uint2 &y) { return x.x < y.x || (x.x == y.x && x.y < y.y); });
-        df_cpy_ptr.push_back((uint32_t)df_cpy.size());
+    {
+        std::vector<std::vector<uint2>> range((p->df_nval + p->copy_range - 1) / p->copy_range);
+        parallel_items(range.size(), table_threads(), [&](unsigned, size_t i) {
+            const uint32_t b = (uint32_t)i * p->copy_range, e = std::min<uint32_t>(p->df_nval, b + p->copy_range);
+            for (uint32_t q = b; q < e; ++q)
+                if (df_vpos[q] != UINT32_MAX) range[i].push_back(make_uint2(df_vpos[q], q - b));
+            std::sort(range[i].begin(), range[i].end(),
+                      [](const uint2 &x, const uint2 &y) { return x.x < y.x || (x.x == y.x && x.y < y.y); });
+        });
+        df_cpy.reserve(p->df_nval);
+        for (const auto &r : range) {
+            df_cpy.insert(df_cpy.end(), r.begin(), r.end());
+            df_cpy_ptr.push_back((uint32_t)df_cpy.size());
+        }
     }
 
     // Refinement / refresh tables from the analysis.
@@ -2662,6 +2637,47 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     }
 
     // ---------------- upload everything into one arena ------------------
+    if (factor_steps.valid()) factor_steps.get();
+    p->nwin = (int)wins.size();
+    for (const Window &w : wins) {
+        p->win_steps += w.l1 - w.l0;
+        p->win_nslot = std::max<uint32_t>(p->win_nslot, (uint32_t)w.pos.size());
+        p->win_slots.push_back((uint32_t)w.pos.size());
+    }
+    T.umap = std::vector<uint32_t>();
+    factor_segments(*p, T, phases, wins);
+    p->units = (int64_t)(T.cln.size() / 64);
+    // The batched kernels' leading grid steps: those ahead of the first LDS
+    // window with at least a workgroup's worth of lanes per matrix (a
+    // narrower step takes one pass of the per-matrix workgroup anyway).
+    {
+        const int lim = std::min({wins.empty() ? P.num_lev : std::min(wins[0].l0, P.num_lev),
+                                  p->batch_grid_opt < 0 ? 0 : p->batch_grid_opt > 0 ? p->batch_grid_opt : INT32_MAX});
+        const uint32_t per_wave = launch::il_items_per_wave();
+        for (int l = 0; l < lim && level_lanes(T, l) >= (uint32_t)p->fused_threads; ++l) {
+            const uint32_t ml = T.ment_long[l], nm = T.ment_ptr[l + 1] - T.ment_ptr[l];
+            const uint32_t items = (T.ctask_ptr[l + 1] - T.ctask_ptr[l]) * 64 + (nm - ml) +
+                                   (l > 0 ? T.dvd_ptr[l] - T.dvd_ptr[l - 1] : 0u);   // + previous step's divisions
+            p->grid_waves.push_back(ml + (items + per_wave - 1) / per_wave);
+        }
+        p->batch_grid_lev = (int)p->grid_waves.size();
+    }
+    // Division items: those of the columns of each of the batched kernels'
+    // grid steps but the last run with the next grid step (kept step by
+    // step); the rest run in one pass after the last step (the single path
+    // runs them all there).  Each step's items, and the rest, are in
+    // position order: a wave's items are then consecutive L entries of a
+    // column (each column's first entry first) and read and write whole
+    // lines.
+    {
+        const auto by_pos = [](const uint2 &a, const uint2 &b) { return a.x < b.x; };
+        const int early = std::max(p->batch_grid_lev - 1, 0);
+        for (int l = 0; l < early; ++l)
+            std::sort(T.dvd.begin() + T.dvd_ptr[l], T.dvd.begin() + T.dvd_ptr[l + 1], by_pos);
+        std::sort(T.dvd.begin() + T.dvd_ptr[early], T.dvd.end(), by_pos);
+    }
+
+
     Uploader U;
     const size_t o_colptr = U.put(P.sym_c_ptr, n + 1);
     std::vector<uint32_t> gcols;   // columns of the pattern, long ones first (GESP sums)
