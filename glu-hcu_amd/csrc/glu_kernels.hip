@@ -998,6 +998,7 @@ __device__ __forceinline__ void factor_window(const WinDev &W, float *__restrict
 // value (updates divide on the fly) and no step writes L(:,k) or U(k,k)
 // after column k's step, so the values are those of the per-step order,
 // one barrier-bound pass per step less.
+template <bool kDivide>
 __device__ __forceinline__ void factor_all_wg(const FactorDev &F, float *__restrict__ val, float *slots, float pert,
                                               int perturb, float *wlds, int l0, uint32_t d0)
 {
@@ -1009,6 +1010,7 @@ __device__ __forceinline__ void factor_all_wg(const FactorDev &F, float *__restr
         l = W.l1;
     }
     factor_levels_wg<false>(F, val, l, F.num_lev + 1, pert, perturb, wlds);
+    if (!kDivide) return;   // (the last step ended with a barrier; a launch of their own follows)
     // the divisions, eight items a lane at a time (their loads issued
     // together); items are independent: an item writes its L entry and, for
     // a perturbed pivot, the pivot, which the column's other items divide
@@ -2633,8 +2635,9 @@ __device__ __forceinline__ void wg_values(const MatDesc *Md, const MatIO &io, in
 // Steps 1-4 (l0 = 0), or, after the launches of steps [0, l0) (interleaved,
 // k_factor_grid_il, or phases; GESP value in io.norms[0]), |b|_inf into
 // io.norms[1] with x = 0 and r = b, steps l0.. of step 3 and step 4.
-// d0: the first division item still to do.
-template <bool kCopy>
+// d0: the first division item still to do.  Not kFinish: without the divisions
+// and the copy, which launches of their own do; the GESP value in io.norms[0].
+template <bool kCopy, bool kFinish = true>
 __device__ __forceinline__ void wg_factor(const MatDesc *Md, const MatIO &io, int perturb, double *sh, float *wlds,
                                           int l0, uint32_t d0)
 {
@@ -2662,7 +2665,7 @@ __device__ __forceinline__ void wg_factor(const MatDesc *Md, const MatIO &io, in
     {
         FactorDev F = Md->f;
         globalize(F);
-        factor_all_wg(F, io.lu, g_lds_vec, pert, perturb, wlds, l0, d0);
+        factor_all_wg<kFinish>(F, io.lu, g_lds_vec, pert, perturb, wlds, l0, d0);
     }
 
     // 4. the factors copied into the sweeps' task-contiguous layout, built
@@ -2701,6 +2704,7 @@ __device__ __forceinline__ void wg_factor(const MatDesc *Md, const MatIO &io, in
         }
     }
     if (tid == 0 && io.norms && (l0 == 0 || io.b)) io.norms[1] = bnorm;
+    if (!kFinish && tid == 0) io.norms[0] = (double)pert;
 }
 
 // Workgroup sum in a fixed order (deterministic): each wave's butterfly,
@@ -3314,6 +3318,7 @@ __global__ void __launch_bounds__(256) k_sw_prod(const SwProd *__restrict__ prod
 // assembly of all of them side by side (items {member, block | bin | first
 // wave}).
 constexpr uint32_t kGroupValues = 1024;
+constexpr uint32_t kGroupSpread = 64;   // workgroups a member of the divisions and the copy
 
 __global__ void __launch_bounds__(256) k_group_values(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
                                                       const uint2 *__restrict__ items)
@@ -3371,8 +3376,9 @@ __global__ void __launch_bounds__(256) k_group_assemble(const PhaseDev *__restri
 }
 
 // Then workgroup g runs matrix order[g] with its own tables, from step
-// l0[order[g]].
-template <bool kCopy>
+// l0[order[g]]; the divisions and the copy for the sweeps follow over many
+// workgroups a member, the group leaving most of the card idle otherwise (16
+// patterns of about 30,000: the factor kernel 445 -> 172 us, these 11 and 29).
 __global__ void __launch_bounds__(1024) k_batch_group_factor(const MatDesc *__restrict__ descs,
                                                              const MatIO *__restrict__ ios,
                                                              const uint32_t *__restrict__ order,
@@ -3383,7 +3389,32 @@ __global__ void __launch_bounds__(1024) k_batch_group_factor(const MatDesc *__re
     const uint32_t m = order[blockIdx.x];
     MatIO io = ios[m];
     globalize(io);
-    wg_factor<kCopy>(descs + m, io, perturb, sh, wl[threadIdx.x / kWave], l0[m], 0u);
+    wg_factor<false, false>(descs + m, io, perturb, sh, wl[threadIdx.x / kWave], l0[m], 0u);
+}
+
+__global__ void __launch_bounds__(256) k_group_divide(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
+                                                      const uint32_t *__restrict__ order, int perturb)
+{
+    const uint32_t m = order[blockIdx.y];
+    const float pert = perturb ? (float)glb(ios[m].norms)[0] : 0.f;
+    const uint2 *dvd = glb(descs[m].f.dvd);
+    const uint32_t nd = glb(descs[m].f.dvd_ptr)[descs[m].f.num_lev];
+    float *lu = glb(ios[m].lu);
+    for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < nd; t += gridDim.x * 256)
+        factor_divide(lu, dvd[t], pert, perturb);
+}
+
+__global__ void __launch_bounds__(256) k_group_copy(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
+                                                    const uint32_t *__restrict__ order)
+{
+    const uint32_t m = order[blockIdx.y], nval = descs[m].s.df_nval;
+    const uint32_t *src = glb(descs[m].s.df_src);
+    const float *lu = glb(ios[m].lu);
+    float *to = glb(ios[m].lucsr);
+    for (uint32_t q = blockIdx.x * 256 + threadIdx.x; q < nval; q += gridDim.x * 256) {
+        const uint32_t p = src[q];
+        to[q] = p != ~0u ? lu[p] : 0.f;
+    }
 }
 
 template <int kMode>
@@ -3785,10 +3816,10 @@ void batch_group(const MatDesc *descs, const void *ios, const uint32_t *order, i
                  int maxit, int perturb, int threads, int mode, size_t fact_lds, size_t ref_lds, hipStream_t st)
 {
     const MatIO *io = static_cast<const MatIO *>(ios);
-    if (mode == kSweepLevels)
-        k_batch_group_factor<false><<<count, threads, fact_lds, st>>>(descs, io, order, l0, perturb);
-    else
-        k_batch_group_factor<true><<<count, threads, fact_lds, st>>>(descs, io, order, l0, perturb);
+    const dim3 spread(kGroupSpread, count);
+    k_batch_group_factor<<<count, threads, fact_lds, st>>>(descs, io, order, l0, perturb);
+    k_group_divide<<<spread, 256, 0, st>>>(descs, io, order, perturb);
+    if (mode != kSweepLevels) k_group_copy<<<spread, 256, 0, st>>>(descs, io, order);
     if (mode == kSweepLds)
         k_batch_group_refine<kSweepLds><<<count, threads, ref_lds, st>>>(descs, io, order, tol, maxit);
     else if (mode == kSweepFlags)   // per matrix: vector in LDS where it fits ref_lds
@@ -3850,8 +3881,7 @@ size_t enable_lds()
         reinterpret_cast<const void *>(&k_batch_same_fused<kSweepLds>),
         reinterpret_cast<const void *>(&k_batch_same_refine<kSweepFlags>),
         reinterpret_cast<const void *>(&k_batch_same_refine<kSweepLevels>),
-        reinterpret_cast<const void *>(&k_batch_group_factor<true>),
-        reinterpret_cast<const void *>(&k_batch_group_factor<false>),
+        reinterpret_cast<const void *>(&k_batch_group_factor),
         reinterpret_cast<const void *>(&k_batch_group_refine<kSweepLds>),
         reinterpret_cast<const void *>(&k_batch_group_refine<kSweepFlags>),
         reinterpret_cast<const void *>(&k_batch_group_refine<kSweepLevels>),

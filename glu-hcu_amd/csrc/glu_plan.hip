@@ -3954,7 +3954,7 @@ extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, c
     for (int i = nsplit; i < count; ++i) {
         const glu_plan *p = g->plans[g->order[i]];
         nmax = std::max<size_t>(nmax, p->n);
-        tmax = std::max<size_t>(tmax, sizeof(float) * std::max(p->win_nslot + kWinExtra, p->copy_range));
+        tmax = std::max<size_t>(tmax, sizeof(float) * (p->win_nslot + kWinExtra));
     }
     const int mode = sweep_mode((uint32_t)nmax, cap);
     // ready bits only for the largest order: each matrix whose vector fits
