@@ -214,17 +214,20 @@ struct DfDev {
 };
 
 // A triangular sweep as streams of chunks: the layout of the sweeps whose
-// vector is in LDS, values being their own ready marks.  A chunk is a wave's
-// unit: 64 lanes of four entries.  A row takes 1, 2, 4, 8 or 16 lanes
+// vector is in LDS.  A chunk is a wave's unit: 64 lanes of four entries, rows
+// of one level, which run in one step of the sweep.  A row takes 1, 2, 4, 8 or 16 lanes
 // (aligned), lane j of the row its entries 4 j .. 4 j + 3 in the order the row
-// consumes them, rows of any size side by side in schedule order;
+// consumes them, rows of any size side by side;
 // a row of more than 64 summed entries takes chunks of its own, lane j of
 // such a chunk holding entries j, 64 + j, 128 + j and 192 + j of its 256.
-//   meta[64 c + lane] = {slots of entries 0, 1 (16 bits each), of 2, 3,
-//     row slot | log2 lanes << 16 | kSwTree | kSwOn, the chunk's header}; in a
-//     chunk of a long row kSwEntry << e (the lane has entry e) and its entries
-//   values: value c stride + 4 lane + e is entry e's, c stride + 256 + lane
-//     the row's pivot (div sweeps; at the lane that stores the row)
+// Only the lanes a chunk uses are stored, a multiple of four (a chain of
+// levels of one row each is a chunk a row): F its first lane, u its lanes.
+//   meta[F + lane] = {slots of entries 0, 1 (16 bits each), of 2, 3,
+//     row slot | log2 lanes << 16 | kSwTree | kSwOn, by lane: the chunk's
+//     header; F and u of the wave's chunk two after}; in a chunk of a long row
+//     kSwEntry << e (the lane has entry e) and its entries
+//   values (L = 4, in div sweeps 5, a lane): value F L + 4 lane + e is entry
+//     e's, F L + 4 u + lane the row's pivot (at the lane that stores the row)
 //   a row's right-hand side: rhs[rpos[slot]], at its first lane
 // Slots number the rows of a part (one workgroup's rows); the two after them
 // hold 0 (places without an entry: value 0) and 1 (entries whose column is
@@ -250,7 +253,7 @@ constexpr uint32_t kSwPreShift = 16, kSwPreMask = 15u, kSwRemShift = 20, kSwRemM
 constexpr uint32_t kSwCountShift = 20;   // meta.z of a long row's chunk: its entries
 
 struct SwPart {
-    uint32_t wp;               // wptr[wp + w] .. wptr[wp + w + 1]: wave w's chunks
+    uint32_t wp;               // wave[wp + w]: wave w's chunks
     uint32_t s0, nslot;        // rows row[s0 + slot], right-hand sides rpos[s0 + slot]
     uint32_t steps;
 };
@@ -261,15 +264,14 @@ struct SwProd {
 };
 
 struct SwDev {
-    const uint4 *meta;         // [64 chunks]
-    const uint32_t *wptr;
+    const uint4 *meta;         // [lanes]
+    const uint4 *wave;         // {chunks, F of the first, F of the second, their u | u << 8}
     const SwPart *part;
     const uint32_t *row, *rpos;
     const SwProd *prod;
     uint32_t nprod, nwave;     // nwave: streams per part
-    uint32_t stride, voff;     // floats per chunk; this sweep's first value in the copy
+    uint32_t voff;             // this sweep's first value in the copy
     int32_t div;
-    uint32_t pad;
 };
 
 // The split sweeps of one matrix (a vector beyond LDS): head parts and tail

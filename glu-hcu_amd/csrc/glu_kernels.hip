@@ -1789,7 +1789,7 @@ __device__ __forceinline__ void globalize(TriDev &T)
 __device__ __forceinline__ void globalize(SwDev &D)
 {
     D.meta = glb(D.meta);
-    D.wptr = glb(D.wptr);
+    D.wave = glb(D.wave);
     D.part = glb(D.part);
     D.row = glb(D.row);
     D.rpos = glb(D.rpos);
@@ -2204,6 +2204,7 @@ struct SwChunk {
     uint4 m;
     float4 v;
     float r, d;
+    uint32_t u;   // lanes (uniform)
 };
 
 // a / d with the work on d done ahead (the divisor is known long before the
@@ -2265,30 +2266,34 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
                                          const float *__restrict__ rhs, float *xs, float *slice)
 {
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    uint32_t k = __builtin_amdgcn_readfirstlane(w < D.nwave ? D.wptr[P.wp + w] : 0u);
-    const uint32_t k1 = __builtin_amdgcn_readfirstlane(w < D.nwave ? D.wptr[P.wp + w + 1] : 0u);
+    const uint4 mine = w < D.nwave ? D.wave[P.wp + w] : make_uint4(0u, 0u, 0u, 0u);
+    uint32_t k = 0;
+    const uint32_t k1 = __builtin_amdgcn_readfirstlane(mine.x);
     const uint32_t steps = __builtin_amdgcn_readfirstlane(P.steps);
     if (k >= k1) {
         for (uint32_t s = 0; s < steps; ++s) __syncthreads();
         return;
     }
-    const uint32_t lane = threadIdx.x & (kWave - 1), doff = D.div ? 256u : 0u, stride = D.stride;
+    const uint32_t lane = threadIdx.x & (kWave - 1), per_lane = D.div ? 5u : 4u;
     const uint4 *meta = uniform(D.meta);
     const float *val = uniform(sv), *rh = uniform(rhs);
-    auto load = [&](uint32_t q) {
-        q = min(q, k1 - 1);
-        const float *c = val + (size_t)q * stride, *rr = rh + (size_t)q * kWave;   // (scalar bases, the lane's offset)
-        const uint4 *m = meta + (size_t)q * kWave;
+    // the chunk of lanes [f, f + u) (scalar bases, the lane's offset; lanes
+    // past it read the last's and take no part)
+    auto load = [&](uint32_t f, uint32_t u) {
+        const uint32_t l = min(lane, u - 1);
+        const float *c = val + (size_t)f * per_lane;
         SwChunk t;
-        t.m = m[lane];
-        t.v = reinterpret_cast<const float4 *>(c)[lane];
-        t.r = rr[lane];
-        t.d = (c + doff)[lane];
+        t.m = (meta + f)[l];
+        t.v = reinterpret_cast<const float4 *>(c)[l];
+        t.r = (rh + f)[l];
+        t.d = (c + (D.div ? 4 * u : 0u))[l];
+        t.u = u;
         return t;
     };
-    SwChunk c0 = load(k);
+    const uint32_t us = __builtin_amdgcn_readfirstlane(mine.w);
+    SwChunk c0 = load(__builtin_amdgcn_readfirstlane(mine.y), us & 255u);
     asm volatile("" ::: "memory");   // (in this order, which the waits count on)
-    SwChunk c1 = load(k + 1), c2;
+    SwChunk c1 = load(__builtin_amdgcn_readfirstlane(mine.z), us >> 8), c2;
     uint32_t done = 0;   // steps
     // of the long rows open: running value (exact: the same in every lane), right-hand side
     float acc_a = 0.f, acc_b = 0.f, first_a = 0.f, first_b = 0.f;
@@ -2301,15 +2306,16 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
     auto run = [&](uint32_t q, const SwChunk &t, SwChunk &next) __attribute__((always_inline)) {
         const uint32_t h = __builtin_amdgcn_readfirstlane(t.m.w), step = h & kSwStepMask;
         if (q < k1 && done < step) meet();
-        next = load(q + 2);
+        next = load(__builtin_amdgcn_readlane(t.m.w, 1), __builtin_amdgcn_readlane(t.m.w, 2));
         if (q >= k1) return;
         // (byte addresses)
         uint32_t a0 = base + ((t.m.x & 0xffffu) << 2), a1 = base + ((t.m.x >> 16) << 2);
         uint32_t a2 = base + ((t.m.y & 0xffffu) << 2), a3 = base + ((t.m.y >> 16) << 2);
-        uint32_t row = t.m.z & 0xffffu;
-        const uint32_t lg = (t.m.z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
-        const bool tree = !kExact && (t.m.z & kSwTree);
-        const bool stores = (h & kSwLong) ? lane == 0 : (t.m.z & kSwOn) && (tree ? j == 0 : j == g - 1u);
+        const uint32_t z = lane < t.u ? t.m.z : 0u;
+        uint32_t row = z & 0xffffu;
+        const uint32_t lg = (z >> 16) & 7u, g = 1u << lg, j = lane & (g - 1u);
+        const bool tree = !kExact && (z & kSwTree);
+        const bool stores = (h & kSwLong) ? lane == 0 : (z & kSwOn) && (tree ? j == 0 : j == g - 1u);
         const uint64_t S = __ballot(stores);
         SwDiv dv{1.f, 1.f, true};
         if (D.div) dv = sw_div_prepare(t.d);
@@ -2319,7 +2325,7 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
         if (kExact) {
             const bool ahead = done < step;
             if (h & kSwLong) {
-                const uint32_t early = (h >> kSwEarlyShift) & kSwEarlyMask, count = t.m.z >> kSwCountShift;   // (uniform)
+                const uint32_t early = (h >> kSwEarlyShift) & kSwEarlyMask, count = __builtin_amdgcn_readfirstlane(z) >> kSwCountShift;   // (uniform)
                 const bool second = h & kSwTrack;
                 float acc = second ? acc_b : acc_a;
                 // the entries [lo, hi) of the chunk among its u-th 64
@@ -2416,7 +2422,7 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
         } else {
             uint32_t lanes = 1;   // of the chunk's widest row summed in order
             if (!(h & kSwLong))
-                while (__ballot((t.m.z & kSwOn) && !tree && g > lanes)) lanes *= 2;
+                while (__ballot((z & kSwOn) && !tree && g > lanes)) lanes *= 2;
             while (done < step) meet();
             const float p0 = t.v.x * at(a0), p1 = t.v.y * at(a1), p2 = t.v.z * at(a2), p3 = t.v.w * at(a3);
             if (h & kSwLong) {
@@ -2424,10 +2430,10 @@ __device__ __forceinline__ void sw_steps(const SwDev &D, const SwPart &P, const 
                 const bool second = h & kSwTrack;
                 const float first = (h & kSwFirst) ? t.r : second ? first_b : first_a;
                 float s = second ? acc_b : acc_a;
-                if (t.m.z & kSwEntry) s = (h & kSwFirst) ? p0 : s + p0;
-                if (t.m.z & (kSwEntry << 1)) s += p1;
-                if (t.m.z & (kSwEntry << 2)) s += p2;
-                if (t.m.z & (kSwEntry << 3)) s += p3;
+                if (z & kSwEntry) s = (h & kSwFirst) ? p0 : s + p0;
+                if (z & (kSwEntry << 1)) s += p1;
+                if (z & (kSwEntry << 2)) s += p2;
+                if (z & (kSwEntry << 3)) s += p3;
                 if (second) acc_b = s, first_b = first;
                 else acc_a = s, first_a = first;
                 if (!(h & kSwLast)) return;
@@ -2550,7 +2556,7 @@ __device__ __forceinline__ void sw_both(const SwDev &A, const SwDev &B, const fl
 enum : int {
     kSweepLevels = 0,   // level-synchronous sweeps, correction vector in global memory
     kSweepFlags = 1,    // dataflow sweeps, ready bits in LDS, vector in global memory
-    kSweepLds = 2,      // dataflow sweeps, vector in LDS, values as their own ready marks
+    kSweepLds = 2,      // sweeps a level a step, vector in LDS
 };
 
 // One workgroup runs one matrix: value refresh, GESP value, factorization

@@ -1847,11 +1847,13 @@ bool check_df(const DfHost &D, uint32_t n, uint32_t nnz, const char *name, std::
 // rows in schedule order, each row's entries, and whether the refinement sums
 // the row's products (the rows that table gives a group of lanes).
 struct SwHost {
-    std::vector<uint4> meta;           // [64 chunks]
-    std::vector<uint32_t> hdr, wptr, row, rpos, vsrc;   // vsrc: CSC position of each value (~0: 0)
+    std::vector<uint4> meta;           // [lanes]
+    std::vector<uint4> wave;           // by part and wave (SwDev)
+    std::vector<uint32_t> hdr, first, lanes;   // chunks: header, first lane, lanes
+    std::vector<uint32_t> row, rpos, vsrc;     // vsrc: CSC position of each value (~0: 0)
     std::vector<SwPart> part;
     std::vector<SwProd> prod;          // value index within this sweep
-    uint32_t nwave = 0, stride = 256, nslot_max = 0;
+    uint32_t nwave = 0, per_lane = 4, nslot_max = 0;   // per_lane: values of a lane
 };
 
 // Rows of parts: part_of[r] (UINT32_MAX: not in this sweep), slot_of[r] and
@@ -1879,7 +1881,8 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
 {
     const uint32_t nparts = (uint32_t)Q.count.size();
     S.nwave = waves;
-    S.stride = kSwEntries + (div ? 64 : 0);
+    S.per_lane = div ? 5 : 4;
+    const uint32_t stride = kSwEntries + (div ? 64 : 0);   // of a chunk before its unused lanes go
     // by position: first entry's place in D, the step to the next, level, sum?
     struct Pos {
         uint32_t row, len, base, step, level, pivot;
@@ -1911,13 +1914,13 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
         std::vector<Pos> &R = rows[part];
         const uint32_t nslot = Q.count[part], zero = nslot, one = nslot + 1;
         S.nslot_max = std::max(S.nslot_max, nslot);
-        SwPart P{(uint32_t)S.wptr.size(), (uint32_t)S.row.size(), nslot, 0};
+        SwPart P{(uint32_t)S.wave.size(), (uint32_t)S.row.size(), nslot, 0};
         S.row.resize(P.s0 + nslot);
         S.rpos.resize(P.s0 + nslot);
         auto is_long = [](const Pos &x) { return x.sum && x.len > 64; };
         // the part's chunks in schedule order
         std::vector<uint4> meta;
-        std::vector<uint32_t> hdr, vsrc, wave, rpos(nslot);
+        std::vector<uint32_t> hdr, vsrc, wave, lanes, rpos(nslot);
         struct Prod {
             uint32_t chunk, at, vpos, col;
         };
@@ -1925,7 +1928,8 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
         auto add = [&](uint32_t h) {
             hdr.push_back(h);
             meta.resize(meta.size() + 64, make_uint4(zero | zero << 16, zero | zero << 16, 0u, 0u));
-            vsrc.resize(vsrc.size() + S.stride, UINT32_MAX);
+            vsrc.resize(vsrc.size() + stride, UINT32_MAX);
+            lanes.push_back(0);
         };
         auto put = [&](uint32_t lane, uint32_t e, const Pos &x, uint32_t k) {   // entry k of row x
             const size_t c = hdr.size() - 1, q = x.base + (size_t)k * x.step;
@@ -1933,7 +1937,7 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
             uint32_t slot;
             if (Q.part_of[col] == part) {
                 slot = Q.slot_of[col];
-                vsrc[c * S.stride + 4 * lane + e] = vp;
+                vsrc[c * stride + 4 * lane + e] = vp;
             } else {
                 slot = one;
                 prod.push_back(Prod{(uint32_t)c, 4 * lane + e, vp, col});
@@ -2011,7 +2015,8 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
                         }
                         for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (hdr.size() - 1) + lane].z = slot | bits[lane] | left << kSwCountShift;
                         if (c == 0) rpos[slot] = 64 * (uint32_t)(hdr.size() - 1);
-                        if (c + 1 == nc && div) vsrc[(hdr.size() - 1) * S.stride + kSwEntries] = x.pivot;
+                        if (c + 1 == nc && div) vsrc[(hdr.size() - 1) * stride + kSwEntries] = x.pivot;
+                        lanes.back() = std::min(left, 64u);
                     }
                     continue;
                 }
@@ -2041,8 +2046,9 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
                 rpos[slot] = 64 * (uint32_t)c + used;
                 if (div)   // at the lane that stores the row: the last; a summed row's first too
                     for (uint32_t lane : {used + g - 1, x.sum ? used : used + g - 1})
-                        vsrc[c * S.stride + kSwEntries + lane] = x.pivot;
+                        vsrc[c * stride + kSwEntries + lane] = x.pivot;
                 used += g;
+                lanes.back() = used;
             }
         }
         // stream by stream
@@ -2050,20 +2056,34 @@ void build_sw(const TriHost &H, const DfHost &D, uint32_t n, bool div, const SwP
         std::vector<std::vector<uint32_t>> stream(waves);
         for (size_t c = 0; c < hdr.size(); ++c) stream[wave[c]].push_back((uint32_t)c);
         for (uint32_t w = 0; w < waves; ++w) {
-            S.wptr.push_back((uint32_t)S.hdr.size());
             std::stable_sort(stream[w].begin(), stream[w].end(),
                              [&](uint32_t a, uint32_t b) { return (hdr[a] & kSwStepMask) < (hdr[b] & kSwStepMask); });
+            const size_t k0 = S.hdr.size();
             for (uint32_t c : stream[w]) {
+                const uint32_t u = (std::max(lanes[c], 1u) + 3) & ~3u;
                 at[c] = (uint32_t)S.hdr.size();
                 S.hdr.push_back(hdr[c]);
-                for (uint32_t lane = 0; lane < 64; ++lane) meta[64 * (size_t)c + lane].w = hdr[c];
-                S.meta.insert(S.meta.end(), meta.begin() + 64 * (size_t)c, meta.begin() + 64 * ((size_t)c + 1));
-                S.vsrc.insert(S.vsrc.end(), vsrc.begin() + (size_t)c * S.stride, vsrc.begin() + ((size_t)c + 1) * S.stride);
+                S.first.push_back((uint32_t)S.meta.size());
+                S.lanes.push_back(u);
+                const size_t m = 64 * (size_t)c, v = stride * (size_t)c;
+                meta[m].w = hdr[c];
+                S.meta.insert(S.meta.end(), meta.begin() + m, meta.begin() + m + u);
+                S.vsrc.insert(S.vsrc.end(), vsrc.begin() + v, vsrc.begin() + v + 4 * u);
+                if (div) S.vsrc.insert(S.vsrc.end(), vsrc.begin() + v + kSwEntries, vsrc.begin() + v + kSwEntries + u);
             }
+            // a chunk names the one two after it (the last again)
+            const size_t k1 = S.hdr.size();
+            for (size_t k = k0; k < k1; ++k) {
+                const size_t q = std::min(k + 2, k1 - 1);
+                S.meta[S.first[k] + 1].w = S.first[q];
+                S.meta[S.first[k] + 2].w = S.lanes[q];
+            }
+            const size_t q = std::min(k0 + 1, k1 - 1);
+            S.wave.push_back(k0 == k1 ? make_uint4(0u, 0u, 0u, 0u)
+                                      : make_uint4((uint32_t)(k1 - k0), S.first[k0], S.first[q], S.lanes[k0] | S.lanes[q] << 8));
         }
-        S.wptr.push_back((uint32_t)S.hdr.size());
-        for (uint32_t k = 0; k < nslot; ++k) S.rpos[P.s0 + k] = 64 * at[rpos[k] / 64] + rpos[k] % 64;
-        for (const Prod &q : prod) S.prod.push_back(SwProd{at[q.chunk] * S.stride + q.at, q.vpos, q.col});
+        for (uint32_t k = 0; k < nslot; ++k) S.rpos[P.s0 + k] = S.first[at[rpos[k] / 64]] + rpos[k] % 64;
+        for (const Prod &q : prod) S.prod.push_back(SwProd{S.first[at[q.chunk]] * S.per_lane + q.at, q.vpos, q.col});
         S.part.push_back(P);
     }
 }
@@ -2080,20 +2100,36 @@ bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
         return false;
     };
     const uint32_t nchunk = (uint32_t)S.hdr.size();
-    if (S.meta.size() != 64 * (size_t)nchunk || S.vsrc.size() != (size_t)S.stride * nchunk) return bad("sizes");
+    if (S.first.size() != nchunk || S.lanes.size() != nchunk || S.vsrc.size() != S.per_lane * S.meta.size() ||
+        S.wave.size() != S.part.size() * S.nwave || S.vsrc.size() > 0xffffffffull)
+        return bad("sizes");
+    for (uint32_t c = 0; c < nchunk; ++c)
+        if (S.lanes[c] < 4 || S.lanes[c] > 64 || S.lanes[c] % 4 || S.first[c] % 4 ||
+            (size_t)S.first[c] + S.lanes[c] > S.meta.size())
+            return bad("chunk out of range");
+    uint32_t k0 = 0, k1 = 0;   // a stream's chunks: the streams follow each other
     for (uint32_t v : S.vsrc)
         if (v != UINT32_MAX && v >= nnz) return bad("value position out of range");
     for (const SwProd &q : S.prod)
         if (q.val >= S.vsrc.size() || q.vpos >= nnz) return bad("product out of range");
     for (const SwPart &P : S.part) {
-        if ((size_t)P.wp + S.nwave >= S.wptr.size() || (size_t)P.s0 + P.nslot > S.row.size() || P.nslot > 0xfffdu ||
+        if ((size_t)P.wp + S.nwave > S.wave.size() || (size_t)P.s0 + P.nslot > S.row.size() || P.nslot > 0xfffdu ||
             P.steps > kSwStepMask + 1)
             return bad("part out of range");
         std::vector<uint32_t> set(P.nslot + 2, 0);   // 1 + the row's step
+        const uint32_t part_k0 = k1;
         for (uint32_t pass = 0; pass < 2; ++pass)
             for (uint32_t w = 0; w < S.nwave; ++w) {
-                const uint32_t k0 = S.wptr[P.wp + w], k1 = S.wptr[P.wp + w + 1];
-                if (k0 > k1 || k1 > nchunk) return bad("stream out of range");
+                const uint4 d = S.wave[P.wp + w];
+                k0 = w == 0 ? part_k0 : k1;
+                if (d.x > nchunk - k0) return bad("stream out of range");
+                k1 = k0 + d.x;
+                for (uint32_t c = k0; c < k1; ++c) {
+                    const uint32_t q = std::min(c + 2, k1 - 1), second = std::min(k0 + 1, k1 - 1), l = S.first[c];
+                    if (S.meta[l].w != S.hdr[c] || S.meta[l + 1].w != S.first[q] || S.meta[l + 2].w != S.lanes[q] ||
+                        d.y != S.first[k0] || d.z != S.first[second] || d.w != (S.lanes[k0] | S.lanes[second] << 8))
+                        return bad("a chunk is misplaced");
+                }
                 uint32_t last = 0;
                 bool open[2] = {false, false};   // in a long row
                 uint32_t row_open[2] = {0, 0};
@@ -2102,11 +2138,11 @@ bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
                     if (step < last || step >= P.steps) return bad("step out of range");
                     last = step;
                     auto entry = [&](uint32_t lane, uint32_t e) {
-                        const uint4 &m = S.meta[64 * (size_t)c + lane];
+                        const uint4 &m = S.meta[S.first[c] + lane];
                         const uint32_t v = e < 2 ? m.x : m.y;
                         return (e & 1) ? v >> 16 : v & 0xffffu;
                     };
-                    for (uint32_t lane = 0; lane < 64; ++lane)
+                    for (uint32_t lane = 0; lane < S.lanes[c]; ++lane)
                         for (uint32_t e = 0; e < 4; ++e) {
                             if (entry(lane, e) > P.nslot + 1) return bad("slot out of range");
                             if (pass && set[entry(lane, e)] > step) return bad("an entry's row is not in an earlier step");
@@ -2119,26 +2155,26 @@ bool check_sw(const SwHost &S, uint32_t nnz, const char *name, std::string &err)
                         return once;
                     };
                     if (h & kSwLong) {
-                        const uint32_t z = S.meta[64 * (size_t)c].z, slot = z & 0xffffu;
+                        const uint32_t z = S.meta[S.first[c]].z, slot = z & 0xffffu;
                         const uint32_t n_early = (h >> kSwEarlyShift) & kSwEarlyMask, count = z >> kSwCountShift;
                         const uint32_t tr = (h & kSwTrack) ? 1 : 0;
                         if (open[tr] ? (h & kSwFirst) || slot != row_open[tr] : !(h & kSwFirst)) return bad("a row's chunks are apart");
                         open[tr] = !(h & kSwLast);
                         row_open[tr] = slot;
-                        if (slot >= P.nslot || count > kSwEntries || n_early > count) return bad("long row out of range");
+                        if (slot >= P.nslot || count > kSwEntries || n_early > count || S.lanes[c] < std::min(count, 64u)) return bad("long row out of range");
                         for (uint32_t e = 0; e < n_early && pass; ++e)
                             if (set[entry(e % 64, e / 64)] && set[entry(e % 64, e / 64)] + kSwLead > step) return bad("an entry is taken before it is set");
-                        if ((h & kSwFirst) && S.rpos[P.s0 + slot] != 64 * c) return bad("right-hand side misplaced");
+                        if ((h & kSwFirst) && S.rpos[P.s0 + slot] != S.first[c]) return bad("right-hand side misplaced");
                         if ((h & kSwLast) && !store(slot)) return bad("a row runs twice");
                         continue;
                     }
                     const uint32_t pre = (h >> kSwPreShift) & kSwPreMask, rem = (h >> kSwRemShift) & kSwRemMask;
-                    for (uint32_t lane = 0; lane < 64;) {
-                        const uint32_t z = S.meta[64 * (size_t)c + lane].z, slot = z & 0xffffu, g = 1u << ((z >> 16) & 7u);
-                        if (lane % g || lane + g > 64 || g > 16) return bad("row lanes out of place");
+                    for (uint32_t lane = 0; lane < S.lanes[c];) {
+                        const uint32_t z = S.meta[S.first[c] + lane].z, slot = z & 0xffffu, g = 1u << ((z >> 16) & 7u);
+                        if (lane % g || lane + g > S.lanes[c] || g > 16) return bad("row lanes out of place");
                         if (z & kSwOn) {
                             if (slot >= P.nslot) return bad("row slot out of range");
-                            if (S.rpos[P.s0 + slot] != 64 * c + lane) return bad("right-hand side misplaced");
+                            if (S.rpos[P.s0 + slot] != S.first[c] + lane) return bad("right-hand side misplaced");
                             if (!store(slot)) return bad("a row runs twice");
                             uint32_t n_early = 0;   // lanes done a step ahead
                             while (n_early < std::min(g, pre + 1) && early(lane + n_early, 0) && early(lane + n_early, 1) &&
@@ -2475,7 +2511,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     p->scratch_nval[1] = dtu.idx.size() + dtl.idx.size() + n + 64;
     uint32_t sw_rhs = 0;
     for (const SwHost *h : {&sw[0], &sw[1], &sw[2], &sw[3], &hd[0], &hd[1], &hd[2], &hd[3]})
-        sw_rhs = std::max(sw_rhs, 64 * (uint32_t)h->hdr.size());
+        sw_rhs = std::max(sw_rhs, (uint32_t)h->meta.size());
     p->t32_len = long_lanes ? n : std::max(n, sw_rhs);
     // the value copies (CSC position of each value, ~0 for places without
     // one, which get 0) of A x = b and A' x = b; with the vector beyond LDS,
@@ -2742,7 +2778,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     const size_t o_out = U.reserve(sizeof(float) * most_out);
     const size_t o_wdev = U.reserve(sizeof(WinDev) * std::max<size_t>(wins.size(), 1));
     struct SwOff {
-        size_t meta, wptr, part, row, rpos, prod;
+        size_t meta, wave, part, row, rpos, prod;
     };
     SwOff o_sw[4], o_hd[4];
     for (int q = 0; q < 4; ++q)
@@ -2750,7 +2786,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
             SwHost &h = k ? hd[q] : sw[q];
             if (h.prod.size())   // product values count from the copy's start
                 for (SwProd &e : h.prod) e.val += k ? hd_voff[q] : sw_voff[q];
-            (k ? o_hd : o_sw)[q] = SwOff{U.put(h.meta), U.put(h.wptr), U.put(h.part),
+            (k ? o_hd : o_sw)[q] = SwOff{U.put(h.meta), U.put(h.wave), U.put(h.part),
                                          U.put(h.row), U.put(h.rpos), U.put(h.prod)};
         }
     const size_t o_spl[2] = {U.put(spl_vpos[0]), U.put(spl_vpos[1])};
@@ -2959,14 +2995,13 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     auto swd = [&](const SwHost &h, const SwOff &o, bool div, uint32_t voff) {
         SwDev d{};
         d.meta = reinterpret_cast<const uint4 *>(A + o.meta);
-        d.wptr = u32p(o.wptr);
+        d.wave = reinterpret_cast<const uint4 *>(A + o.wave);
         d.part = reinterpret_cast<const SwPart *>(A + o.part);
         d.row = u32p(o.row);
         d.rpos = u32p(o.rpos);
         d.prod = reinterpret_cast<const SwProd *>(A + o.prod);
         d.nprod = (uint32_t)h.prod.size();
         d.nwave = h.nwave;
-        d.stride = h.stride;
         d.voff = voff;
         d.div = div;
         return d;
