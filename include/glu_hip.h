@@ -191,9 +191,9 @@ glu_status glu_refresh(glu_plan *p, const double *d_ax, float *d_lu, int batch, 
  * x starts from 0.  h_iters/h_eta (host, may be NULL) receive the result
  * (h_iters counts preconditioner solves).  Orders whose FP32 sweep vector
  * fits in LDS run FGMRES(plan krylov) entirely in one workgroup; larger
- * orders run plain refinement with the two sweeps in one workgroup and the
- * FP64 work in grid kernels (or, beyond the sweeps' LDS ready bits, level
- * by level).  Synchronous. */
+ * orders run plain refinement with the sweeps split over workgroups (or in
+ * one) and the FP64 work in grid kernels (or, beyond the sweeps' LDS ready
+ * bits, level by level).  Synchronous. */
 glu_status glu_refine(glu_plan *p, const double *d_ax, const float *d_lu, const double *d_b,
                       double *d_x, double tol, int maxit, int transpose, int *h_iters,
                       double *h_eta, void *stream);
@@ -201,13 +201,14 @@ glu_status glu_refine(glu_plan *p, const double *d_ax, const float *d_lu, const 
 /* glu_refine without any allocation: the same refinement and results (the
  * same kernels), with its scratch (the sweep-layout copy of the factors,
  * the correction and residual vectors, the FGMRES vectors, the iteration
- * count and eta) in a static device array of GLU_NOALLOC_SCRATCH_BYTES per
- * device, which each device that runs it holds until the process ends.
+ * count and eta) in a static device array of twice
+ * GLU_NOALLOC_SCRATCH_BYTES per device, which each device that runs it holds until the process ends.
  * No counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  It calls no hipMalloc/hipFree.  Limits: the
  * order must fit the one-workgroup refinement (n up to ~1.2M) and its
- * scratch must fit the array, else GLU_ERR_ARGUMENT (use glu_refine).
+ * scratch, counted with the ready-bit sweeps' tables, must not exceed
+ * GLU_NOALLOC_SCRATCH_BYTES, else GLU_ERR_ARGUMENT (use glu_refine).
  * Every call on one device shares that device's array: calls that overlap
  * on one device (other streams or threads) race and must not be issued. */
 #define GLU_NOALLOC_SCRATCH_BYTES (64u << 20)
