@@ -328,6 +328,7 @@ struct glu_plan {
     std::vector<PhaseDev> phases;
     std::vector<std::vector<uint32_t>> phase_work;   // chunks of each phase's bins
     int phase_lev = 0;           // steps the phases cover
+    size_t phase_out = 0;        // products of the largest (PhaseDev::out)
     TriHost tri[4];          // lo, up, tup, tlo
     bool tri_dataflow = false;   // fused solve segments run barrier-free
     int solve_df_opt = 0;        // glu_plan_opts.solve_dataflow
@@ -2776,6 +2777,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         most_out = std::max<size_t>(most_out, phases[k].nout);
     }
     const size_t o_out = U.reserve(sizeof(float) * most_out);
+    p->phase_out = most_out;
     const size_t o_wdev = U.reserve(sizeof(WinDev) * std::max<size_t>(wins.size(), 1));
     struct SwOff {
         size_t meta, wave, part, row, rpos, prod;
@@ -3781,6 +3783,7 @@ struct glu_group {
     float *d_t32 = nullptr;
     double *d_r64 = nullptr;
     float *d_lucsr = nullptr;
+    float *d_prod = nullptr;       // the phases' products, a range a member
     double *d_norms = nullptr;
     double *d_kry = nullptr;
     std::vector<size_t> voff;   // per-matrix offset into d_r64
@@ -3800,6 +3803,7 @@ struct glu_group {
         }
         if (ev_in) (void)hipEventDestroy(ev_in);
         if (d_lucsr) (void)hipFree(d_lucsr);
+        if (d_prod) (void)hipFree(d_prod);
         if (d_norms) (void)hipFree(d_norms);
         if (d_kry) (void)hipFree(d_kry);
         if (d_descs) (void)hipFree(d_descs);
@@ -3858,16 +3862,27 @@ extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_gr
     if (ktot) HIP_TRY(hipMalloc(&g->d_kry, sizeof(double) * ktot));
     // The leading launches (for every number of members that may be split
     // off): blocks of values, then bins (those with the most work first) and
-    // assembly blocks of each phase round.
+    // assembly blocks of each phase round.  A member's products go to a range
+    // of its own: a plan may be several members, and is in use outside the
+    // group (a split-off member's factorization, glu_factor on another stream).
     {
         std::vector<int32_t> l0(count, 0);
-        for (int i = 0; i < count; ++i)
+        std::vector<size_t> poff(count, 0);
+        size_t ptot = 0;
+        for (int i = 0; i < count; ++i) {
             l0[i] = plans[i]->phases.size() <= kGroupRounds ? plans[i]->phase_lev : 0;
+            poff[i] = ptot;
+            if (l0[i]) ptot += (plans[i]->phase_out + 63) & ~(size_t)63;
+        }
+        if (ptot) HIP_TRY(hipMalloc(&g->d_prod, sizeof(float) * ptot));
         std::vector<PhaseDev> ph[kGroupRounds];
         for (uint32_t r = 0; r < kGroupRounds; ++r) {
             ph[r].resize(count);
             for (int i = 0; i < count; ++i)
-                if (l0[i] && r < plans[i]->phases.size()) ph[r][i] = plans[i]->phases[r];
+                if (l0[i] && r < plans[i]->phases.size()) {
+                    ph[r][i] = plans[i]->phases[r];
+                    ph[r][i].out = g->d_prod + poff[i];
+                }
         }
         std::vector<uint2> items;
         size_t first[kMaxGroupSplit + 1][1 + 2 * kGroupRounds];
@@ -3958,11 +3973,18 @@ extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, c
     // CUs the fused launch leaves idle, then the one-workgroup refinement,
     // the same kernel the fused launch runs (same workgroup size and restart
     // length), so the results are the same bits.  Only members whose
-    // refinement keeps its vector in LDS qualify.
+    // refinement keeps its vector in LDS qualify, and one member of a plan
+    // (that path works in the plan's scratch; the fused launch in the group's).
     int want = g->split_req >= 0 ? g->split_req : (count >= 4 ? 1 : 0);
     want = std::min(want, count - 1);
     int nsplit = 0;
-    while (nsplit < want && sweep_mode(g->plans[g->order[nsplit]]->n, cap) == 2) ++nsplit;
+    const auto apart = [&](const glu_plan *p) {   // not a split-off member's plan
+        for (int j = 0; j < nsplit; ++j)
+            if (g->plans[g->order[j]] == p) return false;
+        return true;
+    };
+    while (nsplit < want && sweep_mode(g->plans[g->order[nsplit]]->n, cap) == 2 && apart(g->plans[g->order[nsplit]]))
+        ++nsplit;
     if (nsplit > 0) {
         if (!g->ev_in) HIP_TRY(hipEventCreateWithFlags(&g->ev_in, hipEventDisableTiming));
         HIP_TRY(hipEventRecord(g->ev_in, st));

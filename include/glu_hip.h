@@ -263,13 +263,17 @@ glu_status glu_abft_check(glu_plan *p, int batch, const float *d_lu, const float
  * ---------------------------------------------------------------------- */
 typedef struct glu_group glu_group;
 
+/* A plan may be named more than once (a block instanced several times, other
+ * values): the fused launch reads its tables and works in scratch of the
+ * group's own, a range a member. */
 glu_status glu_group_create(glu_plan *const *plans, int count, glu_group **out);
 void glu_group_destroy(glu_group *g);
 /* Members run through the single-matrix path alongside the fused launch:
  * the `count` heaviest (0..2; -1, the default: one in a group of four or
  * more), on streams of their own, while the fused launch takes the rest.
  * Results are the same bits either way.  Only members whose refinement
- * vector fits in LDS are moved.  (No counterpart in the reference: part of
+ * vector fits in LDS are moved, and one member of a plan at most (they work
+ * in the plan's scratch).  (No counterpart in the reference: part of
  * the uneven batch this library adds.) */
 glu_status glu_group_set_split(glu_group *g, int count);
 /* Host arrays of `count` device pointers each, in plan order. */
