@@ -3841,8 +3841,8 @@ extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_gr
         vtot += p->n;
         g->toff.push_back(ttot);
         ttot += p->t32_len;
-        g->foff.push_back(ftot);
-        ftot += p->df_nval;
+        g->foff.push_back(ftot);   // (whole lines: the sweeps load 16 bytes a lane)
+        ftot += ((size_t)p->df_nval + 63) & ~(size_t)63;
         g->threads = std::max(g->threads, p->fused_threads);
         // heaviest first: levels dominate the latency, updates the work
         work[i] = {-(int64_t)(p->num_lev + p->tri[0].lvl_ptr.size() + p->tri[1].lvl_ptr.size()) * 64 - p->updates,
