@@ -1260,14 +1260,14 @@ struct Phase {
 
 constexpr uint32_t kPhaseWaves = 8;
 constexpr uint32_t kPhaseBins = 512;       // two workgroups a CU
-constexpr uint32_t kPhaseSlots = 19000;    // entries of a bin (76 KB: two a CU)
+constexpr uint32_t kPhaseSlots = 19000;    // entries of a bin, at most (76 KB: two a CU)
 constexpr int kMinPhase = 4;               // steps
 
 // The steps from l0 on that make a phase, at most to `limit`: as many as keep
-// every component's entries within a bin.  Components of the columns of steps
-// [l0, e): joined by entries of L or U between them.  Returns e (l0: none)
-// and each column's component (UINT32_MAX: not in the phase).
-int phase_end(const glu_pattern &P, int l0, int limit, std::vector<uint32_t> &comp)
+// every component's entries within a bin (of bin_slots).  Components of the
+// columns of steps [l0, e): joined by entries of L or U between them.  Returns
+// e (l0: none) and each column's component (UINT32_MAX: not in the phase).
+int phase_end(const glu_pattern &P, int l0, int limit, uint32_t bin_slots, std::vector<uint32_t> &comp)
 {
     const uint32_t n = P.n;
     std::vector<uint32_t> parent(n), ent(n);
@@ -1302,7 +1302,7 @@ int phase_end(const glu_pattern &P, int l0, int limit, std::vector<uint32_t> &co
     int e = l0;
     for (bool fits = true; e < limit && fits; e += fits)
         for (int t = P.level_ptr[e]; t < P.level_ptr[e + 1]; ++t)
-            fits = add((uint32_t)P.level_idx[t]) <= kPhaseSlots && fits;
+            fits = add((uint32_t)P.level_idx[t]) <= bin_slots && fits;
     reset();   // (without the step that did not fit)
     for (int l = l0; l < e; ++l)
         for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) (void)add((uint32_t)P.level_idx[t]);
@@ -1316,7 +1316,7 @@ int phase_end(const glu_pattern &P, int l0, int limit, std::vector<uint32_t> &co
 // columns' components comp.  False: an update would cross components (the
 // pattern's levels do not order it; the steps stay as they are).
 bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &level_of,
-                 const std::vector<uint32_t> &comp, Phase &ph)
+                 const std::vector<uint32_t> &comp, uint32_t bin_slots, Phase &ph)
 {
     const uint32_t n = P.n;
     const unsigned threads = table_threads();
@@ -1346,7 +1346,7 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
     for (uint32_t c : order) {
         uint32_t to = UINT32_MAX;
         for (uint32_t b = 0; b < nbin; ++b)
-            if (fill[b] + size[c] <= kPhaseSlots && (to == UINT32_MAX || load[b] < load[to])) to = b;
+            if (fill[b] + size[c] <= bin_slots && (to == UINT32_MAX || load[b] < load[to])) to = b;
         if (to == UINT32_MAX) {   // no room: one more bin
             to = (uint32_t)load.size();
             load.push_back(0);
@@ -1555,20 +1555,21 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
     return true;
 }
 
-// The phases ahead of step `limit` (the first LDS window's).
-void choose_phases(const glu_pattern &P, const Tables &T, int limit, std::vector<Phase> &phases)
+// The phases ahead of step `limit` (the first LDS window's), their bins of
+// bin_slots entries at most.
+void choose_phases(const glu_pattern &P, const Tables &T, int limit, uint32_t bin_slots, std::vector<Phase> &phases)
 {
     std::vector<int> level_of(P.n, 0);
     for (int l = 0; l < P.num_lev; ++l)
         for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) level_of[P.level_idx[t]] = l;
     std::vector<uint32_t> comp;
     for (int l = 0; l < limit;) {
-        const int e = phase_end(P, l, limit, comp);
+        const int e = phase_end(P, l, limit, bin_slots, comp);
         if (e - l < kMinPhase) break;
         Phase ph;
         ph.l0 = l;
         ph.l1 = e;
-        if (!build_phase(P, T, level_of, comp, ph)) break;
+        if (!build_phase(P, T, level_of, comp, bin_slots, ph)) break;
         phases.push_back(std::move(ph));
         l = e;
     }
@@ -2208,10 +2209,12 @@ struct SwSplit {
 
 constexpr uint32_t kHeadWaves = 8;
 constexpr uint32_t kHeadParts = 512;    // two workgroups a CU
-constexpr uint32_t kHeadSlots = 16384;  // 64 KB of LDS
+constexpr uint32_t kHeadSlots = 16384;  // at most (64 KB of LDS)
 
+// cap_slots: rows a workgroup's LDS holds.
 bool choose_split(const glu_pattern &P, uint32_t cap_slots, uint32_t tail_waves, SwSplit &S)
 {
+    const uint32_t head_slots = std::min(cap_slots, kHeadSlots);
     const uint32_t n = P.n;
     std::vector<uint32_t> ht(n, 0), wgt(n);
     uint32_t top = 0;
@@ -2267,7 +2270,7 @@ bool choose_split(const glu_pattern &P, uint32_t cap_slots, uint32_t tail_waves,
         }
         if (h < next_try) continue;
         next_try = h + std::max(1u, h / 4);
-        if (max_n > kHeadSlots) break;
+        if (max_n > head_slots) break;
         const uint32_t tail = n - rows_at[h];
         if (tail > cap_slots) continue;
         const double head_chunks = std::max((double)max_w, (double)head_w / kHeadParts) / 64.0;
@@ -2313,7 +2316,7 @@ bool choose_split(const glu_pattern &P, uint32_t cap_slots, uint32_t tail_waves,
     for (uint32_t c : order) {
         uint32_t to = UINT32_MAX;
         for (uint32_t k = 0; k < nparts; ++k)
-            if (rows[k] + size[c] <= kHeadSlots && (to == UINT32_MAX || load[k] < load[to])) to = k;
+            if (rows[k] + size[c] <= head_slots && (to == UINT32_MAX || load[k] < load[to])) to = k;
         if (to == UINT32_MAX) return false;
         load[to] += weight[c];
         rows[to] += size[c];
@@ -2401,6 +2404,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     // (slots are 16-bit numbers)
     uint32_t budget = std::min<uint32_t>((uint32_t)(p->lds_cap / sizeof(float)), 0xffffu);
     budget -= std::min(budget, kWinExtra);
+    const uint32_t bin_slots = std::min(budget, kPhaseSlots);
     if (p->win_values) budget = std::min(budget, p->win_values);
     // Built side by side on host threads: the windows, the four triangular
     // sweeps (L, U; U', L' for A' x = b: rows of U' are columns of U with the
@@ -2480,7 +2484,7 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     std::vector<Phase> phases;
     const auto windows_and_phases = [&]() {
         choose_windows(T, P.num_lev, P.nnz, budget, (uint32_t)p->fuse_units, p->max_windows, wg_waves, wins);
-        choose_phases(P, T, wins.empty() ? 0 : std::min(wins[0].l0, P.num_lev), phases);
+        choose_phases(P, T, wins.empty() ? 0 : std::min(wins[0].l0, P.num_lev), bin_slots, phases);
     };
     std::future<void> factor_steps;   // (waits in its destructor, before what it works on goes)
     try {
@@ -2492,7 +2496,8 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         if (item < 4)
             sweep_tables((int)item);
         else
-            split = choose_split(P, (uint32_t)std::min<size_t>(p->lds_cap / sizeof(float), 0xffffu) - 2, wg_waves, spl);
+            split = choose_split(P, (uint32_t)std::min<size_t>(std::max<size_t>(p->lds_cap / sizeof(float), 2), 0xffffu) - 2,
+                                 wg_waves, spl);
     });
     for (int q = 0; q < 4; ++q)
         if (!good[q]) return fail(GLU_ERR_INVALID, errs[q]);
