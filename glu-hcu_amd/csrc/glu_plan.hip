@@ -608,8 +608,8 @@ struct LevelItems {
 // level l, every (i in L_k, j in U_k) update targets the CSC position of
 // (i,j) in column j; the fill closure of the pattern guarantees it exists
 // (checked).  Targets that two or more columns of the level update become
-// merge entries whose sources keep the level's column order (level_idx lists
-// a level's columns in increasing order); all other updates are items.
+// merge entries whose sources keep the order in which level_idx lists the
+// level's columns; all other updates are items.
 // The update map is built per target column and the items per level, each
 // on host threads; levels are then concatenated in order, so the tables do
 // not depend on the thread count.
@@ -1379,18 +1379,21 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
             slot[pos[i]] = (uint16_t)i;
         }
     });
-    // products per later entry: column j's pivots of the phase in order of
-    // step and number; cnt by position, then each product's place
+    // products per later entry: column j's pivots of the phase in schedule
+    // order (step by step, a step's columns as level_idx lists them, the order
+    // of every other path); cnt by position, then each product's place
     std::vector<uint32_t> cnt(P.nnz, 0), base(P.nnz, 0);
     std::vector<uint32_t> csc2csr(P.nnz);
     for (uint32_t q = 0; q < P.nnz; ++q) csc2csr[T.upos[q]] = q;
     std::atomic<bool> crossed(false);
+    std::vector<int> place_of(n);
+    for (int t = 0; t < (int)n; ++t) place_of[P.level_idx[t]] = t;
     auto each_outside = [&](uint32_t j, std::vector<std::pair<int, uint32_t>> &ks, auto f) {
         ks.clear();
         for (uint32_t p = P.sym_c_ptr[j]; p < P.l_col_ptr[j]; ++p)
-            if (comp[P.sym_r_idx[p]] != UINT32_MAX) ks.push_back({level_of[P.sym_r_idx[p]], p});
-        std::sort(ks.begin(), ks.end());   // (positions of a column ascend with the pivots)
-        for (const auto &[lev, p] : ks) {
+            if (comp[P.sym_r_idx[p]] != UINT32_MAX) ks.push_back({place_of[P.sym_r_idx[p]], p});
+        std::sort(ks.begin(), ks.end());
+        for (const auto &[at_place, p] : ks) {
             const uint32_t k = P.sym_r_idx[p], L = P.sym_c_ptr[k + 1] - P.l_col_ptr[k] - 1;
             const uint64_t at = T.moff[k] + (uint64_t)(csc2csr[p] - P.csr_diag_ptr[k] - 1) * L;
             for (uint32_t ii = 0; ii < L; ++ii) {
@@ -1503,7 +1506,7 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
             std::vector<uint32_t> cur;   // next source of each merge entry
             for (uint16_t t : order)
                 if (M.count[t] >= 2) cur.push_back(M.first[t]);
-            // the columns of a step ascend, so a merge entry's sources come in order
+            // (the bin lists its columns in schedule order, so a merge entry's sources come in it)
             for (size_t c = i; c < e; ++c) {
                 const uint32_t k = cols[b][c], dpos = P.l_col_ptr[k], L = P.sym_c_ptr[k + 1] - dpos - 1;
                 if (L == 0) continue;

@@ -79,3 +79,11 @@ def test_streams(checker, pattern, name, values):
 def test_bins_fit_small_limits(checker, pattern, name, bin_values):
     """Bins of a device with less LDS: none holds more values than it may."""
     assert _check(checker, pattern(name), 60, bin_values)["largest"] <= bin_values
+
+
+@pytest.mark.parametrize("name", list(CASES))
+@pytest.mark.parametrize("values", [60, 700])
+def test_levels_listed_downward(checker, pattern, name, values):
+    """A caller's pattern may list a level's columns in any order: the phases
+    subtract in that order too, as the other steps do."""
+    _check(checker, pattern(name), values, 19000, reverse=1)
