@@ -338,6 +338,7 @@ struct glu_plan {
     float *d_tlucsr = nullptr;   // glu_refine's A' x = b value copy
     uint32_t t32_len = 0;        // floats of a matrix's sweep scratch (SolveDev::t32_len)
     uint64_t scratch_nval[2] = {0, 0};   // value copies the scratch limit of glu_refine_noalloc counts (A, A')
+    uint32_t rhs_len[2] = {0, 0};        // lanes of the longer of the two sweeps' streams (A, A')
     // one matrix's sweeps outside the batch kernels (A, A'): value copy,
     // right-hand sides, vector by row; allocated on first use, never moved
     struct Single {
@@ -345,7 +346,6 @@ struct glu_plan {
     } single[2];
     bool has_split = false;      // vector beyond LDS: split sweeps (split[0]: A, [1]: A')
     SplitDev split[2] = {};
-    uint32_t split_rhs = 0;      // floats of their right-hand sides
     // LDS windows allowed (from the last level); windows hold narrow steps
     // only, so small orders get one whatever the cap, and n=500k MNA gains
     // up to ~16 (refactor 14.3 -> 12.4 ms; no change beyond)
@@ -2518,10 +2518,9 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     }
     p->scratch_nval[0] = dlo.idx.size() + dup.idx.size() + n + 64;
     p->scratch_nval[1] = dtu.idx.size() + dtl.idx.size() + n + 64;
-    uint32_t sw_rhs = 0;
-    for (const SwHost *h : {&sw[0], &sw[1], &sw[2], &sw[3], &hd[0], &hd[1], &hd[2], &hd[3]})
-        sw_rhs = std::max(sw_rhs, (uint32_t)h->meta.size());
-    p->t32_len = long_lanes ? n : std::max(n, sw_rhs);
+    for (int q = 0; q < 4; ++q)
+        for (const SwHost *h : {&sw[q], &hd[q]}) p->rhs_len[q / 2] = std::max(p->rhs_len[q / 2], (uint32_t)h->meta.size());
+    p->t32_len = long_lanes ? n : std::max({n, p->rhs_len[0], p->rhs_len[1]});
     // the value copies (CSC position of each value, ~0 for places without
     // one, which get 0) of A x = b and A' x = b; with the vector beyond LDS,
     // those of the dataflow tables (slots, then the pivots), and the split
@@ -3020,7 +3019,6 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         for (int q = 0; q < 4; ++q) S.sw[q] = swd(sw[q], o_sw[q], divs[q], sw_voff[q]);
     S.t32_len = p->t32_len;
     p->has_split = split;
-    p->split_rhs = sw_rhs;
     if (split)
         for (int t = 0; t < 2; ++t) {
             SplitDev &d = p->split[t];
@@ -3217,7 +3215,7 @@ glu_status ensure_single(glu_plan *p, int transpose)
     glu_plan::Single &q = p->single[transpose];
     if (q.buf) return GLU_OK;
     const size_t nval = p->has_split ? p->split[transpose].nval : transpose ? p->tdf_nval : p->df_nval;
-    const size_t rhs = p->has_split ? p->split_rhs : p->t32_len;
+    const size_t rhs = p->has_split ? p->rhs_len[transpose] : p->t32_len;
     const size_t a = (nval + 63) & ~(size_t)63, b = (rhs + 63) & ~(size_t)63;
     HIP_TRY(hipMalloc(&q.buf, sizeof(float) * (a + b + p->n)));
     q.lucsr = q.buf;
@@ -3546,7 +3544,7 @@ extern "C" glu_status glu_refine(glu_plan *p, const double *d_ax, const float *d
 
 namespace {
 
-constexpr size_t kScratchBytes = 2 * (size_t)GLU_NOALLOC_SCRATCH_BYTES;   // see glu_refine_noalloc's layout
+constexpr size_t kScratchBytes = GLU_NOALLOC_SCRATCH_BYTES / 2 * (size_t)5;   // see noalloc_layout
 constexpr int kScratchDevices = 64;
 
 // One copy per device, held until the process ends.  Host code never uses
@@ -3578,6 +3576,55 @@ glu_status scratch_base(unsigned char **out)
 
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
+// The scratch of glu_refine_noalloc in sweep mode `mode` (t: A' x = b): sweep
+// value copy, right-hand sides and vector, residual, norms (one-workgroup
+// path: FP64 |b| slots, FGMRES vectors, iteration count + eta; grid path: the
+// four norm words).  limit: what GLU_NOALLOC_SCRATCH_BYTES counts, the same
+// with the dataflow tables' slots in the copy and no right-hand sides.
+//
+// Every order within the limit fits kScratchBytes.  One workgroup (mode 2): a
+// sweep's streams have at most (slots + 64 n) / 3 lanes (the most by slots: a
+// row of 65 entries, 128 slots and 64 lanes, and one of 320, 320 and 128), so
+// with 4 and 5 values a lane and the right-hand sides the layout takes at most
+// 2 limit + 207.4 n floats, and n <= 39,718 (the vector and the ready bits in
+// 160 KB): 160 MiB.  Split sweeps (mode 1) take the split's copy when it
+// fits, else the one workgroup's, which is what the limit counts (the same
+// bits).
+struct NoallocLayout {
+    bool split = false;
+    uint32_t nval = 0;
+    size_t val = 0, rhs = 0, t32 = 0, r64 = 0, norms = 0, kry = 0, out = 0, bytes = 0, limit = 0;
+};
+
+NoallocLayout noalloc_layout(const glu_plan &p, int mode, int t)
+{
+    const size_t n = p.n, kry = mode == 2 && p.krylov ? sizeof(double) * (3 * (size_t)p.krylov + 1) * n : 0;
+    NoallocLayout L;
+    L.split = mode == 1 && p.has_split;
+    for (;;) {
+        size_t off = 0;
+        auto take = [&](size_t bytes) {
+            const size_t o = off;
+            off = align256(off + bytes);
+            return o;
+        };
+        L.nval = L.split ? p.split[t].nval : t ? p.tdf_nval : p.df_nval;
+        L.val = take(sizeof(float) * (size_t)L.nval);
+        L.rhs = take(L.split ? sizeof(float) * (size_t)p.rhs_len[t] : 0);
+        L.t32 = take(sizeof(float) * (mode == 2 ? std::max<size_t>(p.rhs_len[t], n) : n));
+        L.r64 = take(sizeof(double) * n);
+        L.norms = take(4 * sizeof(unsigned long long));
+        L.kry = take(kry);
+        L.out = take(16);
+        L.bytes = off;
+        if (!L.split || L.bytes <= kScratchBytes) break;
+        L.split = false;
+    }
+    L.limit = align256(sizeof(float) * (size_t)p.scratch_nval[t]) + align256(sizeof(float) * n) +
+              align256(sizeof(double) * n) + align256(4 * sizeof(unsigned long long)) + align256(kry) + align256(16);
+    return L;
+}
+
 }  // namespace
 
 extern "C" glu_status glu_refine_noalloc(glu_plan *p, const double *d_ax, const float *d_lu, const double *d_b,
@@ -3592,52 +3639,28 @@ extern "C" glu_status glu_refine_noalloc(glu_plan *p, const double *d_ax, const 
         return fail(GLU_ERR_ARGUMENT, "order " + std::to_string(n) +
                                           " is beyond the dataflow sweeps (their ready bits exceed LDS): "
                                           "use glu_refine");
-    // The limit counts the copy with the dataflow tables' slots, the vector,
-    // the residual, the norms, the FGMRES vectors and the results; the
-    // layout below may take up to twice that (the array holds it).
     const int t = transpose ? 1 : 0;
-    const size_t kry = mode == 2 && p->krylov ? sizeof(double) * (3 * (size_t)p->krylov + 1) * n : 0;
-    const size_t need = align256(sizeof(float) * (size_t)p->scratch_nval[t]) + align256(sizeof(float) * (size_t)n) +
-                        align256(sizeof(double) * (size_t)n) + align256(4 * sizeof(unsigned long long)) +
-                        align256(kry) + align256(16);
-    // scratch layout: sweep value copy, right-hand sides and vector,
-    // residual, norms (one-workgroup path: FP64 |b| slots, FGMRES vectors,
-    // iteration count + eta; grid path: the four norm words)
-    const bool split = mode == 1 && p->has_split;
-    const uint32_t nval = split ? p->split[t].nval : transpose ? p->tdf_nval : p->df_nval;
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        const size_t o = off;
-        off = align256(off + bytes);
-        return o;
-    };
-    const size_t o_val = take(sizeof(float) * (size_t)nval);
-    const size_t o_rhs = take(split ? sizeof(float) * (size_t)p->split_rhs : 0);
-    const size_t o_t32 = take(sizeof(float) * (size_t)std::max(p->t32_len, n));
-    const size_t o_r64 = take(sizeof(double) * (size_t)n);
-    const size_t o_norms = take(4 * sizeof(unsigned long long));
-    const size_t o_kry = take(kry);
-    const size_t o_out = take(16);
-    if (need > GLU_NOALLOC_SCRATCH_BYTES || off > kScratchBytes)
-        return fail(GLU_ERR_ARGUMENT, "refinement needs " + std::to_string(need) + " bytes of scratch; the static " +
+    const NoallocLayout L = noalloc_layout(*p, mode, t);
+    if (L.limit > GLU_NOALLOC_SCRATCH_BYTES || L.bytes > kScratchBytes)
+        return fail(GLU_ERR_ARGUMENT, "refinement needs " + std::to_string(L.limit) + " bytes of scratch; the static " +
                                           "scratch holds " + std::to_string(GLU_NOALLOC_SCRATCH_BYTES) + ": use glu_refine");
     unsigned char *base = nullptr;
     glu_status s = scratch_base(&base);
     if (s != GLU_OK) return s;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    float *lucsr = reinterpret_cast<float *>(base + o_val);
-    float *t32 = reinterpret_cast<float *>(base + o_t32);
-    double *r64 = reinterpret_cast<double *>(base + o_r64);
+    float *lucsr = reinterpret_cast<float *>(base + L.val);
+    float *t32 = reinterpret_cast<float *>(base + L.t32);
+    double *r64 = reinterpret_cast<double *>(base + L.r64);
     if (mode == 2)   // as glu_refine: everything in one workgroup
         return refine_one_wg(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, lucsr, t32, r64,
-                             reinterpret_cast<double *>(base + o_norms),
-                             p->krylov ? reinterpret_cast<double *>(base + o_kry) : nullptr,
-                             reinterpret_cast<char *>(base + o_out), h_iters, h_eta, st);
+                             reinterpret_cast<double *>(base + L.norms),
+                             p->krylov ? reinterpret_cast<double *>(base + L.kry) : nullptr,
+                             reinterpret_cast<char *>(base + L.out), h_iters, h_eta, st);
     // as glu_refine: the split sweeps, or both sweeps in one workgroup
-    launch::copy_df(split ? p->split[t].src : transpose ? p->S.tdf_src : p->S.df_src, nval, d_lu, lucsr, st);
+    launch::copy_df(L.split ? p->split[t].src : transpose ? p->S.tdf_src : p->S.df_src, L.nval, d_lu, lucsr, st);
     return refine_host_loop(p, d_ax, d_lu, d_b, d_x, tol, maxit, transpose, lucsr,
-                            split ? reinterpret_cast<float *>(base + o_rhs) : nullptr, t32, r64,
-                            reinterpret_cast<unsigned long long *>(base + o_norms), h_iters, h_eta, st);
+                            L.split ? reinterpret_cast<float *>(base + L.rhs) : nullptr, t32, r64,
+                            reinterpret_cast<unsigned long long *>(base + L.norms), h_iters, h_eta, st);
 }
 
 extern "C" glu_status glu_adjoint_values(glu_plan *p, const double *d_lam, const double *d_x, double *d_grad_ax,

@@ -201,8 +201,9 @@ glu_status glu_refine(glu_plan *p, const double *d_ax, const float *d_lu, const 
 /* glu_refine without any allocation: the same refinement and results (the
  * same kernels), with its scratch (the sweep-layout copy of the factors,
  * the correction and residual vectors, the FGMRES vectors, the iteration
- * count and eta) in a static device array of twice
- * GLU_NOALLOC_SCRATCH_BYTES per device, which each device that runs it holds until the process ends.
+ * count and eta) in a static device array of two and a half times
+ * GLU_NOALLOC_SCRATCH_BYTES per device, which each device that runs it
+ * holds until the process ends.
  * No counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  It calls no hipMalloc/hipFree.  Limits: the

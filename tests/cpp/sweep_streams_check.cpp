@@ -180,6 +180,9 @@ int main(int argc, char **argv)
         }
         lanes += tl[q].meta.size() + hd[q].meta.size();
         slots += D.idx.size();
+        // (glu_refine_noalloc's scratch rests on this)
+        if (whole && 3 * (uint64_t)tl[q].meta.size() > D.idx.size() + 64 * (uint64_t)n)
+            die("lanes exceed a third of the slots and 64 a row", tl[q].meta.size(), D.idx.size());
         // planted mistakes: a slot or a value position past the end, a step
         // too early, a chunk left out, a right-hand side elsewhere
         const SwHost &S = tl[q];
