@@ -3209,6 +3209,15 @@ glu_status ensure_batch(glu_plan *p, int batch)
     return GLU_OK;
 }
 
+// Is the caller capturing a graph on st?
+bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();   // (the null stream beside a capture: the launches report it)
+    return false;
+}
+
 // The buffers of one matrix's sweeps (p->single[transpose]).
 glu_status ensure_single(glu_plan *p, int transpose)
 {
@@ -3342,8 +3351,11 @@ extern "C" glu_status glu_solve(glu_plan *p, const float *d_lu, const float *d_b
     // 1: the split sweeps, or (A x = b) one workgroup with the ready bits in
     // LDS; 0: level by level.  All give the reference's arithmetic.
     int mode = p->tri_dataflow ? sweep_mode(p->n, launch::enable_lds()) : 0;
+    if (mode == 1 && !p->has_split && transpose) mode = 0;
+    // the other modes' buffers come with their first call; in a capture, which
+    // cannot allocate, that call runs level by level
+    if (mode != 0 && !p->single[transpose].buf && capturing(st)) mode = 0;
     const bool split = mode == 1 && p->has_split;
-    if (mode == 1 && !split && transpose) mode = 0;
     if (mode != 0) {
         glu_status s = ensure_single(p, transpose);   // (before any graph capture)
         if (s != GLU_OK) return s;
@@ -3381,7 +3393,7 @@ extern "C" glu_status glu_solve(glu_plan *p, const float *d_lu, const float *d_b
         return GLU_OK;
     };
     if (!p->use_graph) return issue(st);
-    return replay(p, p->g_solve[transpose], d_lu, d_b, d_x, 0, st, issue);
+    return replay(p, p->g_solve[transpose], d_lu, d_b, d_x, mode, st, issue);
 }
 
 extern "C" glu_status glu_refresh(glu_plan *p, const double *d_ax, float *d_lu, int batch, void *stream)
