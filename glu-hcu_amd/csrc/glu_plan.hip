@@ -18,6 +18,7 @@
 #include <exception>
 #include <memory>
 #include <mutex>
+#include <stdexcept>
 #include <string>
 #include <atomic>
 #include <system_error>
@@ -116,6 +117,21 @@ static glu_status fail(glu_status s, const std::string &msg)
     } while (0)
 
 extern "C" const char *glu_last_error(void) { return g_err.c_str(); }
+
+// f() with C++ exceptions as status codes (nothing may leave a C entry).
+template <typename F>
+static glu_status guarded(F f)
+{
+    try {
+        return f();
+    } catch (const std::bad_alloc &) {
+        return fail(GLU_ERR_MEMORY, "out of host memory");
+    } catch (const std::length_error &) {
+        return fail(GLU_ERR_MEMORY, "a table is too large for host memory");
+    } catch (const std::exception &e) {
+        return fail(GLU_ERR_GENERAL, e.what());
+    }
+}
 
 // ---------------------------------------------------------------------------
 // analysis object
@@ -3238,11 +3254,7 @@ glu_status ensure_single(glu_plan *p, int transpose)
 extern "C" glu_status glu_plan_create(const glu_pattern *pat, const glu_plan_opts *opts, glu_plan **out)
 {
     if (!pat || !out) return fail(GLU_ERR_ARGUMENT, "null argument");
-    try {
-        return build_plan(*pat, nullptr, opts, out);
-    } catch (const std::bad_alloc &) {
-        return fail(GLU_ERR_MEMORY, "out of host memory");
-    }
+    return guarded([&] { return build_plan(*pat, nullptr, opts, out); });
 }
 
 extern "C" glu_status glu_plan_create_from_analysis(const glu_analysis *a, const glu_plan_opts *opts,
@@ -3250,11 +3262,7 @@ extern "C" glu_status glu_plan_create_from_analysis(const glu_analysis *a, const
 {
     if (!a || !out) return fail(GLU_ERR_ARGUMENT, "null argument");
     glu_pattern P = pattern_of(a->sym);
-    try {
-        return build_plan(P, a, opts, out);
-    } catch (const std::bad_alloc &) {
-        return fail(GLU_ERR_MEMORY, "out of host memory");
-    }
+    return guarded([&] { return build_plan(P, a, opts, out); });
 }
 
 extern "C" void glu_plan_destroy(glu_plan *p) { delete p; }
@@ -3858,7 +3866,9 @@ struct glu_group {
     }
 };
 
-extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_group **out)
+namespace {
+
+glu_status group_create(glu_plan *const *plans, int count, glu_group **out)
 {
     if (!plans || count <= 0 || !out) return fail(GLU_ERR_ARGUMENT, "bad argument");
     *out = nullptr;
@@ -3983,6 +3993,13 @@ extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_gr
     return GLU_OK;
 }
 
+}  // namespace
+
+extern "C" glu_status glu_group_create(glu_plan *const *plans, int count, glu_group **out)
+{
+    return guarded([&] { return group_create(plans, count, out); });
+}
+
 extern "C" void glu_group_destroy(glu_group *g) { delete g; }
 
 extern "C" glu_status glu_group_set_split(glu_group *g, int count)
@@ -3992,9 +4009,11 @@ extern "C" glu_status glu_group_set_split(glu_group *g, int count)
     return GLU_OK;
 }
 
-extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, const double *const *d_b,
-                                      double *const *d_x, float *const *d_lu, double tol, int maxit,
-                                      int32_t *d_iters, double *d_eta, unsigned flags, void *stream)
+namespace {
+
+glu_status group_solve(glu_group *g, const double *const *d_ax, const double *const *d_b, double *const *d_x,
+                       float *const *d_lu, double tol, int maxit, int32_t *d_iters, double *d_eta, unsigned flags,
+                       void *stream)
 {
     if (!g || !d_ax || !d_b || !d_x || !d_lu || !d_iters || !d_eta || maxit <= 0)
         return fail(GLU_ERR_ARGUMENT, "bad argument");
@@ -4076,4 +4095,13 @@ extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, c
     // ios is read by the kernel from device memory; the host copy may go.
     HIP_TRY(hipStreamSynchronize(st));
     return GLU_OK;
+}
+
+}  // namespace
+
+extern "C" glu_status glu_group_solve(glu_group *g, const double *const *d_ax, const double *const *d_b,
+                                      double *const *d_x, float *const *d_lu, double tol, int maxit,
+                                      int32_t *d_iters, double *d_eta, unsigned flags, void *stream)
+{
+    return guarded([&] { return group_solve(g, d_ax, d_b, d_x, d_lu, tol, maxit, d_iters, d_eta, flags, stream); });
 }
