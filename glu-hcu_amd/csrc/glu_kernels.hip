@@ -3324,7 +3324,9 @@ __global__ void __launch_bounds__(256) k_sw_prod(const SwProd *__restrict__ prod
 // assembly of all of them side by side (items {member, block | bin | first
 // wave}).
 constexpr uint32_t kGroupValues = 1024;
-constexpr uint32_t kGroupSpread = 64;   // workgroups a member of the divisions and the copy
+// workgroups a member of the divisions and the copy (in one dimension, for any
+// number of members; at most kGroupGrid in all: 2^32 threads)
+constexpr uint32_t kGroupSpread = 64, kGroupGrid = (1u << 24) - 1;
 
 __global__ void __launch_bounds__(256) k_group_values(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
                                                       const uint2 *__restrict__ items)
@@ -3399,25 +3401,25 @@ __global__ void __launch_bounds__(1024) k_batch_group_factor(const MatDesc *__re
 }
 
 __global__ void __launch_bounds__(256) k_group_divide(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
-                                                      const uint32_t *__restrict__ order, int perturb)
+                                                      const uint32_t *__restrict__ order, uint32_t spread, int perturb)
 {
-    const uint32_t m = order[blockIdx.y];
+    const uint32_t m = order[blockIdx.x / spread];
     const float pert = perturb ? (float)glb(ios[m].norms)[0] : 0.f;
     const uint2 *dvd = glb(descs[m].f.dvd);
     const uint32_t nd = glb(descs[m].f.dvd_ptr)[descs[m].f.num_lev];
     float *lu = glb(ios[m].lu);
-    for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < nd; t += gridDim.x * 256)
+    for (uint32_t t = blockIdx.x % spread * 256 + threadIdx.x; t < nd; t += spread * 256)
         factor_divide(lu, dvd[t], pert, perturb);
 }
 
 __global__ void __launch_bounds__(256) k_group_copy(const MatDesc *__restrict__ descs, const MatIO *__restrict__ ios,
-                                                    const uint32_t *__restrict__ order)
+                                                    const uint32_t *__restrict__ order, uint32_t spread)
 {
-    const uint32_t m = order[blockIdx.y], nval = descs[m].s.df_nval;
+    const uint32_t m = order[blockIdx.x / spread], nval = descs[m].s.df_nval;
     const uint32_t *src = glb(descs[m].s.df_src);
     const float *lu = glb(ios[m].lu);
     float *to = glb(ios[m].lucsr);
-    for (uint32_t q = blockIdx.x * 256 + threadIdx.x; q < nval; q += gridDim.x * 256) {
+    for (uint32_t q = blockIdx.x % spread * 256 + threadIdx.x; q < nval; q += spread * 256) {
         const uint32_t p = src[q];
         to[q] = p != ~0u ? lu[p] : 0.f;
     }
@@ -3822,10 +3824,10 @@ void batch_group(const MatDesc *descs, const void *ios, const uint32_t *order, i
                  int maxit, int perturb, int threads, int mode, size_t fact_lds, size_t ref_lds, hipStream_t st)
 {
     const MatIO *io = static_cast<const MatIO *>(ios);
-    const dim3 spread(kGroupSpread, count);
+    const uint32_t spread = std::min(kGroupSpread, std::max(1u, kGroupGrid / (uint32_t)count));
     k_batch_group_factor<<<count, threads, fact_lds, st>>>(descs, io, order, l0, perturb);
-    k_group_divide<<<spread, 256, 0, st>>>(descs, io, order, perturb);
-    if (mode != kSweepLevels) k_group_copy<<<spread, 256, 0, st>>>(descs, io, order);
+    k_group_divide<<<spread * count, 256, 0, st>>>(descs, io, order, spread, perturb);
+    if (mode != kSweepLevels) k_group_copy<<<spread * count, 256, 0, st>>>(descs, io, order, spread);
     if (mode == kSweepLds)
         k_batch_group_refine<kSweepLds><<<count, threads, ref_lds, st>>>(descs, io, order, tol, maxit);
     else if (mode == kSweepFlags)   // per matrix: vector in LDS where it fits ref_lds
