@@ -2209,9 +2209,11 @@ struct SwChunk {
 
 // a / d with the work on d done ahead (the divisor is known long before the
 // row's value is).  r: the reciprocal with one Newton step; the quotient then
-// takes the two corrections of the compiler's own division of operands that
-// need no scaling, so the result is its result, correctly rounded.  Operands
-// outside [2^-30, 2^30] (d) and [2^-64, 2^64] (a) take the full division.
+// takes the two corrections of an FP32 division of operands that need no
+// scaling as LLVM's AMDGPU backend expands it (LowerFDIV32), so the result is
+// that of a / d, correctly rounded.  Operands outside [2^-30, 2^30) (d) and
+// [2^-64, 2^64) (a) take the full division; inside, no correction leaves the
+// normal range (the smallest, a's 2^-64 less 48 bits, is 2^-112).
 struct SwDiv {
     float d, r;
     bool plain;   // d in range

@@ -1519,9 +1519,6 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
                     nsrc += M.count[t];
                 }
             src.resize(nsrc);
-            std::vector<uint32_t> cur;   // next source of each merge entry
-            for (uint16_t t : order)
-                if (M.count[t] >= 2) cur.push_back(M.first[t]);
             // (the bin lists its columns in schedule order, so a merge entry's sources come in it)
             for (size_t c = i; c < e; ++c) {
                 const uint32_t k = cols[b][c], dpos = P.l_col_ptr[k], L = P.sym_c_ptr[k + 1] - dpos - 1;
