@@ -1330,8 +1330,12 @@ int phase_end(const glu_pattern &P, int l0, int limit, uint32_t bin_slots, std::
 
 // The streams and the assembly of the phase of steps [ph.l0, ph.l1) with the
 // columns' components comp.  False: an update would cross components (the
-// pattern's levels do not order it; the steps stay as they are).
-bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &level_of,
+// pattern's levels do not order it; the steps stay as they are).  The update
+// map of the phase's columns, which nothing else reads from here on, is
+// overwritten: updates of later entries get their products' places (kPlace).
+constexpr uint32_t kPlace = 0x80000000u;   // (positions are below 2^31)
+
+bool build_phase(const glu_pattern &P, Tables &T, const std::vector<int> &level_of,
                  const std::vector<uint32_t> &comp, uint32_t bin_slots, Phase &ph)
 {
     const uint32_t n = P.n;
@@ -1398,17 +1402,17 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
     // products per later entry: column j's pivots of the phase in schedule
     // order (step by step, a step's columns as level_idx lists them, the order
     // of every other path); cnt by position, then each product's place
-    std::vector<uint32_t> cnt(P.nnz, 0), base(P.nnz, 0);
+    std::vector<uint32_t> cnt(P.nnz, 0);
     std::vector<uint32_t> csc2csr(P.nnz);
     for (uint32_t q = 0; q < P.nnz; ++q) csc2csr[T.upos[q]] = q;
     std::atomic<bool> crossed(false);
     std::vector<int> place_of(n);
     for (int t = 0; t < (int)n; ++t) place_of[P.level_idx[t]] = t;
-    auto each_outside = [&](uint32_t j, std::vector<std::pair<int, uint32_t>> &ks, auto f) {
+    auto each_outside = [&](uint32_t j, bool in_order, std::vector<std::pair<int, uint32_t>> &ks, auto f) {
         ks.clear();
         for (uint32_t p = P.sym_c_ptr[j]; p < P.l_col_ptr[j]; ++p)
             if (comp[P.sym_r_idx[p]] != UINT32_MAX) ks.push_back({place_of[P.sym_r_idx[p]], p});
-        std::sort(ks.begin(), ks.end());
+        if (in_order) std::sort(ks.begin(), ks.end());
         for (const auto &[at_place, p] : ks) {
             const uint32_t k = P.sym_r_idx[p], L = P.sym_c_ptr[k + 1] - P.l_col_ptr[k] - 1;
             const uint64_t at = T.moff[k] + (uint64_t)(csc2csr[p] - P.csr_diag_ptr[k] - 1) * L;
@@ -1424,44 +1428,43 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
     const size_t items = (n + kCols - 1) / kCols;
     parallel_items(items, threads, [&](unsigned w, size_t item) {
         for (uint32_t j = (uint32_t)item * kCols; j < std::min<uint32_t>(n, (uint32_t)(item + 1) * kCols); ++j)
-            each_outside(j, scratch[w], [&](uint64_t, uint32_t t) { ++cnt[t]; });
+            each_outside(j, false, scratch[w], [&](uint64_t, uint32_t t) { ++cnt[t]; });
     });
     if (crossed.load()) return false;
     // entries by product count: groups of 64 of about the same, waves for the rest
-    std::vector<uint32_t> few, many;
+    std::vector<uint32_t> few, many, with(kAsmLane + 2, 0);   // with[c]: entries of more than c products, at most kAsmLane
     for (uint32_t p = 0; p < P.nnz; ++p)
-        if (cnt[p]) (cnt[p] <= kAsmLane ? few : many).push_back(p);
-    const auto most = [&](uint32_t a, uint32_t b) { return cnt[a] > cnt[b]; };
-    std::stable_sort(few.begin(), few.end(), most);
-    std::stable_sort(many.begin(), many.end(), most);
+        if (cnt[p] > kAsmLane) many.push_back(p);
+        else if (cnt[p]) ++with[cnt[p] - 1];
+    for (uint32_t c = kAsmLane; c-- > 0;) with[c] += with[c + 1];
+    few.resize(with[0]);
+    for (uint32_t p = 0; p < P.nnz; ++p)   // most products first, then by position
+        if (cnt[p] && cnt[p] <= kAsmLane) few[with[cnt[p]]++] = p;
+    std::stable_sort(many.begin(), many.end(), [&](uint32_t a, uint32_t b) { return cnt[a] > cnt[b]; });
     uint64_t out = 0;
-    std::vector<uint8_t> lane64(P.nnz, 0);   // product stride 64 (grouped) or 1
+    std::vector<uint32_t> next(P.nnz, UINT32_MAX);   // place of the entry's next product; kPlace: 64 apart
     for (size_t i = 0; i < few.size(); i += 64) {
         const uint32_t m = cnt[few[i]];
         ph.grp.push_back(make_uint2((uint32_t)out, m));
         for (size_t k = i; k < i + 64; ++k) {
             ph.tgt.push_back(k < few.size() ? few[k] : UINT32_MAX);
             ph.cnt.push_back(k < few.size() ? (uint8_t)cnt[few[k]] : 0);
-            if (k < few.size()) {
-                base[few[k]] = (uint32_t)(out + (k - i));
-                lane64[few[k]] = 1;
-            }
+            if (k < few.size()) next[few[k]] = kPlace | (uint32_t)(out + (k - i));
         }
         out += 64 * (uint64_t)m;
     }
     for (uint32_t p : many) {
         ph.wav.push_back(AsmWave{p, (uint32_t)out, cnt[p], 0});
-        base[p] = (uint32_t)out;
+        next[p] = (uint32_t)out;
         out += (cnt[p] + 63u) & ~63u;
     }
-    if (out >= UINT32_MAX) return false;
+    if (out >= kPlace) return false;
     ph.nout = (uint32_t)out;
-    std::vector<uint32_t> place(T.umap.size(), UINT32_MAX);   // by update, as umap
-    std::fill(cnt.begin(), cnt.end(), 0);
     parallel_items(items, threads, [&](unsigned w, size_t item) {
         for (uint32_t j = (uint32_t)item * kCols; j < std::min<uint32_t>(n, (uint32_t)(item + 1) * kCols); ++j)
-            each_outside(j, scratch[w], [&](uint64_t at, uint32_t t) {
-                place[at] = base[t] + cnt[t]++ * (lane64[t] ? 64u : 1u);
+            each_outside(j, true, scratch[w], [&](uint64_t at, uint32_t t) {
+                T.umap[at] = kPlace | next[t];
+                next[t] += (next[t] & kPlace) ? 64u : 1u;
             });
     });
     // each bin's program: its steps' inner updates, then all its products
@@ -1497,8 +1500,8 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
                     const uint32_t U = P.csr_r_ptr[k + 1] - P.csr_diag_ptr[k] - 1;
                     for (uint32_t jj = 0; jj < U; ++jj)
                         for (uint32_t ii = 0; ii < L; ++ii) {
-                            const uint64_t at = T.moff[k] + (uint64_t)jj * L + ii;
-                            if (place[at] == UINT32_MAX) f(k, jj, ii, slot[T.umap[at]]);
+                            const uint32_t t = T.umap[T.moff[k] + (uint64_t)jj * L + ii];
+                            if (!(t & kPlace)) f(k, jj, ii, slot[t]);
                         }
                 }
             };
@@ -1533,9 +1536,9 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
                 for (uint32_t jj = 0; jj < U; ++jj) {
                     const uint16_t u = slot[T.upos[P.csr_diag_ptr[k] + 1 + jj]];
                     for (uint32_t ii = 0; ii < L; ++ii) {
-                        const uint64_t at = T.moff[k] + (uint64_t)jj * L + ii;
-                        if (place[at] != UINT32_MAX) continue;
-                        const uint16_t t = slot[T.umap[at]];
+                        const uint32_t q = T.umap[T.moff[k] + (uint64_t)jj * L + ii];
+                        if (q & kPlace) continue;
+                        const uint16_t t = slot[q];
                         if (M.count[t] >= 2) src[M.first[t]++] = {lslot[ii], u, slot[dpos]};
                         else lists[ii].push_back({u, t});
                     }
@@ -1556,10 +1559,10 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
                     uint16_t u[2];
                     uint32_t o[2], m = 0;
                     for (uint32_t x = jj; x < std::min(jj + 2, U); ++x) {
-                        const uint32_t at = place[T.moff[k] + (uint64_t)x * L + ii];
-                        if (at == UINT32_MAX) continue;
+                        const uint32_t at = T.umap[T.moff[k] + (uint64_t)x * L + ii];
+                        if (!(at & kPlace)) continue;
                         u[m] = slot[T.upos[P.csr_diag_ptr[k] + 1 + x]];
-                        o[m++] = at;
+                        o[m++] = at & ~kPlace;
                     }
                     if (m) B.product(slot[dpos + 1 + ii], slot[dpos], m, u, o);
                 }
@@ -1573,7 +1576,7 @@ bool build_phase(const glu_pattern &P, const Tables &T, const std::vector<int> &
 
 // The phases ahead of step `limit` (the first LDS window's), their bins of
 // bin_slots entries at most.
-void choose_phases(const glu_pattern &P, const Tables &T, int limit, uint32_t bin_slots, std::vector<Phase> &phases)
+void choose_phases(const glu_pattern &P, Tables &T, int limit, uint32_t bin_slots, std::vector<Phase> &phases)
 {
     std::vector<int> level_of(P.n, 0);
     for (int l = 0; l < P.num_lev; ++l)
@@ -2693,6 +2696,11 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
         p->has_scaling = p->has_refine = true;
     }
 
+    std::vector<uint2> cln2(T.cln.size());   // {L position, pivot position} per lane
+    for (size_t q = 0; q < T.cln.size(); ++q) cln2[q] = make_uint2(T.cln[q].x, T.cln[q].y);
+    std::vector<uint4> mrec;
+    merge_records(T.ment, T.msrc_ptr, T.msrc, 0, (uint32_t)T.ment.size(), [](uint32_t q) { return q; }, mrec);
+
     // ---------------- upload everything into one arena ------------------
     if (factor_steps.valid()) factor_steps.get();
     p->nwin = (int)wins.size();
@@ -2752,8 +2760,6 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     const size_t o_cdiag = U.put(P.csr_diag_ptr, n);
     const size_t o_upos = U.put(T.upos);
     const size_t o_cptr = U.put(T.ctask_ptr);
-    std::vector<uint2> cln2(T.cln.size());   // {L position, pivot position} per lane
-    for (size_t q = 0; q < T.cln.size(); ++q) cln2[q] = make_uint2(T.cln[q].x, T.cln[q].y);
     const size_t o_cln = U.put(cln2);
     const size_t o_ctgt = U.put(T.ctgt);
     const size_t o_cup = U.put(T.cup);
@@ -2762,8 +2768,6 @@ glu_status build_plan(const glu_pattern &P, const glu_analysis *a, const glu_pla
     const size_t o_mlong = U.put(T.ment_long);
     const size_t o_msptr = U.put(T.msrc_ptr);
     const size_t o_msrc = U.put(T.msrc);
-    std::vector<uint4> mrec;
-    merge_records(T.ment, T.msrc_ptr, T.msrc, 0, (uint32_t)T.ment.size(), [](uint32_t q) { return q; }, mrec);
     const size_t o_mrec = U.put(mrec);
     const size_t o_dvd = U.put(T.dvd);
     const size_t o_dptr = U.put(T.dvd_ptr);

@@ -211,6 +211,7 @@ int main(int argc, char **argv)
     std::vector<Window> wins;
     choose_windows(T, P.num_lev, P.nnz, budget, kDefaultFuseUnits, 1, waves, wins);
     std::vector<Phase> phases;
+    const std::vector<uint32_t> umap = T.umap;   // (the phases write places over theirs)
     choose_phases(P, T, wins.empty() ? 0 : std::min(wins[0].l0, P.num_lev), bin_values, phases);
     size_t lane = 0, wave = 0, bins = 0, most = 0;
     int steps = 0;
@@ -237,7 +238,7 @@ int main(int argc, char **argv)
                 for (uint32_t jj = 0; jj < rp[k + 1] - u0; ++jj)
                     for (uint32_t ii = 0; ii < L; ++ii) {
                         const float m = v[d + 1 + ii] / gesp(v[d], pert);
-                        float &x = v[T.umap[T.moff[k] + (uint64_t)jj * L + ii]];
+                        float &x = v[umap[T.moff[k] + (uint64_t)jj * L + ii]];
                         x = x + (-(m * v[T.upos[u0 + jj]]));
                     }
             }
