@@ -1279,21 +1279,64 @@ constexpr uint32_t kPhaseBins = 512;       // two workgroups a CU
 constexpr uint32_t kPhaseSlots = 19000;    // entries of a bin, at most (76 KB: two a CU)
 constexpr int kMinPhase = 4;               // steps
 
-// The steps from l0 on that make a phase, at most to `limit`: as many as keep
-// every component's entries within a bin (of bin_slots).  Components of the
-// columns of steps [l0, e): joined by entries of L or U between them.  Returns
-// e (l0: none) and each column's component (UINT32_MAX: not in the phase).
-int phase_end(const glu_pattern &P, int l0, int limit, uint32_t bin_slots, std::vector<uint32_t> &comp)
+// Whether steps gain from being a phase, estimated in us (measured over MNA,
+// mesh and dense patterns).  A step as a launch of its own: 4.1, and 16 ns for
+// each source of its longest merge entry and 20 ns per 1,000 lanes (4.2 to 5 on
+// meshes and dense patterns, 13 where a rail's entry has 500 sources).  A phase:
+// its two launches, 0.3 a step, the updates of the bin with the most at 1 ns
+// (0.36 to 1.2 ns: one workgroup) or all of them at 8 ps (the whole card),
+// and the longest entry's products at 3.5 ns.  What decides is how much of the
+// work falls on one bin: the leading steps of a circuit fall apart into
+// hundreds of components (n=200,003: 42 steps, 30 M updates over 512 bins,
+// 292 us for about 700), a mesh's soon join into a few (a 300 x 300 mesh, all
+// steps in 63 phases of 1 to 237 bins: 93 ms, as launches 9.7) and a dense
+// pattern's are one (n=600: 29 ms, as launches 2.5).
+struct StepCost {
+    double us;
+    uint64_t updates;
+    uint32_t longest;      // sources of its longest merge entry
+};
+
+std::vector<StepCost> step_costs(const glu_pattern &P, const Tables &T, int limit)
+{
+    std::vector<StepCost> cost(limit);
+    for (int l = 0; l < limit; ++l) {
+        StepCost &c = cost[l];
+        c.updates = 0;
+        c.longest = 0;
+        for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) c.updates += T.moff[P.level_idx[t] + 1] - T.moff[P.level_idx[t]];
+        for (uint32_t e = T.ment_ptr[l]; e < T.ment_ptr[l + 1]; ++e) c.longest = std::max(c.longest, T.msrc_ptr[e + 1] - T.msrc_ptr[e]);
+        c.us = 4.1 + 0.016 * c.longest + 2e-5 * level_lanes(T, l);
+    }
+    return cost;
+}
+
+constexpr double kEven = 5.0;
+
+double phase_us(int steps, uint64_t updates, uint64_t most, uint64_t longest)
+{
+    return 10.0 + 0.3 * steps + std::max(1e-3 * (double)most, 8e-6 * (double)updates) + 3.5e-3 * (double)longest;
+}
+
+// The steps from l0 on that make a phase, at most to `limit` and as long as
+// every component's entries fit a bin (of bin_slots): at least kMinPhase, as
+// many as gain the most within kEven (the estimate errs on the bins' side:
+// n=20,000 38 steps 605 us, the 37 it puts 2 us ahead 608).  Components of the columns of steps [l0, e):
+// joined by entries of L or U between them.  Returns e (l0: none) and each
+// column's component (UINT32_MAX: not in the phase).
+int phase_end(const glu_pattern &P, const Tables &T, const std::vector<StepCost> &cost, int l0, int limit, uint32_t bin_slots,
+              std::vector<uint32_t> &comp)
 {
     const uint32_t n = P.n;
     std::vector<uint32_t> parent(n), ent(n);
+    std::vector<uint64_t> work(n);
     std::vector<uint8_t> seen(n);
     auto find = [&](uint32_t r) {
         while (parent[r] != r) r = parent[r] = parent[parent[r]];
         return r;
     };
     // column k joins what it shares an entry with among the columns seen;
-    // returns its component's entries
+    // returns its component
     auto add = [&](uint32_t k) {
         seen[k] = 1;
         auto join = [&](uint32_t r) {
@@ -1302,30 +1345,47 @@ int phase_end(const glu_pattern &P, int l0, int limit, uint32_t bin_slots, std::
             if (a == c) return;
             parent[a] = c;
             ent[c] += ent[a];
+            work[c] += work[a];
         };
         for (uint32_t q = P.csr_r_ptr[k]; q < P.csr_r_ptr[k + 1]; ++q) join(P.csr_c_idx[q]);
         for (uint32_t q = P.sym_c_ptr[k]; q < P.sym_c_ptr[k + 1]; ++q) join(P.sym_r_idx[q]);
-        return ent[find(k)];
+        return find(k);
     };
     auto reset = [&]() {
         for (uint32_t k = 0; k < n; ++k) {
             parent[k] = k;
             ent[k] = (P.sym_c_ptr[k + 1] - P.l_col_ptr[k]) + (P.csr_r_ptr[k + 1] - P.csr_diag_ptr[k] - 1);
+            work[k] = T.moff[k + 1] - T.moff[k];
             seen[k] = 0;
         }
     };
     reset();
-    int e = l0;
-    for (bool fits = true; e < limit && fits; e += fits)
-        for (int t = P.level_ptr[e]; t < P.level_ptr[e + 1]; ++t)
-            fits = add((uint32_t)P.level_idx[t]) <= bin_slots && fits;
-    reset();   // (without the step that did not fit)
-    for (int l = l0; l < e; ++l)
+    int best = l0;
+    double gain = 0.0, launches = 0.0;
+    uint64_t updates = 0, most = 0, longest = 0;
+    for (int e = l0; e < limit; ++e) {
+        bool fits = true;
+        for (int t = P.level_ptr[e]; t < P.level_ptr[e + 1]; ++t) {
+            const uint32_t c = add((uint32_t)P.level_idx[t]);
+            fits = ent[c] <= bin_slots && fits;
+            most = std::max(most, work[c]);
+        }
+        if (!fits) break;
+        launches += cost[e].us;
+        updates += cost[e].updates;
+        longest += cost[e].longest;
+        const int steps = e + 1 - l0;
+        const double g = launches - phase_us(steps, updates, std::max<uint64_t>(most, updates / kPhaseBins), longest);
+        if (steps >= kMinPhase && g > 0.0 && g >= gain - kEven) best = e + 1;
+        gain = std::max(gain, g);
+    }
+    reset();   // (without the steps after the best)
+    for (int l = l0; l < best; ++l)
         for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) (void)add((uint32_t)P.level_idx[t]);
     comp.assign(n, UINT32_MAX);
-    for (int l = l0; l < e; ++l)
+    for (int l = l0; l < best; ++l)
         for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) comp[P.level_idx[t]] = find((uint32_t)P.level_idx[t]);
-    return e;
+    return best;
 }
 
 // The streams and the assembly of the phase of steps [ph.l0, ph.l1) with the
@@ -1581,10 +1641,11 @@ void choose_phases(const glu_pattern &P, Tables &T, int limit, uint32_t bin_slot
     std::vector<int> level_of(P.n, 0);
     for (int l = 0; l < P.num_lev; ++l)
         for (int t = P.level_ptr[l]; t < P.level_ptr[l + 1]; ++t) level_of[P.level_idx[t]] = l;
+    const std::vector<StepCost> cost = step_costs(P, T, limit);
     std::vector<uint32_t> comp;
     for (int l = 0; l < limit;) {
-        const int e = phase_end(P, l, limit, bin_slots, comp);
-        if (e - l < kMinPhase) break;
+        const int e = phase_end(P, T, cost, l, limit, bin_slots, comp);
+        if (e == l) break;
         Phase ph;
         ph.l0 = l;
         ph.l1 = e;

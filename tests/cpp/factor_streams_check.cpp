@@ -213,17 +213,18 @@ int main(int argc, char **argv)
     std::vector<Phase> phases;
     const std::vector<uint32_t> umap = T.umap;   // (the phases write places over theirs)
     choose_phases(P, T, wins.empty() ? 0 : std::min(wins[0].l0, P.num_lev), bin_values, phases);
-    size_t lane = 0, wave = 0, bins = 0, most = 0;
+    size_t lane = 0, wave = 0, bins = 0, most = 0, busiest = 0;   // busiest: chunks of a phase's longest bin a step
     int steps = 0;
     for (const Phase &ph : phases) {
-        for (const uint2 &g : ph.grp) (void)g, lane += 64;
+        lane += 64 * ph.grp.size();
+        for (const Window &w : ph.bin) busiest = std::max(busiest, w.hdr.size() / (size_t)(ph.l1 - ph.l0));
         wave += ph.wav.size();
         bins += ph.bin.size();
         most = std::max<size_t>(most, ph.nslot);
         steps = ph.l1;
     }
-    printf("n=%u levels=%d windows=%zu phases=%zu steps=%d bins=%zu largest=%zu lane_entries=%zu wave_entries=%zu\n", P.n,
-           P.num_lev, wins.size(), phases.size(), steps, bins, most, lane, wave);
+    printf("n=%u levels=%d windows=%zu phases=%zu steps=%d bins=%zu largest=%zu lane_entries=%zu wave_entries=%zu busiest=%zu\n", P.n,
+           P.num_lev, wins.size(), phases.size(), steps, bins, most, lane, wave, busiest);
     if (most > bin_values) die("a bin's values exceed the limit", most, bin_values);
     std::mt19937 g(11);
     std::uniform_real_distribution<float> U(-1.f, 1.f);

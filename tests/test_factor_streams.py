@@ -11,6 +11,7 @@ import subprocess
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from test_gpu_phases import CASES
 from test_sweep_tables import BUILD, HIPCC, PKG, ROOT
@@ -33,6 +34,31 @@ def checker(tmp_path_factory):
     shutil.rmtree(d, ignore_errors=True)
 
 
+def _csc(A):
+    A = sp.csc_matrix(A)
+    A.sort_indices()
+    return A.data.copy(), A.indices.astype(np.int32), A.indptr.astype(np.int32), A.shape[0]
+
+
+def _mesh(m, dims):
+    """Laplacian of an m x m (x m) mesh."""
+    one, line = sp.identity(m), sp.diags([-1.0, 2.0, -1.0], [-1, 0, 1], (m, m))
+    A = 0
+    for d in range(dims):
+        term = sp.identity(1)
+        for k in range(dims):
+            term = sp.kron(term, line if k == d else one)
+        A = A + term
+    return _csc(A)
+
+
+# patterns whose leading steps join into few components
+JOINED = {"dense": lambda: _csc(np.random.default_rng(1).uniform(0.1, 1, (300, 300)) + 300 * np.eye(300)),
+          "mesh2": lambda: _mesh(110, 2), "mesh3": lambda: _mesh(13, 3),
+          "blocks": lambda: _csc(sp.block_diag([np.random.default_rng(k).uniform(0.1, 1, (150, 150)) + 150 * np.eye(150)
+                                                for k in range(12)]))}
+
+
 @pytest.fixture(scope="module")
 def pattern(tmp_path_factory):
     d = tmp_path_factory.mktemp("patterns")
@@ -41,7 +67,7 @@ def pattern(tmp_path_factory):
         path = d / name
         if not path.exists():
             from pyglu.analysis import Analysis
-            an = Analysis(*CASES[name]())
+            an = Analysis(*(CASES.get(name) or JOINED[name])())
             with open(path, "wb") as f:
                 for k in ("sym_c_ptr", "sym_r_idx", "l_col_ptr", "csr_r_ptr", "csr_c_idx", "csr_diag_ptr",
                           "level_ptr", "level_idx"):
@@ -70,7 +96,7 @@ def test_streams(checker, pattern, name, values):
         assert got["phases"]
     if values == 700 and name in ("lane", "wave"):
         assert (got["lane_entries"] > 0, got["wave_entries"] > 0) == (name == "lane", name == "wave")
-    if name in ("unsym300", "unsym1500", "mna2k", "grad"):
+    if name in ("unsym300", "mna2k", "grad"):
         assert got["lane_entries"] and got["wave_entries"]
 
 
@@ -87,3 +113,11 @@ def test_levels_listed_downward(checker, pattern, name, values):
     """A caller's pattern may list a level's columns in any order: the phases
     subtract in that order too, as the other steps do."""
     _check(checker, pattern(name), values, 19000, reverse=1)
+
+
+@pytest.mark.parametrize("name", list(JOINED))
+@pytest.mark.parametrize("values", [700, 39800])
+def test_work_of_a_phase_is_spread(checker, pattern, name, values):
+    """Steps whose work would fall on a few workgroups stay launches over the
+    whole card: 50 ns a chunk on the busiest bin, at most 5 us a step."""
+    assert _check(checker, pattern(name), values, 19000)["busiest"] <= 100
