@@ -1940,6 +1940,33 @@ __device__ __forceinline__ void df2_issue(const DfDev &D, const float *__restric
     }
 }
 
+// A wait for ready bits must leave the units to the wave it waits for.  Of the
+// waves of a SIMD the oldest is served first, so waiting waves that keep a
+// unit busy can hold the others back for good: with the x values of all six
+// entries loaded on every poll, ready or not, four waves of 64 waiting lanes
+// took the whole vector memory unit (6 gathers of 64 lines each a poll), and
+// a younger wave that had the awaited row never got its loads issued (a
+// 300 x 300 mesh, 32 matrices a call: some calls ended by the bound below,
+// after 2^24 polls of 0.74 us, with NaN).  After kEagerPolls polls in a row in
+// which no lane went on, a wave therefore waits by ready bits alone, asleep
+// between them.
+constexpr uint32_t kEagerPolls = 4;
+
+// Until the row of column c is ready in a waiting lane (or spins reaches cap).
+__device__ __forceinline__ void df_quiet(const uint32_t *flags, bool waiting, uint32_t c, uint32_t &spins, uint32_t cap)
+{
+    while (!__ballot(waiting && df_peek(flags, c)) && spins < cap) {
+        ++spins;
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+__device__ __forceinline__ void df_wait(const uint32_t *flags, uint32_t c)
+{
+    for (uint32_t idle = 0; !df_ready(flags, c);)
+        if (++idle > kEagerPolls) __builtin_amdgcn_s_sleep(1);
+}
+
 // A task of lane rows some longer than kDfK entries: each lane walks its
 // row kDfK entries at a time (the slots of entry e at base + 64 e + lane),
 // consuming ready entries in the row's order as the short-row path does.
@@ -1969,7 +1996,9 @@ __device__ __forceinline__ void df2_lane_long(const DfDev &D, const float *__res
             nval[e] = sv[t.base + (kDfK + e) * kWave + lane];
         }
     uint32_t ci = 0, c0 = 0;   // entries consumed, first entry of the chunk
+    uint32_t idle = 0;
     for (uint32_t spins = 0; __ballot(pending) && spins < kSpinCap; ++spins) {
+        const uint32_t before = ci;
         if (pending) {
             if (ci == c0 + kDfK) {
                 // chunk consumed, row not done: the next kDfK entries
@@ -2016,6 +2045,14 @@ __device__ __forceinline__ void df2_lane_long(const DfDev &D, const float *__res
                 pending = false;
             }
         }
+        if (__ballot(ci != before)) {
+            idle = 0;
+        } else if (++idle >= kEagerPolls) {
+            uint32_t c = idx[0];   // the lane's next entry
+#pragma unroll
+            for (uint32_t e = 1; e < kDfK; ++e) c = c0 + e == ci ? idx[e] : c;
+            df_quiet(flags, pending, c, spins, kSpinCap);
+        }
     }
     if (pending) {   // gave up: the row completes with NaN
         x.put(t.row, df_nan());
@@ -2023,9 +2060,6 @@ __device__ __forceinline__ void df2_lane_long(const DfDev &D, const float *__res
     }
 }
 
-// Waits spin on the LDS ready bits without s_sleep: measured on the n=20k
-// batch, the wake-up latency of a sleeping wave costs more (7.08 vs
-// 6.92 ms per batch) than the LDS reads of the spinning ones.
 // kExact: every row's products subtracted one at a time in the row's order
 // (group rows through the wave's LDS slice `lds`, by the group's first
 // lane) — the arithmetic of Symbolic_Matrix::solve, for glu_solve.
@@ -2040,8 +2074,9 @@ __device__ __forceinline__ void df2_run(const DfDev &D, const float *__restrict_
         }
         bool pending = lane < t.cnt;
         float acc = pending ? x.in(t.row) : 0.f;
-        uint32_t ci = 0;
+        uint32_t ci = 0, idle = 0;
         while (__ballot(pending)) {   // unbounded: the plan's tables are checked on the host
+            const uint32_t before = ci;
             if (pending) {
                 // every entry's ready bit and x value read without branches
                 // (independent LDS reads, one wait each), then the ready
@@ -2071,6 +2106,14 @@ __device__ __forceinline__ void df2_run(const DfDev &D, const float *__restrict_
                     pending = false;
                 }
             }
+            if (__ballot(ci != before)) {
+                idle = 0;
+            } else if (++idle >= kEagerPolls && __ballot(pending)) {
+                uint32_t c = t.idx[0], spins = 0;   // the lane's next entry
+#pragma unroll
+                for (uint32_t e = 1; e < kDfK; ++e) c = e == ci ? t.idx[e] : c;
+                df_quiet(flags, pending, c, spins, ~0u);
+            }
         }
         return;
     }
@@ -2097,7 +2140,7 @@ __device__ __forceinline__ void df2_run(const DfDev &D, const float *__restrict_
             }
             float pr = 0.f;
             if (c0 + j < t.len) {
-                while (!df_ready(flags, col)) {}
+                df_wait(flags, col);
                 pr = v * x.get(col);
             }
             a = j == 0 ? carry - pr : pr;
@@ -2123,7 +2166,7 @@ __device__ __forceinline__ void df2_run(const DfDev &D, const float *__restrict_
     }
     float sum = 0.f;
     if (j < t.len) {
-        while (!df_ready(flags, t.idx[0])) {}
+        df_wait(flags, t.idx[0]);
         sum = t.val[0] * x.get(t.idx[0]);
     }
     for (uint32_t c0 = kWave; c0 < t.len; c0 += 4 * kWave) {   // gw == 64 here
@@ -2138,7 +2181,7 @@ __device__ __forceinline__ void df2_run(const DfDev &D, const float *__restrict_
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u)
             if (c0 + u * kWave + j < t.len) {
-                while (!df_ready(flags, col[u])) {}
+                df_wait(flags, col[u]);
                 sum += v[u] * x.get(col[u]);
             }
     }
