@@ -161,7 +161,7 @@ int main(int argc, char **argv)
         for (uint32_t k : p->count)
             if (!whole && k > cap) die("a part's rows exceed the limit", k, cap);
     SwHost hd[4], tl[4];
-    uint64_t lanes = 0, slots = 0, longest = 0;
+    uint64_t lanes = 0, slots = 0, longest = 0, waited = 0, least = 0;
     int planted = 0, caught = 0;
     for (int q = 0; q < 4; ++q) {
         TriHost H;
@@ -183,6 +183,18 @@ int main(int argc, char **argv)
         // (glu_refine_noalloc's scratch rests on this)
         if (whole && 3 * (uint64_t)tl[q].meta.size() > D.idx.size() + 64 * (uint64_t)n)
             die("lanes exceed a third of the slots and 64 a row", tl[q].meta.size(), D.idx.size());
+        // chunks every step waits for: the most a wave has, and the fewest that could be
+        if (whole) {
+            const SwHost &S = tl[q];
+            std::vector<uint32_t> total(S.part[0].steps), most(S.part[0].steps);
+            size_t c = 0;
+            for (uint32_t w = 0; w < waves; ++w) {
+                std::vector<uint32_t> mine(S.part[0].steps);
+                for (uint32_t k = 0; k < S.wave[w].x; ++k, ++c) ++mine[S.hdr[c] & kSwStepMask];
+                for (uint32_t k = 0; k < mine.size(); ++k) total[k] += mine[k], most[k] = std::max(most[k], mine[k]);
+            }
+            for (uint32_t k = 0; k < total.size(); ++k) waited += most[k], least += std::max(1u, (total[k] + waves - 1) / waves);
+        }
         // planted mistakes: a slot or a value position past the end, a step
         // too early, a chunk left out, a right-hand side elsewhere
         const SwHost &S = tl[q];
@@ -250,6 +262,7 @@ int main(int argc, char **argv)
                 if (tree ? !(std::fabs(x[r] - ref[r]) <= tol) : std::memcmp(&x[r], &seq[r], 4) != 0)
                     die("a row differs", r, (size_t)(2 * t + tree));
         }
+    if (whole) printf("chunks waited for: %llu of at least %llu\n", (unsigned long long)waited, (unsigned long long)least);
     printf("ok n=%u parts=%zu tail=%u lanes=%llu slots=%llu planted=%d caught=%d: streams equal the row-by-row solve bit for bit\n",
            n, spl.head.count.size(), spl.tail.count[0], (unsigned long long)lanes, (unsigned long long)slots, planted, caught);
     return planted == caught ? 0 : 1;

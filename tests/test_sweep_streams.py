@@ -10,6 +10,7 @@ import subprocess
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from helpers import mna_case
 from test_gpu_sweeps import _case
@@ -42,6 +43,17 @@ def _pattern(case):
         return _case(2049, (1000, 1500, 449, 511, 513), 2126)
     if case == "one":
         return _case(1, (), 1)
+    if case == "mesh":   # 18 x 18 x 18
+        one, side = sp.identity(18), sp.diags([-1, -1], [-1, 1], (18, 18))
+        line = sp.diags([-1, 6, -1], [-1, 0, 1], (18, 18))
+        A = sp.csc_matrix(sp.kron(sp.kron(one, one), line) + sp.kron(sp.kron(one, side), one) +
+                          sp.kron(sp.kron(side, one), one))
+        A.sort_indices()
+        return A.data, A.indices.astype(np.int32), A.indptr.astype(np.int32), A.shape[0]
+    if case == "blocks":   # 10 dense ones
+        A = sp.csc_matrix(sp.block_diag([np.ones((300, 300)) + 300 * np.identity(300)] * 10))
+        A.sort_indices()
+        return A.data, A.indices.astype(np.int32), A.indptr.astype(np.int32), A.shape[0]
     return mna_case(case)
 
 
@@ -64,6 +76,16 @@ def _check(checker, tmp_path, case, cap, waves):
 @pytest.mark.parametrize("waves", [1, 4, 16])
 def test_whole_orders(checker, tmp_path, case, waves):
     assert "bit for bit" in _check(checker, tmp_path, case, 0, waves)
+
+
+@pytest.mark.parametrize("case,most", [("mesh", 1.1), ("blocks", 1.2)])
+def test_no_wave_is_waited_for(checker, tmp_path, case, most):
+    """A step lasts as long as the wave with the most chunks in it takes: few
+    steps beyond the share of every wave, rows of several chunks (which have
+    waves of their own) or not."""
+    out = _check(checker, tmp_path, case, 0, 16)
+    waited, least = map(int, re.search(r"waited for: (\d+) of at least (\d+)", out).groups())
+    assert least <= waited <= most * least
 
 
 @pytest.mark.parametrize("case,cap", [("mna2k", 300), ("mna2k", 1000), ("small", 700), ("small", 2500), ("batch", 4000),
