@@ -167,6 +167,7 @@ glu_status glu_plan_info(const glu_plan *p, int64_t info[12]);
  * perturb != 0: GESP as numeric.cu:490-506 and :139-140 — pert =
  * 3.45e-4 * max column sum of |val| (FP32, before factorization); a pivot
  * with |d| < pert becomes +pert, only in columns whose L part is non-empty.
+ * Uses scratch of the plan: one call per plan at a time, as glu_solve.
  * ---------------------------------------------------------------------- */
 glu_status glu_factor(glu_plan *p, float *d_val, int perturb, void *stream);
 /* Host buffer in/out, synchronous: the LUonDevice contract. */
